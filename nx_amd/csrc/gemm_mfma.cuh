@@ -31,42 +31,12 @@
 
 namespace hipnx {
 
-typedef float v16f __attribute__((ext_vector_type(16)));
-typedef int v16i __attribute__((ext_vector_type(16)));
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 
 constexpr int SLAB = 128;          // bytes of K per row per slab
 constexpr int CHUNKS = SLAB / 16;  // 16-byte chunks per row
-
-template <int DT> struct Mma;
-template <> struct Mma<HIPNX_BF16> {
-  typedef v16f acc_t;
-  static __device__ __forceinline__ void step(acc_t &c, const v4i &a, const v4i &b) {
-    c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8bf, a), __builtin_bit_cast(v8bf, b), c, 0, 0, 0);
-  }
-};
-template <> struct Mma<HIPNX_F16> {
-  typedef v16f acc_t;
-  static __device__ __forceinline__ void step(acc_t &c, const v4i &a, const v4i &b) {
-    c = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(v8h, a), __builtin_bit_cast(v8h, b), c, 0, 0, 0);
-  }
-};
-template <> struct Mma<HIPNX_S8> {
-  typedef v16i acc_t;
-  static __device__ __forceinline__ void step(acc_t &c, const v4i &a, const v4i &b) {
-    c = __builtin_amdgcn_mfma_i32_32x32x32_i8(a, b, c, 0, 0, 0);
-  }
-};
-template <> struct Mma<HIPNX_F32> {
-  typedef v16f acc_t;
-  static __device__ __forceinline__ void step(acc_t &c, const v4i &a, const v4i &b) {
-#pragma unroll
-    for (int s = 0; s < 4; s++)
-      c = __builtin_amdgcn_mfma_f32_32x32x2f32(__int_as_float(a[s]), __int_as_float(b[s]), c, 0, 0, 0);
-  }
-};
 
 typedef float v4f __attribute__((ext_vector_type(4)));
 
@@ -143,6 +113,11 @@ __device__ __forceinline__ void lds_dma16(const unsigned char *g, unsigned char 
 #pragma clang diagnostic pop
 }
 
+// Sixteen zero bytes in device memory: what a lane of a direct-to-LDS load is pointed at where its piece of a slab lies
+// past the end of K (a partial slab).  Both operands are zero there, so the products add nothing whatever the memory
+// behind the operands holds.
+static __device__ __attribute__((aligned(16))) const unsigned g_zero16[4] = {0, 0, 0, 0};
+
 // K-inner slab loader: ROWS x 128 B, direct to LDS.  The per-lane source pointers (row clamp,
 // row * stride, swizzled chunk) are computed once; per slab only the K offset moves.
 // Rows past `rows_valid` are clamped (loaded from the last valid row; their results are never
@@ -173,6 +148,14 @@ struct KInnerLoader {
     for (int i = 0; i < PER; i++)
       lds_dma16(src[i] + kbyte0, lds + lds_off[i]);
   }
+  // a slab of which only the first `valid` bytes of each row exist (whole 16-byte pieces)
+  __device__ __forceinline__ void issue_partial(int64_t kbyte0, int valid, unsigned char *lds, int wave, int lane) const {
+#pragma unroll
+    for (int i = 0; i < PER; i++) {
+      const int r = (wave + NWAVES * i) * 8 + (lane >> 3);
+      lds_dma16(lds_slot(r, lane & 7) * 16 < valid ? src[i] + kbyte0 : (const unsigned char *)g_zero16, lds + lds_off[i]);
+    }
+  }
   // instruction i of the slab goes out at step i * spread / PER + phase (+ skew, which may be a
   // run-time value); with t, spread and phase known after unrolling the tests fold away
   __device__ __forceinline__ void issue_at(int t, int spread, int phase, int skew, int64_t kbyte0, unsigned char *lds) const {
@@ -189,7 +172,7 @@ struct KInnerLoader {
 //   ES = 4:  4 k x  4 rows -> four 16-byte K-runs (pure register renaming)
 //   ES = 1:  4 k x 16 rows -> sixteen 4-byte K-runs (4 x 4 byte transposes with v_perm_b32)
 // `rows_valid` must be a multiple of the block's row count (the host falls back to a transpose
-// pass otherwise); k never runs past K because K*ES is a multiple of the slab.
+// pass otherwise); of a partial slab the k past the end of K are zero (fetch_partial).
 template <int ES> struct KOuterShape;
 template <> struct KOuterShape<2> { static constexpr int KB = 8, RB = 8; };
 template <> struct KOuterShape<4> { static constexpr int KB = 4, RB = 4; };
@@ -217,6 +200,24 @@ struct KOuterStage {
 #pragma unroll
       for (int j = 0; j < KB; j++)
         v[p][j] = *reinterpret_cast<const v4i *>(g + (k0 + kb * KB + j) * ld + col * ES);
+    }
+  }
+
+  // a slab of which only the first `valid` k exist
+  __device__ __forceinline__ void fetch_partial(const unsigned char *__restrict__ g, int64_t ld, int64_t row0, int64_t rows_valid,
+                                                int64_t k0, int valid, int tid) {
+#pragma unroll
+    for (int p = 0; p < PER; p++) {
+      const int blk = tid + p * NTHREADS;
+      if (blk >= BLOCKS) break;
+      const int rb = blk % (ROWS / RB), kb = blk / (ROWS / RB);
+      int64_t col = row0 + rb * RB;
+      col = col + RB <= rows_valid ? col : rows_valid - RB;
+#pragma unroll
+      for (int j = 0; j < KB; j++) {
+        const int k = kb * KB + j;
+        v[p][j] = k < valid ? *reinterpret_cast<const v4i *>(g + (k0 + k) * ld + col * ES) : v4i{0, 0, 0, 0};
+      }
     }
   }
 
@@ -335,6 +336,14 @@ struct KOuterDmaLoader {
     for (int i = 0; i < PER; i++)
       lds_dma16(src[i] + k0 * ld, lds + lds_off[i]);
   }
+  // a slab of which only the first `valid` k-rows exist
+  __device__ __forceinline__ void issue_partial(int64_t k0, int64_t ld, int valid, unsigned char *lds, int wave, int lane) const {
+#pragma unroll
+    for (int i = 0; i < PER; i++) {
+      const int k = ((wave + NWAVES * i) * 1024 + lane * 16) / RBYTES;
+      lds_dma16(k < valid ? src[i] + k0 * ld : (const unsigned char *)g_zero16, lds + lds_off[i]);
+    }
+  }
   __device__ __forceinline__ void issue_at(int t, int spread, int phase, int skew, int64_t k0, int64_t ld, unsigned char *lds) const {
 #pragma unroll
     for (int i = 0; i < PER; i++)
@@ -379,9 +388,16 @@ struct GemmArgs {
   const unsigned char *l, *r;
   void *out;
   int odt;
-  int64_t M, N, Kb;      // Kb = K in bytes (a multiple of 128 for this kernel)
+  int64_t M, N, Kb;      // Kb = K in bytes, rounded up to whole slabs of 128
   int64_t ld_l, ld_r;    // bytes between consecutive rows (K-inner) or consecutive k (K-outer)
-  int64_t bs_l, bs_r;    // bytes between batch items
+  int64_t bs_l, bs_r;    // bytes between batch items (or between the K ranges of a split)
+  int all_slabs;         // > 0: grid index y is not a batch item but a range of Kb of the all_slabs slabs of K (the last may be shorter)
+  // What exists of a partial last slab, 0 = every slab is whole: bytes of each row of a K-inner operand (a multiple of
+  // 16), k of a K-outer one.  The kernels walk the partial slab FIRST, in the prologue, where its requests are code of
+  // their own (lanes past the end read g_zero16): the loop over the whole slabs pays nothing for it.  (bf16
+  // 2000 x 3000 x 1000: 21.0 us per call.  Contracting the whole slabs in place, the rest from two zero-extended
+  // copies, and adding the two results was seven launches and 48.8 us.)
+  int tail_l, tail_r;
   int tiles_m, tiles_n;
   int group_m;  // tile rows per group of the tile order (see gemm_group_m)
   // s8 x s8 with an f32 output: out = (float)(the s32 sum) * scale -- the conversion and the
@@ -666,6 +682,18 @@ inline int gemm_group_m(int tiles_m, int tiles_n) {
   return g;
 }
 
+// The slabs of K this work-group walks: how many, and whether the partial one is among them.
+__device__ __forceinline__ int gemm_slabs(const GemmArgs &a, int y, bool &partial) {
+  int n = (int)(a.Kb / SLAB);
+  partial = a.tail_l > 0;
+  if (a.all_slabs > 0) {
+    const int left = a.all_slabs - y * n;
+    partial = partial && left <= n;
+    n = min(n, left);
+  }
+  return n;
+}
+
 // Tile order: consecutive work-group ids go to different XCDs (id % 8), so each XCD takes a run of
 // total/8 consecutive positions of the order below; the order walks groups of `group_m` tile rows
 // column by column, which makes such a run a compact rectangle of tiles whose operand panels are
@@ -748,6 +776,19 @@ gemm_pipelined_kernel(GemmArgs a) {
     else if constexpr (R_TR) rtr.issue(kbyte0 / ES, a.ld_r, sB);
     else rregs.fetch(rb, a.ld_r, n0, a.N, kbyte0 / ES, tid);
   };
+  bool partial;
+  const int nslab = gemm_slabs(a, blockIdx.y, partial);
+  const int64_t k_first = partial ? (int64_t)(nslab - 1) * SLAB : 0;  // the walk's slab 0, then the others in order
+  const int64_t k_shift = partial ? -SLAB : 0;
+  auto issue_partial = [&]() {
+    unsigned char *sA = smem, *sB = sA + BM * SLAB;
+    if constexpr (L_KIN) lload.issue_partial(k_first, a.tail_l, sA, wave, lane);
+    else if constexpr (L_TR) ltr.issue_partial(k_first / ES, a.ld_l, a.tail_l, sA, wave, lane);
+    else lregs.fetch_partial(lb, a.ld_l, m0, a.M, k_first / ES, a.tail_l, tid);
+    if constexpr (R_KIN) rload.issue_partial(k_first, a.tail_r, sB, wave, lane);
+    else if constexpr (R_TR) rtr.issue_partial(k_first / ES, a.ld_r, a.tail_r, sB, wave, lane);
+    else rregs.fetch_partial(rb, a.ld_r, n0, a.N, k_first / ES, a.tail_r, tid);
+  };
   auto commit = [&](int stage) {  // register-staged K-outer operands: transposed LDS writes
     unsigned char *sA = smem + stage * STAGE, *sB = sA + BM * SLAB;
     if constexpr (!L_KIN && !L_TR) lregs.store(sA, tid);
@@ -819,10 +860,11 @@ gemm_pipelined_kernel(GemmArgs a) {
                       (R_KIN ? KInnerLoader<BN, NW>::PER : R_TR ? KOuterDmaLoader<TR_ES, R_TR ? BN : 256 * NW, NW>::PER : 0);
   constexpr int INFLIGHT = OPS * (NSTAGE - 2);  // requests of younger slabs that may stay outstanding
   static_assert(INFLIGHT < 64, "vmcnt is a 6-bit counter");
-  const int nslab = (int)(a.Kb / SLAB);
+  if (partial) issue_partial();
+  else issue(0, 0);
 #pragma unroll
-  for (int p = 0; p < NSTAGE - 1; p++)
-    if (p < nslab) issue(p, (int64_t)p * SLAB);
+  for (int p = 1; p < NSTAGE - 1; p++)
+    if (p < nslab) issue(p, (int64_t)p * SLAB + k_shift);
   commit(0);
   if (nslab >= NSTAGE - 1) wait_vmcnt<INFLIGHT>();
   else wait_vmcnt<0>();
@@ -830,7 +872,7 @@ gemm_pipelined_kernel(GemmArgs a) {
   if constexpr (EARLY) {  // the first requests of slab 1 (what the steps behind a barrier would have issued)
     if (1 < nslab) {
 #pragma unroll
-      for (int u = 0; u < POST; u++) issue_early(u, 1, SLAB);
+      for (int u = 0; u < POST; u++) issue_early(u, 1, SLAB + k_shift);
     }
   }
   v4i fa[2][TM16], fb[RING];
@@ -844,7 +886,7 @@ gemm_pipelined_kernel(GemmArgs a) {
     const bool more = s + 1 < nslab;                  // another slab to compute after this one
     const bool request = s + NSTAGE - 1 < nslab;      // another slab to request during this one
     const int req_stage = (s + NSTAGE - 1) % NSTAGE;
-    const int64_t req_kbyte = (int64_t)(s + NSTAGE - 1) * SLAB;
+    const int64_t req_kbyte = (int64_t)(s + NSTAGE - 1) * SLAB + k_shift;
 #pragma unroll
     for (int t = 0; t < STEPS; t++) {
       const int ks = t / TN16, j = t % TN16;
@@ -869,7 +911,7 @@ gemm_pipelined_kernel(GemmArgs a) {
       }
       if constexpr (EARLY) {
         if (t > BAR) {
-          if (s + 2 < nslab) issue_early(t - BAR - 1, s % NSTAGE, (int64_t)(s + 2) * SLAB);
+          if (s + 2 < nslab) issue_early(t - BAR - 1, s % NSTAGE, (int64_t)(s + 2) * SLAB + k_shift);
         } else if (request) issue_early(t + POST, req_stage, req_kbyte);
       } else if (request && t <= BAR) issue_step(t, req_stage, req_kbyte);
 #pragma unroll

@@ -93,6 +93,15 @@ struct PPKInnerLoader {
 #pragma unroll
     for (int i = 0; i < PER; i++) lds_dma16_at(b, off[i], lds + (wave + NWAVES * i) * 1024);
   }
+  // a slab of which only the first `valid` bytes of each row exist (whole 16-byte pieces)
+  __device__ __forceinline__ void issue_partial(int64_t kbyte0, int valid, unsigned char *lds, int wave, int lane) const {
+    const unsigned char *b = base + kbyte0;
+#pragma unroll
+    for (int i = 0; i < PER; i++) {
+      const int r = (wave + NWAVES * i) * 8 + (lane >> 3);
+      lds_dma16(lds_slot16(r, lane & 7) * 16 < valid ? b + off[i] : (const unsigned char *)g_zero16, lds + (wave + NWAVES * i) * 1024);
+    }
+  }
 };
 
 // K-outer columns [col0, col0 + ROWS) of an operand copied k-major ([k][ROWS * ES bytes]) for the
@@ -122,6 +131,15 @@ struct PPKOuterLoader {
     const unsigned char *b = base + k0 * ld;
 #pragma unroll
     for (int i = 0; i < PER; i++) lds_dma16_at(b, off[i], lds + (wave + NWAVES * i) * 1024);
+  }
+  // a slab of which only the first `valid` k-rows exist
+  __device__ __forceinline__ void issue_partial(int64_t k0, int64_t ld, int valid, unsigned char *lds, int wave, int lane) const {
+    const unsigned char *b = base + k0 * ld;
+#pragma unroll
+    for (int i = 0; i < PER; i++) {
+      const int k = ((wave + NWAVES * i) * 1024 + lane * 16) / RBYTES;
+      lds_dma16(k < valid ? b + off[i] : (const unsigned char *)g_zero16, lds + (wave + NWAVES * i) * 1024);
+    }
   }
 };
 
@@ -212,13 +230,24 @@ gemm_pingpong_kernel(GemmArgs a) {
     else return read_fragment_tr<ES, BN>(st + BM * SLAB, wn + 16 * j, ks, lane);
   };
 
-  const int nslab = (int)(a.Kb / SLAB);
+  bool partial;
+  const int nslab = gemm_slabs(a, blockIdx.y, partial);
+  const int64_t k_shift = partial ? -SLAB : 0;  // a partial slab is walked first, the whole ones behind it
   // prologue: slabs 0 and 1 into the two stages; slab 0 must have landed before the first phase
-  issue_r(0, 0);
-  issue_l(0, 0);
+  if (partial) {
+    const int64_t k0 = (int64_t)(nslab - 1) * SLAB;
+    unsigned char *sA = smem + lhalf * (HALF * SLAB), *sB = smem + BM * SLAB;
+    if constexpr (R_KIN) rload.issue_partial(k0, a.tail_r, sB, wave, lane);
+    else rtr.issue_partial(k0 / ES, a.ld_r, a.tail_r, sB, wave, lane);
+    if constexpr (L_KIN) lload.issue_partial(k0, a.tail_l, sA, wave & 3, lane);
+    else ltr.issue_partial(k0 / ES, a.ld_l, a.tail_l, sA, wave & 3, lane);
+  } else {
+    issue_r(0, 0);
+    issue_l(0, 0);
+  }
   if (nslab > 1) {
-    issue_r(1, SLAB);
-    issue_l(1, SLAB);
+    issue_r(1, SLAB + k_shift);
+    issue_l(1, SLAB + k_shift);
     wait_vmcnt<RPER + 4>();
   } else {
     wait_vmcnt<0>();
@@ -248,16 +277,16 @@ gemm_pingpong_kernel(GemmArgs a) {
 #if !(HIPNX_PP_EXP & 1)
       if (ks == 0) {
         if (s >= 1 && s + 1 < nslab) {
-          issue_r((s + 1) & 1, (int64_t)(s + 1) * SLAB);
+          issue_r((s + 1) & 1, (int64_t)(s + 1) * SLAB + k_shift);
           issued_r = true;
         }
       } else if (grp == 0) {
         if (s >= 1 && s + 1 < nslab) {
-          issue_l((s + 1) & 1, (int64_t)(s + 1) * SLAB);
+          issue_l((s + 1) & 1, (int64_t)(s + 1) * SLAB + k_shift);
           issued = true;
         }
       } else if (s + 2 < nslab) {
-        issue_l(s & 1, (int64_t)(s + 2) * SLAB);
+        issue_l(s & 1, (int64_t)(s + 2) * SLAB + k_shift);
         issued = true;
       }
 #endif
@@ -376,12 +405,23 @@ gemm_pingpong128_kernel(GemmArgs a) {
   else lkout.init(lb, a.ld_l, m0, a.M, w4, lane);
   if constexpr (R_KIN) rkin.init(rb, a.ld_r, n0, a.N, w4, lane);
   else rkout.init(rb, a.ld_r, n0, a.N, w4, lane);
+  bool partial;
+  const int nslab1 = gemm_slabs(a, blockIdx.y, partial);
+  const int64_t k_shift = partial ? -SLAB : 0;  // a partial slab is walked first, the whole ones behind it
   // (below, "slab" stands for the SPP slabs of one phase)
-  auto issue = [&](int slab) __attribute__((always_inline)) {
+  auto issue = [&](int slab, bool with_partial = false) __attribute__((always_inline)) {
 #pragma unroll
     for (int u = 0; u < SPP; u++) {
       unsigned char *dst = smem + (slab % NSTAGE) * STAGE + u * SLAB1;
-      const int64_t kbyte0 = ((int64_t)slab * SPP + u) * SLAB;
+      if (with_partial && u == 0) {
+        const int64_t k0 = (int64_t)(nslab1 - 1) * SLAB;
+        if constexpr (L_KIN) lkin.issue_partial(k0, a.tail_l, dst, w4, lane);
+        else lkout.issue_partial(k0 / ES, a.ld_l, a.tail_l, dst, w4, lane);
+        if constexpr (R_KIN) rkin.issue_partial(k0, a.tail_r, dst + BM * SLAB, w4, lane);
+        else rkout.issue_partial(k0 / ES, a.ld_r, a.tail_r, dst + BM * SLAB, w4, lane);
+        continue;
+      }
+      const int64_t kbyte0 = ((int64_t)slab * SPP + u) * SLAB + k_shift;
       if constexpr (L_KIN) lkin.issue(kbyte0, dst, w4);
       else lkout.issue(kbyte0 / ES, a.ld_l, dst, w4);
       if constexpr (R_KIN) rkin.issue(kbyte0, dst + BM * SLAB, w4);
@@ -401,7 +441,7 @@ gemm_pingpong128_kernel(GemmArgs a) {
     for (int ks = 0; ks < 2; ks++) b_rd[ks] = BM * SLAB + row * SLAB + lds_slot16(row, 4 * ks + (lane >> 4)) * 16;
   }
 
-  const int nslab = (int)(a.Kb / (SPP * SLAB));  // the host sends whole phases only
+  const int nslab = nslab1 / SPP;  // the host sends whole phases only
   v4i fa[KS][TM16], fb[KS][TN16];
   auto mem_phase = [&](int p) __attribute__((always_inline)) {
     const unsigned char *cur = smem + (p % NSTAGE) * STAGE;
@@ -448,7 +488,10 @@ gemm_pingpong128_kernel(GemmArgs a) {
   // other one reads); group 1 holds slab 0 and waits for it here, slab 1 is awaited by group 0 in phase 0
 #pragma unroll
   for (int q = 0; q < AHEAD; q++)
-    if (q < nslab && ((q + 1) & 1) == grp) issue(q);
+    if (q < nslab && ((q + 1) & 1) == grp) {
+      if (q == 0 && partial) issue(0, true);
+      else issue(q);
+    }
   if (grp == 1) {
     if (nslab >= AHEAD) wait_vmcnt<(AHEAD - 1) / 2 * REQ>();
     else wait_vmcnt<0>();

@@ -312,6 +312,29 @@ def test_contraction_lengths_off_the_slab_grid_are_padded(ty, M, N, K, layout, h
         check_float_dot(got_rows, want, values(oa), values(ob), "mk,kn->mn", K, f"padded K {ty} {layout}")
 
 
+# The partial slab of K in every kernel that walks slabs: one piece or one k of it, all but one, nothing but a partial
+# slab, an odd number of slabs, K split over work-groups so that the last range is shorter and holds it.
+@pytest.mark.parametrize("ty,M,N,K", [("bf16", 2064, 6160, 72), ("f16", 1000, 6200, 1), ("bf16", 2048, 3080, 191), ("bf16", 520, 392, 1032),
+                                      ("f16", 40, 1024, 1160), ("bf16", 24, 2048, 648), ("bf16", 128, 1024, 4104), ("bf16", 96, 392, 63),
+                                      ("f32", 300, 264, 36), ("f32", 1024, 512, 785), ("f32", 512, 10, 4092), ("f32", 40, 384, 1001),
+                                      ("s8", 2064, 6160, 144), ("s8", 64, 12304, 1168), ("s8", 48, 272, 1297), ("s8", 130, 528, 4112), ("s8", 256, 256, 5)])
+@pytest.mark.parametrize("layout", ["nn", "nt", "tn", "tt"])
+def test_partial_slabs_of_k(ty, M, N, K, layout, hip):
+    """Integer-valued operands: every partial sum is a whole number below 2^24 (4 * 4 * 5000), so each order of
+    additions gives the exact product in f32 and s32 alike."""
+    rng = np.random.default_rng(seed_of(ty, M, N, K, layout, "partial slab"))
+    a, b = rng.integers(-4, 5, size=(M, K)), rng.integers(-4, 5, size=(K, N))
+    la = a if layout[0] == "n" else np.ascontiguousarray(a.T)
+    lb = b if layout[1] == "n" else np.ascontiguousarray(b.T)
+    held = {"s8": lambda x: x.astype(np.int8), "f32": lambda x: x.astype(np.float32), "f16": lambda x: x.astype(np.float16),
+            "bf16": lambda x: (x.astype(np.float32).view(np.uint32) >> 16).astype(np.uint16)}[ty]
+    out = "s32" if ty == "s8" else "f32"
+    got = Nx.dot(from_numpy(held(la), ty, hip), [1 if layout[0] == "n" else 0], from_numpy(held(lb), ty, hip),
+                 [0 if layout[1] == "n" else 1], out_type=out)
+    want = (a.astype(np.float64) @ b.astype(np.float64)).astype(np.int32 if ty == "s8" else np.float32)
+    assert np.array_equal(hip.to_numpy(got), want)
+
+
 @pytest.mark.parametrize("ty,M,N,K", [("bf16", 128, 1024, 4096), ("s8", 128, 1024, 4096), ("f16", 200, 520, 2048), ("f32", 132, 384, 2048),
                                       ("bf16", 768, 4096, 4096), ("f16", 1000, 4100, 4096),
                                       ("s8", 384, 512, 8192), ("bf16", 512, 1024, 2048),
