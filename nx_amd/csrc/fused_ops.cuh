@@ -213,10 +213,11 @@ __device__ __forceinline__ float int_unary(float x) {
 
 // A program that relabels bits or computes on integers can look at the bits of a float it made.  The separate kernels
 // store every NaN they compute as the one quiet NaN (0x7FC00000), so such a program does the same after each float
-// instruction; bits that only pass through (an input, a BITCAST) stay as they are, there as here.
+// instruction that one of those follows (the last store writes the one quiet NaN itself); bits that only pass through (an
+// input, a BITCAST) stay as they are, there as here.
 template <typename P>
-constexpr bool bits_are_observed() {
-  for (int i = 0; i < P::n_instr; i++)
+constexpr bool bits_are_observed_after(int pc) {
+  for (int i = pc + 1; i < P::n_instr; i++)
     if (P::kind[i] == HIPNX_FUSED_BITCAST || (P::flags[i] & HIPNX_FUSED_FLAG_INT) != 0) return true;
   return false;
 }
@@ -288,7 +289,7 @@ __device__ __forceinline__ void static_steps(KernArgs a, const int64_t (&row)[FV
     }  // a float AS_TYPE is the rounding below
     constexpr bool computed = kind == HIPNX_FUSED_UNARY || kind == HIPNX_FUSED_BINARY || kind == HIPNX_FUSED_SELECT || kind == HIPNX_FUSED_AS_TYPE ||
                               (kind == HIPNX_FUSED_SET && (src == HIPNX_FUSED_SRC_ROWSTAT || src == HIPNX_FUSED_SRC_CARRY));
-    if constexpr (dt == HIPNX_F32 && computed && bits_are_observed<P>()) {
+    if constexpr (dt == HIPNX_F32 && computed && bits_are_observed_after<P>(PC)) {
 #pragma unroll
       for (int u = 0; u < FV; u++)
 #pragma unroll

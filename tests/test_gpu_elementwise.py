@@ -172,6 +172,21 @@ def test_unary_math(op, ty, hip, oracle):
     assert_all_close(got, want, rtol, 1e-37 if bits == 32 else 1e-7 if bits == 16 else 1e-300, f"{op} {ty}")
 
 
+@pytest.mark.parametrize("where", ["everywhere", "around the switch of polynomials", "next to one", "tiny", "powers of two from one"])
+def test_f32_erf_inv_follows_the_reference_bit_for_bit(where, hip, oracle):
+    """The f32 kernel has its own logarithm and fuses the polynomials' steps: a few 1e-16 away from the reference's f64
+    value, so a result can differ (by its last bit) only where that value is within 1e-15 of halfway between two floats,
+    about one result in 2^25."""
+    rng = np.random.default_rng(seed_of("erf_inv", where))
+    x = {"everywhere": rng.uniform(-1, 1, 200_000), "around the switch of polynomials": rng.uniform(0.9965, 0.9968, 50_000),
+         "next to one": 1 - np.arange(1, 5000) * 2.0 ** -24, "tiny": rng.uniform(-1, 1, 5000) * 10.0 ** rng.integers(-44, -3, 5000),
+         "powers of two from one": 1 - 2.0 ** -np.arange(1, 25)}[where].astype(np.float32)
+    got = values(Nx.erf_inv(from_numpy(x, "f32", hip))).astype(np.float32)
+    want = values(Nx.erf_inv(from_numpy(x, "f32", oracle))).astype(np.float32)
+    apart = np.abs(got.view(np.int32).astype(np.int64) - want.view(np.int32))
+    assert apart.max() <= 1 and (apart != 0).sum() <= 2
+
+
 @pytest.mark.parametrize("op", ["abs", "negate", "sign", "ceil", "floor", "round", "is_nan", "is_infinity"])
 @pytest.mark.parametrize("ty", FLOAT_TYPES + ["s8", "s32", "s64", "u8", "u32"])
 def test_unary_exact(op, ty, hip, oracle):
