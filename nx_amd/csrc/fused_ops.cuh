@@ -171,12 +171,21 @@ struct Saved {
 // compiler here.
 typedef float RowStats[HIPNX_FUSED_STATS];  // results of the row reductions of earlier stages (fused_row_stages_body)
 
+// what a lane keeps of one vector of its row between stages (fused_row_stages_body)
+struct RowVector {
+  float carry[FE];  // the value the previous stage reduced
+  float held[FE];   // input P::held
+};
+
 template <typename P, int SRC, int ARG, unsigned IMM, bool RAW>
 __device__ __forceinline__ void fetch_static(KernArgs a, const Saved &S, const RowStats &stats, const int64_t (&row)[FV],
-                                             const int64_t (&col)[FV], int valid, const float (*carry)[FE], Vecs &dst) {
-  if constexpr (SRC == HIPNX_FUSED_SRC_CARRY) {  // what the previous stage reduced, at this vector
+                                             const int64_t (&col)[FV], int valid, const RowVector *kept, Vecs &dst) {
+  if constexpr (SRC == HIPNX_FUSED_SRC_CARRY) {
 #pragma unroll
-    for (int e = 0; e < FE; e++) dst[0][e] = (*carry)[e];
+    for (int e = 0; e < FE; e++) dst[0][e] = kept->carry[e];
+  } else if constexpr (SRC == HIPNX_FUSED_SRC_INPUT && ARG == P::held && !RAW) {
+#pragma unroll
+    for (int e = 0; e < FE; e++) dst[0][e] = kept->held[e];
   } else if constexpr (SRC == HIPNX_FUSED_SRC_ROWSTAT) {
 #pragma unroll
     for (int u = 0; u < FV; u++)
@@ -237,14 +246,14 @@ __device__ __forceinline__ void forget_provenance(float &x) { asm volatile("" : 
 // instructions PC .. END-1
 template <typename P, int PC, int END>
 __device__ __forceinline__ void static_steps(KernArgs a, const int64_t (&row)[FV], const int64_t (&col)[FV], Vecs &acc, Saved &S,
-                                             const RowStats &stats, int valid = FE, const float (*carry)[FE] = nullptr) {
+                                             const RowStats &stats, int valid = FE, const RowVector *kept = nullptr) {
   if constexpr (PC < END) {
     constexpr int kind = P::kind[PC], op = P::op[PC], src = P::src[PC], arg = P::arg[PC];
     constexpr int src2 = P::src2[PC], arg2 = P::arg2[PC], flags = P::flags[PC], dt = P::dt[PC];
     constexpr unsigned imm = P::imm[PC], imm2 = P::imm2[PC];
     constexpr bool ints = (flags & HIPNX_FUSED_FLAG_INT) != 0, uns = dt == HIPNX_U32;
     if constexpr (kind == HIPNX_FUSED_SET) {
-      fetch_static<P, src, arg, imm, ints>(a, S, stats, row, col, valid, carry, acc);
+      fetch_static<P, src, arg, imm, ints>(a, S, stats, row, col, valid, kept, acc);
     } else if constexpr (kind == HIPNX_FUSED_UNARY) {
       if constexpr (ints) {
 #pragma unroll
@@ -256,7 +265,7 @@ __device__ __forceinline__ void static_steps(KernArgs a, const int64_t (&row)[FV
       }
     } else if constexpr (kind == HIPNX_FUSED_BINARY) {
       Vecs y;
-      fetch_static<P, src, arg, imm, ints>(a, S, stats, row, col, valid, carry, y);
+      fetch_static<P, src, arg, imm, ints>(a, S, stats, row, col, valid, kept, y);
       if constexpr (ints) {
 #pragma unroll
         for (int u = 0; u < FV; u++)
@@ -267,8 +276,8 @@ __device__ __forceinline__ void static_steps(KernArgs a, const int64_t (&row)[FV
       }
     } else if constexpr (kind == HIPNX_FUSED_SELECT) {
       Vecs y, z;
-      fetch_static<P, src, arg, imm, false>(a, S, stats, row, col, valid, carry, y);
-      fetch_static<P, src2, arg2, imm2, false>(a, S, stats, row, col, valid, carry, z);
+      fetch_static<P, src, arg, imm, false>(a, S, stats, row, col, valid, kept, y);
+      fetch_static<P, src2, arg2, imm2, false>(a, S, stats, row, col, valid, kept, z);
 #pragma unroll
       for (int u = 0; u < FV; u++)
 #pragma unroll
@@ -305,7 +314,7 @@ __device__ __forceinline__ void static_steps(KernArgs a, const int64_t (&row)[FV
         for (int e = 0; e < FE; e++) acc[u][e] = round_to(acc[u][e], dt);
     }
     if constexpr ((flags >> 4) != 0) copy_vecs(S.s[(flags >> 4) - 1], acc);
-    static_steps<P, PC + 1, END>(a, row, col, acc, S, stats, valid, carry);
+    static_steps<P, PC + 1, END>(a, row, col, acc, S, stats, valid, kept);
   }
 }
 
@@ -424,7 +433,8 @@ __device__ __forceinline__ void fused_reduce_rows_body() {
 // takes a row through all stages; a stage walks the row exactly as fused_reduce_rows_body does with
 // TPR = WAVE (same lanes, same order, same reducer), and a statistic is carried on as the value a
 // store to its type and a load would give -- so the result equals the separate kernels', bit for bit.
-// The row is read again by every stage, from the caches: one wave has just read it.
+// A row that a lane's registers hold (P::held: an input that more than one stage reads, at most 16 vectors a lane) is read
+// from memory once; a longer one is read again by every stage.  Bound by memory: HELDNOTE
 template <typename CT>
 __device__ __forceinline__ float as_stored(CT v, int dt) {
   switch (dt) {
@@ -434,20 +444,24 @@ __device__ __forceinline__ float as_stored(CT v, int dt) {
   }
 }
 
-// The walk of a row: lane l takes the vectors l, l + WAVE, ... -- at most P::nv of them when the program
-// carries element values from one stage to the next (their registers are indexed by the trip), any
-// number otherwise.
+// The walk of a row: lane l takes the vectors l, l + P::tpr, ... -- P::nv of them, the last one if it lies in the row,
+// when the program keeps vectors from one stage to the next (P::nv > 0), any number otherwise.  The trips are written out
+// by recursion: what is kept is indexed by the trip and has to stay in registers.  (As a loop with an unroll pragma the
+// compiler left it rolled for 16 trips and turned the index into chains of selects, 16 of them per element.)
+template <typename P, int IT, typename F>
+__device__ __forceinline__ void trips_from(int lane, int64_t cols, F &&body) {
+  if constexpr (IT < P::nv) {
+    const int64_t k = ((int64_t)lane + (int64_t)IT * P::tpr) * FE;
+    if constexpr (IT + 1 < P::nv) body(k, IT);
+    else if (k < cols) body(k, IT);
+    trips_from<P, IT + 1>(lane, cols, body);
+  }
+}
 template <typename P, typename F>
 __device__ __forceinline__ void for_each_vector(int lane, int64_t cols, F &&body) {
-  if constexpr (P::nv > 0) {
-#pragma unroll
-    for (int it = 0; it < P::nv; it++) {
-      const int64_t k = ((int64_t)lane + (int64_t)it * P::tpr) * FE;
-      if (k < cols) body(k, it);
-    }
-  } else {
+  if constexpr (P::nv > 0) trips_from<P, 0>(lane, cols, body);
+  else
     for (int64_t k = (int64_t)lane * FE; k < cols; k += (int64_t)P::tpr * FE) body(k, 0);
-  }
 }
 
 // the reduction of a stage over the P::tpr lanes of a row, left in every lane: within a wave by the
@@ -467,20 +481,29 @@ __device__ __forceinline__ typename R::acc_t row_reduce(typename R::acc_t acc) {
   return acc;
 }
 
-template <typename P, int SEG, typename CARRY>
-__device__ __forceinline__ void row_stage(KernArgs a, int64_t r, int lane, RowStats &stats, CARRY &carry) {
+template <typename P, int SEG, typename KEPT>
+__device__ __forceinline__ void row_stage(KernArgs a, int64_t r, int lane, RowStats &stats, KEPT &kept) {
   // stage SEG: instructions [begin, red) on the row's elements, the reduction at `red`, instructions
   // (red, save) on the statistic, which is kept at `save`; the last stage is [begin, n_instr)
   constexpr int begin = SEG == 0 ? 0 : P::seg_save[SEG - 1] + 1;
   constexpr int red = P::seg_red[SEG], save = P::seg_save[SEG];
   const int64_t cols = a->cols;
+  if constexpr (SEG == P::held_stage) {  // the first stage that reads the held input: all of the lane's part is requested at once
+    for_each_vector<P>(lane, cols, [&](int64_t k, int it) __attribute__((always_inline)) {
+      const int64_t row[FV] = {r}, col[FV] = {k};
+      Vecs x;
+      load_input_as(a, P::held, P::in_dt[P::held], 1, row, col, x);
+#pragma unroll
+      for (int e = 0; e < FE; e++) kept[it].held[e] = x[0][e];
+    });
+  }
   if constexpr (red < 0) {  // the last stage: its value is the result
     void *out = (void *)a->out;
-    for_each_vector<P>(lane, cols, [&](int64_t k, int it) {
+    for_each_vector<P>(lane, cols, [&](int64_t k, int it) __attribute__((always_inline)) {
       const int64_t row[FV] = {r}, col[FV] = {k};
       Vecs x;
       Saved S;
-      static_steps<P, begin, P::n_instr>(a, row, col, x, S, stats, FE, &carry[it]);
+      static_steps<P, begin, P::n_instr>(a, row, col, x, S, stats, FE, &kept[it]);
       if constexpr (result_is_relabelled_bits<P>()) {
         uint4 *p = reinterpret_cast<uint4 *>((uint32_t *)out + r * cols + k);
         p[0] = make_uint4(__float_as_uint(x[0][0]), __float_as_uint(x[0][1]), __float_as_uint(x[0][2]), __float_as_uint(x[0][3]));
@@ -494,16 +517,16 @@ __device__ __forceinline__ void row_stage(KernArgs a, int64_t r, int lane, RowSt
     typedef typename std::conditional<op == HIPNX_RED_SUM, double, float>::type CT;
     typedef PlainReducer<CT, op, false> R;
     typename R::acc_t acc = R::init();
-    for_each_vector<P>(lane, cols, [&](int64_t k, int it) {
+    for_each_vector<P>(lane, cols, [&](int64_t k, int it) __attribute__((always_inline)) {
       const int64_t row[FV] = {r}, col[FV] = {k};
       Vecs x;
       Saved S;
-      static_steps<P, begin, red>(a, row, col, x, S, stats, FE, &carry[it]);
+      static_steps<P, begin, red>(a, row, col, x, S, stats, FE, &kept[it]);
 #pragma unroll
       for (int e = 0; e < FE; e++) acc = R::accumulate(acc, (CT)x[0][e], k + e);
       if constexpr (P::nv > 0) {  // kept for the next stage (after this stage's own reads of the previous one's)
 #pragma unroll
-        for (int e = 0; e < FE; e++) carry[it][e] = x[0][e];
+        for (int e = 0; e < FE; e++) kept[it].carry[e] = x[0][e];
       }
     });
     acc = row_reduce<P, R>(acc);  // the same value in every lane of the row
@@ -518,7 +541,7 @@ __device__ __forceinline__ void row_stage(KernArgs a, int64_t r, int lane, RowSt
       if (lane == 0) store_one<float>((void *)a->out, P::out_dt, r, x[0][0]);  // lane 0 of the row
     } else {
       stats[P::arg[save]] = x[0][0];
-      row_stage<P, SEG + 1>(a, r, lane, stats, carry);
+      row_stage<P, SEG + 1>(a, r, lane, stats, kept);
     }
   }
 }
@@ -531,8 +554,8 @@ __device__ __forceinline__ void fused_row_stages_body() {
   const int64_t r = (int64_t)blockIdx.x * (FBLOCK / P::tpr) + threadIdx.x / P::tpr;
   if (r >= a->rows) return;  // (a whole wave, or with a block per row nobody: no barrier is left waiting)
   RowStats stats = {};
-  float carry[P::nv > 0 ? P::nv : 1][FE];  // (indexed by compile-time trip numbers only: registers)
-  row_stage<P, 0>(a, r, threadIdx.x % P::tpr, stats, carry);
+  RowVector kept[P::nv > 0 ? P::nv : 1];  // (indexed by compile-time trip numbers only: registers)
+  row_stage<P, 0>(a, r, threadIdx.x % P::tpr, stats, kept);
 }
 
 }  // namespace hipnx

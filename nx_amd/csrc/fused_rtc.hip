@@ -47,27 +47,52 @@ static void list_of(std::string &s, const char *name, const char *type, int n, c
   s += "};\n";
 }
 
-// Trips of a lane along a row (of at most 4096 elements), when the program carries element values from
-// stage to stage and so indexes their registers by the trip; 0 when it does not.
-static int carry_trips(const FusedArgs &a) {
+// What the lanes of a stage program keep in registers between stages: element values carried from one stage to the next,
+// and an input that several stages read.
+struct Keeps {
+  int trips = 0;        // vectors of a lane along a row, 0 when nothing is kept
+  int held = -1;        // the input, and the first stage that reads it
+  int held_stage = -1;
+};
+static Keeps what_is_kept(const FusedArgs &a) {
+  Keeps k;
+  const int tpr = a.cols > 4096 ? FBLOCK : WAVE;
+  const int64_t trips = (a.cols + tpr * FE - 1) / (tpr * FE);
+  // which stages read an input along the row, and up to which stage a carried value is waiting to be read
+  unsigned reads[HIPNX_FUSED_MAX_INPUTS] = {};
+  int stage = 0, carried_from = -1;
+  bool stages = false;
   for (int i = 0; i < a.n_instr; i++) {
     const hipnx_fused_instr &q = a.ins[i];
-    const bool reads = q.kind == HIPNX_FUSED_SET || q.kind == HIPNX_FUSED_BINARY || q.kind == HIPNX_FUSED_SELECT;
-    if (reads && (q.src == HIPNX_FUSED_SRC_CARRY || (q.kind == HIPNX_FUSED_SELECT && q.src2 == HIPNX_FUSED_SRC_CARRY)))
-      {
-        const int tpr = a.cols > 4096 ? FBLOCK : WAVE;
-        const int64_t trips = (a.cols + tpr * FE - 1) / (tpr * FE);
-        return trips <= 16 ? (int)trips : 0;  // (the host refuses longer rows for such programs)
-      }
+    auto source = [&](int src, int arg) {
+      if (src == HIPNX_FUSED_SRC_CARRY) carried_from = stage - 1;  // (the last stage that leaves a value somebody reads)
+      if (src == HIPNX_FUSED_SRC_INPUT && a.in_cs[arg] == 1 && !(q.flags & HIPNX_FUSED_FLAG_INT)) reads[arg] |= 1u << stage;
+    };
+    if (q.kind == HIPNX_FUSED_SET || q.kind == HIPNX_FUSED_BINARY || q.kind == HIPNX_FUSED_SELECT) source(q.src, q.arg);
+    if (q.kind == HIPNX_FUSED_SELECT) source(q.src2, q.arg2);
+    if (q.kind == HIPNX_FUSED_ROW_REDUCE) stages = true;
+    if (q.kind == HIPNX_FUSED_ROW_STAT) stage++;
   }
-  return 0;
+  if (!stages || trips > 16) return k;  // (the host refuses longer rows for programs that carry values)
+  if (carried_from >= 0) k.trips = (int)trips;
+  for (int in = 0; in < a.n_inputs; in++) {
+    if (!(reads[in] & (reads[in] - 1)) || k.held >= 0) continue;  // one stage reads it: nothing to gain
+    // a lane has room for 16 vectors (128 of its registers): an input that is still read once a carried value is there
+    // shares them
+    const int last = 31 - __builtin_clz(reads[in]);
+    if (carried_from >= 0 && last > carried_from && trips > 8) continue;
+    k.trips = (int)trips;
+    k.held = in;
+    k.held_stage = __builtin_ctz(reads[in]);
+  }
+  return k;
 }
 
 // everything a compiled kernel is specialised on, as bytes: the cache key
 static std::string make_key(const FusedArgs &a, int reduce_op, bool block_per_row) {
   std::string k;
   k.reserve(16 + 16 * a.n_instr + 8 * a.n_inputs);
-  const int head[5] = {a.n_instr, a.n_inputs, a.out_dt, reduce_op * 2 + (block_per_row ? 1 : 0), carry_trips(a)};
+  const int head[5] = {a.n_instr, a.n_inputs, a.out_dt, reduce_op * 2 + (block_per_row ? 1 : 0), what_is_kept(a).trips};
   k.append((const char *)head, sizeof(head));
   k.append((const char *)a.ins, sizeof(hipnx_fused_instr) * a.n_instr);
   k.append((const char *)a.in_dt, sizeof(int) * a.n_inputs);
@@ -78,8 +103,10 @@ static std::string make_key(const FusedArgs &a, int reduce_op, bool block_per_ro
 // the whole translation unit for one program
 static std::string make_source(const FusedArgs &a, int reduce_op, bool block_per_row, const std::string &name) {
   std::string s = RTC_PREAMBLE;
+  const Keeps keeps = what_is_kept(a);
   s += "namespace hipnx {\nstruct P {\n  static constexpr int n_instr = " + std::to_string(a.n_instr) + ", out_dt = " + std::to_string(a.out_dt) +
-       ", nv = " + std::to_string(carry_trips(a)) + ", tpr = " + (block_per_row ? "FBLOCK" : "WAVE") + ";\n";
+       ", nv = " + std::to_string(keeps.trips) + ", tpr = " + (block_per_row ? "FBLOCK" : "WAVE") + ", held = " + std::to_string(keeps.held) +
+       ", held_stage = " + std::to_string(keeps.held_stage) + ";\n";
   const hipnx_fused_instr *q = a.ins;
   list_of(s, "kind", "int", a.n_instr, [&](int i) { return std::to_string((int)q[i].kind); });
   list_of(s, "op", "int", a.n_instr, [&](int i) { return std::to_string((int)q[i].op); });
