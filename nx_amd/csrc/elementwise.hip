@@ -9,47 +9,17 @@
 #include <type_traits>
 
 #include "elementwise_ops.cuh"
+#include "elementwise_vec.cuh"
 #include "internal.h"
 
 namespace hipnx {
 
-constexpr int E = 8;
-// A lane's vector when the element types are known at compile time: 16 bytes of the WIDEST type involved -- 8 elements of
-// 1 or 2 bytes, 4 of 4 bytes, 2 of 8 bytes.  One 16-byte access per lane with the lanes side by side is what streams
-// fastest here: a wave instruction then covers whole cache lines, where two adjacent 16-byte accesses per lane (eight
-// f32) make every instruction touch twice the lines it fills (f32 multiply: 8.4 M elements 11.3 -> 9.4 us, 268 M
-// elements 5.8 -> 6.2 TB/s; bf16 -> f32 conversion of 8.4 M elements 9.6 -> 7.6 us).  The narrower side of a
-// conversion or comparison moves 8, 4 or 2 bytes per lane, still lanes side by side.
-constexpr int fixed_type_bytes(int dt) {
-  return dt < 0 ? 0
-         : (dt == HIPNX_U8 || dt == HIPNX_S8) ? 1
-         : (dt == HIPNX_U16 || dt == HIPNX_S16 || dt == HIPNX_F16 || dt == HIPNX_BF16 || dt == HIPNX_BF16_RNE) ? 2
-         : (dt == HIPNX_U32 || dt == HIPNX_S32 || dt == HIPNX_F32) ? 4 : 8;
-}
-constexpr int vec_elems(int fix_in, int fix_out) {
-  const int a = fixed_type_bytes(fix_in), b = fixed_type_bytes(fix_out), w = a > b ? a : b;
-  return w == 8 ? 2 : w == 4 ? 4 : 8;  // (types known at run time only: 8 elements)
-}
-constexpr int BLOCK = 256;
 constexpr int MAXR = 8;
 
 struct NdIndex {
   int rank;
   int64_t dims[MAXR], ls[MAXR], rs[MAXR];
 };
-
-// Division of an index below 2^31 by an invariant divisor below 2^31 as one multiplication: the 64-bit
-// division the compiler emits costs every wave some hundred scalar and vector instructions, more than the
-// rest of an 8-element vector's work.
-struct FastDiv32 {
-  uint32_t mul, shr;
-};
-static FastDiv32 make_fastdiv(uint32_t d) {
-  uint32_t shr = 0;
-  while ((1ull << shr) < d) shr++;
-  return FastDiv32{(uint32_t)(((1ull << 32) * ((1ull << shr) - d)) / d + 1), shr};
-}
-__device__ __forceinline__ uint32_t fastdiv(uint32_t n, FastDiv32 f) { return (__umulhi(n, f.mul) + n) >> f.shr; }
 
 // how a vector index splits into (row, column); the FLAT modes cut the flat output into vectors that may run across
 // row ends (rows whose length is not a whole number of vectors) and count `vecs_per_row` as the element count
@@ -377,6 +347,10 @@ as_type_kernel(const void *__restrict__ in, void *__restrict__ out, int idt_, in
 
 // ---- host side ------------------------------------------------------------------------------
 
+// elementwise_flat.hip: whether it took the call
+bool binary_flat(const hipnx_ctx *ctx, int op, int dt, const void *l, const void *r, void *out, int64_t total, int64_t cols,
+                 int64_t l0, int64_t l1, int64_t r0, int64_t r1);
+
 enum { CLS_F32 = 0, CLS_F64 = 1, CLS_I64 = 2, CLS_U64 = 3 };
 
 // Whether a launch over `n` elements moves tensors far larger than the 256 MB last-level cache (the widest of the
@@ -660,6 +634,11 @@ extern "C" int hipnx_binary(hipnx_ctx *ctx, int op, int l_dt, int r_dt, int out_
       a.ls0 = l0; a.rs0 = r0; a.ls1 = (int)l1; a.rs1 = (int)r1;
       a.err = deferred_error_word(ctx);
       a.flat_total = n;
+      if (l_dt == out_dt && r_dt == out_dt && n < (1ll << 31) &&
+          binary_flat(ctx, op, out_dt, l->ptr, r->ptr, out->ptr, n, cols, l0, l1, r0, r1)) {
+        HIPNX_HIP(hipGetLastError());
+        return HIPNX_OK;
+      }
     }
   }
   if (vec_ok) {

@@ -457,3 +457,23 @@ def test_integer_extremes_in_every_pair_of_types(op, lt, rt, hip, oracle):
     ha, oa = both(a, lt, hip, oracle)
     hb, ob = both(b, rt, hip, oracle)
     assert_bits_equal(getattr(Nx, op)(ha, hb), getattr(Nx, op)(oa, ob), f"{op} {lt} {rt}")
+
+
+# A dense tensor with a row of its columns or with one value per row, where rows are not whole vectors of eight: fewer columns
+# than a lane's vector, rows that are whole vectors of four, a last vector cut off; either operand the dense one.
+@pytest.mark.parametrize("rows,cols", [(5, 2), (1001, 3), (77, 7), (33, 10), (513, 100), (1000, 33), (3, 1001), (129, 257), (2, 5)])
+@pytest.mark.parametrize("ty", ["f32", "bf16", "f16"])
+@pytest.mark.parametrize("op", ["add", "subtract", "divide", "max", "atan2"])
+def test_short_rows_with_a_row_or_a_value_per_row(rows, cols, ty, op, hip, oracle):
+    rng = np.random.default_rng(seed_of("flat", rows, cols, ty, op))
+    x = rand_raw(rng, ty, (rows, cols), lo=-4, hi=4)
+    hx, ox = both(x, ty, hip, oracle)
+    for shape in ((1, cols), (rows, 1)):
+        y = rand_raw(rng, ty, shape, lo=1, hi=4)
+        hy, oy = both(y, ty, hip, oracle)
+        for (a, b), (c, d) in (((hx, hy), (ox, oy)), ((hy, hx), (oy, ox))):
+            got, want = getattr(Nx, op)(a, b), getattr(Nx, op)(c, d)
+            if op == "atan2":  # a library function on either side
+                assert_all_close(got, want, {"f32": 1e-6, "bf16": 2.0 ** -7, "f16": 2.0 ** -10}[ty], 0, f"{op} {ty} {rows}x{cols} {shape}")
+            else:
+                assert_bits_equal(got, want, f"{op} {ty} {rows}x{cols} {shape}")
