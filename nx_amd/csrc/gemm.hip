@@ -517,38 +517,38 @@ static int dot_impl(hipnx_ctx *ctx, int l_dt, int r_dt, int out_dt, int64_t batc
             if (t < best) { best = t; splits = cand; }
           }
       } else if (wide) {
-        // An f32 slab is eight times the MFMA work of a 2-byte one (2.6 us per slab of a 128 x 128 tile, 0.55 us
-        // for a 64 x 32 tile, the second pass of a split about 8 us), so a grid that leaves CUs idle is cut much
-        // earlier: the cheapest, by those figures, of whole 128 x 128 tiles, K split up to 64 ways (2 slabs or
-        // more each) and 64 x 32 tiles.  512^3: 41 -> 18 us; 256 x 256 x 16384: 84 -> 40 us.
+        // An f32 slab is eight times the MFMA work of a 2-byte one, so a grid that leaves CUs idle is cut much earlier: the
+        // cheapest, by the figures below, of 128 x 128, 64 x 128 (up to 64 rows a 128-row tile would be half empty; and
+        // a last round that leaves most CUs idle ends sooner in halves) and 64 x 32 tiles, the first two also with K
+        // split up to 64 ways, 2 slabs or more each.  512^3: 41 -> 18 us; 256 x 256 x 16384: 84 -> 40 us.
+        //   A work-group takes `alone` us per slab while it has its CU to itself, waiting for memory much of it; up to
+        //   `resident` of them (as the LDS holds) share a CU and take `shared` us per slab and work-group together,
+        //   near what the MFMAs take: a split that puts two or three work-groups on a CU pays for its second pass
+        //   (784 x 512 x 4096, 52 tiles: 4 splits 58 us, 8 splits 50; 1000 x 700 x 1500, 96 tiles: 2 splits 45 us,
+        //   8 splits 35; 300 x 1000 x 900, 40 tiles: 64 x 32 tiles 29 us, 6 splits of 64 x 128 18.5; 2048^3: 128 x 128
+        //   174 us, 64 x 128, two to a CU, 152).  Fitted to f32 contractions of 100 to 8192 a side in three layouts,
+        //   within a tenth.  (Both operands K-inner: 128 x 128 tiles on the two-group kernel, which holds its CU alone,
+        //   and six stages of 64 x 32 tiles, two to a CU.)
+        struct Tile { int cfg, rows, cols, resident; double alone, shared; };
+        const bool kk = l_kin && r_kin, f64 = l_dt == HIPNX_F64;
+        const Tile tiles[3] = {
+            {GEMM_CFG_128, 128, 128, f64 || kk ? 1 : 2, f64 ? 2.6 : kk ? 2.05 : 2.5, f64 ? 2.6 : kk ? 2.05 : 2.15},
+            {GEMM_CFG_64x128, 64, 128, f64 ? 1 : 3, f64 ? 1.3 : 1.44, f64 ? 1.3 : 1.15},
+            {GEMM_CFG_64x32, 64, 32, f64 ? 1 : kk ? 2 : 6, f64 ? 0.55 : kk ? 0.75 : 0.79, f64 ? 0.55 : kk ? 0.65 : 0.36}};
         if (cfg == GEMM_CFG_128) {
           const int64_t cus = ctx->num_cus;
-          auto rounds = [&](int64_t groups) { return (double)((groups + cus - 1) / cus); };
-          double best = 10.0 + rounds(t128 * batch) * (double)nslab * 2.6;
-          // second launch, then the partial results written and read once (mostly from cache: ~8 MB per us)
-          auto split_cost = [&](int cand) { return 5.0 + 2.0 * (double)cand * (double)(M * N) * 4.0 / 8.0e6; };
-          if (splittable)
-            for (int cand = 2; cand <= 64; cand *= 2) {
-              if (t128 * cand > cus || nslab / cand < 2 || !reaches(cand)) continue;
-              const double t = 10.0 + (double)per_split(cand) * 2.6 + split_cost(cand);
-              if (t < best) { best = t; splits = cand; }
+          double best = 0;
+          for (const Tile &t : tiles) {
+            const int64_t count = ((M + t.rows - 1) / t.rows) * ((N + t.cols - 1) / t.cols) * batch;
+            for (int cand : {1, 2, 3, 4, 6, 8, 12, 16, 24, 32, 48, 64}) {
+              if (cand > 1 && (!splittable || t.cfg == GEMM_CFG_64x32 || count * cand > t.resident * cus || nslab / cand < 2 || !reaches(cand))) continue;
+              const int64_t per_cu = (count * cand + cus - 1) / cus, last = per_cu % t.resident;
+              double us = (double)per_split(cand) * ((double)(per_cu - last) * t.shared + (last ? std::max(t.alone, (double)last * t.shared) : 0.0));
+              // a split's second launch, then the partial results written and read once (mostly from cache: ~8 MB per us)
+              if (cand > 1) us += 5.0 + 2.0 * (double)cand * (double)(M * N) * 4.0 / 8.0e6;
+              if (best == 0 || us < best) { best = us; cfg = t.cfg; splits = cand; }
             }
-          // tiles of 64 x 128, half the MFMA work per slab: up to 64 rows a 128-row tile would be half empty, and a grid
-          // of 128 x 128 tiles whose last round leaves most CUs idle ends sooner in halves (3072^3: 576 tiles in three
-          // rounds, 1152 in five of half the length)
-          {
-            const int64_t tn = ((M + 63) / 64) * ((N + 127) / 128) * batch;
-            const double whole = 10.0 + rounds(tn) * (double)nslab * 1.3;
-            if (whole < best) { best = whole; cfg = GEMM_CFG_64x128; splits = 1; }
-            if (splittable)
-              for (int cand = 2; cand <= 64; cand *= 2) {
-                if (tn * cand > cus || nslab / cand < 2 || !reaches(cand)) continue;
-                const double t = 10.0 + (double)per_split(cand) * 1.3 + split_cost(cand);
-                if (t < best) { best = t; cfg = GEMM_CFG_64x128; splits = cand; }
-              }
           }
-          const int64_t t64 = ((M + 63) / 64) * ((N + 31) / 32) * batch;
-          if (10.0 + rounds(t64) * (double)nslab * 0.55 < best) { cfg = GEMM_CFG_64x32; splits = 1; }
         }
       } else if (splittable && t128 * 2 <= ctx->num_cus && nslab >= (t128 * 4 <= ctx->num_cus ? 32 : 64))
         // (the second pass and the partial results cost about 10 us: worth it from K = 32 slabs on -- 64 where

@@ -856,6 +856,12 @@ gemm_pipelined_kernel(GemmArgs a) {
     if constexpr (R_KIN) rload.issue_at(u, 2 * KInnerLoader<BN, NW>::PER, 1, 0, kbyte0, sB);
     else if constexpr (R_TR) rtr.issue_at(u, 2 * KOuterDmaLoader<TR_ES, R_TR ? BN : 256 * NW, NW>::PER, 1, 0, kbyte0 / ES, a.ld_r, sB);
   };
+  // AHEAD (an operand staged through registers): a slab's requests all go out right behind the barrier that frees its
+  // stage, a whole slab of MFMA work before they are committed.  Requested at the first step of the slab before and
+  // committed at step BAR they had five eighths of one, 0.5 us of f32 work, and with a work-group per CU that was
+  // less than the latency: f32 4096 x 512 x 784 (64 x 128 tiles, W stored [K, N]) 52 -> 47 us.  (Not for f64, whose
+  // registers are all spoken for.)
+  constexpr bool AHEAD = !ALL_DMA && DT != HIPNX_F64;
   constexpr int OPS = (L_KIN ? KInnerLoader<BM, NW>::PER : L_TR ? KOuterDmaLoader<TR_ES, L_TR ? BM : 256 * NW, NW>::PER : 0) +
                       (R_KIN ? KInnerLoader<BN, NW>::PER : R_TR ? KOuterDmaLoader<TR_ES, R_TR ? BN : 256 * NW, NW>::PER : 0);
   constexpr int INFLIGHT = OPS * (NSTAGE - 2);  // requests of younger slabs that may stay outstanding
@@ -869,6 +875,8 @@ gemm_pipelined_kernel(GemmArgs a) {
   if (nslab >= NSTAGE - 1) wait_vmcnt<INFLIGHT>();
   else wait_vmcnt<0>();
   __syncthreads();
+  if constexpr (AHEAD)
+    if (1 < nslab) issue(1, SLAB + k_shift);
   if constexpr (EARLY) {  // the first requests of slab 1 (what the steps behind a barrier would have issued)
     if (1 < nslab) {
 #pragma unroll
@@ -913,7 +921,7 @@ gemm_pipelined_kernel(GemmArgs a) {
         if (t > BAR) {
           if (s + 2 < nslab) issue_early(t - BAR - 1, s % NSTAGE, (int64_t)(s + 2) * SLAB + k_shift);
         } else if (request) issue_early(t + POST, req_stage, req_kbyte);
-      } else if (request && t <= BAR) issue_step(t, req_stage, req_kbyte);
+      } else if (!AHEAD && request && t <= BAR) issue_step(t, req_stage, req_kbyte);
 #pragma unroll
       for (int i = 0; i < TM16; i++) Mma16<DT>::step(acc[i][j], fb[t % RING], fa[ks & 1][i]);
       __builtin_amdgcn_s_setprio(0);
@@ -923,6 +931,8 @@ gemm_pipelined_kernel(GemmArgs a) {
         if (request) wait_vmcnt<INFLIGHT>(); // my loads of the next slab have landed
         else wait_vmcnt<0>();
         __syncthreads();
+        if constexpr (AHEAD)
+          if (s + 2 < nslab) issue(s % NSTAGE, (int64_t)(s + 2) * SLAB + k_shift);
       }
       __builtin_amdgcn_sched_barrier(0);
     }
