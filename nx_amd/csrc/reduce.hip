@@ -21,6 +21,8 @@ static int reduce_op(hipnx_ctx *ctx, bool static_ws, int idt, int odt, int64_t o
 // max / min / all / any: reduce_select.hip
 int reduce_select(hipnx_ctx *ctx, bool static_ws, int op, int idt, int odt, int64_t outer, int64_t red, int64_t inner,
                   const void *in, void *out);
+// one long slab of short rows: reduce_narrow.hip
+int reduce_narrow(hipnx_ctx *ctx, int op, int idt, int odt, int64_t red, int64_t inner, const void *in, void *out);
 
 }  // namespace hipnx
 
@@ -55,13 +57,15 @@ static int reduce_entry(hipnx_ctx *ctx, bool static_ws, int op, int in_dt, int o
   if (outer * inner == 0) return HIPNX_OK;
   // A few columns under a long reduced axis ([N, 3] summed over N) give the column kernel a handful of lanes per
   // segment and its second pass a handful of outputs with a thousand partial results each (f32 [33M, 2]: 7.9 ms,
-  // 0.03 TB/s).  With g rows folded into the columns the tensor is also [outer, red / g, g * inner]: reducing that
-  // view first leaves [outer, g, inner] (sums and products in f64 / 64-bit integers, so the result is still rounded
-  // once; selections in the element's own type), and a second, small reduction finishes.  A single slab (outer = 1)
-  // takes any g -- the red mod g rows left over are reduced on their own into one more row for the second step --
-  // several slabs need a divisor of the axis.
+  // 0.03 TB/s).  One slab of rows that a work-group covers goes to a kernel of its own (reduce_narrow.hip).  Otherwise,
+  // with g rows folded into the columns the tensor is also [outer, red / g, g * inner]: reducing that view first leaves
+  // [outer, g, inner] (sums and products in f64 / 64-bit integers, so the result is still rounded once; selections in
+  // the element's own type), and a second, small reduction finishes.  A single slab (outer = 1) takes any g -- the
+  // red mod g rows left over are reduced on their own into one more row for the second step -- several slabs need a
+  // divisor of the axis.
   const int esize = dtype_size(in_dt);
   if (!static_ws && inner > 1 && inner * esize < 1024 && red >= 4096) {
+    if (outer == 1 && inner <= BLOCK) return reduce_narrow(ctx, op, in_dt, out_dt, red, inner, inb->ptr, out->ptr);
     int64_t g = 4096 / inner < red / 32 ? 4096 / inner : red / 32;
     if (outer == 1) g &= ~(int64_t)7;  // whole vectors in the folded rows
     else while (g >= 16 && red % g != 0) g--;

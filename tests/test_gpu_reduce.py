@@ -306,3 +306,31 @@ def test_infinities_and_nan_in_reductions(ty, op, shape, axes, hip, oracle):
         x = (x.view(np.uint32) >> 16).astype(np.uint16)
     hx, ox = both(x, ty, hip, oracle)
     assert_bits_equal(getattr(Nx, op)(hx, axes=axes), getattr(Nx, op)(ox, axes=axes), f"{op} {ty} {shape} {axes}")
+
+
+# One long slab of short rows: columns that are and are not whole vectors, lanes of a work-group that are all or hardly half
+# used (129 columns), a last folded row cut off after any number of elements, one work-group and many; 257 columns and two
+# slabs stay on the other kernels.
+NARROW = [(4096, 2), (4096, 10), (5003, 3), (4099, 7), (70001, 100), (300007, 4), (4096, 129), (9001, 255), (8192, 256), (4096, 257)]
+
+
+@pytest.mark.parametrize("red,inner", NARROW)
+@pytest.mark.parametrize("ty", ["f32", "bf16", "f16", "f64", "s32", "u8", "s64"])
+def test_long_slabs_of_short_rows(red, inner, ty, hip):
+    """Small whole numbers: every sum is exact in f64 and 64-bit integers, so any order of additions gives the same value."""
+    rng = np.random.default_rng(seed_of("narrow", red, inner, ty))
+    whole = rng.integers(0 if ty == "u8" else -100, 101, size=(red, inner))
+    x = whole.astype(np.float32) if ty == "bf16" else whole.astype(T.numpy_dtype(T.normalize(ty)))
+    if ty == "bf16":
+        x = (x.view(np.uint32) >> 16).astype(np.uint16)  # (up to 100: exact)
+    t = from_numpy(x, ty, hip)
+    if T.is_integer(T.normalize(ty)):
+        assert np.array_equal(hip.to_numpy(Nx.sum(t, axes=[0])).astype(np.int64), whole.sum(axis=0))
+    else:
+        want = whole.sum(axis=0).astype(np.float64)
+        keep = {"f64": 0.0, "f32": 0.0, "f16": 2.0 ** -11, "bf16": 2.0 ** -7}[ty]  # one rounding; bf16 drops its low bits
+        got = values(Nx.sum(t, axes=[0]))
+        inside = np.abs(want) < 65504.0
+        assert (np.abs(got - want)[inside] <= keep * np.abs(want)[inside]).all()
+    for op, np_op in (("reduce_max", np.max), ("reduce_min", np.min)):
+        assert np.array_equal(values(getattr(Nx, op)(t, axes=[0])), np_op(whole, axis=0).astype(np.float64))
