@@ -234,7 +234,23 @@ splitk_combine_kernel(const AT *__restrict__ part, void *__restrict__ out, int o
   for (int64_t v = (int64_t)blockIdx.x * 256 + threadIdx.x; v < nvec; v += (int64_t)gridDim.x * 256) {
     typedef __attribute__((ext_vector_type(4), aligned(4))) AT vec_t;
     vec_t acc = *reinterpret_cast<const vec_t *>(part + v * 4);
-    for (int s = 1; s < splits; s++) {
+    int s = 1;
+    for (; s + 3 < splits; s += 4) {  // four loads in flight; added in split order
+      vec_t p[4];
+#pragma unroll
+      for (int u = 0; u < 4; u++) p[u] = *reinterpret_cast<const vec_t *>(part + (s + u) * mn + v * 4);
+#pragma unroll
+      for (int u = 0; u < 4; u++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) acc[e] += p[u][e];
+    }
+    if (s + 1 < splits) {
+      const vec_t p = *reinterpret_cast<const vec_t *>(part + s * mn + v * 4), q = *reinterpret_cast<const vec_t *>(part + (s + 1) * mn + v * 4);
+#pragma unroll
+      for (int e = 0; e < 4; e++) acc[e] = acc[e] + p[e] + q[e];
+      s += 2;
+    }
+    if (s < splits) {
       const vec_t p = *reinterpret_cast<const vec_t *>(part + s * mn + v * 4);
 #pragma unroll
       for (int e = 0; e < 4; e++) acc[e] += p[e];
