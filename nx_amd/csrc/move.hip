@@ -54,11 +54,18 @@ transpose2d_kernel(const T *__restrict__ in, T *__restrict__ out, int64_t R, int
   const T *src = in + b * R * C;
   T *dst = out + b * R * C;
   const int tx = threadIdx.x % TILE, ty = threadIdx.x / TILE;  // 64 x 4
-  for (int j = ty; j < TILE; j += BLOCK / TILE) {
-    int64_t r = tr * TILE + j, c = tc * TILE + tx;
-    if (r < R && c < C) tile[j][tx] = src[r * C + c];
+  // (every load before the first LDS write: one at a time, each waited for, a tile took the latency sixteen times)
+  constexpr int PER = TILE * TILE / BLOCK;
+  T v[PER];
+#pragma unroll
+  for (int i = 0; i < PER; i++) {
+    const int64_t r = tr * TILE + ty + i * (BLOCK / TILE), c = tc * TILE + tx;
+    v[i] = r < R && c < C ? src[r * C + c] : T();
   }
+#pragma unroll
+  for (int i = 0; i < PER; i++) tile[ty + i * (BLOCK / TILE)][tx] = v[i];
   __syncthreads();
+#pragma unroll
   for (int j = ty; j < TILE; j += BLOCK / TILE) {
     int64_t c = tc * TILE + j, r = tr * TILE + tx;
     if (r < R && c < C) dst[c * R + r] = tile[tx][j];
