@@ -346,7 +346,7 @@ static int dot_impl(hipnx_ctx *ctx, int l_dt, int r_dt, int out_dt, int64_t batc
       if (l_pad || r_pad) mfma = (double)M * (double)N * (double)K * (double)batch >= 16777216.0;
     }
     if (scaled) {
-      if (!(int8_pair && mfma)) return set_error(HIPNX_EUNSUPPORTED, "dot_scaled: s8 x s8 with K at most 65536, M * N >= 256 and rows of whole 16-byte pieces (or 16 M multiply-adds)");
+      if (!(int8_pair && mfma && row_bytes % SLAB == 0)) return set_error(HIPNX_EUNSUPPORTED, "dot_scaled: s8 x s8 with K a multiple of 128 and at most 65536, M * N >= 256");
       if (scale_mode == HIPNX_SCALE_PER_ROW && batch != 1) return set_error(HIPNX_EUNSUPPORTED, "dot_scaled: a scale per row with more than one batch item");
       const int64_t need = scale_mode == HIPNX_SCALE_PER_COLUMN ? N : scale_mode == HIPNX_SCALE_PER_ROW ? M : 1;
       if (int st = check_buf(ctx, scale, (uint64_t)need * 4, "dot_scaled scale")) return st;

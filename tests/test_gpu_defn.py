@@ -707,6 +707,22 @@ def test_scaled_dot_entry_point_refuses_what_it_does_not_take(hip):
         hip.dot_scaled(sc.with_(data=None, shape=(16, 40)), x2, [1], [], w2, [1], [], short, SCALE_PER_COLUMN)
 
 
+@pytest.mark.parametrize("K,contract", [(1000, 1), (1008, 1), (1009, 0)])
+def test_scaled_dot_refuses_every_partial_slab_of_k(hip, K, contract):
+    """Also where the plain contraction walks the partial slab in place or copies the rows: the three calls, same bits."""
+    from nx_amd._lib import EUNSUPPORTED, SCALE_PER_COLUMN, HipNxError
+    rng = np.random.default_rng(K)
+    x, w = rand_s8(rng, (128, K), hip), rand_s8(rng, (144, K) if contract else (K, 144), hip)
+    sc = from_numpy(rng.uniform(1e-3, 1e-2, size=(144,)).astype(np.float32), "f32", hip)
+    with pytest.raises(HipNxError) as err:
+        hip.dot_scaled(sc.with_(data=None, shape=(128, 144)), x, [1], [], w, [contract], [], sc, SCALE_PER_COLUMN)
+    assert err.value.status == EUNSUPPORTED
+
+    def fun(xq, wq, s):
+        return Nx.multiply(Nx.as_type(Nx.dot(xq, [1], wq, [contract], out_type="s32"), "f32"), s)
+    assert_bits_equal(defn.compile(fun, x, w, sc, fuse=True)(x, w, sc), defn.compile(fun, x, w, sc)(x, w, sc), "three calls")
+
+
 # ---- stages over the same rows in one kernel (planned for compiled kernels) ------------------------------
 
 def softmax_rows(x):
