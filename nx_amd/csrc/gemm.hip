@@ -6,8 +6,9 @@
 //       (a partial slab of K is walked with zeros behind its end).  What they cannot take is first copied: a K-outer
 //       operand whose row count is not a multiple of its transpose block (16 s8 / 8 bf16,f16 / 4 f32 rows) by the
 //       tiled transpose, a K-inner one whose rows are not whole 16-byte pieces to rows that are -- where the
-//       contraction is large enough to pay for it (16 M multiply-adds), else the plain kernel.
-//   everything else (f64, wide integers, mixed operand types, tiny problems): dot_generic_kernel,
+//       contraction is large enough to pay for it (16 M multiply-adds).
+//   everything else (f64 whose K is not whole slabs, wide integers, mixed operand types, fewer than 256 outputs, and below
+//     16 M multiply-adds a float K that is not whole 16-byte pieces, in every layout): dot_generic_kernel,
 //     a plain tiled kernel accumulating in f64 or wrapping 64-bit integers.
 //
 // Algorithmic work: 2*B*M*N*K flop; minimum traffic bytes(l) + bytes(r) + bytes(out).
@@ -20,8 +21,8 @@
 
 namespace hipnx {
 
-// Rows of K elements copied to a pitch of whole 16-byte pieces (out_pitch bytes), zeros behind K: what a K-inner operand
-// needs whose rows are not whole pieces, as the direct-to-LDS loads take pieces at 16-byte addresses.  A lane writes one
+// Rows of K elements copied to a pitch of whole 16-byte pieces, zeros behind K: what a K-inner operand
+// needs whose rows are not whole pieces, as the direct-to-LDS loads take whole pieces.  A lane writes one
 // piece; a piece inside its row is one load at whatever address it has, the row's last one is put together by elements.
 // Bound by memory: reads and writes the operand once ([2000, 999] bf16, 8 MB moved: 3 us).
 template <typename T>
@@ -340,10 +341,13 @@ static int dot_impl(hipnx_ctx *ctx, int l_dt, int r_dt, int out_dt, int64_t batc
     mfma = (float_pair || int8_pair) && K > 0 && M * N >= 256;
     if (mfma && l_dt == HIPNX_F64) mfma = row_bytes % SLAB == 0;  // (f64 otherwise adds over k in order, on the plain kernels)
     else if (mfma && row_bytes % 16 != 0) {
-      // rows that are not whole pieces: only a K-inner operand minds, and a copy of it is worth a launch from here on
+      // rows that are not whole pieces: only a K-inner operand minds, and a copy of it is worth a launch from 16 M
+      // multiply-adds on.  Below that floats are summed in f64 on the plain kernels whatever the layout (two K-outer
+      // operands need no copy, but their sums would be f32 where the same product stored otherwise has f64); int8 is
+      // exact on either.
       l_pad = l_layout == HIPNX_K_INNER || l_relay;
       r_pad = r_layout == HIPNX_K_INNER || r_relay;
-      if (l_pad || r_pad) mfma = (double)M * (double)N * (double)K * (double)batch >= 16777216.0;
+      if (l_pad || r_pad || l_dt != HIPNX_S8) mfma = (double)M * (double)N * (double)K * (double)batch >= 16777216.0;
     }
     if (scaled) {
       if (!(int8_pair && mfma && row_bytes % SLAB == 0)) return set_error(HIPNX_EUNSUPPORTED, "dot_scaled: s8 x s8 with K a multiple of 128 and at most 65536, M * N >= 256");

@@ -335,6 +335,22 @@ def test_partial_slabs_of_k(ty, M, N, K, layout, hip):
     assert np.array_equal(hip.to_numpy(got), want)
 
 
+@pytest.mark.parametrize("ty,M,N,K", [("f32", 64, 48, 33), ("f32", 64, 64, 4095), ("f32", 16, 16, 1001), ("bf16", 128, 96, 1001), ("f16", 64, 64, 4001)])
+@pytest.mark.parametrize("layout", ["nn", "nt", "tn", "tt"])
+def test_small_contractions_with_k_off_sixteen_bytes_sum_in_f64_in_every_layout(ty, M, N, K, layout, hip, oracle):
+    """A gradient of a layer over a batch of 33 or 4095 rows is dot(x, [0], d, [0]): both operands K-outer.  Below 16 M
+    multiply-adds it has the reference's f64 sums, in order of k and rounded once, as the same product stored K-inner has:
+    the reference's bits.  (An f32 sum of 33 products of f32 values misses some of 3072 results by a rounding.)"""
+    rng = np.random.default_rng(seed_of(ty, M, N, K, layout, "off sixteen bytes"))
+    a, b = rand_raw(rng, ty, (M, K), lo=-1, hi=1), rand_raw(rng, ty, (K, N), lo=-1, hi=1)
+    la = a if layout[0] == "n" else np.ascontiguousarray(a.T)
+    lb = b if layout[1] == "n" else np.ascontiguousarray(b.T)
+    c1, c2 = [1 if layout[0] == "n" else 0], [0 if layout[1] == "n" else 1]
+    ha, oa = both(la, ty, hip, oracle)
+    hb, ob = both(lb, ty, hip, oracle)
+    assert_bits_equal(Nx.dot(ha, c1, hb, c2, out_type="f32"), Nx.dot(oa, c1, ob, c2, out_type="f32"), f"{ty} {M}x{N}x{K} {layout}")
+
+
 @pytest.mark.parametrize("ty,M,N,K", [("bf16", 128, 1024, 4096), ("s8", 128, 1024, 4096), ("f16", 200, 520, 2048), ("f32", 132, 384, 2048),
                                       ("bf16", 768, 4096, 4096), ("f16", 1000, 4100, 4096),
                                       ("s8", 384, 512, 8192), ("bf16", 512, 1024, 2048),
