@@ -64,9 +64,12 @@ static Keeps what_is_kept(const FusedArgs &a) {
   bool stages = false;
   for (int i = 0; i < a.n_instr; i++) {
     const hipnx_fused_instr &q = a.ins[i];
+    // (a SET or BINARY on integers reads the words as they are in memory; a SELECT reads floats whatever its flags:
+    // the cases of fetch_static)
+    const bool raw = (q.flags & HIPNX_FUSED_FLAG_INT) != 0 && q.kind != HIPNX_FUSED_SELECT;
     auto source = [&](int src, int arg) {
       if (src == HIPNX_FUSED_SRC_CARRY) carried_from = stage - 1;  // (the last stage that leaves a value somebody reads)
-      if (src == HIPNX_FUSED_SRC_INPUT && a.in_cs[arg] == 1 && !(q.flags & HIPNX_FUSED_FLAG_INT)) reads[arg] |= 1u << stage;
+      if (src == HIPNX_FUSED_SRC_INPUT && a.in_cs[arg] == 1 && !raw) reads[arg] |= 1u << stage;
     };
     if (q.kind == HIPNX_FUSED_SET || q.kind == HIPNX_FUSED_BINARY || q.kind == HIPNX_FUSED_SELECT) source(q.src, q.arg);
     if (q.kind == HIPNX_FUSED_SELECT) source(q.src2, q.arg2);

@@ -821,6 +821,25 @@ def test_long_rows_take_a_block_each(name, shape, ty, hip):
     assert calls == [1]
 
 
+def test_a_select_on_integers_reads_a_row_that_later_stages_hold(hip):
+    """A SELECT marked as an integer instruction takes its operands as floats all the same: the stage it stands in is the
+    first that reads the row, and the registers that hold the row for the later stages are filled there."""
+    from nx_amd.tensor import template
+    SET, BINARY, SELECT, AS_TYPE, ROW_REDUCE, ROW_STAT = 0, 2, 3, 4, 6, 7
+    CONST, INPUT, ROWSTAT, ADD, SUM, INT = 0, 1, 3, 0, 0, 2
+    f32, s32 = ("f", 32), ("s", 32)
+    program = [dict(kind=SET, src=CONST, imm=1.0, dt=f32), dict(kind=SELECT, src=INPUT, arg=0, src2=INPUT, arg2=0, flags=INT, dt=s32),
+               dict(kind=AS_TYPE, dt=f32), dict(kind=ROW_REDUCE, op=SUM, dt=f32), dict(kind=ROW_STAT, arg=0, dt=f32),
+               dict(kind=SET, src=INPUT, arg=0, dt=f32), dict(kind=BINARY, op=ADD, src=ROWSTAT, arg=0, dt=f32),
+               dict(kind=ROW_REDUCE, op=SUM, dt=f32), dict(kind=ROW_STAT, arg=1, dt=f32),
+               dict(kind=SET, src=INPUT, arg=0, dt=f32), dict(kind=BINARY, op=ADD, src=ROWSTAT, arg=1, dt=f32)]
+    for rows, cols in ((9, 8), (5, 1024), (3, 4104)):
+        x = np.random.default_rng(cols).integers(-3, 4, size=(rows, cols)).astype(np.float32)  # (every sum below 2^24: exact)
+        got = hip.fused_elementwise(template("f32", (rows, cols)), program, [from_numpy(x, "f32", hip)], (rows, cols, [(cols, 1)]), mode="compiled")
+        total = x.sum(axis=1, keepdims=True, dtype=np.float64)
+        np.testing.assert_array_equal(hip.to_numpy(got), (x + (total + cols * total)).astype(np.float32))
+
+
 def test_rows_too_long_for_carried_values_are_read_again(hip):
     x = rand_float(np.random.default_rng(7), "f32", (2048, 32776), hip)
     planned = defn.compile(softmax_rows, x, fuse="compiled")
