@@ -421,7 +421,11 @@ int hipnx_fused_elementwise(hipnx_ctx *ctx, int n_instr, const hipnx_fused_instr
  * out over the same device functions, compiled for the device once by the run-time compiler (a few
  * hundred milliseconds) and kept with the context -- the role exla/lib/exla/defn.ex's compilation
  * cache plays for a whole function, here for one element-wise group.  Results are bit-identical in
- * both modes.  A program first met while the context is capturing runs interpreted in that capture.
+ * both modes.  A program first met while the context is capturing runs interpreted in that capture (one that exists only
+ * compiled is refused there: HIPNX_EUNSUPPORTED).  A program of stages that keeps an input or values of its rows in registers
+ * is compiled once per number of 512-element steps (2048 above 4096 elements, up to 32768) in a row; a capture that meets
+ * it at another row length takes a kernel that reads the rows again, unless it reads HIPNX_FUSED_SRC_CARRY, provided the
+ * program was compiled at some length on the same side of 4096.
  * A program's constants are part of what it is compiled for: one whose constant changes from call to
  * call compiles again for each value.  The context keeps at most 512 programs (another limit, at least
  * 4: hipnx_fused_set_cache_limit); when that many are held, the next new one first waits for the stream

@@ -51,6 +51,7 @@ static void list_of(std::string &s, const char *name, const char *type, int n, c
 // and an input that several stages read.
 struct Keeps {
   int trips = 0;        // vectors of a lane along a row, 0 when nothing is kept
+  bool carries = false;
   int held = -1;        // the input, and the first stage that reads it
   int held_stage = -1;
 };
@@ -77,7 +78,8 @@ static Keeps what_is_kept(const FusedArgs &a) {
     if (q.kind == HIPNX_FUSED_ROW_STAT) stage++;
   }
   if (!stages || trips > 16) return k;  // (the host refuses longer rows for programs that carry values)
-  if (carried_from >= 0) k.trips = (int)trips;
+  k.carries = carried_from >= 0;
+  if (k.carries) k.trips = (int)trips;
   for (int in = 0; in < a.n_inputs; in++) {
     if (!(reads[in] & (reads[in] - 1)) || k.held >= 0) continue;  // one stage reads it: nothing to gain
     // a lane has room for 16 vectors (128 of its registers): an input that is still read once a carried value is there
@@ -91,25 +93,31 @@ static Keeps what_is_kept(const FusedArgs &a) {
   return k;
 }
 
-// everything a compiled kernel is specialised on, as bytes: the cache key
-static std::string make_key(const FusedArgs &a, int reduce_op, bool block_per_row) {
+// everything a compiled kernel is specialised on, as bytes: the cache key.  The number of vectors kept comes last: the keys of
+// one program's kernels for rows of other lengths differ in it alone.
+static std::string make_key(const FusedArgs &a, const Keeps &keeps, int reduce_op, bool block_per_row) {
   std::string k;
-  k.reserve(16 + 16 * a.n_instr + 8 * a.n_inputs);
-  const int head[5] = {a.n_instr, a.n_inputs, a.out_dt, reduce_op * 2 + (block_per_row ? 1 : 0), what_is_kept(a).trips};
+  k.reserve(20 + 16 * a.n_instr + 8 * a.n_inputs);
+  const int head[4] = {a.n_instr, a.n_inputs, a.out_dt, reduce_op * 2 + (block_per_row ? 1 : 0)};
   k.append((const char *)head, sizeof(head));
   k.append((const char *)a.ins, sizeof(hipnx_fused_instr) * a.n_instr);
   k.append((const char *)a.in_dt, sizeof(int) * a.n_inputs);
   k.append((const char *)a.in_cs, sizeof(int) * a.n_inputs);
+  k.append((const char *)&keeps.trips, sizeof(int));
   return k;
 }
 
+// A program that keeps an input in registers only to read it once could do without, and then takes rows of any length: its
+// module also has that kernel, for a capture that meets a length which has not been compiled (a new module is no work to
+// record).  One that carries values cannot.
+static bool has_kernel_for_any_length(const Keeps &k) { return k.trips > 0 && !k.carries; }
+static std::string any_length(const std::string &name) { return name + "_any"; }
+
 // the whole translation unit for one program
-static std::string make_source(const FusedArgs &a, int reduce_op, bool block_per_row, const std::string &name) {
+static std::string make_source(const FusedArgs &a, const Keeps &keeps, int reduce_op, bool block_per_row, const std::string &name) {
   std::string s = RTC_PREAMBLE;
-  const Keeps keeps = what_is_kept(a);
-  s += "namespace hipnx {\nstruct P {\n  static constexpr int n_instr = " + std::to_string(a.n_instr) + ", out_dt = " + std::to_string(a.out_dt) +
-       ", nv = " + std::to_string(keeps.trips) + ", tpr = " + (block_per_row ? "FBLOCK" : "WAVE") + ", held = " + std::to_string(keeps.held) +
-       ", held_stage = " + std::to_string(keeps.held_stage) + ";\n";
+  s += "namespace hipnx {\nstruct Program {\n  static constexpr int n_instr = " + std::to_string(a.n_instr) + ", out_dt = " + std::to_string(a.out_dt) +
+       ", tpr = " + (block_per_row ? "FBLOCK" : "WAVE") + ";\n";
   const hipnx_fused_instr *q = a.ins;
   list_of(s, "kind", "int", a.n_instr, [&](int i) { return std::to_string((int)q[i].kind); });
   list_of(s, "op", "int", a.n_instr, [&](int i) { return std::to_string((int)q[i].op); });
@@ -136,7 +144,18 @@ static std::string make_source(const FusedArgs &a, int reduce_op, bool block_per
   }
   list_of(s, "seg_red", "int", (int)seg_red.size(), [&](int k) { return std::to_string(seg_red[k]); });
   list_of(s, "seg_save", "int", (int)seg_save.size(), [&](int k) { return std::to_string(seg_save[k]); });
-  s += "};\n}\nusing namespace hipnx;\nextern \"C\" __global__ void __launch_bounds__(FBLOCK) " + name + "(FusedArgs by_value) {\n  (void)by_value;\n";
+  auto keeping = [](const char *p, const Keeps &k) {
+    return std::string("struct ") + p + " : Program {\n  static constexpr int nv = " + std::to_string(k.trips) + ", held = " + std::to_string(k.held) +
+           ", held_stage = " + std::to_string(k.held_stage) + ";\n};\n";
+  };
+  auto kernel = [](const std::string &called) {
+    return "extern \"C\" __global__ void __launch_bounds__(FBLOCK) " + called + "(FusedArgs by_value) {\n  (void)by_value;\n";
+  };
+  s += "};\n" + keeping("P", keeps);
+  if (has_kernel_for_any_length(keeps)) s += keeping("Any", Keeps{});
+  s += "}\nusing namespace hipnx;\n";
+  if (has_kernel_for_any_length(keeps)) s += kernel(any_length(name)) + "  fused_row_stages_body<Any>();\n}\n";
+  s += kernel(name);
   const char *tpr = block_per_row ? "FBLOCK" : "WAVE";
   if (stages) s += "  fused_row_stages_body<P>();\n";
   else switch (reduce_op) {
@@ -149,7 +168,7 @@ static std::string make_source(const FusedArgs &a, int reduce_op, bool block_per
   return s;
 }
 
-static int compile(hipnx_ctx *ctx, const std::string &src, const std::string &name, hipnx_ctx::FusedKernel *out) {
+static int compile(hipnx_ctx *ctx, const std::string &src, const std::string &name, bool with_any, hipnx_ctx::FusedKernel *out) {
   hipDeviceProp_t prop;
   HIPNX_HIP(hipGetDeviceProperties(&prop, ctx->device));
   const std::string arch = std::string("--offload-arch=") + prop.gcnArchName;
@@ -173,6 +192,7 @@ static int compile(hipnx_ctx *ctx, const std::string &src, const std::string &na
   hiprtcDestroyProgram(&prog);
   HIPNX_HIP(hipModuleLoadData(&out->module, code.data()));
   hipError_t e = hipModuleGetFunction(&out->function, out->module, name.c_str());
+  if (e == hipSuccess && with_any) e = hipModuleGetFunction(&out->any_length, out->module, any_length(name).c_str());
   if (e != hipSuccess) {
     (void)hipModuleUnload(out->module);
     return hip_fail(e, "hipModuleGetFunction(fused group)");
@@ -208,10 +228,19 @@ static int trim_cache(hipnx_ctx *ctx) {
 // program is new and the stream is capturing (compiling and loading a module is no work to record).
 int fused_launch_compiled(hipnx_ctx *ctx, const FusedArgs &a, int reduce_op, bool block_per_row, unsigned grid, bool *done) {
   *done = false;
-  const std::string key = make_key(a, reduce_op, block_per_row);
+  const Keeps keeps = what_is_kept(a);
+  const std::string key = make_key(a, keeps, reduce_op, block_per_row);
   auto it = ctx->fused_kernels.find(key);
+  hipFunction_t function = nullptr;
+  if (it == ctx->fused_kernels.end() && ctx->capture) {
+    // the program may be there for rows of another length, with a kernel that takes any
+    const size_t same = key.size() - sizeof(int);
+    for (it = ctx->fused_kernels.begin(); it != ctx->fused_kernels.end(); ++it)
+      if (it->second.any_length && it->first.size() == key.size() && it->first.compare(0, same, key, 0, same) == 0) break;
+    if (it == ctx->fused_kernels.end()) return HIPNX_OK;
+    function = it->second.any_length;
+  }
   if (it == ctx->fused_kernels.end()) {
-    if (ctx->capture) return HIPNX_OK;
     // a name a profile can tell apart: what the kernel is (a map, a map with its row reduction, stages over rows),
     // how long its program is, and a hash of what it is specialised on
     int stages = 0;
@@ -222,15 +251,17 @@ int fused_launch_compiled(hipnx_ctx *ctx, const FusedArgs &a, int reduce_op, boo
     if (ctx->fused_kernels.size() >= ctx->fused_cache_max)
       if (int st = trim_cache(ctx)) return st;
     hipnx_ctx::FusedKernel k{};
-    if (int st = compile(ctx, make_source(a, reduce_op, block_per_row, name), name, &k)) return st;
+    if (int st = compile(ctx, make_source(a, keeps, reduce_op, block_per_row, name), name, has_kernel_for_any_length(keeps), &k)) return st;
+    if (keeps.trips == 0) k.any_length = k.function;
     it = ctx->fused_kernels.emplace(key, k).first;
   }
+  if (!function) function = it->second.function;
   it->second.last_use = ++ctx->fused_clock;
   if (ctx->capture) it->second.in_graph = true;  // a recorded launch refers to the loaded module for as long as the graph lives
   // the argument block is the kernel's one by-value parameter: hand it over as the packed buffer it is
   size_t size = sizeof(FusedArgs);
   void *config[] = {HIP_LAUNCH_PARAM_BUFFER_POINTER, (void *)&a, HIP_LAUNCH_PARAM_BUFFER_SIZE, &size, HIP_LAUNCH_PARAM_END};
-  HIPNX_HIP(hipModuleLaunchKernel(it->second.function, grid, 1, 1, FBLOCK, 1, 1, 0, ctx->stream, nullptr, config));
+  HIPNX_HIP(hipModuleLaunchKernel(function, grid, 1, 1, FBLOCK, 1, 1, 0, ctx->stream, nullptr, config));
   *done = true;
   return HIPNX_OK;
 }

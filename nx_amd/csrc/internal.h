@@ -60,6 +60,7 @@ struct hipnx_ctx {
   struct FusedKernel {
     hipModule_t module;
     hipFunction_t function;
+    hipFunction_t any_length;  // the same program for rows of any length (null: there is none)
     uint64_t last_use;
     bool in_graph;
   };

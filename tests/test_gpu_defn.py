@@ -840,6 +840,56 @@ def test_a_select_on_integers_reads_a_row_that_later_stages_hold(hip):
         np.testing.assert_array_equal(hip.to_numpy(got), (x + (total + cols * total)).astype(np.float32))
 
 
+# one vector a lane, two, three, eight; a block per row: three, eight, nine, sixteen, more than are held
+@pytest.mark.parametrize("ty", ["f32", "bf16"])
+@pytest.mark.parametrize("warmed,others", [((40, 64), [(9, 8), (9, 512), (5, 520), (7, 1024), (5, 1032), (3, 1544), (2049, 4096)]),
+                                           ((3, 4104), [(5, 16384), (3, 16392), (8, 32760), (2048, 32776)])])
+def test_a_program_that_holds_its_row_is_captured_at_other_lengths(warmed, others, ty, hip):
+    """Rows of one length were run, rows of another are met in a capture: the program is there in a form that takes any
+    length, nothing is compiled, and the bits are those of the nodes one by one."""
+    from nx_amd import backend as B
+    shift = {"f32": 0.37, "bf16": 0.375}[ty]  # (a constant no other test uses: a program of this test's own)
+
+    def fun(x):
+        z = Nx.subtract(Nx.add(x, shift), Nx.reduce_max(x, axes=[-1], keep_axes=True))
+        return Nx.subtract(z, Nx.log(Nx.sum(Nx.exp(z), axes=[-1], keep_axes=True)))
+    rng = np.random.default_rng(seed_of(warmed, ty, "one compilation"))
+    before = B.fused_compiled_count()
+    first = rand_float(rng, ty, warmed, hip)
+    assert_bits_equal(defn.compile(fun, first, fuse="compiled")(first), defn.compile(fun, first)(first), f"{warmed}")
+    assert B.fused_compiled_count() == before + 1
+    for shape in others:
+        x = rand_float(rng, ty, shape, hip)
+        want = defn.compile(fun, x)(x)
+        planned = defn.compile(fun, x, fuse="compiled")
+        cluster = planned.roots[0].data.args[0]
+        assert type(cluster).__name__ == "_RowCluster" and not any(ins.get("src") == 4 for ins in cluster.program)
+        launches = []
+        original = hip.fused_elementwise.__func__
+
+        def counting(cls, *a, **k):
+            out = original(cls, *a, **k)  # (a refusal raises: the nodes would run one by one)
+            launches.append(k.get("mode"))
+            return out
+        hip.fused_elementwise = classmethod(counting)
+        B.capture_begin(0)
+        try:
+            out = planned(x)
+        finally:
+            graph = B.capture_end(0)
+            hip.fused_elementwise = classmethod(original)
+        assert launches == ["compiled"] and B.fused_compiled_count() == before + 1, shape
+        for _ in range(3):
+            graph.launch()
+            assert_bits_equal(out, want, f"replay at {shape}")
+            assert_bits_equal(Nx.exp(x), Nx.exp(x), "work between the replays")
+        del out
+        graph.destroy()
+    for shape in others:  # and outside a capture each length has kernels of its own
+        x = rand_float(rng, ty, shape, hip)
+        assert_bits_equal(defn.compile(fun, x, fuse="compiled")(x), defn.compile(fun, x)(x), f"{shape}")
+
+
 def test_rows_too_long_for_carried_values_are_read_again(hip):
     x = rand_float(np.random.default_rng(7), "f32", (2048, 32776), hip)
     planned = defn.compile(softmax_rows, x, fuse="compiled")
