@@ -287,8 +287,9 @@ def test_half_width_tiles_of_the_two_group_kernel(ty, M, N, K, layout, hip, orac
                                       ("bf16", 2, 4100, 2050)])
 @pytest.mark.parametrize("layout", ["nn", "nt", "tn", "tt"])
 def test_contraction_lengths_off_the_slab_grid_are_padded(ty, M, N, K, layout, hip, oracle):
-    """A K that is not a whole number of 128-byte slabs: large problems run on zero-extended copies of the
-    operands (products of two zeros add nothing), so int8 stays exact and floats stay within the bound."""
+    """A K that is not a whole number of 128-byte slabs: the partial slab is walked in place with zeros behind its end
+    (K-inner rows that are not whole 16-byte pieces are first copied to rows that are), and products of two zeros add
+    nothing: int8 stays exact and floats stay within the bound."""
     rng = np.random.default_rng(seed_of(ty, M, N, K, layout, "pad"))
     if ty == "s8":
         a = rng.integers(-127, 128, size=(M, K)).astype(np.int8)
@@ -333,6 +334,79 @@ def test_partial_slabs_of_k(ty, M, N, K, layout, hip):
                  [0 if layout[1] == "n" else 1], out_type=out)
     want = (a.astype(np.float64) @ b.astype(np.float64)).astype(np.int32 if ty == "s8" else np.float32)
     assert np.array_equal(hip.to_numpy(got), want)
+
+
+HELD = {"s8": lambda x: x.astype(np.int8), "f32": lambda x: x.astype(np.float32), "f16": lambda x: x.astype(np.float16),
+        "f64": lambda x: x.astype(np.float64), "bf16": lambda x: (x.astype(np.float32).view(np.uint32) >> 16).astype(np.uint16)}
+
+
+# every copy with a batch: K-inner rows padded, K-outer ones re-laid and padded, one operand copied and the other not, none copied
+@pytest.mark.parametrize("ty,batch,M,N,K", [("bf16", 5, 203, 197, 333), ("bf16", 3, 264, 197, 333), ("f16", 3, 264, 520, 72), ("f32", 4, 160, 131, 250),
+                                            ("s8", 3, 256, 272, 301), ("s8", 2, 130, 528, 1297)])
+@pytest.mark.parametrize("layout", ["nn", "nt", "tn", "tt"])
+def test_batched_contractions_with_a_partial_slab(ty, batch, M, N, K, layout, hip):
+    """Integer-valued operands: every partial sum is a whole number below 2^24, so the product is exact in any order."""
+    rng = np.random.default_rng(seed_of(ty, batch, M, N, K, layout, "batched partial slab"))
+    a, b = rng.integers(-4, 5, size=(batch, M, K)), rng.integers(-4, 5, size=(batch, K, N))
+    la = a if layout[0] == "n" else np.ascontiguousarray(a.transpose(0, 2, 1))
+    lb = b if layout[1] == "n" else np.ascontiguousarray(b.transpose(0, 2, 1))
+    got = Nx.dot(from_numpy(HELD[ty](la), ty, hip), [2 if layout[0] == "n" else 1], [0], from_numpy(HELD[ty](lb), ty, hip),
+                 [1 if layout[1] == "n" else 2], [0], out_type="s32" if ty == "s8" else "f32")
+    assert np.array_equal(hip.to_numpy(got).astype(np.float64), a.astype(np.float64) @ b.astype(np.float64))
+
+
+@pytest.mark.parametrize("ty,M,N,K", [("bf16", 264, 520, 72), ("f16", 520, 392, 1032), ("bf16", 24, 2048, 648), ("bf16", 203, 264, 333),
+                                      ("f32", 132, 64, 36), ("f32", 300, 264, 250)])
+@pytest.mark.parametrize("layout", ["nn", "nt", "tn", "tt"])
+def test_what_lies_behind_the_end_of_k_is_not_read(ty, M, N, K, layout, hip):
+    """NaN in the next row, the next column, the next batch item and behind the operands: it stays out of the results of
+    the others, which are exact (integer-valued operands)."""
+    rng = np.random.default_rng(seed_of(ty, M, N, K, layout, "behind the end"))
+    a, b = rng.integers(-4, 5, size=(3, M, K)).astype(np.float64), rng.integers(-4, 5, size=(3, K, N)).astype(np.float64)
+    a[1], b[2] = np.nan, np.nan
+    a[0, 1::2], b[0, :, 2::3] = np.nan, np.inf
+    la = a if layout[0] == "n" else np.ascontiguousarray(a.transpose(0, 2, 1))
+    lb = b if layout[1] == "n" else np.ascontiguousarray(b.transpose(0, 2, 1))
+
+    def followed_by_nan(x):
+        held = HELD[ty](x)
+        nan = HELD[ty](np.full(256, np.nan))
+        owner = from_numpy(np.concatenate([held.ravel(), nan]), ty, hip)
+        pointer = Nx.Pointer(kind="local", address=Nx.to_pointer(owner).address, data_size=held.size * held.itemsize)
+        return Nx.from_pointer(hip, pointer, ty, held.shape, keep=owner)
+    got = hip.to_numpy(Nx.dot(followed_by_nan(la), [2 if layout[0] == "n" else 1], [0], followed_by_nan(lb), [1 if layout[1] == "n" else 2], [0],
+                              out_type="f32")).astype(np.float64)
+    want = a[0, ::2] @ np.nan_to_num(b[0], posinf=0.0)
+    finite = np.arange(N) % 3 != 2
+    assert np.array_equal(got[0, ::2][:, finite], want[:, finite])
+    assert np.isnan(got[0, 1::2]).all() and not np.isfinite(got[0, ::2][:, ~finite]).any() and np.isnan(got[1:]).all()
+
+
+def at_odd_address(arr, ty, hip, elements):
+    """`arr` on the device, `elements` behind the start of an allocation, as a tensor over borrowed memory."""
+    flat = np.concatenate([np.zeros(elements, arr.dtype), arr.ravel(), np.zeros(3, arr.dtype)])
+    owner = from_numpy(flat, ty, hip)
+    size = arr.itemsize
+    pointer = Nx.Pointer(kind="local", address=Nx.to_pointer(owner).address + elements * size, data_size=arr.size * size)
+    return Nx.from_pointer(hip, pointer, ty, arr.shape, keep=owner)
+
+
+# every operand form a contraction kernel takes where it lies: whole slabs, a partial slab, rows that are copied anyway, f64
+@pytest.mark.parametrize("ty,M,N,K", [("bf16", 264, 520, 128), ("f16", 128, 512, 1032), ("bf16", 24, 2048, 648), ("f32", 132, 64, 36),
+                                      ("f32", 300, 264, 250), ("s8", 64, 304, 1168), ("s8", 272, 256, 512), ("f64", 130, 66, 48)])
+@pytest.mark.parametrize("layout", ["nn", "nt", "tn", "tt"])
+@pytest.mark.parametrize("behind", [(1, 0), (0, 3), (1, 1)])
+def test_operands_that_begin_off_a_sixteen_byte_address(ty, M, N, K, layout, behind, hip):
+    """Borrowed memory may begin anywhere: the kernels' loads into LDS take their 16 bytes at any address.  Integer-valued
+    operands: every partial sum is a whole number below 2^24, so the product is exact in any order."""
+    rng = np.random.default_rng(seed_of(ty, M, N, K, layout, behind, "odd address"))
+    a, b = rng.integers(-4, 5, size=(M, K)), rng.integers(-4, 5, size=(K, N))
+    la = a if layout[0] == "n" else np.ascontiguousarray(a.T)
+    lb = b if layout[1] == "n" else np.ascontiguousarray(b.T)
+    left, right = at_odd_address(HELD[ty](la), ty, hip, behind[0]), at_odd_address(HELD[ty](lb), ty, hip, behind[1])
+    out = {"s8": "s32", "f64": "f64"}.get(ty, "f32")
+    got = Nx.dot(left, [1 if layout[0] == "n" else 0], right, [0 if layout[1] == "n" else 1], out_type=out)
+    assert np.array_equal(hip.to_numpy(got).astype(np.float64), a.astype(np.float64) @ b.astype(np.float64))
 
 
 @pytest.mark.parametrize("ty,M,N,K", [("f32", 64, 48, 33), ("f32", 64, 64, 4095), ("f32", 16, 16, 1001), ("bf16", 128, 96, 1001), ("f16", 64, 64, 4001)])
@@ -505,7 +579,7 @@ def test_few_outputs_over_a_long_contraction_batched(hip, oracle):
 @pytest.mark.parametrize("layout", ["nn", "nt", "tn", "tt"])
 def test_many_rows_against_a_few_columns(M, N, K, ty, layout, hip, oracle):
     """A layer with a few outputs ([60000, 784] . [784, 10]): tiles of 128 x 32, and a K that is not whole slabs
-    contracted in place with its last part from padded copies.  int8 exact, floats within the accumulation bound,
+    with its partial slab walked in place.  int8 exact, floats within the accumulation bound,
     and every output in its own place (rows and columns off every tile edge)."""
     rng = np.random.default_rng(seed_of(M, N, K, ty, layout, "narrow"))
     if ty == "s8":

@@ -334,3 +334,59 @@ def test_long_slabs_of_short_rows(red, inner, ty, hip):
         assert (np.abs(got - want)[inside] <= keep * np.abs(want)[inside]).all()
     for op, np_op in (("reduce_max", np.max), ("reduce_min", np.min)):
         assert np.array_equal(values(getattr(Nx, op)(t, axes=[0])), np_op(whole, axis=0).astype(np.float64))
+
+
+# The same slabs on everything but plain numbers: one work-group and many, whole and ragged vectors, a cut last row
+@pytest.mark.parametrize("red,inner", [(4096, 10), (4099, 7), (9001, 33), (70001, 100)])
+@pytest.mark.parametrize("ty", ["f16", "bf16", "f32", "f64"])
+@pytest.mark.parametrize("op", ["sum", "product", "reduce_max", "reduce_min", "all", "any"])
+def test_special_values_in_long_slabs_of_short_rows(red, inner, ty, op, hip, oracle):
+    """Columns with an infinity, with infinities of both signs, with an infinity and a zero, with a NaN, of negative zeros
+    only, of ones and minus ones (every finite sum and product of which is exact in any order): the reference's bits."""
+    rng = np.random.default_rng(seed_of("narrow special", red, inner, ty, op))
+    x = rng.choice([1.0, -1.0], size=(red, inner))
+    for c in range(inner):
+        at = np.sort(rng.choice(red, size=3, replace=False))
+        kind = c % 7
+        if kind == 0:
+            x[at[0], c] = np.inf
+        elif kind == 1:
+            x[at[0], c], x[at[1], c] = np.inf, -np.inf
+        elif kind == 2:
+            x[at[0], c], x[at[1], c] = -np.inf, 0.0
+        elif kind == 3:
+            x[at[0], c], x[at[1], c] = np.nan, np.inf
+        elif kind == 4:
+            x[:, c] = -0.0
+        elif kind == 5 and op in ("product", "all"):
+            x[at[0], c], x[at[1], c] = -0.0, -1.0
+        elif kind == 6 and op == "any":
+            x[:, c] = 0.0
+            x[at[0], c] = -0.0 if c % 2 else np.nan
+    x[red - 1, inner - 1] = -1.0  # (the last element of the slab counts)
+    x = x.astype(np.float32 if ty == "bf16" else T.numpy_dtype(T.normalize(ty)))
+    if ty == "bf16":
+        x = (x.view(np.uint32) >> 16).astype(np.uint16)
+    hx, ox = both(x, ty, hip, oracle)
+    assert_bits_equal(getattr(Nx, op)(hx, axes=[0]), getattr(Nx, op)(ox, axes=[0]), f"{op} {ty} [{red}, {inner}]")
+
+
+@pytest.mark.parametrize("red,inner", [(4096, 10), (4099, 7), (9001, 33)])
+@pytest.mark.parametrize("ty", ["s8", "u8", "s16", "u16", "s32", "u32", "s64", "u64"])
+@pytest.mark.parametrize("op", ["sum", "product", "reduce_max", "reduce_min", "all", "any"])
+def test_integer_ends_in_long_slabs_of_short_rows(red, inner, ty, op, hip, oracle):
+    """The whole range of each type, u64 values beyond 2^63 among them; products of odd numbers (they wrap and stay odd)."""
+    rng = np.random.default_rng(seed_of("narrow ends", red, inner, ty, op))
+    dtype = T.numpy_dtype(T.normalize(ty))
+    info = np.iinfo(dtype)
+    x = rng.integers(info.min, info.max, size=(red, inner), dtype=dtype, endpoint=True)
+    if op == "product":
+        x |= np.ones((), dtype)
+    if op == "all":
+        x[x == 0] = 1
+        x[red // 3, ::2] = 0
+    if op == "any":
+        x[:] = 0
+        x[red - 1, ::3] = info.max
+    hx, ox = both(x, ty, hip, oracle)
+    assert_bits_equal(getattr(Nx, op)(hx, axes=[0]), getattr(Nx, op)(ox, axes=[0]), f"{op} {ty} [{red}, {inner}]")
