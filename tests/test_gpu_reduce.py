@@ -371,7 +371,7 @@ def test_special_values_in_long_slabs_of_short_rows(red, inner, ty, op, hip, ora
     assert_bits_equal(getattr(Nx, op)(hx, axes=[0]), getattr(Nx, op)(ox, axes=[0]), f"{op} {ty} [{red}, {inner}]")
 
 
-@pytest.mark.parametrize("red,inner", [(4096, 10), (4099, 7), (9001, 33)])
+@pytest.mark.parametrize("red,inner", [(4096, 10), (4099, 7), (9001, 33), (9001, 129)])
 @pytest.mark.parametrize("ty", ["s8", "u8", "s16", "u16", "s32", "u32", "s64", "u64"])
 @pytest.mark.parametrize("op", ["sum", "product", "reduce_max", "reduce_min", "all", "any"])
 def test_integer_ends_in_long_slabs_of_short_rows(red, inner, ty, op, hip, oracle):
