@@ -716,7 +716,7 @@ __device__ __forceinline__ void wait_vmcnt() {  // s_waitcnt vmcnt(N), other cou
   __builtin_amdgcn_s_waitcnt(0x0F70 | (N & 15) | ((N >> 4) << 14));
 }
 
-template <int DT, int WM, int WN, int TM, int TN, bool L_KIN, bool R_KIN, int NSTAGE = 2, bool EARLY = false>
+template <int DT, int WM, int WN, int TM, int TN, bool L_KIN, bool R_KIN, int NSTAGE = 2>
 // (f64: at least two waves per SIMD, i.e. at most 256 registers and all of them VGPRs.  With the 512 that a work-group
 // of four waves may have, the compiler keeps some accumulators in AGPRs and moves them to and fro inside the K loop --
 // 128 copies per slab beside 64 MFMAs, each waiting for the MFMA that last wrote its source: 2048^3 404 -> 329 us,
@@ -842,20 +842,6 @@ gemm_pipelined_kernel(GemmArgs a) {
 
   constexpr bool ALL_DMA = (L_KIN || L_TR) && (R_KIN || R_TR);
   static_assert(NSTAGE == 2 || ALL_DMA, "register-staged operands need the two-stage walk");
-  // EARLY (two stages, every operand by direct-to-LDS loads): the requests of a slab start right
-  // behind the barrier that frees its stage -- in the POST steps that follow the barrier of the slab
-  // before the previous one's successor -- instead of at the next slab's first step, one
-  // instruction per step (l in even, r in odd virtual steps u = 0, 1, ..): the last request then
-  // has POST more steps to land before the barrier that publishes the slab.
-  constexpr int POST = STEPS - 1 - BAR;
-  static_assert(!EARLY || (NSTAGE == 2 && ALL_DMA), "early requests need two stages of direct-to-LDS operands");
-  auto issue_early = [&](int u, int stage, int64_t kbyte0) {
-    unsigned char *sA = smem + stage * STAGE, *sB = sA + BM * SLAB;
-    if constexpr (L_KIN) lload.issue_at(u, 2 * KInnerLoader<BM, NW>::PER, 0, 0, kbyte0, sA);
-    else if constexpr (L_TR) ltr.issue_at(u, 2 * KOuterDmaLoader<TR_ES, L_TR ? BM : 256 * NW, NW>::PER, 0, 0, kbyte0 / ES, a.ld_l, sA);
-    if constexpr (R_KIN) rload.issue_at(u, 2 * KInnerLoader<BN, NW>::PER, 1, 0, kbyte0, sB);
-    else if constexpr (R_TR) rtr.issue_at(u, 2 * KOuterDmaLoader<TR_ES, R_TR ? BN : 256 * NW, NW>::PER, 1, 0, kbyte0 / ES, a.ld_r, sB);
-  };
   // AHEAD (an operand staged through registers): a slab's requests all go out right behind the barrier that frees its
   // stage, a whole slab of MFMA work before they are committed.  Requested at the first step of the slab before and
   // committed at step BAR they had five eighths of one, 0.5 us of f32 work, and with a work-group per CU that was
@@ -877,12 +863,6 @@ gemm_pipelined_kernel(GemmArgs a) {
   __syncthreads();
   if constexpr (AHEAD)
     if (1 < nslab) issue(1, SLAB + k_shift);
-  if constexpr (EARLY) {  // the first requests of slab 1 (what the steps behind a barrier would have issued)
-    if (1 < nslab) {
-#pragma unroll
-      for (int u = 0; u < POST; u++) issue_early(u, 1, SLAB + k_shift);
-    }
-  }
   v4i fa[2][TM16], fb[RING];
 #pragma unroll
   for (int i = 0; i < TM16; i++) fa[0][i] = read_l(smem, 0, i);
@@ -917,11 +897,7 @@ gemm_pipelined_kernel(GemmArgs a) {
         for (int i = 0; i < TM16; i++)
           if (i >= d * TM16 / DIST && i < (d + 1) * TM16 / DIST) fa[0][i] = read_l(nxt, 0, i);
       }
-      if constexpr (EARLY) {
-        if (t > BAR) {
-          if (s + 2 < nslab) issue_early(t - BAR - 1, s % NSTAGE, (int64_t)(s + 2) * SLAB + k_shift);
-        } else if (request) issue_early(t + POST, req_stage, req_kbyte);
-      } else if (!AHEAD && request && t <= BAR) issue_step(t, req_stage, req_kbyte);
+      if (!AHEAD && request && t <= BAR) issue_step(t, req_stage, req_kbyte);
 #pragma unroll
       for (int i = 0; i < TM16; i++) Mma16<DT>::step(acc[i][j], fb[t % RING], fa[ks & 1][i]);
       __builtin_amdgcn_s_setprio(0);
