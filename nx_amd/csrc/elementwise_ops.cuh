@@ -198,11 +198,14 @@ __device__ __forceinline__ double fma_const(double p, double w, double c) {
 // The same for an f32 operand (the f32 class of the kernels).  Bound by f64 instructions, each of which costs a SIMD as
 // much as an f32 one; the form above takes about 190, most of them in the library's log, which serves every double, and
 // in separate products and sums.  Here the logarithm is written for what can occur, y = (1 - x)(1 + x) in [2^-23, 1]:
-// y = 2^k m with m in [1/sqrt(2), sqrt(2)), log m = 2 atanh(s), s = (m - 1) / (m + 1), the series of atanh in z = s^2
+// y = 2^k m with m in [1/sqrt(2), sqrt(2)), found by adding to the high word (as the logarithms of the FreeBSD and musl math
+// libraries do), log m = 2 atanh(s), s = (m - 1) / (m + 1), the series of atanh in z = s^2
 // beyond its first term as a polynomial of degree 6 (interpolated at the Chebyshev points of z in [0, 0.02945]; its
 // error is below 2^-57 of log m), the quotient from v_rcp_f64 and two Newton steps; the polynomials are fused
-// multiply-adds.  The polynomials' argument w - 2.5 has one rounding of its own size as above, p one less per step: both
-// stay nine digits below the f32 result.  No branch but the rare one: w >= 5 is |x| > 0.99662, and everything that is
+// multiply-adds.  The polynomials' argument w - 2.5 has one rounding of its own size as above, p one less per step: against
+// the same polynomials in 80 bits either form is within 3.6e-16 (2^26 arguments, half of them next to +-1, the forms written
+// out for the CPU; none of them rounded to another f32 by either).  So a result is the reference's but where the f64 value
+// lies that close to halfway between two floats: the last bit, about once in 2^25.  No branch but the rare one: w >= 5 is |x| > 0.99662, and everything that is
 // not inside (-1, 1) goes the same way.  2^26 normal samples, the chain behind the cipher: 320 us by the form above,
 // 195 with this log and the compiler's v_fmac, 151 as it is.
 __device__ __forceinline__ float erf_inv_f32(float xf) {
