@@ -11,8 +11,8 @@ namespace hipnx {
 // Bound by memory: a lane takes 16 bytes of the flat output, whatever rows they lie in, and the same of the dense operand;
 // the other operand comes from a row or a column that the caches hold.  (The general kernel does the same with the
 // operands' forms, strides and outer axes as run-time arguments and 64-bit offsets, some hundred instructions per
-// vector: f32 [671088, 100] less
-// a row 122 us, now 78 (6.9 TB/s); times a row 129, now 78.)
+// vector: f32 [671088, 100] less a row 132 us back to back, now 89 (6.0 TB/s); 122 and 77 right behind a pass that read
+// the table.)
 //   L_DENSE: the left operand is the dense one.  PER_ROW: the other holds one value per row, `step` elements apart.
 template <int OP, int FIX, bool L_DENSE, bool PER_ROW>
 __global__ void __launch_bounds__(BLOCK)
