@@ -446,9 +446,9 @@ __device__ __forceinline__ float as_stored(CT v, int dt) {
 }
 
 // The walk of a row: lane l takes the vectors l, l + P::tpr, ... -- P::nv of them, the last one if it lies in the row,
-// when the program keeps vectors from one stage to the next (P::nv > 0), any number otherwise.  The trips are written out
-// by recursion: what is kept is indexed by the trip and has to stay in registers.  (As a loop with an unroll pragma the
-// compiler left it rolled for 16 trips and turned the index into chains of selects, 16 of them per element.)
+// when the program keeps vectors from one stage to the next (P::nv > 0), any number otherwise.  Where it pays (fused_rtc.hip)
+// the trips are written out by recursion: what is kept is indexed by the trip and has to stay in registers.  (As a loop with an
+// unroll pragma the compiler leaves 16 light trips rolled and turns the index into chains of selects, 16 of them per element.)
 template <typename P, int IT, typename F>
 __device__ __forceinline__ void trips_from(int lane, int64_t cols, F &&body) {
   if constexpr (IT < P::nv) {
@@ -460,8 +460,14 @@ __device__ __forceinline__ void trips_from(int lane, int64_t cols, F &&body) {
 }
 template <typename P, typename F>
 __device__ __forceinline__ void for_each_vector(int lane, int64_t cols, F &&body) {
-  if constexpr (P::nv > 0) trips_from<P, 0>(lane, cols, body);
-  else
+  if constexpr (P::nv > 0 && P::written_out) trips_from<P, 0>(lane, cols, body);
+  else if constexpr (P::nv > 0) {
+#pragma unroll
+    for (int it = 0; it < P::nv; it++) {
+      const int64_t k = ((int64_t)lane + (int64_t)it * P::tpr) * FE;
+      if (k < cols) body(k, it);
+    }
+  } else
     for (int64_t k = (int64_t)lane * FE; k < cols; k += (int64_t)P::tpr * FE) body(k, 0);
 }
 

@@ -52,19 +52,55 @@ static void list_of(std::string &s, const char *name, const char *type, int n, c
 struct Keeps {
   int trips = 0;        // vectors of a lane along a row, 0 when nothing is kept
   bool carries = false;
+  bool written_out = false;  // a lane's trips as straight code (fused_ops.cuh, for_each_vector)
   int held = -1;        // the input, and the first stage that reads it
   int held_stage = -1;
 };
+// What a function costs a trip that is written out: the branches it has per element and its code for a vector of eight in KB,
+// read off the compiler's output (the others: no branch, 1 KB or less).
+struct Cost {
+  int branches, kbytes;
+};
+static Cost cost_of(const hipnx_fused_instr &q) {
+  if (q.kind == HIPNX_FUSED_UNARY) switch (q.op) {
+    case HIPNX_TANH: return {1, 2};
+    case HIPNX_ERF: return {1, 3};
+    case HIPNX_SIN: case HIPNX_COS: case HIPNX_TAN: return {2, 7};
+    case HIPNX_ERF_INV: return {4, 9};
+    case HIPNX_SIGMOID: case HIPNX_EXPM1: case HIPNX_RSQRT: return {0, 2};
+    case HIPNX_ERFC: return {0, 3};
+    case HIPNX_SINH: case HIPNX_COSH: return {0, 4};
+    case HIPNX_LOG1P: case HIPNX_ASINH: case HIPNX_ACOSH: case HIPNX_ATANH: return {0, 5};
+  }
+  if (q.kind == HIPNX_FUSED_BINARY) switch (q.op) {
+    case HIPNX_REMAINDER: return {3, 2};
+    case HIPNX_ATAN2: return {0, 3};
+    case HIPNX_POW: return {0, 7};
+  }
+  return {0, 0};
+}
+
 static Keeps what_is_kept(const FusedArgs &a) {
   Keeps k;
+  bool stages = false;
+  for (int i = 0; i < a.n_instr; i++) stages |= a.ins[i].kind == HIPNX_FUSED_ROW_REDUCE;
   const int tpr = a.cols > 4096 ? FBLOCK : WAVE;
   const int64_t trips = (a.cols + tpr * FE - 1) / (tpr * FE);
+  if (!stages || trips > 16) return k;  // (the host refuses longer rows for programs that carry values)
   // which stages read an input along the row, and up to which stage a carried value is waiting to be read
   unsigned reads[HIPNX_FUSED_MAX_INPUTS] = {};
   int stage = 0, carried_from = -1;
-  bool stages = false;
+  bool on_stat = false, rounds = false, rounds_f16 = false;
+  Cost trip = {0, 0};
   for (int i = 0; i < a.n_instr; i++) {
     const hipnx_fused_instr &q = a.ins[i];
+    if (!on_stat) {
+      const Cost c = cost_of(q);
+      trip.branches += c.branches, trip.kbytes += c.kbytes;
+      rounds_f16 |= q.dt == HIPNX_F16;
+      rounds |= q.dt == HIPNX_F16 || q.dt == HIPNX_BF16;
+    }
+    on_stat = q.kind == HIPNX_FUSED_ROW_REDUCE || (on_stat && q.kind != HIPNX_FUSED_ROW_STAT);
     // (a SET or BINARY on integers reads the words as they are in memory; a SELECT reads floats whatever its flags:
     // the cases of fetch_static)
     const bool raw = (q.flags & HIPNX_FUSED_FLAG_INT) != 0 && q.kind != HIPNX_FUSED_SELECT;
@@ -74,12 +110,22 @@ static Keeps what_is_kept(const FusedArgs &a) {
     };
     if (q.kind == HIPNX_FUSED_SET || q.kind == HIPNX_FUSED_BINARY || q.kind == HIPNX_FUSED_SELECT) source(q.src, q.arg);
     if (q.kind == HIPNX_FUSED_SELECT) source(q.src2, q.arg2);
-    if (q.kind == HIPNX_FUSED_ROW_REDUCE) stages = true;
     if (q.kind == HIPNX_FUSED_ROW_STAT) stage++;
   }
-  if (!stages || trips > 16) return k;  // (the host refuses longer rows for programs that carry values)
   k.carries = carried_from >= 0;
   if (k.carries) k.trips = (int)trips;
+  // Written-out trips gain where the compiler can lay one trip's loads and arithmetic over the next's, and hold the row for
+  // one read (a layer norm of sigmoids, f32 4096 x 4096: 57 us as a loop, 38 written out).  A branch per element ends
+  // that, and the straight code then costs its own fetching.  f32, loop / written out: tanh in two stages, 3 trips 36 / 30 us,
+  // 4 trips 34 / 33, 6 trips 35 / 40, 8 trips 39 / 56; erf 3 trips 39 / 40, 4 trips 39 / 44, 8 trips 44 / 79; sin 8 trips 38 / 104.
+  // With 16-bit roundings there is less to gain: tanh in one stage, bf16, 2 trips 26 / 28, 4 trips 26 / 29; and in f16, whose
+  // conversions are instructions too, nothing once a function is long (atan2, 2 to 16 trips, 1 to 8 % slower).
+  // And the code has to stay near what the instruction cache holds (64 KB for two CUs): pow in two stages, 16 trips (240 KB),
+  // 154 / 172 us, and 2.4 s to compile instead of 0.5.
+  if (trip.branches * trips > (rounds ? 1 : 6) || trip.kbytes * trips > 96 || (rounds_f16 && trip.kbytes > 0)) return k;
+  // Carried values alone gain only where the compiler leaves the loop over them rolled: f32, logarithms, 14 trips 37 / 43 us,
+  // 16 trips 51 / 46; square roots, 15 trips 32 / 35, 16 trips 40 / 37.
+  k.written_out = k.carries && trips > 15;
   for (int in = 0; in < a.n_inputs; in++) {
     if (!(reads[in] & (reads[in] - 1)) || k.held >= 0) continue;  // one stage reads it: nothing to gain
     // a lane has room for 16 vectors (128 of its registers): an input that is still read once a carried value is there
@@ -87,6 +133,7 @@ static Keeps what_is_kept(const FusedArgs &a) {
     const int last = 31 - __builtin_clz(reads[in]);
     if (carried_from >= 0 && last > carried_from && trips > 8) continue;
     k.trips = (int)trips;
+    k.written_out = true;
     k.held = in;
     k.held_stage = __builtin_ctz(reads[in]);
   }
@@ -145,7 +192,7 @@ static std::string make_source(const FusedArgs &a, const Keeps &keeps, int reduc
   list_of(s, "seg_red", "int", (int)seg_red.size(), [&](int k) { return std::to_string(seg_red[k]); });
   list_of(s, "seg_save", "int", (int)seg_save.size(), [&](int k) { return std::to_string(seg_save[k]); });
   auto keeping = [](const char *p, const Keeps &k) {
-    return std::string("struct ") + p + " : Program {\n  static constexpr int nv = " + std::to_string(k.trips) + ", held = " + std::to_string(k.held) +
+    return std::string("struct ") + p + " : Program {\n  static constexpr int nv = " + std::to_string(k.trips) + ", written_out = " + std::to_string(k.written_out) + ", held = " + std::to_string(k.held) +
            ", held_stage = " + std::to_string(k.held_stage) + ";\n};\n";
   };
   auto kernel = [](const std::string &called) {

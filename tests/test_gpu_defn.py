@@ -890,6 +890,29 @@ def test_a_program_that_holds_its_row_is_captured_at_other_lengths(warmed, other
         assert_bits_equal(defn.compile(fun, x, fuse="compiled")(x), defn.compile(fun, x)(x), f"{shape}")
 
 
+# Functions with a branch, long ones and short ones on either side of where a program's trips are written out: one, two, three, four
+# vectors a lane; a block per row with four, fifteen (values carried in a loop) and sixteen
+@pytest.mark.parametrize("ty", ["f32", "bf16", "f16"])
+@pytest.mark.parametrize("shape", [(9, 512), (9, 1024), (5, 1536), (5, 2048), (3, 4096), (3, 8192), (3, 30720), (2, 32000)])
+@pytest.mark.parametrize("name", ["tanh", "erf", "sin", "pow", "atan2", "log", "sigmoid"])
+def test_row_stages_of_costly_functions_are_bit_identical(name, shape, ty, hip):
+    function = {"pow": lambda x: Nx.pow(Nx.add(Nx.abs(x), 0.5), 1.25), "atan2": lambda x: Nx.atan2(x, 0.75),
+                "log": lambda x: Nx.log(Nx.add(Nx.abs(x), 1.0))}.get(name, getattr(Nx, name, None))
+
+    def held(x):  # the function again in every stage
+        z = function(x)
+        return Nx.subtract(z, Nx.log(Nx.sum(Nx.exp(Nx.subtract(z, Nx.reduce_max(z, axes=[-1], keep_axes=True))), axes=[-1], keep_axes=True)))
+
+    def carried(x):
+        z = function(x)
+        return Nx.divide(z, Nx.add(Nx.sum(z, axes=[-1], keep_axes=True), 2.0))
+    x = rand_float(np.random.default_rng(seed_of(name, shape, ty)), ty, shape, hip)
+    for fun in (held, carried):
+        planned = defn.compile(fun, x, fuse="compiled")
+        assert type(planned.roots[0].data.args[0]).__name__ == "_RowCluster"
+        assert_bits_equal(planned(x), defn.compile(fun, x)(x), f"{name} {shape} {ty}")
+
+
 def test_rows_too_long_for_carried_values_are_read_again(hip):
     x = rand_float(np.random.default_rng(7), "f32", (2048, 32776), hip)
     planned = defn.compile(softmax_rows, x, fuse="compiled")
