@@ -434,7 +434,7 @@ __device__ __forceinline__ void fused_reduce_rows_body() {
 // TPR = WAVE (same lanes, same order, same reducer), and a statistic is carried on as the value a
 // store to its type and a load would give -- so the result equals the separate kernels', bit for bit.
 // A row that a lane's registers hold (P::held: an input that more than one stage reads, at most 16 vectors a lane) is read
-// from memory once; a longer one is read again by every stage.  Bound by memory: f32 softmax of
+// from memory once; a longer one, and one of a program walked in a loop, is read again by every stage.  Bound by memory: f32 softmax of
 // 8192 x 32000 in 381 us (5.5 TB/s; 600 with a read per stage), f32 layer norm of 16384 x 1024 in 25 us (5.4 TB/s).
 template <typename CT>
 __device__ __forceinline__ float as_stored(CT v, int dt) {

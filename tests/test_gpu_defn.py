@@ -890,11 +890,11 @@ def test_a_program_that_holds_its_row_is_captured_at_other_lengths(warmed, other
         assert_bits_equal(defn.compile(fun, x, fuse="compiled")(x), defn.compile(fun, x)(x), f"{shape}")
 
 
-# Functions with a branch, long ones and short ones on either side of where a program's trips are written out: one, two, three, four
+# Functions with a branch, long ones and short ones on either side of where a program's trips are written out: one, two, four
 # vectors a lane; a block per row with four, fifteen (values carried in a loop) and sixteen
 @pytest.mark.parametrize("ty", ["f32", "bf16", "f16"])
-@pytest.mark.parametrize("shape", [(9, 512), (9, 1024), (5, 1536), (5, 2048), (3, 4096), (3, 8192), (3, 30720), (2, 32000)])
-@pytest.mark.parametrize("name", ["tanh", "erf", "sin", "pow", "atan2", "log", "sigmoid"])
+@pytest.mark.parametrize("shape", [(9, 512), (9, 1024), (5, 2048), (3, 8192), (3, 30720), (2, 32000)])
+@pytest.mark.parametrize("name", ["tanh", "sin", "pow", "atan2", "log"])
 def test_row_stages_of_costly_functions_are_bit_identical(name, shape, ty, hip):
     function = {"pow": lambda x: Nx.pow(Nx.add(Nx.abs(x), 0.5), 1.25), "atan2": lambda x: Nx.atan2(x, 0.75),
                 "log": lambda x: Nx.log(Nx.add(Nx.abs(x), 1.0))}.get(name, getattr(Nx, name, None))
