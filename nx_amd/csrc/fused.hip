@@ -175,7 +175,7 @@ static void launch_fused_combine(const hipnx_ctx *ctx, const FusedArgs &a, int r
 static bool narrow(int dt) { return dt == HIPNX_BF16 || dt == HIPNX_F16 || dt == HIPNX_F32; }
 
 // fused_rtc.hip
-int fused_launch_compiled(hipnx_ctx *ctx, const FusedArgs &a, int reduce_op, bool block_per_row, unsigned grid, bool *done);
+int fused_launch_compiled(hipnx_ctx *ctx, const FusedArgs &a, int reduce_op, bool block_per_row, bool walk, unsigned grid, bool *done);
 
 }  // namespace hipnx
 
@@ -310,8 +310,24 @@ extern "C" int hipnx_fused_elementwise(hipnx_ctx *ctx, int n_instr, const hipnx_
   if (on_stat) return set_error(HIPNX_EINVAL, "fused: the program ends inside a stage's work on its statistic");
   if (n_stats && (reduce_op != -1 || cols == 0))
     return set_error(HIPNX_EUNSUPPORTED, "fused: stages take non-empty rows and no reduction of the result");
+  // rows that are not whole vectors are taken row by row in a compiled kernel (fused_ops.cuh, row_walk), a reduction of their
+  // values as a stage whose statistic is the result; but a flat index space may end in a partial vector there
+  const bool ragged = cols % 8 != 0 && ctx->fused_mode == HIPNX_FUSED_COMPILED && (rows != 1 || n_stats || reduce_op != -1);
+  if (ragged && reduce_op != -1) {
+    if (n_instr + 2 > HIPNX_FUSED_MAX_INSTR || !narrow(prog[n_instr - 1].dt) || !narrow(out_dt))
+      return set_error(HIPNX_EUNSUPPORTED, "fused: a reduction of rows that are not whole vectors after so long a program, or of a non-float value");
+    hipnx_fused_instr q{};
+    q.kind = HIPNX_FUSED_ROW_REDUCE, q.op = (uint8_t)reduce_op, q.dt = (uint8_t)out_dt;
+    a.ins[a.n_instr++] = q;
+    q.kind = HIPNX_FUSED_ROW_STAT, q.op = 0, q.flags = HIPNX_FUSED_FLAG_RESULT;
+    a.ins[a.n_instr++] = q;
+    reduce_op = -1;
+    row_result = true;
+    n_stats = 1;
+  }
+  const bool walk = n_stats || ragged;
   // a few very long rows are split into segments by the separate reduction, whose order the stages follow: not here
-  if (n_stats) {
+  if (walk) {
     int would_be = 1;
     int64_t of_length = cols;
     plan_row_segments(ctx, rows, cols, &would_be, &of_length);
@@ -321,8 +337,8 @@ extern "C" int hipnx_fused_elementwise(hipnx_ctx *ctx, int n_instr, const hipnx_
     return set_error(HIPNX_EUNSUPPORTED, "fused: rows too long to keep a stage's values in registers");
   const int64_t n = rows * cols;
   if (cols % 8 != 0) {
-    // a flat index space (one row) may end in a partial vector -- in a compiled kernel, which handles it
-    if (rows != 1 || reduce_op != -1 || n_stats || ctx->fused_mode != HIPNX_FUSED_COMPILED)
+    // (a flat index space, one row, may end in a partial vector)
+    if (ctx->fused_mode != HIPNX_FUSED_COMPILED)
       return set_error(HIPNX_EUNSUPPORTED, "fused: the row length is not a multiple of 8");
     needs_compiled = true;
   }
@@ -334,7 +350,7 @@ extern "C" int hipnx_fused_elementwise(hipnx_ctx *ctx, int n_instr, const hipnx_
     if (in_row_strides[k] < 0 || (in_col_strides[k] != 0 && in_col_strides[k] != 1))
       return set_error(HIPNX_EINVAL, "fused: input %d has strides (%lld, %d)", k, (long long)in_row_strides[k], in_col_strides[k]);
     // rows of an operand read with vector loads must start on a vector boundary
-    if (in_col_strides[k] == 1 && rows > 1 && in_row_strides[k] % 8 != 0)
+    if (!ragged && in_col_strides[k] == 1 && rows > 1 && in_row_strides[k] % 8 != 0)
       return set_error(HIPNX_EUNSUPPORTED, "fused: rows of input %d are not vector-aligned", k);
     const uint64_t extent = n == 0 ? 0 : (uint64_t)((rows - 1) * in_row_strides[k] + (cols - 1) * in_col_strides[k] + 1);
     if (int st = check_buf(ctx, inputs[k], extent * sz, "fused input")) return st;
@@ -377,19 +393,19 @@ extern "C" int hipnx_fused_elementwise(hipnx_ctx *ctx, int n_instr, const hipnx_
   } release{ctx, partials, partials_cap};
   if (ctx->fused_mode == HIPNX_FUSED_COMPILED) {
     // the same grids as the interpreting kernels below
-    const bool block_per_row = (reduce_op != -1 || n_stats) && a.cols > 4096;
-    int64_t grid = n_stats ? (block_per_row ? a.rows : (a.rows + FBLOCK / WAVE - 1) / (FBLOCK / WAVE))  // a wave or a block per row
+    const bool block_per_row = (reduce_op != -1 || walk) && a.cols > 4096;
+    int64_t grid = walk ? (block_per_row ? a.rows : (a.rows + FBLOCK / WAVE - 1) / (FBLOCK / WAVE))  // a wave or a block per row
                    : reduce_op == -1 ? (a.nvec + (int64_t)FBLOCK * FV - 1) / ((int64_t)FBLOCK * FV)
                    : block_per_row ? a.rows * a.nseg : (a.rows + FBLOCK / WAVE - 1) / (FBLOCK / WAVE);
     // a launch may hold at most 2^32 - 1 lanes: the element-wise kernel loops over what a capped grid leaves, the row
     // kernels take one row (or wave of rows) per work-group and leave larger inputs to the separate callbacks
     const int64_t max_grid = ((1ll << 32) - 1) / FBLOCK;
     if (grid > max_grid) {
-      if (n_stats || reduce_op != -1) return set_error(HIPNX_EUNSUPPORTED, "fused: more rows than one launch holds");
+      if (walk || reduce_op != -1) return set_error(HIPNX_EUNSUPPORTED, "fused: more rows than one launch holds");
       grid = max_grid;
     }
     bool done = false;
-    if (int st = fused_launch_compiled(ctx, a, reduce_op, block_per_row, (unsigned)grid, &done)) return st;
+    if (int st = fused_launch_compiled(ctx, a, reduce_op, block_per_row, walk, (unsigned)grid, &done)) return st;
     if (done) {
       if (a.nseg > 1) {
         launch_fused_combine(ctx, a, reduce_op);

@@ -82,7 +82,8 @@ __device__ __forceinline__ float element_to_f32(uint32_t bits, int dt) {
 }
 
 // input k (element type dt, column stride cs) for the lane's FV vectors: all loads are requested,
-// then converted
+// then converted.  UNAL: the vectors begin at any element (rows that are not whole vectors): the loads claim no alignment.
+template <bool UNAL = false>
 __device__ __forceinline__ void load_input_as(KernArgs a, int k, int dt, int cs, const int64_t (&row)[FV],
                                               const int64_t (&col)[FV], Vecs &dst) {
   const int esz = (dt == HIPNX_U8 || dt == HIPNX_S8) ? 1 : (dt == HIPNX_U32 || dt == HIPNX_S32 || dt == HIPNX_F32) ? 4 : 2;
@@ -96,6 +97,10 @@ __device__ __forceinline__ void load_input_as(KernArgs a, int k, int dt, int cs,
       w[u][0] = esz == 4 ? *reinterpret_cast<const uint32_t *>(p)
                 : esz == 2 ? (uint32_t)*reinterpret_cast<const uint16_t *>(p)
                            : (uint32_t)*reinterpret_cast<const uint8_t *>(p);
+    } else if constexpr (UNAL) {
+      if (esz == 4) __builtin_memcpy(w[u], p, FE * 4);
+      else if (esz == 2) __builtin_memcpy(w[u], p, FE * 2);
+      else __builtin_memcpy(w[u], p, FE);
     } else if (esz == 4) {
       const uint4 lo = *reinterpret_cast<const uint4 *>(p), hi = *reinterpret_cast<const uint4 *>(p + 16);
       w[u][0] = lo.x; w[u][1] = lo.y; w[u][2] = lo.z; w[u][3] = lo.w;
@@ -193,7 +198,7 @@ __device__ __forceinline__ void fetch_static(KernArgs a, const Saved &S, const R
       for (int e = 0; e < FE; e++) dst[u][e] = stats[ARG];
   } else if constexpr (SRC == HIPNX_FUSED_SRC_INPUT) {
     // RAW: the words of a 4-byte input as they are (what the f32 path does with its bits)
-    if (valid == FE) load_input_as(a, ARG, RAW ? (int)HIPNX_F32 : P::in_dt[ARG], P::in_cs[ARG], row, col, dst);
+    if (valid == FE) load_input_as<P::unal>(a, ARG, RAW ? (int)HIPNX_F32 : P::in_dt[ARG], P::in_cs[ARG], row, col, dst);
     else load_input_tail(a, ARG, RAW ? (int)HIPNX_F32 : P::in_dt[ARG], P::in_cs[ARG], row, col, valid, dst);
   } else if constexpr (SRC == HIPNX_FUSED_SRC_SAVED) {
     copy_vecs(dst, S.s[ARG]);
@@ -429,9 +434,9 @@ __device__ __forceinline__ void fused_reduce_rows_body() {
 // ---- several stages over the same rows in one kernel ------------------------------------------------
 // A program with HIPNX_FUSED_ROW_REDUCE markers is a sequence of stages: each stage but the last
 // ends in a reduction of its value along the row, and later stages read that row statistic as an
-// operand (softmax: the row maximum, then the sum of the exponentials, then the division).  One wave
-// takes a row through all stages; a stage walks the row exactly as fused_reduce_rows_body does with
-// TPR = WAVE (same lanes, same order, same reducer), and a statistic is carried on as the value a
+// operand (softmax: the row maximum, then the sum of the exponentials, then the division).  A group of
+// lanes takes a row through all stages; a stage walks the row exactly as the separate reduction does
+// (same lanes, same order, same reducer), and a statistic is carried on as the value a
 // store to its type and a load would give -- so the result equals the separate kernels', bit for bit.
 // A row that a lane's registers hold (P::held: an input that more than one stage reads, at most 16 vectors a lane) is read
 // from memory once; a longer one, and one of a program walked in a loop, is read again by every stage.  Bound by memory: f32 softmax of
@@ -445,37 +450,75 @@ __device__ __forceinline__ float as_stored(CT v, int dt) {
   }
 }
 
-// The walk of a row: lane l takes the vectors l, l + P::tpr, ... -- P::nv of them, the last one if it lies in the row,
-// when the program keeps vectors from one stage to the next (P::nv > 0), any number otherwise.  Where it pays (fused_rtc.hip)
+// How the lanes of a row share it (P::form).  In every form a lane meets its elements in the order in which the separate
+// reduction of rows of that length folds them (reduce_rows_kernel and its short-row forms).
+//   ROW_WHOLE: rows of whole vectors; lane l takes the vectors l, l + tpr, ...
+//   ROW_LANE: rows of at most 16 elements; a lane takes a row (tpr = 1): its vectors, then the P::tail elements behind them.
+//   ROW_GROUP: rows of 17 to 256 elements that are not whole vectors; 8, 16 or 32 lanes, so that each has one vector at most;
+//     the elements behind the last vector one per lane.
+//   ROW_RAGGED: longer rows that are not whole vectors; the elements up to a vector boundary of the BUFFER one per lane, whole
+//     aligned vectors as ROW_WHOLE, the elements behind them one per lane.
+// Rows off the vector grid went node by node before, every intermediate through memory: f32 layer norm of 26248 x 185
+// 106 us, bf16 softmax of 247650 x 178 160 us.
+enum { ROW_WHOLE, ROW_LANE, ROW_GROUP, ROW_RAGGED };
+
+template <int N>
+struct Elements {
+  static constexpr int n = N;
+};
+
+struct RowWalk {
+  int64_t begin, end;  // the vectors of the row, all its lanes': columns [begin, end)
+  int64_t cols;
+};
+template <typename P>
+__device__ __forceinline__ RowWalk row_walk(int64_t r, int64_t cols) {
+  if constexpr (P::form == ROW_RAGGED) {
+    const int64_t head = (FE - r * cols % FE) % FE;
+    return {head, head + (cols - head) / FE * FE, cols};
+  } else if constexpr (P::form == ROW_GROUP) return {0, cols / FE * FE, cols};
+  else return {0, cols, cols};
+}
+
+// A lane's part of a row: body(first column, what is kept of these elements, Elements<how many>).  Whole vectors are the
+// vectors l, l + P::tpr, ... -- P::nv of them, the last one if it lies in the row, when the program keeps vectors from one
+// stage to the next (P::nv > 0), any number otherwise.  Where it pays (fused_rtc.hip)
 // the trips are written out by recursion: what is kept is indexed by the trip and has to stay in registers.  (As a loop with an
 // unroll pragma the compiler leaves 16 light trips rolled and turns the index into chains of selects, 16 of them per element.)
 template <typename P, int IT, typename F>
-__device__ __forceinline__ void trips_from(int lane, int64_t cols, F &&body) {
+__device__ __forceinline__ void trips_from(int lane, const RowWalk &w, RowVector *kept, F &&body) {
   if constexpr (IT < P::nv) {
-    const int64_t k = ((int64_t)lane + (int64_t)IT * P::tpr) * FE;
-    if constexpr (IT + 1 < P::nv) body(k, IT);
-    else if (k < cols) body(k, IT);
-    trips_from<P, IT + 1>(lane, cols, body);
+    const int64_t k = w.begin + ((int64_t)lane + (int64_t)IT * P::tpr) * FE;
+    if constexpr (IT + 1 < P::nv || P::form == ROW_LANE) body(k, kept[IT], Elements<FE>{});
+    else if (k < w.end) body(k, kept[IT], Elements<FE>{});
+    trips_from<P, IT + 1>(lane, w, kept, body);
   }
 }
+// `kept`: of the vectors, then of the element in front of them, then of those behind them
 template <typename P, typename F>
-__device__ __forceinline__ void for_each_vector(int lane, int64_t cols, F &&body) {
-  if constexpr (P::nv > 0 && P::written_out) trips_from<P, 0>(lane, cols, body);
+__device__ __forceinline__ void for_each_vector(int lane, const RowWalk &w, RowVector *kept, F &&body) {
+  constexpr int own = P::nv > 0 ? P::nv : 1;
+  if constexpr (P::form == ROW_RAGGED)
+    if (lane < w.begin) body((int64_t)lane, kept[own], Elements<1>{});
+  if constexpr (P::nv > 0 && (P::written_out || P::form == ROW_LANE)) trips_from<P, 0>(lane, w, kept, body);
   else if constexpr (P::nv > 0) {
 #pragma unroll
     for (int it = 0; it < P::nv; it++) {
-      const int64_t k = ((int64_t)lane + (int64_t)it * P::tpr) * FE;
-      if (k < cols) body(k, it);
+      const int64_t k = w.begin + ((int64_t)lane + (int64_t)it * P::tpr) * FE;
+      if (k < w.end) body(k, kept[it], Elements<FE>{});
     }
-  } else
-    for (int64_t k = (int64_t)lane * FE; k < cols; k += (int64_t)P::tpr * FE) body(k, 0);
+  } else if constexpr (P::form != ROW_LANE)
+    for (int64_t k = w.begin + (int64_t)lane * FE; k < w.end; k += (int64_t)P::tpr * FE) body(k, kept[0], Elements<FE>{});
+  if constexpr (P::form == ROW_LANE && P::tail > 0) body((int64_t)P::nv * FE, kept[own + 1], Elements<P::tail>{});
+  if constexpr (P::form == ROW_GROUP || P::form == ROW_RAGGED)
+    if (w.end + lane < w.cols) body(w.end + lane, kept[own + 1], Elements<1>{});
 }
 
 // the reduction of a stage over the P::tpr lanes of a row, left in every lane: within a wave by the
 // butterfly, across the waves of a block through LDS in the order of fused_reduce_rows_body
 template <typename P, typename R>
 __device__ __forceinline__ typename R::acc_t row_reduce(typename R::acc_t acc) {
-  acc = wave_reduce<R>(acc);
+  acc = wave_reduce<R, (P::tpr < WAVE ? P::tpr : WAVE)>(acc);
   if constexpr (P::tpr > WAVE) {
     __shared__ typename R::acc_t sm[FBLOCK / WAVE];
     __syncthreads();  // the previous stage's readers are done with sm
@@ -488,35 +531,49 @@ __device__ __forceinline__ typename R::acc_t row_reduce(typename R::acc_t acc) {
   return acc;
 }
 
-template <typename P, int SEG, typename KEPT>
-__device__ __forceinline__ void row_stage(KernArgs a, int64_t r, int lane, RowStats &stats, KEPT &kept) {
+template <typename P, int SEG>
+__device__ __forceinline__ void row_stage(KernArgs a, int64_t r, int lane, const RowWalk &walk, RowStats &stats, RowVector *kept) {
   // stage SEG: instructions [begin, red) on the row's elements, the reduction at `red`, instructions
   // (red, save) on the statistic, which is kept at `save`; the last stage is [begin, n_instr)
   constexpr int begin = SEG == 0 ? 0 : P::seg_save[SEG - 1] + 1;
   constexpr int red = P::seg_red[SEG], save = P::seg_save[SEG];
-  const int64_t cols = a->cols;
   if constexpr (SEG == P::held_stage) {  // the first stage that reads the held input: all of the lane's part is requested at once
-    for_each_vector<P>(lane, cols, [&](int64_t k, int it) __attribute__((always_inline)) {
+    for_each_vector<P>(lane, walk, kept, [&](int64_t k, RowVector &mine, auto count) __attribute__((always_inline)) {
+      constexpr int n = decltype(count)::n;
       const int64_t row[FV] = {r}, col[FV] = {k};
       Vecs x;
-      load_input_as(a, P::held, P::in_dt[P::held], 1, row, col, x);
+      if constexpr (n == FE) load_input_as<P::unal>(a, P::held, P::in_dt[P::held], 1, row, col, x);
+      else load_input_tail(a, P::held, P::in_dt[P::held], 1, row, col, n, x);
 #pragma unroll
-      for (int e = 0; e < FE; e++) kept[it].held[e] = x[0][e];
+      for (int e = 0; e < n; e++) mine.held[e] = x[0][e];
     });
   }
   if constexpr (red < 0) {  // the last stage: its value is the result
     void *out = (void *)a->out;
-    for_each_vector<P>(lane, cols, [&](int64_t k, int it) __attribute__((always_inline)) {
-      const int64_t row[FV] = {r}, col[FV] = {k};
+    for_each_vector<P>(lane, walk, kept, [&](int64_t k, RowVector &mine, auto count) __attribute__((always_inline)) {
+      constexpr int n = decltype(count)::n;
+      const int64_t row[FV] = {r}, col[FV] = {k}, at = r * walk.cols + k;
       Vecs x;
       Saved S;
-      static_steps<P, begin, P::n_instr>(a, row, col, x, S, stats, FE, &kept[it]);
-      if constexpr (result_is_relabelled_bits<P>()) {
-        uint4 *p = reinterpret_cast<uint4 *>((uint32_t *)out + r * cols + k);
-        p[0] = make_uint4(__float_as_uint(x[0][0]), __float_as_uint(x[0][1]), __float_as_uint(x[0][2]), __float_as_uint(x[0][3]));
-        p[1] = make_uint4(__float_as_uint(x[0][4]), __float_as_uint(x[0][5]), __float_as_uint(x[0][6]), __float_as_uint(x[0][7]));
+      static_steps<P, begin, P::n_instr>(a, row, col, x, S, stats, n, &mine);
+      if constexpr (n < FE) {
+#pragma unroll
+        for (int e = 0; e < n; e++) {
+          if constexpr (result_is_relabelled_bits<P>()) ((uint32_t *)out)[at + e] = __float_as_uint(x[0][e]);
+          else store_one<float>(out, P::out_dt, at + e, x[0][e]);
+        }
+      } else if constexpr (result_is_relabelled_bits<P>()) {
+        uint32_t bits[FE];
+#pragma unroll
+        for (int e = 0; e < FE; e++) bits[e] = __float_as_uint(x[0][e]);
+        __builtin_memcpy((uint32_t *)out + at, bits, sizeof(bits));
+      } else if constexpr (P::unal) {
+        constexpr int bytes = FE * (P::out_dt == HIPNX_F32 ? 4 : P::out_dt == HIPNX_U8 ? 1 : 2);
+        raw_vec<bytes> v;
+        store_vec<float, FE>(&v, P::out_dt, 0, x[0]);
+        __builtin_memcpy((char *)out + at * (bytes / FE), &v, bytes);
       } else {
-        store_vec<float, FE>(out, P::out_dt, r * cols + k, x[0]);
+        store_vec<float, FE>(out, P::out_dt, at, x[0]);
       }
     });
   } else {
@@ -524,16 +581,17 @@ __device__ __forceinline__ void row_stage(KernArgs a, int64_t r, int lane, RowSt
     typedef typename std::conditional<op == HIPNX_RED_SUM, double, float>::type CT;
     typedef PlainReducer<CT, op, false> R;
     typename R::acc_t acc = R::init();
-    for_each_vector<P>(lane, cols, [&](int64_t k, int it) __attribute__((always_inline)) {
+    for_each_vector<P>(lane, walk, kept, [&](int64_t k, RowVector &mine, auto count) __attribute__((always_inline)) {
+      constexpr int n = decltype(count)::n;
       const int64_t row[FV] = {r}, col[FV] = {k};
       Vecs x;
       Saved S;
-      static_steps<P, begin, red>(a, row, col, x, S, stats, FE, &kept[it]);
+      static_steps<P, begin, red>(a, row, col, x, S, stats, n, &mine);
 #pragma unroll
-      for (int e = 0; e < FE; e++) acc = R::accumulate(acc, (CT)x[0][e], k + e);
-      if constexpr (P::nv > 0) {  // kept for the next stage (after this stage's own reads of the previous one's)
+      for (int e = 0; e < n; e++) acc = R::accumulate(acc, (CT)x[0][e], k + e);
+      if constexpr (P::nv > 0 || P::form == ROW_LANE) {  // kept for the next stage (after this stage's own reads of the previous one's)
 #pragma unroll
-        for (int e = 0; e < FE; e++) kept[it].carry[e] = x[0][e];
+        for (int e = 0; e < n; e++) mine.carry[e] = x[0][e];
       }
     });
     acc = row_reduce<P, R>(acc);  // the same value in every lane of the row
@@ -548,7 +606,7 @@ __device__ __forceinline__ void row_stage(KernArgs a, int64_t r, int lane, RowSt
       if (lane == 0) store_one<float>((void *)a->out, P::out_dt, r, x[0][0]);  // lane 0 of the row
     } else {
       stats[P::arg[save]] = x[0][0];
-      row_stage<P, SEG + 1>(a, r, lane, stats, kept);
+      row_stage<P, SEG + 1>(a, r, lane, walk, stats, kept);
     }
   }
 }
@@ -557,12 +615,12 @@ template <typename P>
 __device__ __forceinline__ void fused_row_stages_body() {
   static_assert(FV == 1, "one vector per lane and step");
   KernArgs a = (KernArgs)__builtin_amdgcn_kernarg_segment_ptr();
-  // P::tpr lanes per row: a wave (rows of at most 4096 elements) or the whole block, as the separate reduction has it
+  // P::tpr lanes per row: a part of a wave, a wave (rows of at most 4096 elements) or the whole block, as the separate reduction has it
   const int64_t r = (int64_t)blockIdx.x * (FBLOCK / P::tpr) + threadIdx.x / P::tpr;
-  if (r >= a->rows) return;  // (a whole wave, or with a block per row nobody: no barrier is left waiting)
+  if (r >= a->rows) return;  // (all lanes of a row, or with a block per row nobody: no barrier is left waiting)
   RowStats stats = {};
-  RowVector kept[P::nv > 0 ? P::nv : 1];  // (indexed by compile-time trip numbers only: registers)
-  row_stage<P, 0>(a, r, threadIdx.x % P::tpr, stats, kept);
+  RowVector kept[(P::nv > 0 ? P::nv : 1) + 2];  // (indexed by compile-time trip numbers only: registers)
+  row_stage<P, 0>(a, r, threadIdx.x % P::tpr, row_walk<P>(r, a->cols), stats, kept);
 }
 
 }  // namespace hipnx

@@ -50,6 +50,8 @@ static void list_of(std::string &s, const char *name, const char *type, int n, c
 // What the lanes of a stage program keep in registers between stages: element values carried from one stage to the next,
 // and an input that several stages read.
 struct Keeps {
+  int form = ROW_WHOLE, tail = 0;  // how lanes share a row (fused_ops.cuh), elements behind the vectors of a ROW_LANE row
+  int tpr = 0;          // lanes per row, 0 where the kernel does not take rows one by one
   int trips = 0;        // vectors of a lane along a row, 0 when nothing is kept
   bool carries = false;
   bool written_out = false;  // a lane's trips as straight code (fused_ops.cuh, for_each_vector)
@@ -80,13 +82,27 @@ static Cost cost_of(const hipnx_fused_instr &q) {
   return {0, 0};
 }
 
-static Keeps what_is_kept(const FusedArgs &a) {
+// Lanes per row and their shares: those of the separate reduction of rows of that length, whose order the stages keep (run_reduce_t
+// of reduce_kernels.cuh).  `walk`: the kernel takes the rows one by one (stages, or rows that are not whole vectors).
+static int class_lanes(const FusedArgs &a) { return a.cols > 4096 ? FBLOCK : WAVE; }
+static void share_row(const FusedArgs &a, bool walk, Keeps &k) {
+  if (!walk) return;
+  k.tpr = class_lanes(a);
+  // (a wave per row of 64 had an eighth of its lanes at work)
+  if (a.cols <= 256) k.tpr = a.cols <= 16 ? 1 : a.cols <= 64 ? 8 : a.cols <= 128 ? 16 : 32;
+  k.form = a.cols <= 16 ? ROW_LANE : a.cols % FE == 0 ? ROW_WHOLE : a.cols <= 256 ? ROW_GROUP : ROW_RAGGED;
+  if (k.form == ROW_LANE) k.trips = (int)(a.cols / FE), k.tail = (int)(a.cols % FE);
+}
+
+static Keeps what_is_kept(const FusedArgs &a, bool walk) {
   Keeps k;
   bool stages = false;
   for (int i = 0; i < a.n_instr; i++) stages |= a.ins[i].kind == HIPNX_FUSED_ROW_REDUCE;
-  const int tpr = a.cols > 4096 ? FBLOCK : WAVE;
-  const int64_t trips = (a.cols + tpr * FE - 1) / (tpr * FE);
-  if (!stages || trips > 16) return k;  // (the host refuses longer rows for programs that carry values)
+  share_row(a, walk, k);
+  if (!stages) return k;
+  // (one trip more where the elements around the vectors are code of their own)
+  const int64_t trips = (a.cols / FE + k.tpr - 1) / k.tpr, written = trips + (a.cols % FE != 0);
+  if (trips > 16) return k;  // (the host refuses longer rows for programs that carry values)
   // which stages read an input along the row, and up to which stage a carried value is waiting to be read
   unsigned reads[HIPNX_FUSED_MAX_INPUTS] = {};
   int stage = 0, carried_from = -1;
@@ -122,7 +138,7 @@ static Keeps what_is_kept(const FusedArgs &a) {
   // conversions are instructions too, nothing once a function is long (atan2, 2 to 16 trips, 1 to 8 % slower).
   // And the code has to stay near what the instruction cache holds (64 KB for two CUs): pow in two stages, 16 trips (240 KB),
   // 154 / 172 us, and 2.4 s to compile instead of 0.5.
-  if (trip.branches * trips > (rounds ? 1 : 6) || trip.kbytes * trips > 96 || (rounds_f16 && trip.kbytes > 0)) return k;
+  if (trip.branches * written > (rounds ? 1 : 6) || trip.kbytes * written > 96 || (rounds_f16 && trip.kbytes > 0)) return k;
   // Carried values alone gain only where the compiler leaves the loop over them rolled: f32, logarithms, 14 trips 37 / 43 us,
   // 16 trips 51 / 46; square roots, 15 trips 32 / 35, 16 trips 40 / 37.
   k.written_out = k.carries && trips > 15;
@@ -140,8 +156,9 @@ static Keeps what_is_kept(const FusedArgs &a) {
   return k;
 }
 
-// everything a compiled kernel is specialised on, as bytes: the cache key.  The number of vectors kept comes last: the keys of
+// everything a compiled kernel is specialised on, as bytes: the cache key.  What the length of a row decides comes last: the keys of
 // one program's kernels for rows of other lengths differ in it alone.
+constexpr size_t LENGTH_KEY = 4 * sizeof(int);
 static std::string make_key(const FusedArgs &a, const Keeps &keeps, int reduce_op, bool block_per_row) {
   std::string k;
   k.reserve(20 + 16 * a.n_instr + 8 * a.n_inputs);
@@ -150,21 +167,23 @@ static std::string make_key(const FusedArgs &a, const Keeps &keeps, int reduce_o
   k.append((const char *)a.ins, sizeof(hipnx_fused_instr) * a.n_instr);
   k.append((const char *)a.in_dt, sizeof(int) * a.n_inputs);
   k.append((const char *)a.in_cs, sizeof(int) * a.n_inputs);
-  k.append((const char *)&keeps.trips, sizeof(int));
+  const int length[4] = {keeps.form, keeps.tpr, keeps.tail, keeps.trips};
+  static_assert(sizeof(length) == LENGTH_KEY, "the part of the key that a row's length decides");
+  k.append((const char *)length, sizeof(length));
   return k;
 }
 
-// A program that keeps an input in registers only to read it once could do without, and then takes rows of any length: its
-// module also has that kernel, for a capture that meets a length which has not been compiled (a new module is no work to
-// record).  One that carries values cannot.
-static bool has_kernel_for_any_length(const Keeps &k) { return k.trips > 0 && !k.carries; }
+// A program that keeps an input in registers only to read it once could do without, and then takes rows of any number of whole
+// vectors (a wave per row, a block per long row): its module also has that kernel, for a capture that meets a length which has
+// not been compiled (a new module is no work to record).  One that carries values cannot.
+static bool is_for_any_length(const FusedArgs &a, const Keeps &k) { return k.form == ROW_WHOLE && k.trips == 0 && (k.tpr == 0 || k.tpr == class_lanes(a)); }
+static bool has_kernel_for_any_length(const FusedArgs &a, const Keeps &k) { return a.cols % FE == 0 && !k.carries && !is_for_any_length(a, k); }
 static std::string any_length(const std::string &name) { return name + "_any"; }
 
 // the whole translation unit for one program
 static std::string make_source(const FusedArgs &a, const Keeps &keeps, int reduce_op, bool block_per_row, const std::string &name) {
   std::string s = RTC_PREAMBLE;
-  s += "namespace hipnx {\nstruct Program {\n  static constexpr int n_instr = " + std::to_string(a.n_instr) + ", out_dt = " + std::to_string(a.out_dt) +
-       ", tpr = " + (block_per_row ? "FBLOCK" : "WAVE") + ";\n";
+  s += "namespace hipnx {\nstruct Program {\n  static constexpr int n_instr = " + std::to_string(a.n_instr) + ", out_dt = " + std::to_string(a.out_dt) + ";\n";
   const hipnx_fused_instr *q = a.ins;
   list_of(s, "kind", "int", a.n_instr, [&](int i) { return std::to_string((int)q[i].kind); });
   list_of(s, "op", "int", a.n_instr, [&](int i) { return std::to_string((int)q[i].op); });
@@ -192,19 +211,22 @@ static std::string make_source(const FusedArgs &a, const Keeps &keeps, int reduc
   list_of(s, "seg_red", "int", (int)seg_red.size(), [&](int k) { return std::to_string(seg_red[k]); });
   list_of(s, "seg_save", "int", (int)seg_save.size(), [&](int k) { return std::to_string(seg_save[k]); });
   auto keeping = [](const char *p, const Keeps &k) {
-    return std::string("struct ") + p + " : Program {\n  static constexpr int nv = " + std::to_string(k.trips) + ", written_out = " + std::to_string(k.written_out) + ", held = " + std::to_string(k.held) +
+    return std::string("struct ") + p + " : Program {\n  static constexpr int form = " + std::to_string(k.form) + ", tpr = " + std::to_string(k.tpr) + ", tail = " + std::to_string(k.tail) +
+           ";\n  static constexpr bool unal = " + (k.form == ROW_WHOLE ? "false" : "true") + ";\n  static constexpr int nv = " + std::to_string(k.trips) + ", written_out = " + std::to_string(k.written_out) + ", held = " + std::to_string(k.held) +
            ", held_stage = " + std::to_string(k.held_stage) + ";\n};\n";
   };
   auto kernel = [](const std::string &called) {
     return "extern \"C\" __global__ void __launch_bounds__(FBLOCK) " + called + "(FusedArgs by_value) {\n  (void)by_value;\n";
   };
   s += "};\n" + keeping("P", keeps);
-  if (has_kernel_for_any_length(keeps)) s += keeping("Any", Keeps{});
+  Keeps any;
+  any.tpr = class_lanes(a);
+  if (has_kernel_for_any_length(a, keeps)) s += keeping("Any", any);
   s += "}\nusing namespace hipnx;\n";
-  if (has_kernel_for_any_length(keeps)) s += kernel(any_length(name)) + "  fused_row_stages_body<Any>();\n}\n";
+  if (has_kernel_for_any_length(a, keeps)) s += kernel(any_length(name)) + "  fused_row_stages_body<Any>();\n}\n";
   s += kernel(name);
   const char *tpr = block_per_row ? "FBLOCK" : "WAVE";
-  if (stages) s += "  fused_row_stages_body<P>();\n";
+  if (stages || keeps.form != ROW_WHOLE) s += "  fused_row_stages_body<P>();\n";
   else switch (reduce_op) {
     case HIPNX_RED_SUM: s += std::string("  fused_reduce_rows_body<RunStatic<P>, PlainReducer<double, HIPNX_RED_SUM, false>, double, ") + tpr + ">();\n"; break;
     case HIPNX_RED_MAX: s += std::string("  fused_reduce_rows_body<RunStatic<P>, PlainReducer<float, HIPNX_RED_MAX, false>, float, ") + tpr + ">();\n"; break;
@@ -273,19 +295,23 @@ static int trim_cache(hipnx_ctx *ctx) {
 // Launches the compiled kernel for `a`, compiling it first if this context has not seen the program.
 // *done = false (and HIPNX_OK) when the caller should run the interpreting kernel instead: the
 // program is new and the stream is capturing (compiling and loading a module is no work to record).
-int fused_launch_compiled(hipnx_ctx *ctx, const FusedArgs &a, int reduce_op, bool block_per_row, unsigned grid, bool *done) {
+// `walk`: a group of lanes takes a row, the grid follows from how many; `grid` is the grid otherwise.
+int fused_launch_compiled(hipnx_ctx *ctx, const FusedArgs &a, int reduce_op, bool block_per_row, bool walk, unsigned grid, bool *done) {
   *done = false;
-  const Keeps keeps = what_is_kept(a);
+  const Keeps keeps = what_is_kept(a, walk);
+  int lanes = keeps.tpr;
   const std::string key = make_key(a, keeps, reduce_op, block_per_row);
   auto it = ctx->fused_kernels.find(key);
   hipFunction_t function = nullptr;
   if (it == ctx->fused_kernels.end() && ctx->capture) {
     // the program may be there for rows of another length, with a kernel that takes any
-    const size_t same = key.size() - sizeof(int);
+    if (a.cols % FE != 0) return HIPNX_OK;
+    const size_t same = key.size() - LENGTH_KEY;
     for (it = ctx->fused_kernels.begin(); it != ctx->fused_kernels.end(); ++it)
       if (it->second.any_length && it->first.size() == key.size() && it->first.compare(0, same, key, 0, same) == 0) break;
     if (it == ctx->fused_kernels.end()) return HIPNX_OK;
     function = it->second.any_length;
+    lanes = class_lanes(a);
   }
   if (it == ctx->fused_kernels.end()) {
     // a name a profile can tell apart: what the kernel is (a map, a map with its row reduction, stages over rows),
@@ -298,8 +324,8 @@ int fused_launch_compiled(hipnx_ctx *ctx, const FusedArgs &a, int reduce_op, boo
     if (ctx->fused_kernels.size() >= ctx->fused_cache_max)
       if (int st = trim_cache(ctx)) return st;
     hipnx_ctx::FusedKernel k{};
-    if (int st = compile(ctx, make_source(a, keeps, reduce_op, block_per_row, name), name, has_kernel_for_any_length(keeps), &k)) return st;
-    if (keeps.trips == 0) k.any_length = k.function;
+    if (int st = compile(ctx, make_source(a, keeps, reduce_op, block_per_row, name), name, has_kernel_for_any_length(a, keeps), &k)) return st;
+    if (is_for_any_length(a, keeps)) k.any_length = k.function;
     it = ctx->fused_kernels.emplace(key, k).first;
   }
   if (!function) function = it->second.function;
@@ -307,6 +333,7 @@ int fused_launch_compiled(hipnx_ctx *ctx, const FusedArgs &a, int reduce_op, boo
   if (ctx->capture) it->second.in_graph = true;  // a recorded launch refers to the loaded module for as long as the graph lives
   // the argument block is the kernel's one by-value parameter: hand it over as the packed buffer it is
   size_t size = sizeof(FusedArgs);
+  if (walk) grid = (unsigned)((a.rows + FBLOCK / lanes - 1) / (FBLOCK / lanes));
   void *config[] = {HIP_LAUNCH_PARAM_BUFFER_POINTER, (void *)&a, HIP_LAUNCH_PARAM_BUFFER_SIZE, &size, HIP_LAUNCH_PARAM_END};
   HIPNX_HIP(hipModuleLaunchKernel(function, grid, 1, 1, FBLOCK, 1, 1, 0, ctx->stream, nullptr, config));
   *done = true;

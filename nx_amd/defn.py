@@ -516,7 +516,7 @@ def _fusable(t: Tensor) -> bool:
     return False
 
 
-def _layout(out_shape, in_shapes, split=None):
+def _layout(out_shape, in_shapes, split=None, any_rows=False):
     """The index space as [rows, cols] with a (row stride, column stride) per input, or None: an
     input is the full shape, one value, one row shared by all rows, or one value per row.  `split`
     fixes the axis where the columns begin (a reduction over the last axis needs the rows it
@@ -525,8 +525,13 @@ def _layout(out_shape, in_shapes, split=None):
     padded = [(1,) * (rank - len(s)) + tuple(s) for s in in_shapes]
     for p in (range(rank + 1) if split is None else [split]):
         rows, cols = prod(out_shape[:p]), prod(out_shape[p:])
-        if cols % 8 and not (_plan["ints"] and split is None and p == 0):
-            continue  # whole vectors of 8 along a row; a compiled kernel over a flat index space takes a partial last one
+        # Whole vectors of 8 along a row; a compiled kernel over a flat index space also takes a partial last one.  Rows of any
+        # length, which it takes one by one, come second -- and not the few very long ones that the reductions cut into segments.
+        ragged = cols % 8 != 0 and not (split is None and p == 0)
+        if cols % 8 and not _plan["ints"]:
+            continue
+        if ragged and (cols == 1 or (split is None and not any_rows) or (cols >= 32768 and rows < 2048)):
+            continue
         strides = []
         for s in padded:
             outer, inner = s[:p], s[p:]
@@ -536,12 +541,12 @@ def _layout(out_shape, in_shapes, split=None):
                 break
             cs = 1 if dense_inner and cols > 1 else 0
             rs = (cols if cs else 1) if dense_outer and rows > 1 else 0
-            if cs and rows > 1 and rs % 8:
+            if cs and rows > 1 and rs % 8 and not ragged:
                 break
             strides.append((rs, cs))
         else:
             return rows, cols, strides
-    return None
+    return _layout(out_shape, in_shapes, any_rows=True) if split is None and _plan["ints"] and not any_rows else None
 
 
 class _Program(list):
@@ -1038,8 +1043,6 @@ def _cluster_rows(roots: List[Tensor]) -> int:
         if rank == 0:
             return False
         cols, rows = full_shape[-1], prod(full_shape[:-1])
-        if cols % 8:
-            return False
         per_row = tuple(full_shape[:-1]) + (1,)
         carry_fits = cols <= 32768  # at most sixteen vectors per lane with a block per row (eight with a wave, <= 4096)
 

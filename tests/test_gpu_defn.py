@@ -821,6 +821,66 @@ def test_long_rows_take_a_block_each(name, shape, ty, hip):
     assert calls == [1]
 
 
+def bias_and_scale_per_row(x, bias):  # no reduction: a row and a value per row against ragged rows
+    return Nx.multiply(Nx.exp(Nx.add(x, bias)), Nx.slice_along_axis(x, 0, 1, axis=len(x.shape) - 1))
+
+
+def sum_of_squares(x):
+    return Nx.sum(Nx.multiply(x, Nx.tanh(x)), axes=[-1])
+
+
+# a lane per row (no vector, one, two; tails of every kind); 8, 16, 32 lanes with one vector each at most; a wave, a block: one
+# vector more or less than whole trips, heads and tails of every length in turn from row to row
+RAGGED_ROWS = [(37, 3), (41, 8), (257, 10), (70, 17), (33, 65), (9, 129), (9, 257), (9, 519), (3, 5, 1001), (8, 4097), (3, 32767), (1, 77)]
+
+
+@pytest.mark.parametrize("ty", ["f32", "bf16"])
+@pytest.mark.parametrize("shape", RAGGED_ROWS)
+@pytest.mark.parametrize("name", ["softmax_rows", "centred_and_scaled", "log_softmax_rows", "log_sum_exp_rows", "sum_of_squares",
+                                  "bias_and_scale_per_row"])
+def test_rows_of_any_length_in_one_launch(name, shape, ty, hip):
+    """The bits of the nodes one by one, and nothing written around the result."""
+    rng = np.random.default_rng(seed_of(name, shape, ty, "ragged"))
+    x = rand_float(rng, ty, shape, hip)
+    with_row = name in ("centred_and_scaled", "bias_and_scale_per_row")
+    args = (x, rand_float(rng, ty, (shape[-1],), hip)) if with_row else (x,)
+    fun = globals()[name]
+    planned = defn.compile(fun, *args, fuse="compiled")
+    launches = []
+    original = hip.fused_elementwise.__func__
+
+    def counting(cls, *a, **k):
+        out = original(cls, *a, **k)  # (a refusal raises: the nodes would run one by one)
+        launches.append(k.get("mode"))
+        return out
+    hip.fused_elementwise = classmethod(counting)
+    try:
+        got = planned(*args)
+    finally:
+        hip.fused_elementwise = classmethod(original)
+    assert launches == ["compiled"], launches
+    assert_bits_equal(got, defn.compile(fun, *args)(*args), f"{name} {shape} {ty}")
+
+
+@pytest.mark.parametrize("ty", ["f32", "bf16", "f16"])
+@pytest.mark.parametrize("shape", [(12, 10), (9, 100), (9, 185), (9, 1001), (3, 8191)])
+def test_ragged_rows_at_any_address_leave_their_neighbours(shape, ty, hip):
+    """Operands and results one element behind a vector boundary; rows of infinities, NaN and the lowest number."""
+    from nx_amd import types as T
+    from test_gpu_elementwise import encode
+    rng = np.random.default_rng(seed_of(shape, ty, "address"))
+    n, size = int(np.prod(shape)), T.size_bytes(T.normalize(ty))
+    words = raw(rand_float(rng, ty, (n + 24,), hip)).copy()
+    special = encode(np.array([np.inf, -np.inf, np.nan, -6.0e4 if ty == "f16" else -3.0e38, 0.0, -0.0]), ty)
+    words[1:1 + special.size] = special
+    words[1 + shape[-1]:1 + 2 * shape[-1]] = special[1]  # a row of -inf
+    store = from_numpy(words, ty, hip)
+    x = Nx.from_pointer(hip, Nx.Pointer(kind="local", address=Nx.to_pointer(store).address + size, data_size=n * size), ty, shape, keep=store)
+    want = defn.compile(softmax_rows, x)(x)
+    assert_bits_equal(defn.compile(softmax_rows, x, fuse="compiled")(x), want, f"{shape} {ty}")
+    np.testing.assert_array_equal(raw(store).view(np.uint8), words.view(np.uint8))
+
+
 def test_a_select_on_integers_reads_a_row_that_later_stages_hold(hip):
     """A SELECT marked as an integer instruction takes its operands as floats all the same: the stage it stands in is the
     first that reads the row, and the registers that hold the row for the later stages are filled there."""
