@@ -48,36 +48,63 @@ pad_rows_kernel(const T *__restrict__ in, unsigned char *__restrict__ out, int64
 }
 
 // Plain tiled contraction for every other type combination.  16 x 16 outputs per block, K
-// walked in slabs of 16 through LDS; operands are decoded to CT (double or wrapping int64).
+// walked in slabs of TK (64; 16 for a short K) through LDS; operands are decoded to CT (double or wrapping int64).
 // lk / rk: 1 when the operand is K-inner ([rows, K]), 0 when K-outer ([K, rows]).
-template <typename CT>
+// LDT / RDT: the operands' types where they are known when the kernel is compiled (the four loads per operand and slab then
+// all go out before one is converted), -1: read from ldt / rdt.
+// Bound by the latency of a slab (about 1 us, mostly its loads), K / 64 of them in a row: few outputs over a long K leave the chip
+// idle.  nseg > 1: the blocks along y are cut into segments of K of seg_len (whole slabs), whose sums go to
+// partial[output * nseg + segment] for dot_reduce_finish_kernel.  In slabs of 16 and with K whole, before / now, us per call:
+// f32 80 x 3 x 6377 394 / 20, 100 x 10 x 2001 118 / 12, 64 x 64 x 4095 264 / 15.5, bf16 5 x 300 x 9999 604 / 33.
+template <typename CT, int TK, int LDT = -1, int RDT = -1>
 __global__ void __launch_bounds__(256)
-dot_generic_kernel(const void *__restrict__ l, const void *__restrict__ r, void *__restrict__ out, int ldt, int rdt,
-                   int odt, int64_t M, int64_t N, int64_t K, int lk, int rk) {
-  constexpr int T = 16;
-  __shared__ CT sA[T][T + 1], sB[T][T + 1];
-  const int tx = threadIdx.x % T, ty = threadIdx.x / T;
+dot_generic_kernel(const void *__restrict__ l, const void *__restrict__ r, void *__restrict__ out, int ldt_, int rdt_,
+                   int odt, int64_t M, int64_t N, int64_t K, int lk, int rk, CT *__restrict__ partial, int64_t seg_len, int nseg) {
+  constexpr int T = 16, PER = T * TK / 256;
+  const int ldt = LDT >= 0 ? LDT : ldt_, rdt = RDT >= 0 ? RDT : rdt_;
+  __shared__ CT sA[T][TK + 1], sB[T][TK + 1];
+  const int tid = threadIdx.x, tx = tid % T, ty = tid / T;
   // (tiles of M along x, which holds 2^31 - 1 groups: [2M, 3] . [3, 3] has 131072 of them; tiles of N along y)
   const int64_t b = blockIdx.z;
-  const int64_t m = (int64_t)blockIdx.x * T + ty, n = (int64_t)blockIdx.y * T + tx;
+  const int seg = (int)(blockIdx.y % nseg);
+  const int64_t m0 = (int64_t)blockIdx.x * T, n0 = (int64_t)(blockIdx.y / nseg) * T, m = m0 + ty, n = n0 + tx;
   const int64_t lbase = b * M * K, rbase = b * N * K;
+  const int64_t k_begin = seg * seg_len, k_end = k_begin + seg_len < K ? k_begin + seg_len : K;
   CT acc = 0;
-  for (int64_t k0 = 0; k0 < K; k0 += T) {
-    {  // sA[ty][tx] = l[m, k0 + tx]; sB[ty][tx] = r[n0 + ty, k0 + tx]
-      const int64_t k = k0 + tx;
-      const int64_t mm = (int64_t)blockIdx.x * T + ty, nn = (int64_t)blockIdx.y * T + ty;
-      sA[ty][tx] = (mm < M && k < K) ? load_one<CT>(l, ldt, lbase + (lk ? mm * K + k : k * M + mm)) : (CT)0;
-      sB[ty][tx] = (nn < N && k < K) ? load_one<CT>(r, rdt, rbase + (rk ? nn * K + k : k * N + nn)) : (CT)0;
+  for (int64_t k0 = k_begin; k0 < k_end; k0 += TK) {
+    CT a[PER], c[PER];
+#pragma unroll
+    for (int q = 0; q < PER; q++) {
+      // consecutive lanes along the operand's contiguous axis
+      const int e = tid + q * 256;
+      const int am = lk ? e / TK : e % T, ak = lk ? e % TK : e / T, bn = rk ? e / TK : e % T, bk = rk ? e % TK : e / T;
+      const int64_t mm = m0 + am, nn = n0 + bn, ka = k0 + ak, kb = k0 + bk;
+      a[q] = (mm < M && ka < k_end) ? load_one<CT>(l, ldt, lbase + (lk ? mm * K + ka : ka * M + mm)) : (CT)0;
+      c[q] = (nn < N && kb < k_end) ? load_one<CT>(r, rdt, rbase + (rk ? nn * K + kb : kb * N + nn)) : (CT)0;
+    }
+#pragma unroll
+    for (int q = 0; q < PER; q++) {
+      const int e = tid + q * 256;
+      const int am = lk ? e / TK : e % T, ak = lk ? e % TK : e / T, bn = rk ? e / TK : e % T, bk = rk ? e % TK : e / T;
+      sA[am][ak] = a[q];
+      sB[bn][bk] = c[q];
     }
     __syncthreads();
+    const int steps = k_end - k0 < TK ? (int)(k_end - k0) : TK;
+    for (int k16 = 0; k16 < steps; k16 += 16) {  // (behind K both are zero)
 #pragma unroll
-    for (int kk = 0; kk < T; kk++) {
-      if constexpr (std::is_same<CT, double>::value) acc = sA[ty][kk] * sB[tx][kk] + acc;
-      else acc = (int64_t)((uint64_t)sA[ty][kk] * (uint64_t)sB[tx][kk] + (uint64_t)acc);
+      for (int kk = k16; kk < k16 + 16; kk++) {
+        if constexpr (std::is_same<CT, double>::value) acc = sA[ty][kk] * sB[tx][kk] + acc;
+        else acc = (int64_t)((uint64_t)sA[ty][kk] * (uint64_t)sB[tx][kk] + (uint64_t)acc);
+      }
     }
     __syncthreads();
   }
-  if (m < M && n < N) store_one<CT>(out, odt, b * M * N + m * N + n, acc);
+  if (m < M && n < N) {
+    const int64_t o = b * M * N + m * N + n;
+    if (nseg > 1) partial[o * nseg + seg] = acc;
+    else store_one<CT>(out, odt, o, acc);
+  }
 }
 
 // Many small matrices (a 3 x 3 transform per point, a 4 x 4 block per item): one lane per output over the whole batch,
@@ -429,10 +456,40 @@ static int dot_impl(hipnx_ctx *ctx, int l_dt, int r_dt, int out_dt, int64_t batc
         HIPNX_HIP(hipGetLastError());
         return HIPNX_OK;
       }
-      if (any_float)
-        hipLaunchKernelGGL((dot_generic_kernel<double>), grid, block, 0, ctx->stream, l->ptr, r->ptr, out->ptr, l_dt, r_dt, out_dt, M, N, K, lk, rk);
-      else
-        hipLaunchKernelGGL((dot_generic_kernel<int64_t>), grid, block, 0, ctx->stream, l->ptr, r->ptr, out->ptr, l_dt, r_dt, out_dt, M, N, K, lk, rk);
+      // Few outputs over a long K (the weight gradient of a layer with a handful of classes: [6377, 80]^T . [6377, 3] is five
+      // tiles): K is cut until every CU has two work-groups, where that saves more slabs than the second pass costs (eight
+      // and more: 1 us each against 5).  Not where a sum's order shows: an f64 operand or result adds over k in order.
+      const bool any_f64 = l_dt == HIPNX_F64 || r_dt == HIPNX_F64 || out_dt == HIPNX_F64;
+      const int64_t tiles = (int64_t)grid.x * grid.y * batch, slabs = (K + 63) / 64;
+      int64_t nseg = any_f64 ? 1 : std::min<int64_t>(2 * (int64_t)ctx->num_cus / tiles, slabs / 2);
+      int64_t seg_len = K;
+      if (nseg > 1) {
+        seg_len = (slabs + nseg - 1) / nseg * 64;
+        nseg = (K + seg_len - 1) / seg_len;
+      }
+      if (nseg < 2 || slabs - seg_len / 64 < 8 || grid.y * nseg > 65535) nseg = 1, seg_len = K;
+      void *ws = nullptr;
+      size_t ws_cap = 0;
+      if (nseg > 1 && pool_alloc(ctx, (size_t)(batch * M * N * nseg) * 8, &ws, &ws_cap) != HIPNX_OK) nseg = 1, seg_len = K;
+      grid.y *= (unsigned)nseg;
+      const dim3 finish((unsigned)std::min<int64_t>((batch * M * N + 255) / 256, 1 << 20));
+#define HIPNX_GENERIC_K(CT, TK, ...) hipLaunchKernelGGL((dot_generic_kernel<CT, TK, ##__VA_ARGS__>), grid, block, 0, ctx->stream, l->ptr, r->ptr, out->ptr, l_dt, r_dt, out_dt, M, N, K, lk, rk, (CT *)ws, seg_len, (int)nseg)
+#define HIPNX_GENERIC(CT, ...) do { if (K <= 32) HIPNX_GENERIC_K(CT, 16, ##__VA_ARGS__); else HIPNX_GENERIC_K(CT, 64, ##__VA_ARGS__); } while (0)
+      if (any_float) {
+        if (l_dt == HIPNX_F32 && r_dt == HIPNX_F32) HIPNX_GENERIC(double, HIPNX_F32, HIPNX_F32);
+        else if (l_dt == HIPNX_BF16 && r_dt == HIPNX_BF16) HIPNX_GENERIC(double, HIPNX_BF16, HIPNX_BF16);
+        else if (l_dt == HIPNX_F16 && r_dt == HIPNX_F16) HIPNX_GENERIC(double, HIPNX_F16, HIPNX_F16);
+        else HIPNX_GENERIC(double);
+        if (nseg > 1)
+          hipLaunchKernelGGL((dot_reduce_finish_kernel<double>), finish, block, 0, ctx->stream, (const double *)ws, out->ptr, out_dt, batch * M * N, (int)nseg);
+      } else {
+        HIPNX_GENERIC(int64_t);
+        if (nseg > 1)
+          hipLaunchKernelGGL((dot_reduce_finish_kernel<int64_t>), finish, block, 0, ctx->stream, (const int64_t *)ws, out->ptr, out_dt, batch * M * N, (int)nseg);
+      }
+#undef HIPNX_GENERIC
+#undef HIPNX_GENERIC_K
+      if (ws) pool_free(ctx, ws, ws_cap);  // later work is ordered on the same stream
       HIPNX_HIP(hipGetLastError());
       return HIPNX_OK;
     }

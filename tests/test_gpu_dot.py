@@ -767,3 +767,23 @@ def test_zero_products_leave_a_positive_zero(ty, m, k, n, hip, oracle):
     assert_bits_equal(Nx.dot(ha, hb), Nx.dot(oa, ob), f"dot {ty} {m}x{k}x{n}")
     assert_bits_equal(Nx.dot(ha, [0], hb, [1]) if m == n else Nx.dot(hb, [0], ha, [1]),
                       Nx.dot(oa, [0], ob, [1]) if m == n else Nx.dot(ob, [0], oa, [1]), f"dot {ty} other axes")
+
+
+@pytest.mark.parametrize("layout", ["nn", "nt", "tn", "tt"])
+@pytest.mark.parametrize("lt,rt,M,N,K", [("f32", "f32", 80, 3, 1601), ("bf16", "bf16", 17, 33, 577), ("f16", "f16", 5, 61, 3333), ("f32", "f32", 16, 16, 640 + 33),
+                                         ("f16", "f32", 20, 12, 1500), ("s32", "s32", 33, 40, 1333), ("f64", "f64", 20, 12, 1501), ("f32", "f32", 40, 9, 31)])
+def test_few_outputs_over_a_long_k_are_cut_into_segments(lt, rt, M, N, K, layout, hip, oracle):
+    """Plain kernels with K cut: integers exact; f64 operands are not cut and add in order of k (the oracle's bits); the others are f64
+    sums in another order, K * 2^-53 of the magnitudes apart at most, rounded once to the result's type."""
+    rng = np.random.default_rng(seed_of(lt, rt, M, N, K, layout, "segments"))
+    arrays = [rng.integers(-999, 999, size=s).astype(np.int32) if t == "s32" else rand_raw(rng, t, s, lo=-1, hi=1)
+              for t, s in ((lt, (M, K) if layout[0] == "n" else (K, M)), (rt, (K, N) if layout[1] == "n" else (N, K)))]
+    (ha, oa), (hb, ob) = both(arrays[0], lt, hip, oracle), both(arrays[1], rt, hip, oracle)
+    axes = [1] if layout[0] == "n" else [0], [0] if layout[1] == "n" else [1]
+    got, want = Nx.dot(ha, axes[0], hb, axes[1]), Nx.dot(oa, axes[0], ob, axes[1])
+    if lt in ("s32", "f64"):
+        assert_bits_equal(got, want, f"{lt} {layout}")
+        return
+    a, b = values(oa) if layout[0] == "n" else values(oa).T, values(ob) if layout[1] == "n" else values(ob).T
+    apart = np.abs(values(got) - values(want))
+    assert (apart <= ULP[got.type] * np.abs(values(want)) + 2 * K * 2.0 ** -53 * (np.abs(a) @ np.abs(b))).all(), f"{lt} {layout}: {apart.max()}"
