@@ -257,6 +257,16 @@ int hipnx_dot(hipnx_ctx *ctx, int l_dt, int r_dt, int out_dt, int64_t batch, int
               int64_t K, int l_layout, int r_layout, const hipnx_buf *l, const hipnx_buf *r,
               hipnx_buf *out);
 
+/* replaces: dot/7 after transpose/3 of an operand (nx/lib/nx/backend.ex:73, 77), without the copy: the operands lie in larger or
+ * permuted tensors.  The batch is batch_outer x batch_inner items; l_strides / r_strides are three strides in elements: along the
+ * first batch axis, along the second, and from row to row (HIPNX_K_INNER: the K elements of a row are contiguous) or from k to k
+ * (HIPNX_K_OUTER: the rows are).  The heads of [batch, positions, heads, dim] are {positions * heads * dim, dim, heads * dim}.
+ * The bits are those of the two calls.  Contractions on the matrix cores whose operands can be read as they lie (K of
+ * whole 16-byte pieces, K-outer rows of whole blocks); anything else is HIPNX_EUNSUPPORTED: copy, then hipnx_dot. */
+int hipnx_dot_strided(hipnx_ctx *ctx, int l_dt, int r_dt, int out_dt, int64_t batch_outer, int64_t batch_inner, int64_t M, int64_t N,
+                      int64_t K, int l_layout, int r_layout, const int64_t *l_strides, const int64_t *r_strides, const hipnx_buf *l,
+                      const hipnx_buf *r, hipnx_buf *out);
+
 /* replaces: the three callbacks of a quantised linear layer in one -- dot/7 with an s32 result, as_type/2
  * to f32 and multiply/3 by the scales (nx/lib/nx/backend.ex:77, 68, 115), i.e.
  * Nx.multiply(Nx.as_type(Nx.dot(x, w), :f32), scales) on s8 operands.  out[b, m, n] (f32) =

@@ -95,6 +95,8 @@ PROTOTYPES = {
     "hipnx_argreduce": [_ctx_p, C.c_int, C.c_int, C.c_int, C.c_int, C.c_int64, C.c_int64, C.c_int64, _buf_p, _buf_p],
     "hipnx_dot": [_ctx_p, C.c_int, C.c_int, C.c_int, C.c_int64, C.c_int64, C.c_int64, C.c_int64, C.c_int, C.c_int,
                   _buf_p, _buf_p, _buf_p],
+    "hipnx_dot_strided": [_ctx_p, C.c_int, C.c_int, C.c_int, C.c_int64, C.c_int64, C.c_int64, C.c_int64, C.c_int64, C.c_int, C.c_int,
+                          _i64p, _i64p, _buf_p, _buf_p, _buf_p],
     "hipnx_dot_scaled": [_ctx_p, C.c_int, C.c_int, C.c_int64, C.c_int64, C.c_int64, C.c_int64, C.c_int, C.c_int,
                          _buf_p, _buf_p, C.c_int, _buf_p, _buf_p],
     "hipnx_transpose": [_ctx_p, C.c_int, C.c_int, _i64p, _intp, _buf_p, _buf_p],

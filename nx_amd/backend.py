@@ -638,6 +638,65 @@ class HipNxBackend:
 
     _dot_plans = {}
 
+    @classmethod
+    def dot_views(cls, out: Tensor, l: Tensor, l_axes, c1, b1, r: Tensor, r_axes, c2, b2) -> Tensor:
+        """`dot(transpose(l, l_axes), c1, b1, transpose(r, r_axes), c2, b2)` without the copies (axes of None: the operand as it
+        is): the contraction reads its operands where they lie.  The evaluator offers it when a transpose feeds a dot
+        and nobody else (backend.ex:73, 77).  Raises HipNxError with status EUNSUPPORTED for what the kernels cannot take
+        that way: the caller then makes the separate calls."""
+        dev = cls._device_of(l, r)
+        l, r = cls._from_nx(l, dev), cls._from_nx(r, dev)
+        key = (l.shape, l_axes, tuple(c1), r.shape, r_axes, tuple(c2), len(b1), out.type)
+        plan = cls._view_plans.get(key)
+        if plan is None:
+            if len(cls._view_plans) >= 4096:
+                cls._view_plans.clear()
+            plan = cls._view_plans[key] = cls._plan_views(l.shape, l_axes, c1, r.shape, r_axes, c2, len(b1)) or ()
+        if not plan or out.type[1] < 8:
+            raise L.HipNxError(L.EUNSUPPORTED, "dot_views: operands that are not strided matrices")
+        outer, inner, K, l_layout, M, l_strides, r_layout, N, r_strides = plan
+        res = cls._alloc(out, dev)
+        status = L.lib.hipnx_dot_strided(res.data.ref.ctx, T.code(l.type), T.code(r.type), _out_code(out.type), outer, inner, M, N, K,
+                                         l_layout, r_layout, l_strides, r_strides, cls._handle(l), cls._handle(r), res.data.ref.handle)
+        if status:
+            L.check(status)
+        return res
+
+    _view_plans = {}
+
+    @staticmethod
+    def _plan_views(l_shape, l_axes, c1, r_shape, r_axes, c2, nb):
+        """The call's extents, layouts and strides, or None where an operand is not a matrix per batch item with one of its
+        axes contiguous, or the batch more than two axes."""
+        def as_one(axes):
+            """(extent, stride) of neighbouring axes [(extent, stride), ...] walked as one, or None."""
+            axes = [a for a in axes if a[0] != 1]
+            if any(a[1] != b[0] * b[1] for a, b in zip(axes, axes[1:])):
+                return None
+            return prod(a[0] for a in axes), axes[-1][1] if axes else 0
+        pairs = sorted(zip(c1, c2))
+        sides = []
+        for shape, axes, contract in ((l_shape, l_axes, [p[0] for p in pairs]), (r_shape, r_axes, [p[1] for p in pairs])):
+            dense = HipNxBackend._dense_strides(shape)
+            walk = [(shape[a], dense[a]) for a in (axes if axes is not None else range(len(shape)))]
+            kept, folded = as_one([w for i, w in enumerate(walk) if i >= nb and i not in contract]), as_one([walk[i] for i in contract])
+            if kept is None or folded is None:
+                return None
+            (rows, row_stride), (K, k_stride) = kept, folded
+            if k_stride == 1:
+                sides.append((walk[:nb], K_INNER, rows, K, row_stride or K))
+            elif row_stride == 1:
+                sides.append((walk[:nb], K_OUTER, rows, K, k_stride or rows))
+            else:
+                return None
+        (lb, l_layout, M, K, l_ld), (rb, r_layout, N, _, r_ld) = sides
+        for cut in range(nb + 1):
+            parts = [as_one(b) for b in (lb[:cut], lb[cut:], rb[:cut], rb[cut:])]
+            if None not in parts:
+                (outer, l0), (inner, l1), (_, r0), (_, r1) = parts
+                return outer, inner, K, l_layout, M, L.i64_array((l0, l1, l_ld)), r_layout, N, L.i64_array((r0, r1, r_ld))
+        return None
+
     # ---- data movement ---------------------------------------------------------------------
     @classmethod
     def dot_scaled(cls, out: Tensor, l: Tensor, c1, b1, r: Tensor, c2, b2, scale: Tensor, mode: int) -> Tensor:

@@ -313,10 +313,19 @@ static int pad_rows(hipnx_ctx *ctx, int esz, int64_t rows, int64_t K, const hipn
   return HIPNX_OK;
 }
 
+// Operands contracted where they lie in a larger tensor, in bytes: from row to row (K-inner) or from k to k (K-outer), and from item
+// to item along the two axes of the batch; `inner` items along the second.
+struct DotView {
+  int64_t inner, ld_l, bs_l, ts_l, ld_r, bs_r, ts_r;
+};
+
 // scale_mode != NONE: the scaled form (out_dt is then f32 over an s32 sum)
+// view: strided operands, whose extents the caller has checked; only what the MFMA kernels take as it lies (otherwise HIPNX_EUNSUPPORTED,
+// and nothing has been launched)
 static int dot_impl(hipnx_ctx *ctx, int l_dt, int r_dt, int out_dt, int64_t batch, int64_t M, int64_t N,
                     int64_t K, int l_layout, int r_layout, const hipnx_buf *l, const hipnx_buf *r,
-                    hipnx_buf *out, int scale_mode, const hipnx_buf *scale) {
+                    hipnx_buf *out, int scale_mode, const hipnx_buf *scale, const DotView *view = nullptr) {
+  if (view && batch > 65535) return set_error(HIPNX_EUNSUPPORTED, "dot_strided: more than 65535 batch items");
   // More batch items than a grid's second dimension holds (100000 small matrices): runs of 65535 items, each over
   // borrowed handles on its part of the three buffers.
   if (batch > 65535 && M > 0 && N > 0 && l && r && out && dtype_size(l_dt) > 0 && dtype_size(r_dt) > 0 && out_dtype_size(out_dt) > 0 && K >= 0) {
@@ -359,6 +368,8 @@ static int dot_impl(hipnx_ctx *ctx, int l_dt, int r_dt, int out_dt, int64_t batc
     if (int st = check_buf(ctx, r, (uint64_t)batch * N * K * dtype_size(r_dt), "dot rhs")) return st;
     if (int st = check_buf(ctx, out, (uint64_t)batch * M * N * out_dtype_size(out_dt), "dot out")) return st;
     if (batch * M * N == 0) return HIPNX_OK;
+    if (view && (l_relay || r_relay || K * dtype_size(l_dt) % 16 != 0))
+      return set_error(HIPNX_EUNSUPPORTED, "dot_strided: operands that the kernels cannot take as they lie");
     if (batch > 65535) return set_error(HIPNX_EUNSUPPORTED, "dot: more than 65535 batch items");
 
     const bool float_pair = l_dt == r_dt && (l_dt == HIPNX_BF16 || l_dt == HIPNX_F16 || l_dt == HIPNX_F32 || l_dt == HIPNX_F64) && is_float(out_dt);
@@ -388,7 +399,7 @@ static int dot_impl(hipnx_ctx *ctx, int l_dt, int r_dt, int out_dt, int64_t batc
     // tile would be all but empty, and its f32 work costs more than the bytes -- [1, 8192] . [8192, 8192]^T 105 us)
     const bool few_vectors = dtype_size(l_dt) >= 4 && dtype_size(r_dt) >= 4 && K >= 1024 &&
                              ((M <= 4 && r_layout == HIPNX_K_INNER) || (N <= 4 && l_layout == HIPNX_K_INNER));
-    if (!scaled && ((M <= 32 && N <= 32 && (K >= 4096 || (M * N <= 4 && K >= 128))) || few_vectors) && M * N <= 65535 && batch * M * N <= 65535 && !(!is_float(l_dt) && !is_float(r_dt) && is_float(out_dt))) {
+    if (!scaled && !view && ((M <= 32 && N <= 32 && (K >= 4096 || (M * N <= 4 && K >= 128))) || few_vectors) && M * N <= 65535 && batch * M * N <= 65535 && !(!is_float(l_dt) && !is_float(r_dt) && is_float(out_dt))) {
       const bool any_float = is_float(l_dt) || is_float(r_dt);
       const int lk = l_layout == HIPNX_K_INNER, rk = r_layout == HIPNX_K_INNER;
       const int64_t l_sm = lk ? K : 1, l_sk = lk ? 1 : M, r_sn = rk ? K : 1, r_sk = rk ? 1 : N;
@@ -425,7 +436,7 @@ static int dot_impl(hipnx_ctx *ctx, int l_dt, int r_dt, int out_dt, int64_t batc
 
     // many small matrices (up to 64 outputs, K up to 64): a lane per output over the whole batch (16 x 16 x 16 items are
     // faster on the tiled kernels: 51 us against 175 us for 8192 of them)
-    if (!scaled && M * N <= 64 && K <= 64 && batch >= 64 && !(!is_float(l_dt) && !is_float(r_dt) && is_float(out_dt))) {
+    if (!scaled && !view && M * N <= 64 && K <= 64 && batch >= 64 && !(!is_float(l_dt) && !is_float(r_dt) && is_float(out_dt))) {
       const bool any_float = is_float(l_dt) || is_float(r_dt);
       const int lk = l_layout == HIPNX_K_INNER, rk = r_layout == HIPNX_K_INNER;
       const int64_t blocks = (batch * M * N + 255) / 256;
@@ -438,6 +449,7 @@ static int dot_impl(hipnx_ctx *ctx, int l_dt, int r_dt, int out_dt, int64_t batc
       return HIPNX_OK;
     }
 
+    if (view && !mfma) return set_error(HIPNX_EUNSUPPORTED, "dot_strided: a contraction that is not for the matrix cores");
     if (!mfma) {
       const bool any_float = is_float(l_dt) || is_float(r_dt);
       if (!any_float && is_float(out_dt)) return set_error(HIPNX_EUNSUPPORTED, "dot: integer operands with a float output");
@@ -545,6 +557,11 @@ static int dot_impl(hipnx_ctx *ctx, int l_dt, int r_dt, int out_dt, int64_t batc
       a.ld_r = !r_kin ? N * esz : r_pad ? pitch : row_bytes;
       a.bs_l = l_pad ? M * pitch : M * row_bytes;
       a.bs_r = r_pad ? N * pitch : N * row_bytes;
+      if (view) {
+        a.ld_l = view->ld_l, a.bs_l = view->bs_l, a.ts_l = view->ts_l;
+        a.ld_r = view->ld_r, a.bs_r = view->bs_r, a.ts_r = view->ts_r;
+        a.batch_inner = (int)view->inner;
+      }
       a.tail_l = (int)(l_kin ? (over + 15) / 16 * 16 : over / esz);
       a.tail_r = (int)(r_kin ? (over + 15) / 16 * 16 : over / esz);
       a.scale = scale_mode != HIPNX_SCALE_NONE ? (const float *)scale->ptr : nullptr;
@@ -641,6 +658,7 @@ static int dot_impl(hipnx_ctx *ctx, int l_dt, int r_dt, int out_dt, int64_t batc
         GemmArgs p = a;
         p.Kb = per_split(splits) * SLAB;
         p.all_slabs = (int)nslab;
+        p.batch_inner = 0;
         p.bs_l = l_kin ? p.Kb : (p.Kb / esz) * a.ld_l;  // split s begins p.Kb bytes (or that many k-rows) further on
         p.bs_r = r_kin ? p.Kb : (p.Kb / esz) * a.ld_r;
         p.out = ws;
@@ -681,6 +699,34 @@ extern "C" int hipnx_dot(hipnx_ctx *ctx, int l_dt, int r_dt, int out_dt, int64_t
                          int64_t K, int l_layout, int r_layout, const hipnx_buf *l, const hipnx_buf *r,
                          hipnx_buf *out) {
   return dot_impl(ctx, l_dt, r_dt, out_dt, batch, M, N, K, l_layout, r_layout, l, r, out, HIPNX_SCALE_NONE, nullptr);
+}
+
+extern "C" int hipnx_dot_strided(hipnx_ctx *ctx, int l_dt, int r_dt, int out_dt, int64_t batch_outer, int64_t batch_inner, int64_t M,
+                                 int64_t N, int64_t K, int l_layout, int r_layout, const int64_t *l_strides, const int64_t *r_strides,
+                                 const hipnx_buf *l, const hipnx_buf *r, hipnx_buf *out) {
+  const int lsz = dtype_size(l_dt), rsz = dtype_size(r_dt);
+  if (lsz < 0 || rsz < 0) return set_error(HIPNX_EINVAL, "dot_strided: unknown element type");
+  if (!l_strides || !r_strides || batch_outer < 0 || batch_inner < 0 || M < 0 || N < 0 || K < 0 || (batch_inner > 0 && batch_outer > INT64_MAX / batch_inner))
+    return set_error(HIPNX_EINVAL, "dot_strided: bad extents or strides");
+  if ((l_layout != HIPNX_K_INNER && l_layout != HIPNX_K_OUTER) || (r_layout != HIPNX_K_INNER && r_layout != HIPNX_K_OUTER))
+    return set_error(HIPNX_EINVAL, "dot_strided: unknown operand layout");
+  const int64_t batch = batch_outer * batch_inner;
+  if (batch * M * N > 0 && K > 0) {
+    Enter in(ctx);
+    if (in.status) return in.status;
+    for (int side = 0; side < 2; side++) {
+      const int64_t *s = side ? r_strides : l_strides, rows = side ? N : M;
+      const bool kin = (side ? r_layout : l_layout) == HIPNX_K_INNER;
+      for (int i = 0; i < 3; i++)
+        if (s[i] < 0 || s[i] > (1ll << 40)) return set_error(HIPNX_EINVAL, "dot_strided: a stride of %lld elements", (long long)s[i]);
+      // runs that overlap within an item, or that are read as neighbours without being ones, are no operand
+      if (s[2] < (kin ? K : rows)) return set_error(HIPNX_EINVAL, "dot_strided: rows of an operand overlap");
+      const int64_t last = (batch_outer - 1) * s[0] + (batch_inner - 1) * s[1] + ((kin ? rows : K) - 1) * s[2] + (kin ? K : rows);
+      if (int st = check_buf(ctx, side ? r : l, (uint64_t)last * (side ? rsz : lsz), side ? "dot_strided rhs" : "dot_strided lhs")) return st;
+    }
+  }
+  const DotView v{batch_inner, l_strides[2] * lsz, l_strides[0] * lsz, l_strides[1] * lsz, r_strides[2] * rsz, r_strides[0] * rsz, r_strides[1] * rsz};
+  return dot_impl(ctx, l_dt, r_dt, out_dt, batch, M, N, K, l_layout, r_layout, l, r, out, HIPNX_SCALE_NONE, nullptr, &v);
 }
 
 extern "C" int hipnx_dot_scaled(hipnx_ctx *ctx, int l_dt, int r_dt, int64_t batch, int64_t M, int64_t N, int64_t K,

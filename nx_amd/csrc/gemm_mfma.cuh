@@ -391,6 +391,10 @@ struct GemmArgs {
   int64_t M, N, Kb;      // Kb = K in bytes, rounded up to whole slabs of 128
   int64_t ld_l, ld_r;    // bytes between consecutive rows (K-inner) or consecutive k (K-outer)
   int64_t bs_l, bs_r;    // bytes between batch items (or between the K ranges of a split)
+  // > 0: the batch is two axes, batch_inner items along the second, ts_l / ts_r bytes apart along it and bs_l / bs_r along the
+  // first (the heads of [batch, positions, heads, dim], contracted where they lie)
+  int batch_inner;
+  int64_t ts_l, ts_r;
   int all_slabs;         // > 0: grid index y is not a batch item but a range of Kb of the all_slabs slabs of K (the last may be shorter)
   // What exists of a partial last slab, 0 = every slab is whole: bytes of each row of a K-inner operand (a multiple of
   // 16), k of a K-outer one.  The kernels walk the partial slab FIRST, in the prologue, where its requests are code of
@@ -405,6 +409,18 @@ struct GemmArgs {
   const float *scale;
   int scale_mode;  // HIPNX_SCALE_NONE / PER_COLUMN (scale[n]) / PER_ROW (scale[m]) / ONE (scale[0])
 };
+
+// where batch item b of the operands begins
+__device__ __forceinline__ void gemm_batch_item(const GemmArgs &a, int b, const unsigned char *&l, const unsigned char *&r) {
+  if (a.batch_inner > 0) {
+    const int outer = b / a.batch_inner, inner = b - outer * a.batch_inner;
+    l = a.l + outer * a.bs_l + inner * a.ts_l;
+    r = a.r + outer * a.bs_r + inner * a.ts_r;
+  } else {
+    l = a.l + b * a.bs_l;
+    r = a.r + b * a.bs_r;
+  }
+}
 
 // Epilogue of one wave: for 16x16 tile (i, j) a lane holds m = 16*i + lane%16 and
 // n = 16*j + 4*(lane/16) + 0..3.  ODT is a compile-time constant here, so the typed stores fold
@@ -735,8 +751,8 @@ gemm_pipelined_kernel(GemmArgs a) {
   int tm, tn;
   gemm_tile_position(a, blockIdx.x, tm, tn);
   const int64_t b = blockIdx.y;
-  const unsigned char *lb = a.l + b * a.bs_l;
-  const unsigned char *rb = a.r + b * a.bs_r;
+  const unsigned char *lb, *rb;
+  gemm_batch_item(a, blockIdx.y, lb, rb);
   const int64_t m0 = (int64_t)tm * BM, n0 = (int64_t)tn * BN;
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;

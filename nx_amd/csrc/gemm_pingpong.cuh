@@ -166,8 +166,8 @@ gemm_pingpong_kernel(GemmArgs a) {
   int tm, tn;
   gemm_tile_position(a, blockIdx.x, tm, tn);
   const int64_t b = blockIdx.y;
-  const unsigned char *lb = a.l + b * a.bs_l;
-  const unsigned char *rb = a.r + b * a.bs_r;
+  const unsigned char *lb, *rb;
+  gemm_batch_item(a, blockIdx.y, lb, rb);
   const int64_t m0 = (int64_t)tm * BM, n0 = (int64_t)tn * BN;
 
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -379,8 +379,8 @@ gemm_pingpong128_kernel(GemmArgs a) {
   int tm, tn;
   gemm_tile_position(a, blockIdx.x, tm, tn);
   const int64_t b = blockIdx.y;
-  const unsigned char *lb = a.l + b * a.bs_l;
-  const unsigned char *rb = a.r + b * a.bs_r;
+  const unsigned char *lb, *rb;
+  gemm_batch_item(a, blockIdx.y, lb, rb);
   const int64_t m0 = (int64_t)tm * BM, n0 = (int64_t)tn * BN;
 
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);

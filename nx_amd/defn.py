@@ -788,6 +788,28 @@ def _absorb_scales(order: List[Tensor], uses) -> int:
     return found
 
 
+def _absorb_transposes(order: List[Tensor], uses) -> int:
+    """dot(transpose(x), ...) becomes one `dot_views` node when nobody else reads the transposed copy: a backend that can
+    contract an operand where it lies makes no copy (the heads split off a projected activation)."""
+    found = 0
+    for node in order:
+        e = node.data
+        if e.op != "dot":
+            continue
+        l, c1, b1, r, c2, b2 = e.args
+        sides = []
+        for t in (l, r):
+            inner = t.data
+            single = isinstance(inner, Expr) and inner.op == "transpose" and inner.scope == 0 and uses.get(inner.id) == 1
+            sides.append((inner.args[0], tuple(inner.args[1])) if single else (t, None))
+        if sides[0][1] is None and sides[1][1] is None:
+            continue
+        (l, l_axes), (r, r_axes) = sides
+        e.op, e.args = "dot_views", [l, l_axes, c1, b1, r, r_axes, c2, b2]
+        found += 1
+    return found
+
+
 def _fuse_planned(roots: List[Tensor]) -> int:
     order, uses, seen, parents = [], {}, set(), {}
 
@@ -818,7 +840,7 @@ def _fuse_planned(roots: List[Tensor]) -> int:
         walk(r)
     if any(t.data.op in ("while", "cond", "elem") for t in order):
         return 0  # bodies of nested scopes read root-scope nodes that the counts above do not see
-    if _absorb_scales(order, uses):
+    if _absorb_scales(order, uses) + _absorb_transposes(order, uses):
         uses.clear()
         seen.clear()
         parents.clear()
@@ -1333,7 +1355,7 @@ class _Scope:
 
 
 # nodes that `apply` does not evaluate as a callback on its evaluated operands
-_EVALUATED_APART = frozenset(["parameter", "elem", "while", "cond", "fused", "dot_scaled", "block"]) | frozenset(CREATION_OPS)
+_EVALUATED_APART = frozenset(["parameter", "elem", "while", "cond", "fused", "dot_scaled", "dot_views", "block"]) | frozenset(CREATION_OPS)
 
 
 class _Run:
@@ -1449,6 +1471,20 @@ class _Run:
                         raise
             summed = mod.dot(out.with_(type=("s", 32)), lv, c1, b1, rv, c2, b2)
             return mod.multiply(out, mod.as_type(out, summed), sv)
+        if op == "dot_views":
+            l, l_axes, c1, b1, r, r_axes, c2, b2 = e.args
+            lv, rv = self.eval(l, scope), self.eval(r, scope)
+            mod, out = self.pick([lv, rv]), x.with_(data=None)
+            one_call = getattr(mod, "dot_views", None)
+            if one_call is not None:
+                try:
+                    return one_call(out, lv, l_axes, c1, b1, rv, r_axes, c2, b2)
+                except Exception as err:  # operands the kernels cannot read where they lie
+                    if getattr(err, "status", None) != _EUNSUPPORTED:
+                        raise
+            lv, rv = (v if axes is None else mod.transpose(v.with_(data=None, shape=tuple(v.shape[a] for a in axes)), v, list(axes))
+                      for v, axes in ((lv, l_axes), (rv, r_axes)))
+            return mod.dot(out, lv, c1, b1, rv, c2, b2)
         if op == "block":
             struct, in_args, fun = e.args
             args = [self.eval(a, scope) for a in in_args]

@@ -1138,3 +1138,85 @@ def test_fused_groups_on_special_values(ty, hip):
                 assert_bits_equal(defn.compile(fun, *args, fuse=True)(*args), want, f"{name}, {ty}, {mode}")
     finally:
         set_mode("interpreted")
+
+
+def split_heads(t, heads):
+    return Nx.transpose(Nx.reshape(t, (t.shape[0], t.shape[1], heads, t.shape[2] // heads)), axes=[0, 2, 1, 3])
+
+
+# scores of heads split off projected activations: whole and partial slabs of K, one query (decoding), odd numbers of keys, every
+# kernel the tile choice can come to; K that is not whole 16-byte pieces is copied as before
+@pytest.mark.parametrize("ty", ["bf16", "f16", "f32", "s8"])
+@pytest.mark.parametrize("batch,heads,queries,keys,dim", [(2, 3, 40, 72, 64), (1, 4, 1, 333, 128), (3, 2, 130, 257, 72), (2, 8, 256, 512, 64),
+                                                          (1, 2, 512, 640, 1024), (2, 2, 17, 65, 33), (1, 1, 24, 48, 64)])
+def test_a_dot_reads_transposed_operands_where_they_lie(batch, heads, queries, keys, dim, ty, hip):
+    rng = np.random.default_rng(seed_of(batch, heads, queries, keys, dim, ty))
+
+    def rand(*shape):
+        if ty == "s8":
+            return from_numpy(rng.integers(-99, 100, size=shape).astype(np.int8), "s8", hip)
+        return rand_float(rng, ty, shape, hip)
+    q, k, p = rand(batch, queries, heads * dim), rand(batch, keys, heads * dim), rand(batch, heads, queries, keys)
+    out = {"out_type": "s32"} if ty == "s8" else {}
+
+    def scores(a, b):
+        return Nx.dot(split_heads(a, heads), [3], [0, 1], split_heads(b, heads), [3], [0, 1], **out)
+
+    def mixed(a, b):  # the right operand K-outer, where it lies (the values of an attention)
+        return Nx.dot(a, [3], [0, 1], split_heads(b, heads), [2], [0, 1], **out)
+    copies = []
+    original = hip.transpose.__func__
+
+    def counting(cls, *a, **kw):
+        copies.append(1)
+        return original(cls, *a, **kw)
+    for fun, args, row_block in ((scores, (q, k), 1), (mixed, (p, k), {"bf16": 8, "f16": 8, "f32": 4, "s8": 16}[ty])):
+        want = defn.compile(fun, *args)(*args)
+        planned = defn.compile(fun, *args, fuse="compiled")
+        assert planned.roots[0].data.op == "dot_views"
+        copies.clear()
+        hip.transpose = classmethod(counting)
+        try:
+            got = planned(*args)
+        finally:
+            hip.transpose = classmethod(original)
+        assert_bits_equal(got, want, f"{fun.__name__} {ty}")
+        esz, K = {"s8": 1, "f32": 4}.get(ty, 2), dim if fun is scores else keys
+        direct = K * esz % 16 == 0 and (fun is scores or dim % row_block == 0) and queries * (keys if fun is scores else dim) >= 256
+        assert (not copies) == direct, (fun.__name__, ty, copies)
+
+
+def test_other_orders_of_a_dots_operands(hip, oracle):
+    """Operands whose kept or contracted axes are not neighbours, three batch axes, a transposed operand with a second reader."""
+    rng = np.random.default_rng(77)
+    a, b = rand_float(rng, "bf16", (4, 32, 6, 64), hip), rand_float(rng, "bf16", (6, 4, 48, 64), hip)
+
+    def apart(x, y):          # kept axes (0, 2) of x are not neighbours in memory once 1 is contracted with 3
+        return Nx.dot(Nx.transpose(x, axes=[1, 3, 0, 2]), [0, 1], Nx.reshape(Nx.transpose(y, axes=[3, 0, 1, 2]), (32, 64, 36)), [0, 1])
+
+    def batched(x, y):        # batch axes in another order on either side
+        return Nx.dot(Nx.transpose(x, axes=[0, 2, 1, 3]), [3], [0, 1], Nx.transpose(y, axes=[1, 0, 2, 3]), [3], [0, 1])
+
+    def read_twice(x, y):
+        t = Nx.transpose(x, axes=[0, 2, 1, 3])
+        return Nx.add(Nx.dot(t, [3], [0, 1], Nx.transpose(y, axes=[1, 0, 2, 3]), [3], [0, 1]), Nx.sum(t))
+    for fun in (apart, batched, read_twice):
+        assert_bits_equal(defn.compile(fun, a, b, fuse="compiled")(a, b), defn.compile(fun, a, b)(a, b), fun.__name__)
+
+
+def test_dot_strided_refuses_what_is_not_there(hip):
+    """Strides that reach past an operand's end, overlapping rows, extents below zero: an error, and nothing is launched."""
+    from nx_amd.backend import K_INNER
+    x = rand_float(np.random.default_rng(1), "bf16", (4, 32, 64), hip)
+    out = rand_float(np.random.default_rng(2), "bf16", (4, 32, 32), hip)
+    good = (0, 32 * 64, 64)
+
+    def call(ls, rs, K=64, M=32, outer=1, inner=4):
+        return L.lib.hipnx_dot_strided(_Context.get(0), T_BF16, T_BF16, T_BF16, outer, inner, M, 32, K, K_INNER, K_INNER,
+                                       L.i64_array(ls), L.i64_array(rs), x.data.ref.handle, x.data.ref.handle, out.data.ref.handle)
+    from nx_amd import types as T
+    T_BF16 = T.code(("bf", 16))
+    assert call(good, good) == 0
+    for bad in ((0, 32 * 64 + 8, 64), (0, 32 * 64, 72), (8, 32 * 64, 64), (0, 32 * 64, 56), (0, -64, 64), (0, 32 * 64, 1 << 41)):
+        assert call(bad, good, outer=2 if bad[0] else 1, inner=4) != 0 and call(good, bad, outer=2 if bad[0] else 1) != 0, bad
+    assert call(good, good, M=-1) != 0 and call(good, good, K=72) != 0
