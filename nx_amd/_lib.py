@@ -7,6 +7,7 @@ from __future__ import annotations
 
 import ctypes as C
 import functools
+import importlib.util
 import os
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
@@ -168,3 +169,11 @@ def broadcast_stride_array(shape: tuple, out_shape: tuple):
 def int_array(values):
     values = list(values)
     return (C.c_int * max(len(values), 1))(*values)
+
+# calls laid out natively (csrc/calls.c): as much part of the library as libhipnx.so, there is no fallback either
+_CALLS_PATH = os.path.join(_HERE, "lib", "hipnx_calls.so")
+if not os.path.exists(_CALLS_PATH):
+    raise ImportError(f"hipnx_calls.so not found at {_CALLS_PATH}: build it first (make -C nx_amd/csrc)")
+_spec = importlib.util.spec_from_file_location("hipnx_calls", _CALLS_PATH)
+native = importlib.util.module_from_spec(_spec)
+_spec.loader.exec_module(native)

@@ -20,6 +20,7 @@ from math import prod
 import numpy as np
 
 from . import _lib as L
+from ._lib import native
 from . import shape as S
 from . import types as T
 from .tensor import Tensor, number_to_binary, pack_sub_byte, unpack_sub_byte, wrap_to_type
@@ -69,51 +70,36 @@ class _Context:
             return ctx
 
 
-class _Ref:
-    """Owns one device buffer.  Metadata-only callbacks (reshape / squeeze / bitcast) share it;
-    it is deallocated when the last sharer is, or by the garbage collector."""
-
-    __slots__ = ("ctx", "handle", "nbytes", "sharers", "keep")
-
-    def __init__(self, ctx, nbytes: int, address=None, keep=None, ipc_handle=None):
-        self.ctx = ctx
-        self.handle = C.c_void_p()
-        self.nbytes = nbytes
-        self.sharers = 1
-        self.keep = keep  # the owner of borrowed memory, kept alive with the handle
-        if ipc_handle is not None:  # another process's device memory, opened through its IPC handle
-            raw = C.create_string_buffer(bytes(ipc_handle), L.IPC_HANDLE_BYTES)
-            L.check(L.lib.hipnx_buf_ipc_import(ctx, raw, nbytes, C.byref(self.handle)))
-        elif address is None:
-            L.check(L.lib.hipnx_buf_alloc(ctx, nbytes, C.byref(self.handle)))
-        else:  # someone else's device memory: the handle never frees it
-            L.check(L.lib.hipnx_buf_wrap(ctx, C.c_void_p(address), nbytes, C.byref(self.handle)))
-
-    def __del__(self, _destroy=L.lib.hipnx_buf_destroy):
-        try:
-            handle = self.handle
-        except AttributeError:  # the constructor raised before it had one
-            return
-        if handle is not None and handle.value:
-            try:
-                _destroy(handle)
-            except Exception:  # interpreter shutdown
-                pass
-            self.handle = None
+# Owns one device buffer (csrc/calls.c).  Metadata-only callbacks (reshape / squeeze / bitcast) share it;
+# it is deallocated when the last sharer is, or by the garbage collector.
+_Ref = native.Ref
 
 
-def _fresh_ref(ctx, nbytes: int, _new=object.__new__, _alloc=L.lib.hipnx_buf_alloc, _byref=C.byref, _handle=C.c_void_p) -> _Ref:
-    """A buffer of the pool for a callback's result: `_Ref(ctx, nbytes)` without the argument handling of the
-    general constructor (every callback allocates one)."""
-    ref = _new(_Ref)
-    ref.ctx = ctx
-    ref.handle = handle = _handle()
-    ref.nbytes = nbytes
-    ref.sharers = 1
-    ref.keep = None
-    status = _alloc(ctx, nbytes, _byref(handle))
-    if status:
-        L.check(status)
+def _wrapped_ref(ctx, nbytes: int, address, keep=None) -> _Ref:
+    """Someone else's device memory: the handle never frees it.  `keep`: its owner, kept alive with the handle."""
+    handle = C.c_void_p()
+    L.check(L.lib.hipnx_buf_wrap(ctx, C.c_void_p(address), nbytes, C.byref(handle)))
+    return _Ref(ctx, handle.value, nbytes, keep)
+
+
+def _imported_ref(ctx, nbytes: int, ipc_handle) -> _Ref:
+    """Another process's device memory, opened through its IPC handle."""
+    handle = C.c_void_p()
+    raw = C.create_string_buffer(bytes(ipc_handle), L.IPC_HANDLE_BYTES)
+    L.check(L.lib.hipnx_buf_ipc_import(ctx, raw, nbytes, C.byref(handle)))
+    return _Ref(ctx, handle.value, nbytes)
+
+
+_recorder = [None]  # the recording of a traced function that is going on, if any
+
+
+def _fresh_ref(ctx, nbytes: int, _fresh=native.fresh) -> _Ref:
+    """A buffer of the pool for a callback's result."""
+    ref = _fresh(ctx, ctx.value, nbytes)
+    if ref.__class__ is int:
+        L.check(ref)
+    if _recorder[0] is not None:
+        _recorder[0].allocated(ref)
     return ref
 
 
@@ -401,6 +387,50 @@ class HipNxBackend:
         if status:
             L.check(status)
         return cls._narrow(res) if narrow else res
+
+    @classmethod
+    def prepared(cls, kind: str, name, out: Tensor, *args):
+        """A callable that issues this callback again on tensors of the same types and shapes (csrc/calls.c), or None
+        where the callback is more than one library call.  The front end keeps it per signature, under the present settings."""
+        tensors = [a for a in args if isinstance(a, Tensor)]
+        device = tensors[0].data.device
+        if any(t.data.__class__ is not cls or t.data.device != device or t.type[1] < 8 for t in tensors) or out.type[1] < 8:
+            return None
+        ctx, opts, arrays = _Context.get(device), args[-1], ()
+        if kind == "binary":
+            plan = _binary_plans.get((args[0].type, args[0].shape, args[1].type, args[1].shape, out.type, out.shape))
+            if plan is None:
+                return None
+            lc, rc, oc, rank, dims, ls, rs, _, _ = plan
+            arrays = (dims, ls, rs)
+            fn, laid = "hipnx_binary", [BINARY_OPS.index(name), lc, rc, oc, rank] + [C.addressof(a) for a in arrays]
+        elif kind == "unary":
+            fn, laid = "hipnx_unary", [UNARY_OPS.index(name), T.code(args[0].type), T.code(out.type), out.size]
+        elif kind == "reduce":
+            axes = opts.get("axes")
+            plan = _reduce_plans.get((args[0].type, args[0].shape, out.type, None if axes is None else tuple(axes)))
+            if plan is None:
+                return None
+            fn, laid = "hipnx_reduce", [_REDUCTIONS[name]] + list(plan[:5])
+        elif kind == "argreduce":
+            axis = opts.get("axis")
+            _, outer, red, inner = cls._view_for_axes(args[0], None if axis is None else [axis])
+            fn, laid = "hipnx_argreduce", [("argmax", "argmin").index(name), ("low", "high").index(opts["tie_break"]), T.code(args[0].type),
+                                           T.code(out.type), outer, red, inner]
+        elif kind == "dot":
+            l, c1, b1, r, c2, _ = args
+            _, _, _, K, batch, ((l_layout, M), (r_layout, N)) = cls._dot_plans[(l.shape, tuple(c1), len(b1), r.shape, tuple(c2))]
+            if l_layout is None or r_layout is None:
+                return None
+            fn, laid = "hipnx_dot", [T.code(l.type), T.code(r.type), _out_code(out.type), batch, M, N, K, l_layout, r_layout]
+        else:  # "take": whole entries of the first axis
+            t, indices = tensors
+            arrays = (L.i64_array(t.shape),)
+            fn, laid = "hipnx_gather", [T.size_bytes(t.type), len(t.shape), C.addressof(arrays[0]), T.code(indices.type), indices.size, 1, _bounds["policy"]]
+        laid = [ctx.value] + laid
+        first, n = len(laid), len(tensors)
+        return native.prepare(C.cast(getattr(L.lib, fn), C.c_void_p).value, laid + [0] * (n + 1), list(range(first, first + n)), first + n,
+                              out.size * T.size_bytes(out.type), ctx, ctx.value, device, out.type, out.shape, out.names, arrays)
 
     @classmethod
     def _unary(cls, op: int, out: Tensor, t: Tensor) -> Tensor:
@@ -1041,11 +1071,11 @@ class HipNxBackend:
         if pointer.kind == "ipc":
             if pointer.handle is None or len(pointer.handle) != L.IPC_HANDLE_BYTES:
                 raise ValueError(f"an :ipc pointer carries a handle of {L.IPC_HANDLE_BYTES} bytes")
-            ref = _Ref(_Context.get(backend_opts["device"]), size, ipc_handle=pointer.handle)
+            ref = _imported_ref(_Context.get(backend_opts["device"]), size, pointer.handle)
             return Tensor(cls(ref, backend_opts["device"]), ty, tuple(shape), tuple(opts.get("names") or ()))
         if pointer.kind != "local":
             raise ValueError(f"expected a pointer of kind :local or :ipc, got: {pointer.kind!r}")
-        ref = _Ref(_Context.get(backend_opts["device"]), size, address=pointer.address, keep=opts.get("keep"))
+        ref = _wrapped_ref(_Context.get(backend_opts["device"]), size, pointer.address, keep=opts.get("keep"))
         return Tensor(cls(ref, backend_opts["device"]), ty, tuple(shape), tuple(opts.get("names") or ()))
 
     @classmethod
@@ -1096,7 +1126,7 @@ class HipNxBackend:
         for t in inputs:
             if t.data.released:
                 raise L.HipNxError(L.EFREED, "tensor has been deallocated")
-        handles = handle_array(*[t.data.ref.handle.value for t in inputs])
+        handles = handle_array(*[t.data.ref.handle for t in inputs])
         ctx = _Context.get(dev)
         ref = _fresh_ref(ctx, nbytes)
         status = L.lib.hipnx_fused_elementwise(ctx, len(program), prog_ptr, len(inputs), handles, dts, rs, cs, rows, cols,
@@ -1166,6 +1196,7 @@ def _install():
 
 
 _install()
+native.setup(C.cast(L.lib.hipnx_buf_alloc, C.c_void_p).value, C.cast(L.lib.hipnx_buf_destroy, C.c_void_p).value, Tensor, HipNxBackend)
 
 
 def sync(device: int = 0) -> None:
@@ -1258,6 +1289,7 @@ def bounds_policy(policy: str) -> str:
         raise ValueError(f"expected one of {sorted(names)!r}, got: {policy!r}")
     previous = next(k for k, v in names.items() if v == _bounds["policy"])
     _bounds["policy"] = names[policy]
+    _settings_changed()
     return previous
 
 
@@ -1271,7 +1303,22 @@ def bf16_rounding(mode: str) -> str:
         raise ValueError(f'expected "truncate" or "nearest_even", got: {mode!r}')
     previous = _bf16["rounding"]
     _bf16["rounding"] = mode
+    _settings_changed()
     return previous
+
+
+_epoch = [0]
+
+
+def settings_epoch() -> int:
+    """Grows with every change of a setting that calls are laid out under (bounds policy, bf16 rounding, fused mode)."""
+    return _epoch[0]
+
+
+def _settings_changed() -> None:
+    from . import nx
+    _epoch[0] += 1
+    nx._ready.clear()
 
 
 def fused_mode(mode: str, device: int = 0) -> None:
@@ -1280,6 +1327,7 @@ def fused_mode(mode: str, device: int = 0) -> None:
     first use, and kept).  Results are bit-identical."""
     _set_fused_mode(mode, device)
     _fused_modes[device] = mode
+    _settings_changed()
 
 
 def _set_fused_mode(mode: str, device: int) -> None:
@@ -1309,6 +1357,7 @@ def _advise_huge_pages(address: int, n: int) -> None:
         lo, hi = (address + huge - 1) & ~(huge - 1), (address + n) & ~(huge - 1)
         if hi > lo:
             _libc.madvise(C.c_void_p(lo), hi - lo, 14)  # MADV_HUGEPAGE
+_REDUCTIONS = {"sum": RED_SUM, "product": RED_PRODUCT, "reduce_max": RED_MAX, "reduce_min": RED_MIN, "all": RED_ALL, "any": RED_ANY}
 _reduce_plans = {}  # (types, shape and axes of a reduction callback) -> its type codes, [outer, red, inner] view, result bytes
 _binary_plans = {}  # (types and shapes of a binary callback) -> its type codes, shape and stride arrays, result bytes
 _fused_modes = {}  # device -> the mode chosen with fused_mode/2: what a call that names none runs in

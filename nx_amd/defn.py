@@ -21,6 +21,7 @@ from __future__ import annotations
 import math
 import itertools
 import operator
+import sys
 import threading
 from math import prod
 from typing import Any, Callable, Dict, List, Optional, Tuple
@@ -1517,6 +1518,9 @@ class _Run:
         return self.backend[0] if mod is HostBinary else mod
 
 
+_RECORD_AT = 3
+
+
 class Compiled:
     """A traced function: call it with arguments of the traced shapes and types."""
 
@@ -1525,6 +1529,7 @@ class Compiled:
         self.n_params = len(templates)
         self.plans: Dict[Any, _Plan] = {}
         self.plan = _Plan(roots, 0, self.plans)
+        self.calls, self.replay = 0, None
 
     def _params(self, args):
         leaves: list = []
@@ -1538,6 +1543,21 @@ class Compiled:
         return params
 
     def _evaluate(self, params):
+        """Through the recorded library calls where there is a recording that applies (replay.py): the third evaluation is
+        recorded, by which time every program is compiled and every fallback has been found."""
+        if self.replay is not None:
+            results = self.replay.run(params)
+            if results is not None:
+                return results
+        self.calls += 1
+        if self.calls == _RECORD_AT and (backend := sys.modules.get(__package__ + ".backend")) is not None:
+            if all(p.data.__class__ is backend.HipNxBackend for p in params):
+                from .replay import record
+                results, self.replay = record(self._walk, params)
+                return results
+        return self._walk(params)
+
+    def _walk(self, params):
         run = _Run(self.plans, _runtime_backend(params))
         root = _Scope(self.plan, None, params)
         results = []

@@ -206,11 +206,40 @@ _PRED = ["equal", "not_equal", "greater", "less", "greater_equal", "less_equal",
          "logical_xor"]
 
 
+# Calls the backend has laid out for operands of these types and shapes, by front-end function and arguments (a backend that offers
+# `prepared`): the front end's and the backend's work on types, axes and layouts is a function of these alone.  A call that
+# does not apply to the operands it is given (on another backend or device, deallocated) or is refused answers None and the
+# general path takes over.
+_ready = {}
+
+
+def _make_ready(key, mod, *args):
+    if "prepared" in mod.__dict__:  # (not asked of the expression builder, to which any name is an operation)
+        if len(_ready) >= 4096:
+            _ready.clear()
+        call = mod.prepared(*args)
+        if call is not None:
+            _ready[key] = call
+
+
 def _number_or_type(x):
     return x if isinstance(x, (int, float)) and not isinstance(x, bool) else to_tensor(x).type
 
 
 def _binary(name, left, right, out_type_fun):
+    key = None
+    if left.__class__ is Tensor:
+        if right.__class__ is Tensor:
+            key, r = (name, left.type, left.shape, right.type, right.shape), right
+        # (the type of a result with a number depends on what kind of number it is; beside an integer tensor on its sign)
+        elif right.__class__ is float or (right.__class__ is int and left.type[0] != "u" and left.type[0] != "s"):
+            key, r = (name, left.type, left.shape, right.__class__), None
+        if key is not None:
+            ready = _ready.get(key)
+            if ready is not None:
+                out = ready(left, to_tensor(right) if r is None else r)
+                if out is not None:
+                    return out
     if left.__class__ is Tensor and right.__class__ is Tensor:  # the common case: no number to look at
         ty = left.type if left.type == right.type else T.merge(left.type, right.type)
         l, r = left, right
@@ -220,7 +249,12 @@ def _binary(name, left, right, out_type_fun):
     ls, rs = l.shape, r.shape
     out = template(out_type_fun(ty), ls if ls == rs or rs == () else rs if ls == () else S.binary_broadcast(ls, rs))
     lb, rb = l.data.__class__, r.data.__class__
-    return getattr(lb if lb is rb else _impl(l, r), name)(out, l, r)
+    if lb is not rb:
+        return getattr(_impl(l, r), name)(out, l, r)
+    res = getattr(lb, name)(out, l, r)
+    if key is not None:
+        _make_ready(key, lb, "binary", name, out, l, r)
+    return res
 
 
 def _def_binary():
@@ -253,7 +287,17 @@ def _def_unary():
     for name in _MATH:  # nx.ex:8592-8598: out type = to_floating
         def math_fun(t, _n=name):
             t = to_tensor(t)
-            return getattr(_impl(t), _n)(t.with_(data=None, type=T.to_floating(t.type)), t)
+            key = (_n, t.type, t.shape, t.names)
+            ready = _ready.get(key)
+            if ready is not None:
+                res = ready(t)
+                if res is not None:
+                    return res
+            mod, out = _impl(t), t.with_(data=None, type=T.to_floating(t.type))
+            res = getattr(mod, _n)(out, t)
+            if mod is t.data.__class__:
+                _make_ready(key, mod, "unary", _n, out, t)
+            return res
         g[name] = math_fun
     for name in ["negate", "sign"]:  # nx.ex:8703-8731
         g[name] = (lambda n: lambda t: getattr(_impl(to_tensor(t)), n)(to_tensor(t).with_(data=None), to_tensor(t)))(name)
@@ -297,6 +341,11 @@ def _aggregate(t, op, out_type, axes=None, keep_axes=False):
     # the axes and the result's shape depend on the shape and the options only: worked out once per signature
     try:
         key = (t.shape, axes if axes is None else tuple(axes), keep_axes)
+        ready = _ready.get((op, t.type, out_type) + key)
+        if ready is not None:
+            res = ready(t)
+            if res is not None:
+                return res
         known = _aggregate_shapes.get(key)
     except TypeError:  # axes that are no list of integers: the checks below say so
         key = known = None
@@ -316,7 +365,11 @@ def _aggregate(t, op, out_type, axes=None, keep_axes=False):
     axes, shape_ = known
     if axes == []:
         return as_type(t, out_type)
-    return getattr(t.data.__class__, op)(template(out_type, shape_), t, {"axes": None if axes is None else list(axes), "keep_axes": keep_axes})
+    mod, out, opts = t.data.__class__, template(out_type, shape_), {"axes": None if axes is None else list(axes), "keep_axes": keep_axes}
+    res = getattr(mod, op)(out, t, opts)
+    if key is not None:
+        _make_ready((op, t.type, out_type) + key, mod, "reduce", op, out, t, opts)
+    return res
 
 
 _aggregate_shapes = {}  # (shape, axes, keep_axes) -> (normalised axes, shape of the result)
@@ -355,13 +408,22 @@ def _argmin_or_max(t, op, axis=None, tie_break="low", keep_axis=False, type=("s"
     if tie_break not in ("low", "high"):
         raise ValueError(f"unknown value for :tie_break, expected :high or :low, got: {tie_break!r}")
     t = to_tensor(t)
+    key = (op, t.type, t.shape, axis, tie_break, keep_axis, type) if axis is None or axis.__class__ is int else None
+    ready = _ready.get(key)
+    if ready is not None:
+        res = ready(t)
+        if res is not None:
+            return res
     if axis is not None:
         axis = S.normalize_axis(t.shape, axis)
         shape_ = S.contract(t.shape, [axis], keep_axis)
     else:
         shape_ = ()
-    out = template(T.normalize(type), shape_)
-    return getattr(_impl(t), op)(out, t, {"tie_break": tie_break, "axis": axis, "keep_axis": keep_axis})
+    mod, out, opts = _impl(t), template(T.normalize(type), shape_), {"tie_break": tie_break, "axis": axis, "keep_axis": keep_axis}
+    res = getattr(mod, op)(out, t, opts)
+    if key is not None and mod is t.data.__class__:
+        _make_ready(key, mod, "argreduce", op, out, t, opts)
+    return res
 
 
 def argmax(t, **opts):
@@ -380,34 +442,51 @@ def dot(t1, *args, out_type=None):
     `out_type` is not part of the reference's front end: it sets the template type handed to the
     `dot` callback (both reference backends honour `out.type` whatever the operand types,
     binary_backend.ex:549-559) and is how a s8 x s8 -> s32 contraction is requested."""
+    try:
+        key = ("dot", out_type, t1.type, t1.shape) + tuple([(a.type, a.shape) if a.__class__ is Tensor else tuple(a) for a in args])
+        ready = _ready.get(key)
+    except (TypeError, AttributeError):  # numbers, axes that are no lists of integers: the general path and its checks
+        return _dot(t1, args, out_type, None)
+    if ready is not None:
+        res = ready(t1, args[0] if len(args) == 1 else args[len(args) // 2])
+        if res is not None:
+            return res
+    return _dot(t1, args, out_type, key)
+
+
+def _dot(t1, args, out_type, key):
     if len(args) == 1:
         t1, t2 = to_tensor(t1), to_tensor(args[0])
         n, m = len(t1.shape), len(t2.shape)
         if n == 0 or m == 0:
             return globals()["multiply"](t1, t2)
         if m == 1:
-            return dot(t1, [n - 1], [], t2, [0], [], out_type=out_type)
+            return _dot(t1, ([n - 1], [], t2, [0], []), out_type, key)
         if n == 1:
-            return dot(t1, [0], [], t2, [m - 2], [], out_type=out_type)
-        return dot(t1, [n - 1], [], t2, [m - 2], [], out_type=out_type)
+            return _dot(t1, ([0], [], t2, [m - 2], []), out_type, key)
+        return _dot(t1, ([n - 1], [], t2, [m - 2], []), out_type, key)
     if len(args) == 3:
         c1, t2, c2 = args
-        return dot(t1, c1, [], t2, c2, [], out_type=out_type)
+        return _dot(t1, (c1, [], t2, c2, []), out_type, key)
     c1, b1, t2, c2, b2 = args
     t1, t2 = to_tensor(t1), to_tensor(t2)
     ty = T.normalize(out_type) if out_type is not None else T.binary_type(t1.type, t2.type)
     # the axes and the output shape depend on the shapes and the axes given only: worked out once per signature
-    key = (t1.shape, tuple(c1), tuple(b1), t2.shape, tuple(c2), tuple(b2))
-    plan = _DOT_PLANS.get(key)
+    signature = (t1.shape, tuple(c1), tuple(b1), t2.shape, tuple(c2), tuple(b2))
+    plan = _DOT_PLANS.get(signature)
     if plan is None:
         n1, n2 = S.normalize_axes(t1.shape, c1), S.normalize_axes(t2.shape, c2)
         m1, m2 = S.normalize_axes(t1.shape, b1), S.normalize_axes(t2.shape, b2)
         plan = (n1, m1, n2, m2, S.dot(t1.shape, n1, m1, t2.shape, n2, m2))
         if len(_DOT_PLANS) >= 4096:
             _DOT_PLANS.clear()
-        _DOT_PLANS[key] = plan
+        _DOT_PLANS[signature] = plan
     c1, b1, c2, b2, shape = plan
-    return _impl(t1, t2).dot(template(ty, shape), t1, c1, b1, t2, c2, b2)
+    mod, out = _impl(t1, t2), template(ty, shape)
+    res = mod.dot(out, t1, c1, b1, t2, c2, b2)
+    if key is not None and mod is t1.data.__class__ and mod is t2.data.__class__:
+        _make_ready(key, mod, "dot", "dot", out, t1, c1, b1, t2, c2, b2)
+    return res
 
 
 _DOT_PLANS = {}
@@ -575,6 +654,12 @@ def take(t, indices, axis=0):
     """Nx.take/3 (nx.ex:14732-14821), non-vectorised path: wraps the default gather-based
     implementation in a `Nx.Block.Take` so a backend can do it natively."""
     t, indices = to_tensor(t), to_tensor(indices)
+    key = ("take", t.type, t.shape, indices.type, indices.shape) if axis.__class__ is int and axis == 0 else None
+    ready = _ready.get(key)
+    if ready is not None:
+        res = ready(t, indices)
+        if res is not None:
+            return res
     if not T.is_integer(indices.type):
         raise ValueError(f"indices must be an integer tensor, got {indices.type!r}")
     axis = S.normalize_axis(t.shape, axis)
@@ -589,7 +674,10 @@ def take(t, indices, axis=0):
         leading, trailing = tensor_axes[:axis], tensor_axes[axis:]
         return transpose(gather(tensor_, gather_indices, axes=[axis]), leading + indices_axes + trailing)
 
-    return block(BlockTake(axis), [t, indices], out, default)
+    res = block(BlockTake(axis), [t, indices], out, default)
+    if key is not None and t.data.__class__ is indices.data.__class__:
+        _make_ready(key, t.data.__class__, "take", "take", out, t, indices)
+    return res
 
 
 # ---- one step off the hot path: creation, selection, windows -------------------------------------

@@ -1220,3 +1220,190 @@ def test_dot_strided_refuses_what_is_not_there(hip):
     for bad in ((0, 32 * 64 + 8, 64), (0, 32 * 64, 72), (8, 32 * 64, 64), (0, 32 * 64, 56), (0, -64, 64), (0, 32 * 64, 1 << 41)):
         assert call(bad, good, outer=2 if bad[0] else 1, inner=4) != 0 and call(good, bad, outer=2 if bad[0] else 1) != 0, bad
     assert call(good, good, M=-1) != 0 and call(good, good, K=72) != 0
+
+
+# ---- traced functions and callbacks issued natively (nx_amd/replay.py, csrc/calls.c) ----------------------
+
+def replayed_functions(hip):
+    rng = np.random.default_rng(99)
+
+    def r(*shape, ty="f32"):
+        return lambda: rand_float(rng, ty, shape, hip)
+
+    def words(*shape):
+        return lambda: from_numpy(rng.integers(0, 2 ** 32, size=shape, dtype=np.uint32), "u32", hip)
+
+    def normalised(x, g):
+        return centred_and_scaled(x, g), Nx.sum(x, axes=[0]), Nx.add(Nx.multiply(x, 0.5), 3)
+
+    def step(x, w, b):
+        h = Nx.max(Nx.add(Nx.dot(x, w), b), 0.0)
+        return Nx.subtract(w, Nx.multiply(Nx.dot(x, [0], h, [0]), 0.1)), Nx.mean(h)
+
+    def moved(x):
+        return Nx.concatenate([Nx.reverse(x, axes=[1]), Nx.transpose(Nx.transpose(x))], axis=0), Nx.slice_along_axis(x, 1, 2, axis=1), Nx.select(Nx.greater(x, 0.0), x, 0.0)
+
+    def picked(x, t):
+        best = Nx.argmax(x, axis=1, type="u32")
+        return best, Nx.take(t, best)
+    return {"normalised": (normalised, [r(9, 24), r(24)]), "softmax": (softmax_rows, [r(6, 33, ty="bf16")]), "step": (step, [r(16, 24), r(24, 40), r(40)]),
+            "moved": (moved, [r(5, 8)]), "picked": (picked, [r(7, 50), r(50, 16, ty="bf16")]),
+            "normal": (lambda k: Random.normal(k, shape=(1001,))[0], [words(2)])}
+
+
+@pytest.mark.parametrize("name", ["normalised", "softmax", "step", "moved", "picked", "normal"])
+def test_a_recorded_function_gives_each_call_its_own_results(name, hip):
+    """Every call after the recording on operands of its own, earlier results kept, dropped and deallocated in between: the
+    bits of the nodes one by one, results in buffers of their own, and no memory that stays behind."""
+    fun, makers = replayed_functions(hip)[name]
+    planned = defn.compile(fun, *[m() for m in makers], fuse="compiled")
+    plain = defn.compile(fun, *[m() for m in makers])
+    kept, wanted = [], []
+    for i in range(9):
+        args = [m() for m in makers]
+        want = plain._walk(args)
+        got = planned._evaluate(args)
+        for g, w in zip(got, want):
+            assert_bits_equal(g, w, f"{name}, call {i}")
+        kept.append(got)
+        wanted.append(want)
+        if i == 5:
+            for t in kept.pop(0):
+                assert Nx.backend_deallocate(t) == "ok" and Nx.backend_deallocate(t) == "already_deallocated"
+            wanted.pop(0)
+    assert planned.replay is not None, "not recorded"
+    for got, want in zip(kept, wanted):
+        for g, w in zip(got, want):
+            assert_bits_equal(g, w, f"{name}, kept")
+    assert len({Nx.to_pointer(t).address for got in kept for t in got}) == sum(len(got) for got in kept)
+    args = [m() for m in makers]
+    del kept, wanted, got, want, g, w
+    gc.collect()
+    planned._evaluate(args)
+    before = mem_stats()["live"]
+    for _ in range(5):
+        planned._evaluate(args)
+    assert mem_stats()["live"] == before
+
+
+def test_a_recording_is_left_where_it_does_not_apply(hip):
+    from nx_amd import HostBinary
+    from nx_amd import backend as B
+
+    def fun(x, t):
+        return Nx.as_type(x, "bf16"), Nx.take(t, Nx.as_type(Nx.reduce_max(x, axes=[1]), "s32"))
+    x = from_numpy(np.arange(12, dtype=np.float32).reshape(3, 4) / 4 + 0.1234, "f32", hip)
+    t = rand_float(np.random.default_rng(3), "f32", (4, 8), hip)
+    planned, plain = defn.compile(fun, x, t, fuse="compiled"), defn.compile(fun, x, t)
+    for _ in range(5):
+        planned(x, t)
+    assert planned.replay is not None
+
+    def same(*args):
+        for g, w in zip(planned._evaluate(list(args)), plain._walk(list(args))):
+            assert_bits_equal(g, w, "")
+    same(x, t)
+    previous = B.bf16_rounding("nearest_even")     # a setting the calls were laid out under
+    try:
+        same(x, t)
+    finally:
+        B.bf16_rounding(previous)
+    same(x, Nx.backend_copy(t, HostBinary, {}))   # an operand elsewhere
+    far = from_numpy(np.full((3, 4), 77.0, dtype=np.float32), "f32", hip)
+    for _ in range(2):                              # what the library refuses is reported as ever
+        with pytest.raises(Exception, match="index 77 is out of bounds"):
+            planned(far, t)
+    previous = B.bounds_policy("clamp")
+    try:
+        same(far, t)
+    finally:
+        B.bounds_policy(previous)
+    gone = Nx.backend_copy(x, hip, {"device": 0})
+    Nx.backend_deallocate(gone)
+    with pytest.raises(L.HipNxError):
+        planned(gone, t)
+    same(x, t)
+    with pytest.raises(ValueError):
+        planned(t, x)
+
+
+def test_what_cannot_be_recorded_is_evaluated(hip):
+    """One buffer under two parameters when the recording would be made, parameters and constants handed through, one buffer
+    under two results, control flow."""
+    x = rand_float(np.random.default_rng(5), "f32", (4, 8), hip)
+    y = rand_float(np.random.default_rng(6), "f32", (4, 8), hip)
+    twice = defn.compile(lambda a, b: Nx.subtract(Nx.multiply(a, 2.0), b), x, y, fuse="compiled")
+    for _ in range(5):
+        twice(x, x)
+    assert twice.replay is None
+    assert_bits_equal(twice(x, y), Nx.subtract(Nx.multiply(x, 2.0), y), "other operands afterwards")
+    for fun in (lambda a: (a, Nx.exp(a)), lambda a: (lambda e: (e, Nx.reshape(e, (32,))))(Nx.exp(a)),
+                lambda a: defn.cond(Nx.greater(Nx.sum(a), 1.0e9), lambda: Nx.negate(a), lambda: Nx.exp(a))):
+        planned, plain = defn.compile(fun, x), defn.compile(fun, x)
+        for i in range(6):
+            z = rand_float(np.random.default_rng(i), "f32", (4, 8), hip)
+            for g, w in zip(planned._evaluate([z]), plain._walk([z])):
+                assert_bits_equal(g, w, "")
+        assert planned.replay is None
+
+
+def test_recorded_functions_and_callbacks_from_several_threads(hip):
+    import threading
+    rng = np.random.default_rng(8)
+    x, g = rand_float(rng, "f32", (33, 40), hip), rand_float(rng, "f32", (40,), hip)
+    planned = defn.compile(centred_and_scaled, x, g, fuse="compiled")
+    inputs = [rand_float(rng, "f32", (33, 40), hip) for _ in range(4)]
+    wants = [defn.compile(centred_and_scaled, x, g)(i, g) for i in inputs]
+    eager = [Nx.sum(Nx.exp(Nx.multiply(Nx.add(i, i), 0.5)), axes=[1]) for i in inputs]
+    errors = []
+
+    def work(k):
+        try:
+            for _ in range(40):  # (the recording happens while the others evaluate)
+                assert_bits_equal(planned(inputs[k], g), wants[k], f"thread {k}")
+                assert_bits_equal(Nx.sum(Nx.exp(Nx.multiply(Nx.add(inputs[k], inputs[k]), 0.5)), axes=[1]), eager[k], f"thread {k}, eager")
+        except BaseException as e:  # noqa: BLE001
+            errors.append(e)
+    threads = [threading.Thread(target=work, args=(k,)) for k in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not errors, errors[0]
+
+
+def test_callbacks_laid_out_once_follow_their_operands(hip):
+    """The same signature again and again: numbers that change, operands elsewhere or gone, settings that change."""
+    from nx_amd import backend as B
+    x = rand_float(np.random.default_rng(1), "f32", (6, 10), hip)
+    v = hip.to_numpy(x)
+    for c in (0.5, -3.25, 0.0, -0.0, 7.0):
+        np.testing.assert_array_equal(hip.to_numpy(Nx.multiply(x, c)).view(np.uint32), (v * np.float32(c)).view(np.uint32))
+        np.testing.assert_array_equal(hip.to_numpy(Nx.add(x, int(c))), v + np.float32(int(c)))
+    u = from_numpy(np.arange(60, dtype=np.uint8).reshape(6, 10), "u8", hip)
+    assert Nx.add(u, 1).type == ("u", 8) and Nx.add(u, -1).type == ("s", 16) and Nx.add(u, 1.5).type == ("f", 32)
+    gone = Nx.backend_copy(x, hip, {"device": 0})
+    Nx.add(gone, x)
+    Nx.backend_deallocate(gone)
+    for call in (lambda: Nx.add(gone, x), lambda: Nx.exp(gone), lambda: Nx.sum(gone, axes=[1]), lambda: Nx.argmax(gone, axis=1), lambda: Nx.dot(gone, Nx.transpose(x))):
+        with pytest.raises(L.HipNxError):
+            call()
+    t = rand_float(np.random.default_rng(2), "f32", (5, 4), hip)
+    near, far = from_numpy(np.array([1, 4], np.int32), "s32", hip), from_numpy(np.array([1, 9], np.int32), "s32", hip)
+    Nx.take(t, near)
+    with pytest.raises(Exception, match="index 9 is out of bounds"):
+        Nx.take(t, far)
+    previous = B.bounds_policy("clamp")
+    try:
+        np.testing.assert_array_equal(hip.to_numpy(Nx.take(t, far)), hip.to_numpy(t)[[1, 4]])
+    finally:
+        B.bounds_policy(previous)
+    b = from_numpy(np.array([[1.01, 1.0], [1.0, 1.0]], np.float32), "f32", hip)
+    y = Nx.as_type(b, "bf16")
+    for mode in ("truncate", "nearest_even", "truncate"):
+        previous = B.bf16_rounding(mode)
+        try:
+            want = defn.compile(lambda p, q: Nx.dot(p, [1], q, [0]), y, y)._walk([y, y])[0]
+            assert_bits_equal(Nx.dot(y, [1], y, [0]), want, mode)
+        finally:
+            B.bf16_rounding(previous)
