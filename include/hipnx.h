@@ -360,6 +360,8 @@ int hipnx_narrow_int(hipnx_ctx *ctx, hipnx_buf *buf, int64_t n, int bits, int is
  * counter whose output is dropped).  Not a Nx.Backend callback: a binding calls it from its
  * own random module when the key lives on the device. */
 int hipnx_threefry2x32(hipnx_ctx *ctx, const hipnx_buf *key, int64_t n, hipnx_buf *out);
+/* key number `index` of the `parts` that Nx.Random.split makes of a key (random.ex:148-152): two u32 words */
+int hipnx_threefry_key(hipnx_ctx *ctx, const hipnx_buf *key, int parts, int index, hipnx_buf *out);
 
 /* ---- fused element-wise chains ----------------------------------------------------------------
  * replaces: a group of element-wise callbacks that the reference's evaluator issues one by one
@@ -424,6 +426,14 @@ int hipnx_fused_elementwise(hipnx_ctx *ctx, int n_instr, const hipnx_fused_instr
                             const hipnx_buf *const *inputs, const int *in_dts, const int64_t *in_row_strides,
                             const int *in_col_strides, int64_t rows, int64_t cols, int reduce_op, int out_dt,
                             hipnx_buf *out);
+
+/* The same over a flat index space of n elements of which input `words` (u32, column stride 1) is not in memory: its buffer holds
+ * a key (two u32 words), and its elements are the words of hipnx_threefry2x32 for n counters under that key -- or, key_parts
+ * > 0, under key number key_index of the key_parts that it splits into (hipnx_threefry_key).  The program's other inputs
+ * have a column stride of 1 (n elements) or 0 (one).  HIPNX_FUSED_COMPILED only; no stages. */
+int hipnx_fused_words(hipnx_ctx *ctx, int n_instr, const hipnx_fused_instr *prog, int n_inputs, const hipnx_buf *const *inputs,
+                      const int *in_dts, const int *in_col_strides, int words, int key_parts, int key_index, int64_t n,
+                      int out_dt, hipnx_buf *out);
 
 /* How hipnx_fused_elementwise runs a program on this context.  HIPNX_FUSED_INTERPRETED (the default):
  * one pair of kernels decodes any program, instruction by instruction.  HIPNX_FUSED_COMPILED: each

@@ -1079,14 +1079,16 @@ class HipNxBackend:
         return Tensor(cls(ref, backend_opts["device"]), ty, tuple(shape), tuple(opts.get("names") or ()))
 
     @classmethod
-    def fused_elementwise(cls, out: Tensor, program, inputs, layout, reduce_op: int = -1, mode=None) -> Tensor:
+    def fused_elementwise(cls, out: Tensor, program, inputs, layout, reduce_op: int = -1, mode=None, words=None) -> Tensor:
         """A group of element-wise nodes in one kernel (the evaluator offers it groups it has found
         in a traced function).  `program` is a list of dicts with the fields of `hipnx_fused_instr`
         (`dt` as a type tuple); `layout` is (rows, cols, [(row_stride, col_stride) per input]).
         `reduce_op` (RED_SUM / RED_MAX / RED_MIN) reduces the group's value along its rows without
         storing it; `out` is then the reduction's template.  Raises HipNxError with status
         EUNSUPPORTED when the shapes do not fit the kernel: the caller then runs the nodes one by one.
-        `mode` ("interpreted" / "compiled") runs this call in that mode whatever the device is set to."""
+        `mode` ("interpreted" / "compiled") runs this call in that mode whatever the device is set to.
+        `words` (input number, parts, index): that input is a key (key `index` of the `parts` it splits into, if any), and what
+        the program reads are the random words of `threefry2x32` under it, made where they are used."""
         dev = cls._device_of(*inputs) if inputs else 0
         # the library is switched when a call wants another mode than the last call had, not around every call:
         # the groups of a traced function all want the same one
@@ -1111,7 +1113,7 @@ class HipNxBackend:
                 pass
         n = max(len(inputs), 1)
         # types and strides repeat from call to call of a traced function: kept with the layout they belong to
-        if getattr(program, "packed", None) is not prog:  # a plain list: its packed form lives for this call only
+        if getattr(program, "packed", None) is not prog and words is None:  # a plain list: its packed form lives for this call only
             return cls._fused_call(out, prog, len(program), inputs, layout, reduce_op, dev)
         key = (id(layout), id(prog), out.type, out.shape, *[t.type for t in inputs])
         cached = _fused_arrays.get(key)
@@ -1129,8 +1131,11 @@ class HipNxBackend:
         handles = handle_array(*[t.data.ref.handle for t in inputs])
         ctx = _Context.get(dev)
         ref = _fresh_ref(ctx, nbytes)
-        status = L.lib.hipnx_fused_elementwise(ctx, len(program), prog_ptr, len(inputs), handles, dts, rs, cs, rows, cols,
-                                               reduce_op, out_code, ref.handle)
+        if words is not None:
+            status = L.lib.hipnx_fused_words(ctx, len(program), prog_ptr, len(inputs), handles, dts, cs, *words, cols, out_code, ref.handle)
+        else:
+            status = L.lib.hipnx_fused_elementwise(ctx, len(program), prog_ptr, len(inputs), handles, dts, rs, cs, rows, cols,
+                                                   reduce_op, out_code, ref.handle)
         if status:
             L.check(status)
         return out.with_(data=HipNxBackend(ref, dev))
@@ -1157,6 +1162,15 @@ class HipNxBackend:
         key = cls._from_nx(key, dev)
         res = cls._alloc(out, dev)
         L.check(L.lib.hipnx_threefry2x32(res.data.ref.ctx, cls._handle(key), out.size, res.data.ref.handle))
+        return res
+
+    @classmethod
+    def random_key(cls, out: Tensor, key: Tensor, parts: int, index: int) -> Tensor:
+        """Nx.Random.split(key, parts)[index] (random.ex:148-152) in one launch, where a slice of the split is two."""
+        dev = cls._device_of(key)
+        key = cls._from_nx(key, dev)
+        res = cls._alloc(out, dev)
+        L.check(L.lib.hipnx_threefry_key(res.data.ref.ctx, cls._handle(key), parts, index, res.data.ref.handle))
         return res
 
     @classmethod

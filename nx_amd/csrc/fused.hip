@@ -21,6 +21,8 @@
 // Programs with 32-bit integer instructions or bitcasts (flags bit 1, HIPNX_FUSED_BITCAST) exist only
 // compiled (fused_rtc.hip); the kernels here refuse them.
 // Bound by HBM: bytes(inputs) + bytes(out).
+#include <algorithm>
+
 #include "fused_ops.cuh"
 #include "internal.h"
 #include "reduce_kernels.cuh"
@@ -181,10 +183,11 @@ int fused_launch_compiled(hipnx_ctx *ctx, const FusedArgs &a, int reduce_op, boo
 
 using namespace hipnx;
 
-extern "C" int hipnx_fused_elementwise(hipnx_ctx *ctx, int n_instr, const hipnx_fused_instr *prog, int n_inputs,
-                                       const hipnx_buf *const *inputs, const int *in_dts, const int64_t *in_row_strides,
-                                       const int *in_col_strides, int64_t rows, int64_t cols, int reduce_op, int out_dt,
-                                       hipnx_buf *out) {
+// words >= 0: that input is a key, and what the program reads are the cipher's words (see hipnx_fused_words)
+static int fused_impl(hipnx_ctx *ctx, int n_instr, const hipnx_fused_instr *prog, int n_inputs,
+                      const hipnx_buf *const *inputs, const int *in_dts, const int64_t *in_row_strides,
+                      const int *in_col_strides, int64_t rows, int64_t cols, int reduce_op, int out_dt,
+                      hipnx_buf *out, int words, int key_parts, int key_index) {
   Enter in(ctx);
   if (in.status) return in.status;
   if (n_instr < 1 || n_instr > HIPNX_FUSED_MAX_INSTR || !prog)
@@ -199,6 +202,10 @@ extern "C" int hipnx_fused_elementwise(hipnx_ctx *ctx, int n_instr, const hipnx_
   FusedArgs a{};
   a.n_instr = n_instr;
   a.n_inputs = n_inputs;
+  a.words = words;
+  a.key_parts = key_parts;
+  a.key_index = key_index;
+  if (words >= 0 && ctx->fused_mode != HIPNX_FUSED_COMPILED) return set_error(HIPNX_EUNSUPPORTED, "fused: random words need the compiled mode");
   unsigned saved = 0;  // slots that hold a value so far
   unsigned raw_inputs = 0;  // inputs whose words are loaded unconverted
   bool have_acc = false, full = false, needs_compiled = false;
@@ -326,6 +333,10 @@ extern "C" int hipnx_fused_elementwise(hipnx_ctx *ctx, int n_instr, const hipnx_
     n_stats = 1;
   }
   const bool walk = n_stats || ragged;
+  if (words >= 0) {
+    if (n_stats || reduce_op != -1) return set_error(HIPNX_EUNSUPPORTED, "fused: random words under a reduction");
+    needs_compiled = true;
+  }
   // a few very long rows are split into segments by the separate reduction, whose order the stages follow: not here
   if (walk) {
     int would_be = 1;
@@ -352,7 +363,11 @@ extern "C" int hipnx_fused_elementwise(hipnx_ctx *ctx, int n_instr, const hipnx_
     // rows of an operand read with vector loads must start on a vector boundary
     if (!ragged && in_col_strides[k] == 1 && rows > 1 && in_row_strides[k] % 8 != 0)
       return set_error(HIPNX_EUNSUPPORTED, "fused: rows of input %d are not vector-aligned", k);
-    const uint64_t extent = n == 0 ? 0 : (uint64_t)((rows - 1) * in_row_strides[k] + (cols - 1) * in_col_strides[k] + 1);
+    if (k == words) {
+      if (dt != HIPNX_U32 || in_col_strides[k] != 1) return set_error(HIPNX_EINVAL, "fused: random words are u32, one per element");
+      if (int st = check_buf(ctx, inputs[k], 8, "fused key")) return st;
+    }
+    const uint64_t extent = n == 0 || k == words ? 0 : (uint64_t)((rows - 1) * in_row_strides[k] + (cols - 1) * in_col_strides[k] + 1);
     if (int st = check_buf(ctx, inputs[k], extent * sz, "fused input")) return st;
     a.in[k] = inputs[k]->ptr;
     a.in_dt[k] = dt;
@@ -400,6 +415,8 @@ extern "C" int hipnx_fused_elementwise(hipnx_ctx *ctx, int n_instr, const hipnx_
     // a launch may hold at most 2^32 - 1 lanes: the element-wise kernel loops over what a capped grid leaves, the row
     // kernels take one row (or wave of rows) per work-group and leave larger inputs to the separate callbacks
     const int64_t max_grid = ((1ll << 32) - 1) / FBLOCK;
+    // a lane takes sixteen words a trip; sixteen work-groups to a CU share out what there is (each derives the key once)
+    if (words >= 0) grid = std::min<int64_t>((n + 16 * FBLOCK - 1) / (16 * FBLOCK), 16 * (int64_t)ctx->num_cus);
     if (grid > max_grid) {
       if (walk || reduce_op != -1) return set_error(HIPNX_EUNSUPPORTED, "fused: more rows than one launch holds");
       grid = max_grid;
@@ -431,4 +448,21 @@ extern "C" int hipnx_fused_elementwise(hipnx_ctx *ctx, int n_instr, const hipnx_
   else hipLaunchKernelGGL((fused_elementwise_kernel<false>), dim3((unsigned)blocks), dim3(FBLOCK), 0, ctx->stream, a);
   HIPNX_HIP(hipGetLastError());
   return HIPNX_OK;
+}
+
+extern "C" int hipnx_fused_elementwise(hipnx_ctx *ctx, int n_instr, const hipnx_fused_instr *prog, int n_inputs,
+                                       const hipnx_buf *const *inputs, const int *in_dts, const int64_t *in_row_strides,
+                                       const int *in_col_strides, int64_t rows, int64_t cols, int reduce_op, int out_dt,
+                                       hipnx_buf *out) {
+  return fused_impl(ctx, n_instr, prog, n_inputs, inputs, in_dts, in_row_strides, in_col_strides, rows, cols, reduce_op, out_dt, out, -1, 0, 0);
+}
+
+extern "C" int hipnx_fused_words(hipnx_ctx *ctx, int n_instr, const hipnx_fused_instr *prog, int n_inputs, const hipnx_buf *const *inputs,
+                                 const int *in_dts, const int *in_col_strides, int words, int key_parts, int key_index, int64_t n,
+                                 int out_dt, hipnx_buf *out) {
+  if (words < 0 || words >= n_inputs || n_inputs > HIPNX_FUSED_MAX_INPUTS) return set_error(HIPNX_EINVAL, "fused_words: input %d of %d", words, n_inputs);
+  if (key_parts < 0 || key_parts > 1 << 30 || (key_parts > 0 && (key_index < 0 || key_index >= key_parts)))
+    return set_error(HIPNX_EINVAL, "fused_words: key %d of %d", key_index, key_parts);
+  const int64_t row_strides[HIPNX_FUSED_MAX_INPUTS] = {};
+  return fused_impl(ctx, n_instr, prog, n_inputs, inputs, in_dts, row_strides, in_col_strides, 1, n, -1, out_dt, out, words, key_parts, key_index);
 }

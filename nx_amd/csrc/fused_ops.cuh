@@ -8,6 +8,7 @@
 #pragma once
 #include "elementwise_ops.cuh"
 #include "reduce_ops.cuh"
+#include "threefry.cuh"
 
 namespace hipnx {
 
@@ -28,13 +29,16 @@ struct FusedArgs {
   int64_t in_rs[HIPNX_FUSED_MAX_INPUTS];  // element stride between rows (0 = the same row for all)
   int in_cs[HIPNX_FUSED_MAX_INPUTS];      // element stride along a row: 1, or 0 = one value per row
   void *out;
-  int out_dt, unused;
+  int out_dt;
+  int words;  // the input that is not in memory: in[words] holds a key, and the input is the cipher's words (-1: there is none)
   int64_t rows, cols, vecs_per_row, nvec;
   // a reduction of the result along rows that are cut into segments (nseg > 1): segment `seg` of a row covers the
   // columns [seg * seg_len, min(cols, (seg + 1) * seg_len)) and leaves its raw accumulator in partial[row * nseg + seg]
   int64_t seg_len;
   void *partial;
-  int nseg, unused2;
+  int nseg;
+  int key_parts, key_index;  // the key is number key_index of the key_parts that in[words] splits into (0 parts: in[words] itself)
+  int unused;
 };
 
 // The argument block is read where the launch put it (the kernel-argument segment, constant address
@@ -188,6 +192,9 @@ __device__ __forceinline__ void fetch_static(KernArgs a, const Saved &S, const R
   if constexpr (SRC == HIPNX_FUSED_SRC_CARRY) {
 #pragma unroll
     for (int e = 0; e < FE; e++) dst[0][e] = kept->carry[e];
+  } else if constexpr (SRC == HIPNX_FUSED_SRC_INPUT && ARG == P::words) {
+#pragma unroll
+    for (int e = 0; e < FE; e++) dst[0][e] = RAW ? kept->held[e] : element_to_f32(__float_as_uint(kept->held[e]), HIPNX_U32);
   } else if constexpr (SRC == HIPNX_FUSED_SRC_INPUT && ARG == P::held && !RAW) {
 #pragma unroll
     for (int e = 0; e < FE; e++) dst[0][e] = kept->held[e];
@@ -380,6 +387,61 @@ __device__ __forceinline__ void fused_elementwise_body() {
         p[1] = make_uint4(__float_as_uint(acc[u][4]), __float_as_uint(acc[u][5]), __float_as_uint(acc[u][6]), __float_as_uint(acc[u][7]));
       } else {
         store_vec<float, FE>(out, odt, at, acc[u]);
+      }
+    }
+  }
+}
+
+// A group over random words that exist only here: a lane enciphers eight counter pairs and takes the program over the two vectors
+// of words they give, elements i .. i + 7 and half + i .. half + i + 7 (the order of threefry2x32_kernel, nx/lib/nx/random.ex:214-229).
+// Bound by vector instructions, the cipher's (35 an element) and the program's (66 for normal samples); the words' way
+// through memory and the launches in front of it are gone: 2^26 normal samples 227 -> 183 us a pass, 664464 of them 27.7 -> 10.8.
+template <typename P>
+__device__ __forceinline__ void fused_words_body() {
+  KernArgs a = (KernArgs)__builtin_amdgcn_kernarg_segment_ptr();
+  const uint32_t *key = (const uint32_t *)a->in[P::words];
+  uint32_t key1 = __builtin_amdgcn_readfirstlane(key[0]), key2 = __builtin_amdgcn_readfirstlane(key[1]);
+  if (a->key_parts > 0) threefry_sub_key(key1, key2, a->key_parts, a->key_index);
+  const int64_t n = a->cols, half = (n + 1) / 2, groups = (half + FE - 1) / FE;
+  for (int64_t g = (int64_t)blockIdx.x * FBLOCK + threadIdx.x; g < groups; g += (int64_t)gridDim.x * FBLOCK) {
+    uint32_t w[2][FE];
+#pragma unroll
+    for (int e = 0; e < FE; e++) {
+      w[0][e] = (uint32_t)(g * FE + e);
+      w[1][e] = half + g * FE + e < n ? (uint32_t)(half + g * FE + e) : 0u;
+      threefry_pair(w[0][e], w[1][e], key1, key2);
+    }
+#pragma unroll 1
+    for (int side = 0; side < 2; side++) {
+      const int64_t at = side * half + g * FE, left = (side ? n : half) - at;
+      const int valid = left < FE ? (int)left : FE;
+      if (valid <= 0) break;
+      RowVector words;
+#pragma unroll
+      for (int e = 0; e < FE; e++) words.held[e] = __uint_as_float(side ? w[1][e] : w[0][e]);
+      const int64_t row[FV] = {0}, col[FV] = {at};
+      Vecs x;
+      Saved S;
+      const RowStats none = {};
+      static_steps<P, 0, P::n_instr>(a, row, col, x, S, none, valid, &words);
+      void *out = (void *)a->out;
+      constexpr bool raw = result_is_relabelled_bits<P>();
+      constexpr int bytes = FE * (raw || P::out_dt == HIPNX_F32 ? 4 : P::out_dt == HIPNX_U8 ? 1 : 2);
+      raw_vec<bytes> v;
+      if constexpr (raw) {
+        uint32_t bits[FE];
+#pragma unroll
+        for (int e = 0; e < FE; e++) bits[e] = __float_as_uint(x[0][e]);
+        __builtin_memcpy(&v, bits, bytes);
+      } else store_vec<float, FE>(&v, P::out_dt, 0, x[0]);
+      if (valid == FE) __builtin_memcpy((char *)out + at * (bytes / FE), &v, bytes);
+      else {
+#pragma unroll
+        for (int e = 0; e < FE - 1; e++)
+          if (e < valid) {
+            if constexpr (raw) ((uint32_t *)out)[at + e] = __float_as_uint(x[0][e]);
+            else store_one<float>(out, P::out_dt, at + e, x[0][e]);
+          }
       }
     }
   }

@@ -161,8 +161,8 @@ static Keeps what_is_kept(const FusedArgs &a, bool walk) {
 constexpr size_t LENGTH_KEY = 4 * sizeof(int);
 static std::string make_key(const FusedArgs &a, const Keeps &keeps, int reduce_op, bool block_per_row) {
   std::string k;
-  k.reserve(20 + 16 * a.n_instr + 8 * a.n_inputs);
-  const int head[4] = {a.n_instr, a.n_inputs, a.out_dt, reduce_op * 2 + (block_per_row ? 1 : 0)};
+  k.reserve(40 + 16 * a.n_instr + 8 * a.n_inputs);
+  const int head[5] = {a.n_instr, a.n_inputs, a.out_dt, reduce_op * 2 + (block_per_row ? 1 : 0), a.words};
   k.append((const char *)head, sizeof(head));
   k.append((const char *)a.ins, sizeof(hipnx_fused_instr) * a.n_instr);
   k.append((const char *)a.in_dt, sizeof(int) * a.n_inputs);
@@ -183,7 +183,7 @@ static std::string any_length(const std::string &name) { return name + "_any"; }
 // the whole translation unit for one program
 static std::string make_source(const FusedArgs &a, const Keeps &keeps, int reduce_op, bool block_per_row, const std::string &name) {
   std::string s = RTC_PREAMBLE;
-  s += "namespace hipnx {\nstruct Program {\n  static constexpr int n_instr = " + std::to_string(a.n_instr) + ", out_dt = " + std::to_string(a.out_dt) + ";\n";
+  s += "namespace hipnx {\nstruct Program {\n  static constexpr int n_instr = " + std::to_string(a.n_instr) + ", out_dt = " + std::to_string(a.out_dt) + ", words = " + std::to_string(a.words) + ";\n";
   const hipnx_fused_instr *q = a.ins;
   list_of(s, "kind", "int", a.n_instr, [&](int i) { return std::to_string((int)q[i].kind); });
   list_of(s, "op", "int", a.n_instr, [&](int i) { return std::to_string((int)q[i].op); });
@@ -210,9 +210,9 @@ static std::string make_source(const FusedArgs &a, const Keeps &keeps, int reduc
   }
   list_of(s, "seg_red", "int", (int)seg_red.size(), [&](int k) { return std::to_string(seg_red[k]); });
   list_of(s, "seg_save", "int", (int)seg_save.size(), [&](int k) { return std::to_string(seg_save[k]); });
-  auto keeping = [](const char *p, const Keeps &k) {
+  auto keeping = [&](const char *p, const Keeps &k) {
     return std::string("struct ") + p + " : Program {\n  static constexpr int form = " + std::to_string(k.form) + ", tpr = " + std::to_string(k.tpr) + ", tail = " + std::to_string(k.tail) +
-           ";\n  static constexpr bool unal = " + (k.form == ROW_WHOLE ? "false" : "true") + ";\n  static constexpr int nv = " + std::to_string(k.trips) + ", written_out = " + std::to_string(k.written_out) + ", held = " + std::to_string(k.held) +
+           ";\n  static constexpr bool unal = " + (k.form == ROW_WHOLE && a.words < 0 ? "false" : "true") + ";\n  static constexpr int nv = " + std::to_string(k.trips) + ", written_out = " + std::to_string(k.written_out) + ", held = " + std::to_string(k.held) +
            ", held_stage = " + std::to_string(k.held_stage) + ";\n};\n";
   };
   auto kernel = [](const std::string &called) {
@@ -226,7 +226,8 @@ static std::string make_source(const FusedArgs &a, const Keeps &keeps, int reduc
   if (has_kernel_for_any_length(a, keeps)) s += kernel(any_length(name)) + "  fused_row_stages_body<Any>();\n}\n";
   s += kernel(name);
   const char *tpr = block_per_row ? "FBLOCK" : "WAVE";
-  if (stages || keeps.form != ROW_WHOLE) s += "  fused_row_stages_body<P>();\n";
+  if (a.words >= 0) s += "  fused_words_body<P>();\n";
+  else if (stages || keeps.form != ROW_WHOLE) s += "  fused_row_stages_body<P>();\n";
   else switch (reduce_op) {
     case HIPNX_RED_SUM: s += std::string("  fused_reduce_rows_body<RunStatic<P>, PlainReducer<double, HIPNX_RED_SUM, false>, double, ") + tpr + ">();\n"; break;
     case HIPNX_RED_MAX: s += std::string("  fused_reduce_rows_body<RunStatic<P>, PlainReducer<float, HIPNX_RED_MAX, false>, float, ") + tpr + ">();\n"; break;
@@ -319,7 +320,7 @@ int fused_launch_compiled(hipnx_ctx *ctx, const FusedArgs &a, int reduce_op, boo
     int stages = 0;
     for (int i = 0; i < a.n_instr; i++) stages += a.ins[i].kind == HIPNX_FUSED_ROW_REDUCE;
     char name[96];
-    snprintf(name, sizeof(name), "fused_%s_%dinstr_%08zx", stages ? "stages" : reduce_op != -1 ? "map_reduce" : "map", a.n_instr,
+    snprintf(name, sizeof(name), "fused_%s_%dinstr_%08zx", a.words >= 0 ? "words" : stages ? "stages" : reduce_op != -1 ? "map_reduce" : "map", a.n_instr,
              std::hash<std::string>{}(key) & 0xFFFFFFFFu);
     if (ctx->fused_kernels.size() >= ctx->fused_cache_max)
       if (int st = trim_cache(ctx)) return st;

@@ -5,32 +5,12 @@
 //   n is odd and i is the last pair -- and writes out[i] and out[half + i].
 // Bound by integer work, not by the HBM writes: about 75 vector operations per 8 output bytes.
 #include "internal.h"
+#include "threefry.cuh"
 
 namespace hipnx {
 
 constexpr int RBLOCK = 256;
 constexpr int RPAIRS = 4;  // counter pairs per lane: one 16-byte store into each half of the output
-
-__device__ __forceinline__ uint32_t rotl32(uint32_t x, int r) { return (x << r) | (x >> (32 - r)); }
-
-// 20 rounds on one counter pair, key already split into the three schedule words
-__device__ __forceinline__ void threefry_pair(uint32_t &x1, uint32_t &x2, uint32_t key1, uint32_t key2) {
-  uint32_t k1 = key2, k2 = key1 ^ key2 ^ 0x1BD11BDAu, k3 = key1;
-  x1 += key1;
-  x2 += key2;
-  constexpr int R[2][4] = {{13, 15, 26, 6}, {17, 29, 16, 24}};
-#pragma unroll
-  for (int g = 1; g <= 5; g++) {
-#pragma unroll
-    for (int r = 0; r < 4; r++) {
-      x1 += x2;
-      x2 = rotl32(x2, R[(g - 1) & 1][r]) ^ x1;
-    }
-    x1 += k1;
-    x2 += k2 + (uint32_t)g;
-    const uint32_t t = k1; k1 = k2; k2 = k3; k3 = t;
-  }
-}
 
 // One lane takes RPAIRS consecutive pairs.  `vec` says that half is a multiple of RPAIRS and the output 16-byte aligned, so both
 // stores of a lane whose pairs all exist are 16-byte aligned; every other lane stores word by word.
@@ -61,6 +41,12 @@ threefry2x32_kernel(const uint32_t *__restrict__ key, uint32_t *__restrict__ out
   }
 }
 
+__global__ void threefry_key_kernel(const uint32_t *__restrict__ key, uint32_t *__restrict__ out, uint32_t parts, uint32_t index) {
+  uint32_t key1 = key[0], key2 = key[1];
+  threefry_sub_key(key1, key2, parts, index);
+  if (threadIdx.x == 0) out[0] = key1, out[1] = key2;
+}
+
 }  // namespace hipnx
 
 using namespace hipnx;
@@ -78,6 +64,17 @@ extern "C" int hipnx_threefry2x32(hipnx_ctx *ctx, const hipnx_buf *key, int64_t 
   if (blocks > ((1ll << 32) - 1) / RBLOCK) blocks = ((1ll << 32) - 1) / RBLOCK;  // a launch may hold at most 2^32 - 1 lanes
   hipLaunchKernelGGL(threefry2x32_kernel, dim3((unsigned)blocks), dim3(RBLOCK), 0, ctx->stream,
                      (const uint32_t *)key->ptr, (uint32_t *)out->ptr, n, half, (int)(half % RPAIRS == 0 && (uintptr_t)out->ptr % 16 == 0));
+  HIPNX_HIP(hipGetLastError());
+  return HIPNX_OK;
+}
+
+extern "C" int hipnx_threefry_key(hipnx_ctx *ctx, const hipnx_buf *key, int parts, int index, hipnx_buf *out) {
+  Enter in(ctx);
+  if (in.status) return in.status;
+  if (parts < 1 || parts > 1 << 30 || index < 0 || index >= parts) return set_error(HIPNX_EINVAL, "threefry_key: key %d of %d", index, parts);
+  if (int st = check_buf(ctx, key, 8, "threefry_key key")) return st;
+  if (int st = check_buf(ctx, out, 8, "threefry_key out")) return st;
+  hipLaunchKernelGGL(threefry_key_kernel, dim3(1), dim3(64), 0, ctx->stream, (const uint32_t *)key->ptr, (uint32_t *)out->ptr, (uint32_t)parts, (uint32_t)index);
   HIPNX_HIP(hipGetLastError());
   return HIPNX_OK;
 }

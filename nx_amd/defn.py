@@ -559,6 +559,8 @@ class _Group:
     """One fused group: the member nodes in evaluation order, its external inputs, and the program
     for the backend's accumulator machine (None when the group does not fit it)."""
 
+    words = None  # (input number, parts, index): that operand is a key, and the input its random words (_absorb_random)
+
     def __init__(self, root: Tensor, members: List[Tensor], inputs: List[Tensor]):
         self.root, self.members, self.inputs = root, members, inputs
         # planned for compiled execution (integer instructions allowed): ask the backend for that mode
@@ -707,10 +709,14 @@ class _Group:
             return getattr(run.pick([value]), name)(out, value, opts)
         if fused is not None:
             try:
-                return fused(out, self.program, values, self.layout, **self.how)
+                return fused(out, self.program, values, self.layout, **self.how, **({"words": self.words} if self.words else {}))
             except Exception as e:  # e.g. integer instructions met while the device is capturing
                 if getattr(e, "status", None) != _EUNSUPPORTED:
                     raise
+        if self.words:
+            at, parts, index = self.words
+            values = list(values)
+            values[at] = _random().threefry2x32(_sub_key(values[at], parts, index), self.inputs[at].shape)
         # node by node, on the callbacks (a backend without the kernel, or a group that does not fit)
         done = {t.data.id: v for t, v in zip(self.inputs, values)}
         for m in self.members:
@@ -971,7 +977,72 @@ def _fuse_planned(roots: List[Tensor]) -> int:
         e.op, e.args = "fused", [both, inner.args[1]]
     if _plan["ints"]:  # planned for compiled kernels: groups over the same rows become stages of one
         _cluster_rows(roots)
+        _absorb_random(roots)
     return formed
+
+
+def _random():
+    from . import random
+    return random
+
+
+def _sub_key(key: Tensor, parts: int, index: int) -> Tensor:
+    return _random()._at(_random().split(key, parts), index) if parts else key
+
+
+def _split_of(t: Tensor):
+    """(key, parts, index) when `t` is key number `index` of a key split into `parts` (Nx.Random.split/2 and an access), or None."""
+    if t.shape != (2,) or t.data.op != "squeeze":
+        return None
+    cut = t.data.args[0]
+    if cut.data.op != "slice":
+        return None
+    keys, starts, lengths, strides = cut.data.args
+    if not (isinstance(keys, Tensor) and keys.data.op == "block" and isinstance(keys.data.args[0], Nx.BlockThreefry) and len(keys.shape) == 2):
+        return None
+    starts = [s if isinstance(s, int) else _const(s) for s in starts]
+    if keys.shape[1] != 2 or list(lengths) != [1, 2] or list(strides) != [1, 1] or starts[1] != 0 or not isinstance(starts[0], int) or not 0 <= starts[0] < keys.shape[0]:
+        return None
+    return keys.data.args[1][0], keys.shape[0], starts[0]
+
+
+def _absorb_random(roots: List[Tensor]) -> None:
+    """A group over a flat index space that alone reads random words makes them itself, from the key; a key that is one of a
+    split is derived where it is used (the words' way through memory, the split and its slice were three launches more)."""
+    order, uses, seen = [], {}, set()
+
+    def walk(t):
+        e = t.data
+        if e.op in ("constant", "tensor") or e.scope != 0:
+            return
+        uses[e.id] = uses.get(e.id, 0) + 1
+        if e.id in seen:
+            return
+        seen.add(e.id)
+        for child in _children(e):
+            if isinstance(child, Tensor):
+                walk(child)
+        order.append(t)
+    for r in roots:
+        walk(r)
+    for node in order:
+        e = node.data
+        if e.op != "fused" or not isinstance(e.args[0], _Group) or e.args[0].reduce is not None or not e.args[0].program or not e.args[0].layout:
+            continue
+        group, inputs = e.args
+        rows, cols, strides = group.layout
+        for k, t in enumerate(inputs):
+            d = t.data
+            if (rows == 1 and d.op == "block" and isinstance(d.args[0], Nx.BlockThreefry) and uses[d.id] == 1 and t.size == cols > 1
+                    and strides[k][1] == 1 and t.type == ("u", 32)):
+                key, parts, index = _split_of(d.args[1][0]) or (d.args[1][0], 0, 0)
+                group.words = (k, parts, index)
+                e.args = [group, inputs[:k] + [key] + inputs[k + 1:]]
+                break
+    for node in order:
+        split = _split_of(node)
+        if split is not None:
+            node.data.op, node.data.args = "random_key", list(split)
 
 
 def _over_last_axis(opts, rank: int) -> bool:
@@ -1356,7 +1427,7 @@ class _Scope:
 
 
 # nodes that `apply` does not evaluate as a callback on its evaluated operands
-_EVALUATED_APART = frozenset(["parameter", "elem", "while", "cond", "fused", "dot_scaled", "dot_views", "block"]) | frozenset(CREATION_OPS)
+_EVALUATED_APART = frozenset(["parameter", "elem", "while", "cond", "fused", "dot_scaled", "dot_views", "random_key", "block"]) | frozenset(CREATION_OPS)
 
 
 class _Run:
@@ -1486,6 +1557,12 @@ class _Run:
             lv, rv = (v if axes is None else mod.transpose(v.with_(data=None, shape=tuple(v.shape[a] for a in axes)), v, list(axes))
                       for v, axes in ((lv, l_axes), (rv, r_axes)))
             return mod.dot(out, lv, c1, b1, rv, c2, b2)
+        if op == "random_key":
+            key, parts, index = e.args
+            key = self.eval(key, scope)
+            mod = self.pick([key])
+            one_call = getattr(mod, "random_key", None)
+            return one_call(x.with_(data=None), key, parts, index) if one_call is not None else _sub_key(key, parts, index)
         if op == "block":
             struct, in_args, fun = e.args
             args = [self.eval(a, scope) for a in in_args]

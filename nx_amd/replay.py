@@ -21,7 +21,7 @@ from ._lib import native
 # entry points whose effect is their result buffer's content, a function of their arguments
 _RECORDED = frozenset("hipnx_" + n for n in (
     "binary", "unary", "as_type", "reduce", "argreduce", "dot", "dot_strided", "dot_scaled", "transpose", "broadcast", "gather", "select", "clip",
-    "concat", "strided_copy", "iota", "eye", "narrow_int", "threefry2x32", "fused_elementwise"))
+    "concat", "strided_copy", "iota", "eye", "narrow_int", "threefry2x32", "threefry_key", "fused_elementwise", "fused_words"))
 _lock = threading.Lock()
 
 
@@ -65,7 +65,7 @@ class _Recorder:
                 try:
                     self._drain()
                     self.ops.append(("call", C.cast(real, C.c_void_p).value, [self._argument(a, t) for a, t in zip(args, real.argtypes)]))
-                    if name == "hipnx_fused_elementwise":
+                    if name in ("hipnx_fused_elementwise", "hipnx_fused_words"):
                         self.modes.add(B._fused_set.get(self.device, "interpreted"))
                 except _Unrecordable:
                     self.failed = True

@@ -9,7 +9,7 @@ import pytest
 from nx_amd import nx as Nx
 from nx_amd import random as Random
 from random_support import CASES, check_random_case
-from support import assert_all_close, assert_bits_equal, seed_of
+from support import assert_all_close, assert_bits_equal, from_numpy, seed_of
 
 pytestmark = pytest.mark.gpu
 
@@ -108,3 +108,30 @@ def test_known_answers_hold_through_the_composition_too(hip):
             check_random_case(case, hip)
     finally:
         Random.compose_only(previous)
+
+
+# a lane has two vectors of eight words: one, less and more than a lane's, halves off the vector grid, several trips of the grid
+@pytest.mark.parametrize("shape", [(1,), (2,), (7,), (15,), (16,), (17,), (33, 31), (4096,), (100003,), (1 << 24,)])
+def test_words_made_inside_a_compiled_group(shape, hip):
+    """A traced sample makes its words where it uses them and derives its key there: two launches, the bits of the separate calls."""
+    from nx_amd import defn
+    key = Random.key(20 + len(shape) + shape[0], backend=hip)
+    other = from_numpy(np.linspace(-1, 1, int(np.prod(shape)), dtype=np.float32).reshape(shape), "f32", hip)
+    functions = {"normal": lambda k, o: Random.normal(k, shape=shape), "uniform": lambda k, o: Random.uniform(k, -2.0, 3.0, shape=shape),
+                 "noisy": lambda k, o: Nx.add(o, Nx.multiply(0.25, Random.normal_split(k, shape=shape))),
+                 "bits": lambda k, o: Nx.bitwise_xor(Nx.right_shift(Random.random_bits(k, shape=shape), 3), 12345),
+                 "third of five": lambda k, o: Random.uniform_split(Random._at(Random.split(k, 5), 2), shape=shape)}
+    for name, fun in functions.items():
+        planned = defn.compile(fun, key, other, fuse="compiled")
+        group = next(r.data.args[0] for r in planned.roots if r.data.op == "fused")
+        assert group.words is not None or shape == (1,), name
+        calls = []
+        original = hip.threefry2x32.__func__
+        hip.threefry2x32 = classmethod(lambda cls, *a: (calls.append(1), original(cls, *a))[1])
+        try:
+            got = planned._evaluate([key, other])
+        finally:
+            hip.threefry2x32 = classmethod(original)
+        assert not calls or shape == (1,), name
+        for g, w in zip(got, defn.compile(fun, key, other)._walk([key, other])):
+            assert_bits_equal(g, w, f"{name} {shape}")
