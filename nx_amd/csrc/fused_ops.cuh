@@ -217,6 +217,13 @@ __device__ __forceinline__ void fetch_static(KernArgs a, const Saved &S, const R
   }
 }
 
+// What an arithmetic instruction computes is never a NaN whose set bits all lie in the half that truncation to bf16 drops
+// (a computed NaN is a quiet one): the bits can be cut without looking.  (A value that only passes through can be.)
+constexpr bool computes_quiet_nan(int kind, int op) {
+  return (kind == HIPNX_FUSED_UNARY && (op == HIPNX_EXP || op == HIPNX_LOG || op == HIPNX_SQRT || op == HIPNX_RSQRT || op == HIPNX_TANH)) ||
+         (kind == HIPNX_FUSED_BINARY && (op == HIPNX_ADD || op == HIPNX_SUBTRACT || op == HIPNX_MULTIPLY || op == HIPNX_DIVIDE));
+}
+
 // 32-bit integers travel through the lane's vectors as raw bits; an operation on them widens to
 // the 64-bit integer class of the separate kernels and keeps the low word, as their stores do
 template <int OP, bool UNS>
@@ -319,7 +326,12 @@ __device__ __forceinline__ void static_steps(KernArgs a, const int64_t (&row)[FV
           acc[u][e] = __uint_as_float((b & 0x7FFFFFFFu) > 0x7F800000u ? 0x7FC00000u : b);
         }
     }
-    if constexpr (dt == HIPNX_BF16 || dt == HIPNX_F16) {
+    if constexpr (dt == HIPNX_BF16 && !ints && computes_quiet_nan(kind, op) && !bits_are_observed_after<P>(PC)) {
+#pragma unroll
+      for (int u = 0; u < FV; u++)
+#pragma unroll
+        for (int e = 0; e < FE; e++) acc[u][e] = __uint_as_float(__float_as_uint(acc[u][e]) & 0xFFFF0000u);
+    } else if constexpr (dt == HIPNX_BF16 || dt == HIPNX_F16) {
 #pragma unroll
       for (int u = 0; u < FV; u++)
 #pragma unroll

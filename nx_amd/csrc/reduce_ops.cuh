@@ -56,7 +56,6 @@ struct PlainReducer {
   // (for all / any an element counts as true unless it equals 0 -- NaN included,
   // binary_backend.ex:1293-1314)
   static __device__ __forceinline__ acc_t accumulate(acc_t a, CT x, int64_t) { return combine(a, x); }
-  static __device__ __forceinline__ acc_t shfl_xor(acc_t a, int m) { return __shfl_xor(a, m, WAVE); }
 };
 
 template <typename CT>
@@ -111,20 +110,69 @@ struct ArgReducer {
     if constexpr (FP) take |= x != x;
     return take ? acc_t{x, (int)idx} : a;
   }
-  static __device__ __forceinline__ acc_t shfl_xor(acc_t a, int m) {
-    acc_t r;
-    r.v = __shfl_xor(a.v, m, WAVE);
-    r.i = __shfl_xor(a.i, m, WAVE);
-    return r;
-  }
 };
+
+// ---- values of other lanes ---------------------------------------------------------------------
+// In vector instructions: a shuffle through the LDS crossbar is a round trip of about a hundred clocks, two for a 64-bit value,
+// and the six steps of a wave's reduction wait for one another.  Lane i ^ M of the wave, for M below 16 (DPP: a permutation of
+// four lanes, of a row of sixteen).
+template <int M>
+__device__ __forceinline__ uint32_t xor_lane_word(uint32_t v) {
+  static_assert(M == 1 || M == 2 || M == 4 || M == 8, "within a row of sixteen lanes");
+  const int x = (int)v;
+  if constexpr (M == 1) return (uint32_t)__builtin_amdgcn_update_dpp(x, x, 0xB1, 0xF, 0xF, false);       // quad_perm 1 0 3 2
+  else if constexpr (M == 2) return (uint32_t)__builtin_amdgcn_update_dpp(x, x, 0x4E, 0xF, 0xF, false);  // quad_perm 2 3 0 1
+  else if constexpr (M == 4) {  // the even quads from four lanes up, the odd ones from four lanes down
+    const int up = __builtin_amdgcn_update_dpp(x, x, 0x104, 0xF, 0x5, false);
+    return (uint32_t)__builtin_amdgcn_update_dpp(up, x, 0x114, 0xF, 0xA, false);
+  } else return (uint32_t)__builtin_amdgcn_update_dpp(x, x, 0x128, 0xF, 0xF, false);  // row_ror:8
+}
+template <int M, typename T>
+__device__ __forceinline__ T xor_lane(T v) {
+  static_assert(sizeof(T) % 4 == 0, "whole words");
+  uint32_t w[sizeof(T) / 4];
+  __builtin_memcpy(w, &v, sizeof(T));
+#pragma unroll
+  for (unsigned i = 0; i < sizeof(T) / 4; i++) w[i] = xor_lane_word<M>(w[i]);
+  __builtin_memcpy(&v, w, sizeof(T));
+  return v;
+}
+// for M = 16 or 32: of the two lanes that differ in bit M, the lower one's value and the upper one's, in both
+template <int M, typename T>
+__device__ __forceinline__ void lower_and_upper(T v, T &lower, T &upper) {
+  static_assert(M == 16 || M == 32, "across the rows of a wave");
+  uint32_t w[sizeof(T) / 4], lo[sizeof(T) / 4], hi[sizeof(T) / 4];
+  __builtin_memcpy(w, &v, sizeof(T));
+#pragma unroll
+  for (unsigned i = 0; i < sizeof(T) / 4; i++) {
+    const auto s = [&] {
+      if constexpr (M == 16) return __builtin_amdgcn_permlane16_swap(w[i], w[i], false, false);
+      else return __builtin_amdgcn_permlane32_swap(w[i], w[i], false, false);
+    }();
+    lo[i] = s[0];
+    hi[i] = s[1];
+  }
+  __builtin_memcpy(&lower, lo, sizeof(T));
+  __builtin_memcpy(&upper, hi, sizeof(T));
+}
 
 // combines across the aligned groups of WIDTH lanes (a power of two, the whole wave by default); lane 0 of a
 // group ends with its result.  The steps for a narrower group are the last steps of the wave's.
 template <typename R, int WIDTH = WAVE>
 __device__ __forceinline__ typename R::acc_t wave_reduce(typename R::acc_t a) {
-#pragma unroll
-  for (int m = WIDTH / 2; m >= 1; m >>= 1) a = R::combine(a, R::shfl_xor(a, m));
+  typename R::acc_t lower, upper;
+  if constexpr (WIDTH > 32) {
+    lower_and_upper<32>(a, lower, upper);
+    a = R::combine(lower, upper);
+  }
+  if constexpr (WIDTH > 16) {
+    lower_and_upper<16>(a, lower, upper);
+    a = R::combine(lower, upper);
+  }
+  if constexpr (WIDTH > 8) a = R::combine(a, xor_lane<8>(a));
+  if constexpr (WIDTH > 4) a = R::combine(a, xor_lane<4>(a));
+  if constexpr (WIDTH > 2) a = R::combine(a, xor_lane<2>(a));
+  if constexpr (WIDTH > 1) a = R::combine(a, xor_lane<1>(a));
   return a;
 }
 
