@@ -435,6 +435,17 @@ int hipnx_fused_words(hipnx_ctx *ctx, int n_instr, const hipnx_fused_instr *prog
                       const int *in_dts, const int *in_col_strides, int words, int key_parts, int key_index, int64_t n,
                       int out_dt, hipnx_buf *out);
 
+/* A program of stages of which input `scores` is the result of a contraction that is not stored: out[b, m, n] of hipnx_dot_strided
+ * for bf16 or f16 operands whose rows are K-inner and a result of their type, with rows = batch_outer * batch_inner * M and n along the
+ * columns (the scores of an attention under their softmax).  strides: {first batch axis, second, row} of the left operand, then of
+ * the right one; operands: the two buffers; inputs[scores] is not looked at.  K of 32 to 256 in whole steps of 32, at most 4096
+ * columns, HIPNX_FUSED_COMPILED; anything else, and shapes that are faster in two calls, are HIPNX_EUNSUPPORTED.  A sum over K is
+ * added in order of k in f32, rounded to the operands' type once. */
+int hipnx_fused_scores(hipnx_ctx *ctx, int n_instr, const hipnx_fused_instr *prog, int n_inputs, const hipnx_buf *const *inputs,
+                       const int *in_dts, const int64_t *in_row_strides, const int *in_col_strides, int64_t cols, int scores,
+                       int64_t batch_outer, int64_t batch_inner, int64_t M, int64_t K, const int64_t *strides,
+                       const hipnx_buf *const *operands, int out_dt, hipnx_buf *out);
+
 /* How hipnx_fused_elementwise runs a program on this context.  HIPNX_FUSED_INTERPRETED (the default):
  * one pair of kernels decodes any program, instruction by instruction.  HIPNX_FUSED_COMPILED: each
  * distinct program (instructions, input types and column strides, result type, reduction) is written

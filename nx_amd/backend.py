@@ -1100,17 +1100,7 @@ class HipNxBackend:
         rows, cols, strides = layout
         prog = getattr(program, "packed", None)
         if prog is None:
-            prog = (L.FusedInstr * len(program))()
-            for q, ins in zip(prog, program):
-                q.kind, q.op, q.src, q.arg = ins["kind"], ins.get("op", 0), ins.get("src", 0), ins.get("arg", 0)
-                q.src2, q.arg2, q.flags, q.dt = ins.get("src2", 0), ins.get("arg2", 0), ins.get("flags", 0), T.code(ins["dt"])
-                q.imm.f, q.imm2.f = ins.get("imm", 0.0), ins.get("imm2", 0.0)
-                if "imm_bits" in ins:  # the constant of an integer instruction, as the bits it is
-                    q.imm.bits = ins["imm_bits"]
-            try:
-                program.packed = prog  # a caller's list type with room for the packed form keeps it
-            except AttributeError:
-                pass
+            prog = _pack(program)
         n = max(len(inputs), 1)
         # types and strides repeat from call to call of a traced function: kept with the layout they belong to
         if getattr(program, "packed", None) is not prog and words is None:  # a plain list: its packed form lives for this call only
@@ -1136,6 +1126,43 @@ class HipNxBackend:
         else:
             status = L.lib.hipnx_fused_elementwise(ctx, len(program), prog_ptr, len(inputs), handles, dts, rs, cs, rows, cols,
                                                    reduce_op, out_code, ref.handle)
+        if status:
+            L.check(status)
+        return out.with_(data=HipNxBackend(ref, dev))
+
+    @classmethod
+    def fused_scores(cls, out: Tensor, program, inputs, layout, at: int, dot, mode=None) -> Tensor:
+        """`fused_elementwise` for a program of stages whose input number `at` is the contraction `dot` = (left, its axes,
+        contracted axes, batch axes, right, its axes, contracted axes, batch axes; see `dot_views`): its result is made
+        inside the kernel and never stored.  Raises HipNxError with status EUNSUPPORTED where the two calls have to be made."""
+        l, l_axes, c1, b1, r, r_axes, c2, b2 = dot
+        dev = cls._device_of(l, r)
+        if any(t.data.__class__ is not HipNxBackend for t in inputs) or r.data.__class__ is not HipNxBackend or _bf16["rounding"] != "truncate":
+            raise L.HipNxError(L.EUNSUPPORTED, "fused_scores: operands elsewhere, or another rounding of the contraction's result")
+        wanted = mode if mode is not None else _fused_modes.get(dev, "interpreted")
+        if _fused_set.get(dev, "interpreted") != wanted:
+            _set_fused_mode(wanted, dev)
+        rows, cols, strides = layout
+        key = ("scores", id(layout), id(program), out.type, out.shape, l.type, l.shape, l_axes, r.type, r.shape, r_axes, *[t.type for t in inputs])
+        cached = _fused_arrays.get(key)
+        if cached is None or cached[0] is not layout or cached[1] is not program:
+            views = cls._plan_views(l.shape, l_axes, c1, r.shape, r_axes, c2, len(b1))
+            if views is None or views[3] != K_INNER or views[6] != K_INNER or views[7] != cols or l.type != r.type:
+                raise L.HipNxError(L.EUNSUPPORTED, "fused_scores: operands that are not rows of contiguous elements")
+            outer, inner, K, _, M, l_strides, _, _, r_strides = views
+            n, types = len(inputs), [l.type if i == at else t.type for i, t in enumerate(inputs)]
+            if len(_fused_arrays) > 4096:
+                _fused_arrays.clear()
+            cached = _fused_arrays[key] = (layout, program, (C.c_int * n)(*[T.code(t) for t in types]), (C.c_int64 * n)(*[s[0] for s in strides]),
+                                           (C.c_int * n)(*[s[1] for s in strides]), (C.c_int64 * 6)(*l_strides, *r_strides),
+                                           (outer, inner, M, K), T.code(out.type), out.size * T.size_bytes(out.type), _packed(program))
+        _, _, dts, rs, cs, operand_strides, extents, out_code, nbytes, prog_ptr = cached
+        handles = (C.c_void_p * len(inputs))(*[cls._handle(t) for t in inputs])
+        operands = (C.c_void_p * 2)(cls._handle(l), cls._handle(r))
+        ctx = _Context.get(dev)
+        ref = _fresh_ref(ctx, nbytes)
+        status = L.lib.hipnx_fused_scores(ctx, len(program), prog_ptr, len(inputs), handles, dts, rs, cs, cols, at, *extents, operand_strides,
+                                          operands, out_code, ref.handle)
         if status:
             L.check(status)
         return out.with_(data=HipNxBackend(ref, dev))
@@ -1187,6 +1214,27 @@ class HipNxBackend:
         if isinstance(struct, BlockThreefry):
             return cls.threefry2x32(out, args[0])
         return fun(struct, *args)
+
+
+def _pack(program):
+    """The instructions as the C ABI takes them; a caller's list type with room for the packed form keeps it."""
+    prog = (L.FusedInstr * len(program))()
+    for q, ins in zip(prog, program):
+        q.kind, q.op, q.src, q.arg = ins["kind"], ins.get("op", 0), ins.get("src", 0), ins.get("arg", 0)
+        q.src2, q.arg2, q.flags, q.dt = ins.get("src2", 0), ins.get("arg2", 0), ins.get("flags", 0), T.code(ins["dt"])
+        q.imm.f, q.imm2.f = ins.get("imm", 0.0), ins.get("imm2", 0.0)
+        if "imm_bits" in ins:  # the constant of an integer instruction, as the bits it is
+            q.imm.bits = ins["imm_bits"]
+    try:
+        program.packed = prog
+    except AttributeError:
+        pass
+    return prog
+
+
+def _packed(program):
+    prog = getattr(program, "packed", None)
+    return C.cast(prog if prog is not None else _pack(program), C.c_void_p)
 
 
 def _install():

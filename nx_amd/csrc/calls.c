@@ -14,12 +14,13 @@
 #include <structmember.h>
 #include <stdint.h>
 
-#define MAX_ARGS 16
+#define MAX_ARGS 20
 typedef int (*entry_t)(int64_t, int64_t, int64_t, int64_t, int64_t, int64_t, int64_t, int64_t, int64_t, int64_t, int64_t, int64_t,
-                       int64_t, int64_t, int64_t, int64_t);
+                       int64_t, int64_t, int64_t, int64_t, int64_t, int64_t, int64_t, int64_t);
 
 static int enter(int64_t fn, const int64_t *a) {
-  return ((entry_t)(intptr_t)fn)(a[0], a[1], a[2], a[3], a[4], a[5], a[6], a[7], a[8], a[9], a[10], a[11], a[12], a[13], a[14], a[15]);
+  return ((entry_t)(intptr_t)fn)(a[0], a[1], a[2], a[3], a[4], a[5], a[6], a[7], a[8], a[9], a[10], a[11], a[12], a[13], a[14], a[15],
+                                a[16], a[17], a[18], a[19]);
 }
 
 static int (*buf_alloc)(void *, size_t, void **);

@@ -177,17 +177,25 @@ static void launch_fused_combine(const hipnx_ctx *ctx, const FusedArgs &a, int r
 static bool narrow(int dt) { return dt == HIPNX_BF16 || dt == HIPNX_F16 || dt == HIPNX_F32; }
 
 // fused_rtc.hip
-int fused_launch_compiled(hipnx_ctx *ctx, const FusedArgs &a, int reduce_op, bool block_per_row, bool walk, unsigned grid, bool *done);
+int fused_launch_compiled(hipnx_ctx *ctx, const FusedArgs &a, int reduce_op, bool block_per_row, bool walk, int scores_k, unsigned grid, bool *done);
 
 }  // namespace hipnx
 
 using namespace hipnx;
 
+// An input that is a contraction's result (hipnx_fused_scores)
+struct Scores {
+  int input = -1, K = 0;
+  int64_t batch_outer = 0, batch_inner = 0, M = 0;
+  const int64_t *l_strides = nullptr, *r_strides = nullptr;
+  const hipnx_buf *l = nullptr, *r = nullptr;
+};
+
 // words >= 0: that input is a key, and what the program reads are the cipher's words (see hipnx_fused_words)
 static int fused_impl(hipnx_ctx *ctx, int n_instr, const hipnx_fused_instr *prog, int n_inputs,
                       const hipnx_buf *const *inputs, const int *in_dts, const int64_t *in_row_strides,
                       const int *in_col_strides, int64_t rows, int64_t cols, int reduce_op, int out_dt,
-                      hipnx_buf *out, int words, int key_parts, int key_index) {
+                      hipnx_buf *out, int words, int key_parts, int key_index, const Scores &scores = Scores()) {
   Enter in(ctx);
   if (in.status) return in.status;
   if (n_instr < 1 || n_instr > HIPNX_FUSED_MAX_INSTR || !prog)
@@ -205,6 +213,7 @@ static int fused_impl(hipnx_ctx *ctx, int n_instr, const hipnx_fused_instr *prog
   a.words = words;
   a.key_parts = key_parts;
   a.key_index = key_index;
+  a.scores = scores.input;
   if (words >= 0 && ctx->fused_mode != HIPNX_FUSED_COMPILED) return set_error(HIPNX_EUNSUPPORTED, "fused: random words need the compiled mode");
   unsigned saved = 0;  // slots that hold a value so far
   unsigned raw_inputs = 0;  // inputs whose words are loaded unconverted
@@ -337,6 +346,34 @@ static int fused_impl(hipnx_ctx *ctx, int n_instr, const hipnx_fused_instr *prog
     if (n_stats || reduce_op != -1) return set_error(HIPNX_EUNSUPPORTED, "fused: random words under a reduction");
     needs_compiled = true;
   }
+  if (scores.input >= 0) {
+    const Scores &c = scores;
+    const int dt = in_dts[c.input];
+    if (!n_stats || reduce_op != -1 || cols > 4096 || ctx->fused_mode != HIPNX_FUSED_COMPILED)
+      return set_error(HIPNX_EUNSUPPORTED, "fused_scores: a program of stages over at most 4096 columns");
+    if ((dt != HIPNX_BF16 && dt != HIPNX_F16) || c.K < 32 || c.K > 256 || c.K % 32 != 0)
+      return set_error(HIPNX_EUNSUPPORTED, "fused_scores: bf16 or f16 operands with K of 32 to 256 in whole steps of 32");
+    if (c.batch_outer < 1 || c.batch_inner < 1 || c.M < 1 || c.batch_outer > (1ll << 31) / c.batch_inner || c.M > (1ll << 31) / (c.batch_outer * c.batch_inner) ||
+        c.batch_outer * c.batch_inner * c.M != rows || in_row_strides[c.input] != (rows > 1 ? cols : 0) || in_col_strides[c.input] != 1)
+      return set_error(HIPNX_EINVAL, "fused_scores: extents that do not make the program's rows");
+    // (fewer than 256 results per item are summed in f64 by the separate contraction.  And a block pulls all of an item's right
+    // operand through one CU, about 0.1 MB a us: with few blocks a large one is better spread over the chip)
+    const int64_t blocks = c.batch_outer * c.batch_inner * ((c.M + SCORE_ROWS - 1) / SCORE_ROWS);
+    if (c.M * cols < 256 || (blocks < (int64_t)ctx->num_cus && cols * c.K > 65536))
+      return set_error(HIPNX_EUNSUPPORTED, "fused_scores: left to the separate contraction");
+    for (int side = 0; side < 2; side++) {
+      const int64_t *st = side ? c.r_strides : c.l_strides;
+      for (int i = 0; i < 3; i++)
+        if (st[i] < 0 || st[i] > (1ll << 40)) return set_error(HIPNX_EINVAL, "fused_scores: a stride of %lld elements", (long long)st[i]);
+      const int64_t last = (c.batch_outer - 1) * st[0] + (c.batch_inner - 1) * st[1] + ((side ? cols : c.M) - 1) * st[2] + c.K;
+      if (int s = check_buf(ctx, side ? c.r : c.l, (uint64_t)last * 2, side ? "fused_scores rhs" : "fused_scores lhs")) return s;
+    }
+    a.scores_inner = (int)c.batch_inner;
+    a.scores_rows = c.M;
+    a.l = c.l->ptr, a.r = c.r->ptr;
+    a.l_outer = c.l_strides[0], a.l_inner = c.l_strides[1], a.l_ld = c.l_strides[2];
+    a.r_outer = c.r_strides[0], a.r_inner = c.r_strides[1], a.r_ld = c.r_strides[2];
+  }
   // a few very long rows are split into segments by the separate reduction, whose order the stages follow: not here
   if (walk) {
     int would_be = 1;
@@ -366,6 +403,12 @@ static int fused_impl(hipnx_ctx *ctx, int n_instr, const hipnx_fused_instr *prog
     if (k == words) {
       if (dt != HIPNX_U32 || in_col_strides[k] != 1) return set_error(HIPNX_EINVAL, "fused: random words are u32, one per element");
       if (int st = check_buf(ctx, inputs[k], 8, "fused key")) return st;
+    }
+    if (k == scores.input) {  // (not in memory)
+      a.in_dt[k] = dt;
+      a.in_rs[k] = in_row_strides[k];
+      a.in_cs[k] = in_col_strides[k];
+      continue;
     }
     const uint64_t extent = n == 0 || k == words ? 0 : (uint64_t)((rows - 1) * in_row_strides[k] + (cols - 1) * in_col_strides[k] + 1);
     if (int st = check_buf(ctx, inputs[k], extent * sz, "fused input")) return st;
@@ -421,8 +464,9 @@ static int fused_impl(hipnx_ctx *ctx, int n_instr, const hipnx_fused_instr *prog
       if (walk || reduce_op != -1) return set_error(HIPNX_EUNSUPPORTED, "fused: more rows than one launch holds");
       grid = max_grid;
     }
+    if (scores.input >= 0) grid = scores.batch_outer * scores.batch_inner * ((scores.M + SCORE_ROWS - 1) / SCORE_ROWS);
     bool done = false;
-    if (int st = fused_launch_compiled(ctx, a, reduce_op, block_per_row, walk, (unsigned)grid, &done)) return st;
+    if (int st = fused_launch_compiled(ctx, a, reduce_op, block_per_row, walk, scores.K, (unsigned)grid, &done)) return st;
     if (done) {
       if (a.nseg > 1) {
         launch_fused_combine(ctx, a, reduce_op);
@@ -465,4 +509,18 @@ extern "C" int hipnx_fused_words(hipnx_ctx *ctx, int n_instr, const hipnx_fused_
     return set_error(HIPNX_EINVAL, "fused_words: key %d of %d", key_index, key_parts);
   const int64_t row_strides[HIPNX_FUSED_MAX_INPUTS] = {};
   return fused_impl(ctx, n_instr, prog, n_inputs, inputs, in_dts, row_strides, in_col_strides, 1, n, -1, out_dt, out, words, key_parts, key_index);
+}
+
+extern "C" int hipnx_fused_scores(hipnx_ctx *ctx, int n_instr, const hipnx_fused_instr *prog, int n_inputs, const hipnx_buf *const *inputs,
+                                  const int *in_dts, const int64_t *in_row_strides, const int *in_col_strides, int64_t cols, int scores,
+                                  int64_t batch_outer, int64_t batch_inner, int64_t M, int64_t K, const int64_t *strides,
+                                  const hipnx_buf *const *operands, int out_dt, hipnx_buf *out) {
+  if (scores < 0 || scores >= n_inputs || n_inputs > HIPNX_FUSED_MAX_INPUTS || !in_dts || !in_row_strides || !in_col_strides || !strides || !operands)
+    return set_error(HIPNX_EINVAL, "fused_scores: input %d of %d", scores, n_inputs);
+  if (batch_outer < 1 || batch_inner < 1 || M < 1 || K < 1 || K > 1 << 30 || batch_outer > 1 << 30 || batch_inner > 1 << 30 || M > (1ll << 40) / (batch_outer * batch_inner))
+    return set_error(HIPNX_EUNSUPPORTED, "fused_scores: empty or enormous extents");
+  Scores s;
+  s.input = scores, s.K = (int)K, s.batch_outer = batch_outer, s.batch_inner = batch_inner, s.M = M;
+  s.l_strides = strides, s.r_strides = strides + 3, s.l = operands[0], s.r = operands[1];
+  return fused_impl(ctx, n_instr, prog, n_inputs, inputs, in_dts, in_row_strides, in_col_strides, batch_outer * batch_inner * M, cols, -1, out_dt, out, -1, 0, 0, s);
 }

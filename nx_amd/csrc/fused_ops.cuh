@@ -37,6 +37,12 @@ struct FusedArgs {
   int64_t seg_len;
   void *partial;
   int nseg;
+  // the input that is the result of a contraction and not in memory (-1: there is none): rows of l against rows of r, K contiguous
+  // elements each, `scores_rows` rows of l per batch item; strides in elements along the batch's two axes and from row to row
+  int scores, scores_inner;
+  int64_t scores_rows;
+  const void *l, *r;
+  int64_t l_outer, l_inner, l_ld, r_outer, r_inner, r_ld;
   int key_parts, key_index;  // the key is number key_index of the key_parts that in[words] splits into (0 parts: in[words] itself)
   int unused;
 };
@@ -186,6 +192,44 @@ struct RowVector {
   float held[FE];   // input P::held
 };
 
+// How the lanes of a row share it (P::form).  In every form a lane meets its elements in the order in which the separate
+// reduction of rows of that length folds them (reduce_rows_kernel and its short-row forms).
+//   ROW_WHOLE: rows of whole vectors; lane l takes the vectors l, l + tpr, ...
+//   ROW_LANE: rows of at most 16 elements; a lane takes a row (tpr = 1): its vectors, then the P::tail elements behind them.
+//   ROW_GROUP: rows of 17 to 256 elements that are not whole vectors; 8, 16 or 32 lanes, so that each has one vector at most;
+//     the elements behind the last vector one per lane.
+//   ROW_RAGGED: longer rows that are not whole vectors; the elements up to a vector boundary of the BUFFER one per lane, whole
+//     aligned vectors as ROW_WHOLE, the elements behind them one per lane.
+// Rows off the vector grid went node by node before, every intermediate through memory: f32 layer norm of 26248 x 185
+// 106 us, bf16 softmax of 247650 x 178 160 us.
+enum { ROW_WHOLE, ROW_LANE, ROW_GROUP, ROW_RAGGED };
+
+// ---- a contraction's result as an input (fused_scores_body) ----
+constexpr int SCORE_ROWS = 16;
+// the block's rows of it in LDS: row i's column c at element c + score_shift of row i, so that the vectors of a ROW_RAGGED row are
+// aligned; a pitch that sets the sixteen rows four banks apart
+template <typename P>
+__device__ __forceinline__ uint16_t *score_row(int i) {
+  __shared__ __attribute__((aligned(16))) uint16_t sm[SCORE_ROWS * (P::scores_cols + 8)];
+  return sm + i * (P::scores_cols + 8);
+}
+__device__ __forceinline__ int score_shift(int64_t r, int64_t cols, bool ragged) { return ragged ? (int)(r * cols & 7) : 0; }
+template <typename P>
+__device__ __forceinline__ void load_scores(KernArgs a, int64_t r, int64_t k, int valid, Vecs &dst) {
+  const int i = (int)((uint32_t)r % (uint32_t)a->scores_rows) % SCORE_ROWS;
+  const uint16_t *p = score_row<P>(i) + k + score_shift(r, a->cols, P::form == ROW_RAGGED);
+  uint32_t w[FE];
+  if (valid == FE) {
+    const uint4 v = *reinterpret_cast<const uint4 *>(p);
+    w[0] = v.x & 0xFFFFu, w[1] = v.x >> 16, w[2] = v.y & 0xFFFFu, w[3] = v.y >> 16, w[4] = v.z & 0xFFFFu, w[5] = v.z >> 16, w[6] = v.w & 0xFFFFu, w[7] = v.w >> 16;
+  } else {
+#pragma unroll
+    for (int e = 0; e < FE; e++) w[e] = e < valid ? p[e] : 0u;
+  }
+#pragma unroll
+  for (int e = 0; e < FE; e++) dst[0][e] = element_to_f32(w[e], P::in_dt[P::scores < 0 ? 0 : P::scores]);
+}
+
 template <typename P, int SRC, int ARG, unsigned IMM, bool RAW>
 __device__ __forceinline__ void fetch_static(KernArgs a, const Saved &S, const RowStats &stats, const int64_t (&row)[FV],
                                              const int64_t (&col)[FV], int valid, const RowVector *kept, Vecs &dst) {
@@ -204,6 +248,10 @@ __device__ __forceinline__ void fetch_static(KernArgs a, const Saved &S, const R
 #pragma unroll
       for (int e = 0; e < FE; e++) dst[u][e] = stats[ARG];
   } else if constexpr (SRC == HIPNX_FUSED_SRC_INPUT) {
+    if constexpr (ARG == P::scores) {
+      load_scores<P>(a, row[0], col[0], valid, dst);
+      return;
+    }
     // RAW: the words of a 4-byte input as they are (what the f32 path does with its bits)
     if (valid == FE) load_input_as<P::unal>(a, ARG, RAW ? (int)HIPNX_F32 : P::in_dt[ARG], P::in_cs[ARG], row, col, dst);
     else load_input_tail(a, ARG, RAW ? (int)HIPNX_F32 : P::in_dt[ARG], P::in_cs[ARG], row, col, valid, dst);
@@ -524,18 +572,6 @@ __device__ __forceinline__ float as_stored(CT v, int dt) {
   }
 }
 
-// How the lanes of a row share it (P::form).  In every form a lane meets its elements in the order in which the separate
-// reduction of rows of that length folds them (reduce_rows_kernel and its short-row forms).
-//   ROW_WHOLE: rows of whole vectors; lane l takes the vectors l, l + tpr, ...
-//   ROW_LANE: rows of at most 16 elements; a lane takes a row (tpr = 1): its vectors, then the P::tail elements behind them.
-//   ROW_GROUP: rows of 17 to 256 elements that are not whole vectors; 8, 16 or 32 lanes, so that each has one vector at most;
-//     the elements behind the last vector one per lane.
-//   ROW_RAGGED: longer rows that are not whole vectors; the elements up to a vector boundary of the BUFFER one per lane, whole
-//     aligned vectors as ROW_WHOLE, the elements behind them one per lane.
-// Rows off the vector grid went node by node before, every intermediate through memory: f32 layer norm of 26248 x 185
-// 106 us, bf16 softmax of 247650 x 178 160 us.
-enum { ROW_WHOLE, ROW_LANE, ROW_GROUP, ROW_RAGGED };
-
 template <int N>
 struct Elements {
   static constexpr int n = N;
@@ -616,7 +652,8 @@ __device__ __forceinline__ void row_stage(KernArgs a, int64_t r, int lane, const
       constexpr int n = decltype(count)::n;
       const int64_t row[FV] = {r}, col[FV] = {k};
       Vecs x;
-      if constexpr (n == FE) load_input_as<P::unal>(a, P::held, P::in_dt[P::held], 1, row, col, x);
+      if constexpr (P::held == P::scores) load_scores<P>(a, r, k, n, x);
+      else if constexpr (n == FE) load_input_as<P::unal>(a, P::held, P::in_dt[P::held], 1, row, col, x);
       else load_input_tail(a, P::held, P::in_dt[P::held], 1, row, col, n, x);
 #pragma unroll
       for (int e = 0; e < n; e++) mine.held[e] = x[0][e];
@@ -695,6 +732,90 @@ __device__ __forceinline__ void fused_row_stages_body() {
   RowStats stats = {};
   RowVector kept[(P::nv > 0 ? P::nv : 1) + 2];  // (indexed by compile-time trip numbers only: registers)
   row_stage<P, 0>(a, r, threadIdx.x % P::tpr, row_walk<P>(r, a->cols), stats, kept);
+}
+
+// Stages over the rows of a contraction whose result exists only here (attention probabilities: scores, scaling, softmax).  A block
+// takes sixteen rows of l against all rows of r: each wave contracts every fourth tile of sixteen columns with operands
+// loaded straight into MFMA registers (no wave shares a row of r, and r is in the L2 for the blocks of the same batch item,
+// which follow one another on one XCD), rounds the sums to the contraction's type and leaves them in LDS; then the row
+// stages run as they do over a tensor.  P::scores_k: K, in whole steps of 32.
+// Bound by the stages' vector instructions and the result's way to memory: bf16 4 x 8 x 512 x 512 from 64-element rows, f32 result,
+// 26 us of kernels and 23.8 us a pass in two -> 21.9 us a pass in one; one query against 368 keys 10.2 -> 6.2.
+template <int DT>
+struct ScoreMma;
+typedef float score4 __attribute__((ext_vector_type(4)));
+typedef int score_words __attribute__((ext_vector_type(4)));
+template <>
+struct ScoreMma<HIPNX_BF16> {
+  static __device__ __forceinline__ score4 step(score_words a, score_words b, score4 c) {
+    typedef __bf16 v8 __attribute__((ext_vector_type(8)));
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8, a), __builtin_bit_cast(v8, b), c, 0, 0, 0);
+  }
+};
+template <>
+struct ScoreMma<HIPNX_F16> {
+  static __device__ __forceinline__ score4 step(score_words a, score_words b, score4 c) {
+    typedef _Float16 v8 __attribute__((ext_vector_type(8)));
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8, a), __builtin_bit_cast(v8, b), c, 0, 0, 0);
+  }
+};
+
+template <typename P>
+__device__ __forceinline__ void fused_scores_body() {
+  KernArgs a = (KernArgs)__builtin_amdgcn_kernarg_segment_ptr();
+  typedef score_words __attribute__((aligned(2))) words_any;
+  constexpr int STEPS = P::scores_k / 32, TILES = STEPS <= 2 ? 4 : STEPS <= 4 ? 2 : 1;  // column tiles in flight: up to 32 registers of operands
+  constexpr int DT = P::in_dt[P::scores];
+  const int lane = threadIdx.x % WAVE, wave = threadIdx.x / WAVE;
+  const int64_t cols = a->cols, M = a->scores_rows, tiles_m = (M + SCORE_ROWS - 1) / SCORE_ROWS;
+  int64_t block = blockIdx.x;
+  if (gridDim.x % 8 == 0) block = (int64_t)(blockIdx.x % 8) * (gridDim.x / 8) + blockIdx.x / 8;
+  const int64_t item = block / tiles_m, m0 = (block - item * tiles_m) * SCORE_ROWS;
+  const int64_t outer = item / a->scores_inner, inner = item - outer * a->scores_inner;
+  {
+    const uint16_t *l = (const uint16_t *)a->l + outer * a->l_outer + inner * a->l_inner, *r = (const uint16_t *)a->r + outer * a->r_outer + inner * a->r_inner;
+    const int64_t m = m0 + lane % 16 < M ? m0 + lane % 16 : M - 1;  // (rows past the edge: any row; they are not used)
+    score_words x[STEPS];
+#pragma unroll
+    for (int s = 0; s < STEPS; s++) x[s] = *reinterpret_cast<const words_any *>(l + m * a->l_ld + s * 32 + lane / 16 * 8);
+    uint16_t *row = score_row<P>(lane % 16);
+    const int shift = score_shift(item * M + m0 + lane % 16, cols, P::form == ROW_RAGGED);
+    const bool whole = cols % 4 == 0;  // four neighbouring columns lie in the row together, eight bytes aligned
+    for (int64_t n0 = wave * 16; n0 < cols; n0 += 64 * TILES) {
+      score_words y[TILES][STEPS];
+#pragma unroll
+      for (int t = 0; t < TILES; t++) {
+        int64_t n = n0 + t * 64 + lane % 16;
+        n = n < cols ? n : cols - 1;
+#pragma unroll
+        for (int s = 0; s < STEPS; s++) y[t][s] = *reinterpret_cast<const words_any *>(r + n * a->r_ld + s * 32 + lane / 16 * 8);
+      }
+#pragma unroll
+      for (int t = 0; t < TILES; t++) {
+        score4 acc = {0, 0, 0, 0};
+#pragma unroll
+        for (int s = 0; s < STEPS; s++) acc = ScoreMma<DT>::step(y[t][s], x[s], acc);
+        const int64_t n = n0 + t * 64 + lane / 16 * 4;  // a lane has four columns of row lane % 16
+        uint16_t h[4];
+#pragma unroll
+        for (int e = 0; e < 4; e++) h[e] = DT == HIPNX_BF16 ? conv<float>::to_bf16(acc[e]) : conv<float>::to_f16(acc[e]);
+        if (whole) {
+          if (n < cols) *reinterpret_cast<uint2 *>(row + n + shift) = make_uint2(h[0] | (uint32_t)h[1] << 16, h[2] | (uint32_t)h[3] << 16);
+        } else {
+#pragma unroll
+          for (int e = 0; e < 4; e++)
+            if (n + e < cols) row[n + e + shift] = h[e];
+        }
+      }
+    }
+  }
+  __syncthreads();
+  for (int i = threadIdx.x / P::tpr; i < SCORE_ROWS && m0 + i < M; i += FBLOCK / P::tpr) {  // (a row's lanes go on or stop together)
+    const int64_t r = item * M + m0 + i;
+    RowStats stats = {};
+    RowVector kept[(P::nv > 0 ? P::nv : 1) + 2];
+    row_stage<P, 0>(a, r, threadIdx.x % P::tpr, row_walk<P>(r, cols), stats, kept);
+  }
 }
 
 }  // namespace hipnx

@@ -159,10 +159,12 @@ static Keeps what_is_kept(const FusedArgs &a, bool walk) {
 // everything a compiled kernel is specialised on, as bytes: the cache key.  What the length of a row decides comes last: the keys of
 // one program's kernels for rows of other lengths differ in it alone.
 constexpr size_t LENGTH_KEY = 4 * sizeof(int);
-static std::string make_key(const FusedArgs &a, const Keeps &keeps, int reduce_op, bool block_per_row) {
+// columns of a contraction's result that LDS has room for: whole steps of 512, one kernel for all lengths of a step
+static int scores_class(const FusedArgs &a) { return a.scores < 0 ? 0 : (int)((a.cols + 511) / 512 * 512); }
+static std::string make_key(const FusedArgs &a, const Keeps &keeps, int reduce_op, bool block_per_row, int scores_k) {
   std::string k;
   k.reserve(40 + 16 * a.n_instr + 8 * a.n_inputs);
-  const int head[5] = {a.n_instr, a.n_inputs, a.out_dt, reduce_op * 2 + (block_per_row ? 1 : 0), a.words};
+  const int head[8] = {a.n_instr, a.n_inputs, a.out_dt, reduce_op * 2 + (block_per_row ? 1 : 0), a.words, a.scores, scores_class(a), scores_k};
   k.append((const char *)head, sizeof(head));
   k.append((const char *)a.ins, sizeof(hipnx_fused_instr) * a.n_instr);
   k.append((const char *)a.in_dt, sizeof(int) * a.n_inputs);
@@ -176,14 +178,15 @@ static std::string make_key(const FusedArgs &a, const Keeps &keeps, int reduce_o
 // A program that keeps an input in registers only to read it once could do without, and then takes rows of any number of whole
 // vectors (a wave per row, a block per long row): its module also has that kernel, for a capture that meets a length which has
 // not been compiled (a new module is no work to record).  One that carries values cannot.
-static bool is_for_any_length(const FusedArgs &a, const Keeps &k) { return k.form == ROW_WHOLE && k.trips == 0 && (k.tpr == 0 || k.tpr == class_lanes(a)); }
-static bool has_kernel_for_any_length(const FusedArgs &a, const Keeps &k) { return a.cols % FE == 0 && !k.carries && !is_for_any_length(a, k); }
+static bool is_for_any_length(const FusedArgs &a, const Keeps &k) { return a.scores < 0 && k.form == ROW_WHOLE && k.trips == 0 && (k.tpr == 0 || k.tpr == class_lanes(a)); }
+static bool has_kernel_for_any_length(const FusedArgs &a, const Keeps &k) { return a.scores < 0 && a.cols % FE == 0 && !k.carries && !is_for_any_length(a, k); }
 static std::string any_length(const std::string &name) { return name + "_any"; }
 
 // the whole translation unit for one program
-static std::string make_source(const FusedArgs &a, const Keeps &keeps, int reduce_op, bool block_per_row, const std::string &name) {
+static std::string make_source(const FusedArgs &a, const Keeps &keeps, int reduce_op, bool block_per_row, int scores_k, const std::string &name) {
   std::string s = RTC_PREAMBLE;
-  s += "namespace hipnx {\nstruct Program {\n  static constexpr int n_instr = " + std::to_string(a.n_instr) + ", out_dt = " + std::to_string(a.out_dt) + ", words = " + std::to_string(a.words) + ";\n";
+  s += "namespace hipnx {\nstruct Program {\n  static constexpr int n_instr = " + std::to_string(a.n_instr) + ", out_dt = " + std::to_string(a.out_dt) + ", words = " + std::to_string(a.words) +
+       ", scores = " + std::to_string(a.scores < 0 ? -2 : a.scores) + ", scores_cols = " + std::to_string(scores_class(a)) + ", scores_k = " + std::to_string(scores_k) + ";\n";
   const hipnx_fused_instr *q = a.ins;
   list_of(s, "kind", "int", a.n_instr, [&](int i) { return std::to_string((int)q[i].kind); });
   list_of(s, "op", "int", a.n_instr, [&](int i) { return std::to_string((int)q[i].op); });
@@ -227,6 +230,7 @@ static std::string make_source(const FusedArgs &a, const Keeps &keeps, int reduc
   s += kernel(name);
   const char *tpr = block_per_row ? "FBLOCK" : "WAVE";
   if (a.words >= 0) s += "  fused_words_body<P>();\n";
+  else if (a.scores >= 0) s += "  fused_scores_body<P>();\n";
   else if (stages || keeps.form != ROW_WHOLE) s += "  fused_row_stages_body<P>();\n";
   else switch (reduce_op) {
     case HIPNX_RED_SUM: s += std::string("  fused_reduce_rows_body<RunStatic<P>, PlainReducer<double, HIPNX_RED_SUM, false>, double, ") + tpr + ">();\n"; break;
@@ -297,11 +301,11 @@ static int trim_cache(hipnx_ctx *ctx) {
 // *done = false (and HIPNX_OK) when the caller should run the interpreting kernel instead: the
 // program is new and the stream is capturing (compiling and loading a module is no work to record).
 // `walk`: a group of lanes takes a row, the grid follows from how many; `grid` is the grid otherwise.
-int fused_launch_compiled(hipnx_ctx *ctx, const FusedArgs &a, int reduce_op, bool block_per_row, bool walk, unsigned grid, bool *done) {
+int fused_launch_compiled(hipnx_ctx *ctx, const FusedArgs &a, int reduce_op, bool block_per_row, bool walk, int scores_k, unsigned grid, bool *done) {
   *done = false;
   const Keeps keeps = what_is_kept(a, walk);
   int lanes = keeps.tpr;
-  const std::string key = make_key(a, keeps, reduce_op, block_per_row);
+  const std::string key = make_key(a, keeps, reduce_op, block_per_row, scores_k);
   auto it = ctx->fused_kernels.find(key);
   hipFunction_t function = nullptr;
   if (it == ctx->fused_kernels.end() && ctx->capture) {
@@ -320,12 +324,12 @@ int fused_launch_compiled(hipnx_ctx *ctx, const FusedArgs &a, int reduce_op, boo
     int stages = 0;
     for (int i = 0; i < a.n_instr; i++) stages += a.ins[i].kind == HIPNX_FUSED_ROW_REDUCE;
     char name[96];
-    snprintf(name, sizeof(name), "fused_%s_%dinstr_%08zx", a.words >= 0 ? "words" : stages ? "stages" : reduce_op != -1 ? "map_reduce" : "map", a.n_instr,
+    snprintf(name, sizeof(name), "fused_%s_%dinstr_%08zx", a.words >= 0 ? "words" : a.scores >= 0 ? "scores" : stages ? "stages" : reduce_op != -1 ? "map_reduce" : "map", a.n_instr,
              std::hash<std::string>{}(key) & 0xFFFFFFFFu);
     if (ctx->fused_kernels.size() >= ctx->fused_cache_max)
       if (int st = trim_cache(ctx)) return st;
     hipnx_ctx::FusedKernel k{};
-    if (int st = compile(ctx, make_source(a, keeps, reduce_op, block_per_row, name), name, has_kernel_for_any_length(a, keeps), &k)) return st;
+    if (int st = compile(ctx, make_source(a, keeps, reduce_op, block_per_row, scores_k, name), name, has_kernel_for_any_length(a, keeps), &k)) return st;
     if (is_for_any_length(a, keeps)) k.any_length = k.function;
     it = ctx->fused_kernels.emplace(key, k).first;
   }
@@ -334,7 +338,7 @@ int fused_launch_compiled(hipnx_ctx *ctx, const FusedArgs &a, int reduce_op, boo
   if (ctx->capture) it->second.in_graph = true;  // a recorded launch refers to the loaded module for as long as the graph lives
   // the argument block is the kernel's one by-value parameter: hand it over as the packed buffer it is
   size_t size = sizeof(FusedArgs);
-  if (walk) grid = (unsigned)((a.rows + FBLOCK / lanes - 1) / (FBLOCK / lanes));
+  if (walk && a.scores < 0) grid = (unsigned)((a.rows + FBLOCK / lanes - 1) / (FBLOCK / lanes));
   void *config[] = {HIP_LAUNCH_PARAM_BUFFER_POINTER, (void *)&a, HIP_LAUNCH_PARAM_BUFFER_SIZE, &size, HIP_LAUNCH_PARAM_END};
   HIPNX_HIP(hipModuleLaunchKernel(function, grid, 1, 1, FBLOCK, 1, 1, 0, ctx->stream, nullptr, config));
   *done = true;

@@ -817,6 +817,39 @@ def _absorb_transposes(order: List[Tensor], uses) -> int:
     return found
 
 
+def _dot_views(mod, out: Tensor, l, l_axes, c1, b1, r, r_axes, c2, b2):
+    """dot(transpose(l), ..., transpose(r), ...) on backend `mod`, without the copies where it can (axes of None: as it is)."""
+    one_call = getattr(mod, "dot_views", None) if l_axes is not None or r_axes is not None else None
+    if one_call is not None:
+        try:
+            return one_call(out, l, l_axes, c1, b1, r, r_axes, c2, b2)
+        except Exception as err:  # operands the kernels cannot read where they lie
+            if getattr(err, "status", None) != _EUNSUPPORTED:
+                raise
+    l, r = (v if axes is None else mod.transpose(v.with_(data=None, shape=tuple(v.shape[a] for a in axes)), v, list(axes))
+            for v, axes in ((l, l_axes), (r, r_axes)))
+    return mod.dot(out, l, c1, b1, r, c2, b2)
+
+
+def _absorb_scores(order: List[Tensor], uses) -> None:
+    """Row stages over the result of a contraction that nobody else reads contract it themselves (attention probabilities)."""
+    for node in order:
+        e = node.data
+        if e.op != "fused" or not isinstance(e.args[0], _RowCluster):
+            continue
+        cluster, inputs = e.args
+        for at, t in enumerate(inputs):
+            d = t.data
+            if d.op not in ("dot", "dot_views") or d.scope != 0 or uses[d.id] != 1 or t.type not in (("bf", 16), ("f", 16)):
+                continue
+            l, l_axes, c1, b1, r, r_axes, c2, b2 = d.args if d.op == "dot_views" else [d.args[0], None, *d.args[1:4], None, *d.args[4:]]
+            rows, cols, strides = cluster.layout
+            if l.type == t.type and r.type == t.type and rows > 1 and strides[at] == (cols, 1):
+                cluster.scores = (at, l_axes, c1, b1, r_axes, c2, b2)
+                e.args = [cluster, inputs[:at] + [l] + inputs[at + 1:] + [r]]
+                break
+
+
 def _fuse_planned(roots: List[Tensor]) -> int:
     order, uses, seen, parents = [], {}, set(), {}
 
@@ -977,7 +1010,8 @@ def _fuse_planned(roots: List[Tensor]) -> int:
         e.op, e.args = "fused", [both, inner.args[1]]
     if _plan["ints"]:  # planned for compiled kernels: groups over the same rows become stages of one
         _cluster_rows(roots)
-        _absorb_random(roots)
+        _absorb_random(*_readers(roots))
+        _absorb_scores(*_readers(roots))
     return formed
 
 
@@ -1006,9 +1040,8 @@ def _split_of(t: Tensor):
     return keys.data.args[1][0], keys.shape[0], starts[0]
 
 
-def _absorb_random(roots: List[Tensor]) -> None:
-    """A group over a flat index space that alone reads random words makes them itself, from the key; a key that is one of a
-    split is derived where it is used (the words' way through memory, the split and its slice were three launches more)."""
+def _readers(roots: List[Tensor]):
+    """The root scope's nodes in evaluation order, and how often each is read."""
     order, uses, seen = [], {}, set()
 
     def walk(t):
@@ -1025,6 +1058,12 @@ def _absorb_random(roots: List[Tensor]) -> None:
         order.append(t)
     for r in roots:
         walk(r)
+    return order, uses
+
+
+def _absorb_random(order: List[Tensor], uses) -> None:
+    """A group over a flat index space that alone reads random words makes them itself, from the key; a key that is one of a
+    split is derived where it is used (the words' way through memory, the split and its slice were three launches more)."""
     for node in order:
         e = node.data
         if e.op != "fused" or not isinstance(e.args[0], _Group) or e.args[0].reduce is not None or not e.args[0].program or not e.args[0].layout:
@@ -1062,13 +1101,26 @@ class _RowCluster:
     reduce = None
     how = {"mode": "compiled"}
     split_rows = False
+    scores = None  # (input number, the rest of a dot_views node's arguments): that input is a contraction's result (_absorb_scores)
 
     def __init__(self, steps, inputs, program, layout, n_stages):
         self.steps, self.inputs, self.program, self.layout, self.n_stages = steps, inputs, program, layout, n_stages
         self.root = steps[-1]
 
     def run(self, run: "_Run", out: Tensor, values: List[Tensor]):
-        fused = getattr(run.pick(values), "fused_elementwise", None)
+        mod = run.pick(values)
+        if self.scores is not None:
+            at, l_axes, c1, b1, r_axes, c2, b2 = self.scores
+            l, r, values = values[at], values[-1], values[:-1]
+            one_call = getattr(mod, "fused_scores", None)
+            if one_call is not None:
+                try:
+                    return one_call(out, self.program, values, self.layout, at, (l, l_axes, c1, b1, r, r_axes, c2, b2), **self.how)
+                except Exception as e:  # a shape that the separate contraction is for
+                    if getattr(e, "status", None) != _EUNSUPPORTED:
+                        raise
+            values[at] = _dot_views(mod, self.inputs[at].with_(data=None), l, l_axes, c1, b1, r, r_axes, c2, b2)
+        fused = getattr(mod, "fused_elementwise", None)
         if fused is not None and not self.split_rows:
             try:
                 return fused(out, self.program, values, self.layout, **self.how)
@@ -1547,16 +1599,7 @@ class _Run:
             l, l_axes, c1, b1, r, r_axes, c2, b2 = e.args
             lv, rv = self.eval(l, scope), self.eval(r, scope)
             mod, out = self.pick([lv, rv]), x.with_(data=None)
-            one_call = getattr(mod, "dot_views", None)
-            if one_call is not None:
-                try:
-                    return one_call(out, lv, l_axes, c1, b1, rv, r_axes, c2, b2)
-                except Exception as err:  # operands the kernels cannot read where they lie
-                    if getattr(err, "status", None) != _EUNSUPPORTED:
-                        raise
-            lv, rv = (v if axes is None else mod.transpose(v.with_(data=None, shape=tuple(v.shape[a] for a in axes)), v, list(axes))
-                      for v, axes in ((lv, l_axes), (rv, r_axes)))
-            return mod.dot(out, lv, c1, b1, rv, c2, b2)
+            return _dot_views(mod, out, lv, l_axes, c1, b1, rv, r_axes, c2, b2)
         if op == "random_key":
             key, parts, index = e.args
             key = self.eval(key, scope)

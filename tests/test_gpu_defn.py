@@ -1407,3 +1407,75 @@ def test_callbacks_laid_out_once_follow_their_operands(hip):
             assert_bits_equal(Nx.dot(y, [1], y, [0]), want, mode)
         finally:
             B.bf16_rounding(previous)
+
+
+def attention_probabilities(q, k, heads, mask=None, log=False):
+    scores = Nx.dot(split_heads(q, heads), [3], [0, 1], split_heads(k, heads), [3], [0, 1])
+    z = Nx.multiply(Nx.as_type(scores, "f32"), 0.125)
+    if mask is not None:
+        z = Nx.add(z, mask)
+    return log_softmax_rows(z) if log else softmax_rows(z)
+
+
+# one query row and rows around a block's sixteen; rows of columns in every form (whole vectors, 8 to 32 lanes, heads and tails),
+# steps of 512 columns; K of one to eight steps
+@pytest.mark.parametrize("ty", ["bf16", "f16"])
+@pytest.mark.parametrize("batch,heads,queries,keys,dim", [(2, 3, 1, 320, 64), (3, 2, 16, 16, 32), (2, 2, 17, 100, 64), (1, 5, 33, 185, 128), (2, 4, 31, 512, 64),
+                                                          (1, 3, 40, 513, 96), (2, 2, 64, 1001, 64), (1, 2, 20, 2041, 32), (14, 1, 300, 4096, 32), (4, 16, 18, 250, 256)])
+def test_row_stages_contract_their_scores_themselves(batch, heads, queries, keys, dim, ty, hip):
+    """On whole numbers, whose sums are exact in any order: the bits of the nodes one by one, and no contraction of its own."""
+    rng = np.random.default_rng(seed_of(batch, heads, queries, keys, dim, ty))
+
+    def whole(*shape):
+        v = rng.integers(-2, 3, size=shape).astype(np.float32)
+        return from_numpy((v.view(np.uint32) >> 16).astype(np.uint16) if ty == "bf16" else v.astype(np.float16), ty, hip)
+    q, k = whole(batch, queries, heads * dim), whole(batch, keys, heads * dim)
+    guard = whole(64)
+    before = raw(guard).copy()
+    mask = rand_float(rng, "f32", (batch, heads, queries, keys), hip)
+    calls = []
+    original = hip.fused_scores.__func__
+
+    def counting(cls, *a, **kw):
+        out = original(cls, *a, **kw)  # (a refusal raises)
+        calls.append(1)
+        return out
+    for fun, args in ((lambda a, b: attention_probabilities(a, b, heads), (q, k)), (lambda a, b: attention_probabilities(a, b, heads, log=True), (q, k)),
+                      (lambda a, b, m: attention_probabilities(a, b, heads, m), (q, k, mask))):
+        planned = defn.compile(fun, *args, fuse="compiled")
+        if len(args) == 3:  # (the masked scores are a tensor of their own: two full-size operands)
+            assert_bits_equal(planned(*args), defn.compile(fun, *args)(*args), f"{ty}, mask")
+            continue
+        assert planned.roots[0].data.args[0].scores is not None
+        calls.clear()
+        hip.fused_scores = classmethod(counting)
+        try:
+            got = planned(*args)
+        finally:
+            hip.fused_scores = classmethod(original)
+        assert calls == [1]
+        assert_bits_equal(got, defn.compile(fun, *args)(*args), f"{ty}")
+    np.testing.assert_array_equal(raw(guard), before)
+
+
+@pytest.mark.parametrize("ty", ["bf16", "f16"])
+def test_scores_that_are_left_to_the_contraction(ty, hip):
+    """K off the steps of 32, few results per item (summed in f64 there), rows of more than 4096, one block per item over a large right
+    operand, the other rounding: two calls, the same values as ever."""
+    from nx_amd import backend as B
+    rng = np.random.default_rng(seed_of(ty, "left"))
+    for batch, heads, queries, keys, dim in ((2, 2, 20, 64, 40), (1, 4, 1, 100, 64), (1, 1, 8, 4104, 32), (1, 2, 1, 2048, 128)):
+        q, k = rand_float(rng, ty, (batch, queries, heads * dim), hip), rand_float(rng, ty, (batch, keys, heads * dim), hip)
+        fun = lambda a, b: attention_probabilities(a, b, heads)  # noqa: E731
+        planned, want = defn.compile(fun, q, k, fuse="compiled"), defn.compile(fun, q, k)(q, k)
+        for _ in range(4):
+            assert_bits_equal(planned(q, k), want, f"{queries} x {keys} x {dim}")
+        assert planned.replay is not None  # (a refusal does not keep the two calls from being recorded)
+    q, k = rand_float(rng, ty, (2, 20, 128), hip), rand_float(rng, ty, (2, 64, 128), hip)
+    fun = lambda a, b: attention_probabilities(a, b, 2)  # noqa: E731
+    planned = defn.compile(fun, q, k, fuse="compiled")
+    previous = B.bf16_rounding("nearest_even")
+    try:
+        assert_bits_equal(planned(q, k), defn.compile(fun, q, k)(q, k), "nearest even")
+    finally:
+        B.bf16_rounding(previous)
