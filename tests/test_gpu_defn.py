@@ -1327,6 +1327,33 @@ def test_a_recording_is_left_where_it_does_not_apply(hip):
         planned(t, x)
 
 
+@pytest.mark.parametrize("ty", ["f32", "bf16", "f16"])
+@pytest.mark.parametrize("cols", [10, 72, 185, 512, 1001])
+def test_quotients_of_exponentials_are_divisions(cols, ty, hip):
+    """exp(x) / s over rows whose exponentials lie on both sides of every bound of the quick quotient: zeros, subnormal numbers,
+    infinities, NaN; divisors of all sizes."""
+    rng = np.random.default_rng(seed_of(cols, ty, "quotients"))
+    span = {"f16": 9.0, "bf16": 100.0, "f32": 104.0}[ty]
+    x = rng.uniform(-span, 0, (64, cols)).astype(np.float32)
+    x[:16] = rng.uniform(-3, 3, (16, cols))
+    x[16:24, ::3] = -np.inf
+    x[24:28, 1::5] = 60.0 if ty != "f16" else 9.0
+    x[28:30, 2::7], x[30, 3], x[31, 4] = 80.0 if ty != "f16" else 10.0, np.inf, np.nan
+    scale = np.float32(2.0) ** rng.integers(-60, 60, (64, 1)).astype(np.float32) * rng.uniform(1, 2, (64, 1)).astype(np.float32)
+    s = from_numpy(scale, "f32", hip)
+    t = from_numpy((x.view(np.uint32) >> 16).astype(np.uint16) if ty == "bf16" else x.astype(np.float16 if ty == "f16" else np.float32), ty, hip)
+
+    def softmaxed(v):
+        e = Nx.exp(v)
+        return Nx.divide(e, Nx.sum(e, axes=[-1], keep_axes=True))
+
+    def scaled(v, w):  # the divisor's size set by an operand
+        e = Nx.exp(Nx.as_type(v, "f32"))
+        return Nx.divide(e, Nx.multiply(Nx.sum(Nx.multiply(e, w), axes=[-1], keep_axes=True), 0.37))
+    for fun, args in ((softmaxed, (t,)), (scaled, (t, s))):
+        assert_bits_equal(defn.compile(fun, *args, fuse="compiled")(*args), defn.compile(fun, *args)(*args), f"{fun.__name__} {cols} {ty}")
+
+
 def test_what_cannot_be_recorded_is_evaluated(hip):
     """One buffer under two parameters when the recording would be made, parameters and constants handed through, one buffer
     under two results, control flow."""
