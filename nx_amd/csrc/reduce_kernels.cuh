@@ -267,6 +267,49 @@ reduce_cols_kernel(const void *__restrict__ in, void *__restrict__ out, typename
   }
 }
 
+// Columns of a few thousand rows at most, few enough of them to leave the chip idle (a bias gradient, the mean of a small table): a
+// work-group of 1024 lanes takes X adjacent columns, its 1024 / X rows of lanes a run of the reduced axis each, eight loads in
+// flight, and the runs are folded in order in LDS.  Bound by latency: four round trips of a lane and ten steps in LDS.  (One lane
+// per column walked all of it, or it was two launches; us per call, then / now: f32 [48, 3] 12.2 / 3.5, [144, 915] 16.7 / 3.7,
+// [2048, 8] 9.4 / 4.0, [4000, 100] 23.2 / 5.8, [2000, 2000] 9.4 / 6.3.)
+constexpr int COLS_ONCE = 1024;
+constexpr int cols_once_run = 32;  // rows of a lane at most
+inline int cols_once_x(int64_t red, int64_t inner) {  // the widest group that covers the axis
+  int x = inner <= 8 ? 8 : inner <= 16 ? 16 : inner <= 32 ? 32 : 64;
+  while (x > 8 && red > cols_once_run * (COLS_ONCE / x)) x /= 2;
+  return x;
+}
+template <typename R, typename CT, int IDT, int X>
+__global__ void __launch_bounds__(COLS_ONCE)
+reduce_cols_once_kernel(const void *__restrict__ in, void *__restrict__ out, int odt, int red, int64_t inner) {
+  typedef typename R::acc_t acc_t;
+  constexpr int Y = COLS_ONCE / X;
+  __shared__ acc_t sm[COLS_ONCE];
+  const int tx = threadIdx.x % X, ty = threadIdx.x / X;
+  const int64_t col = (int64_t)blockIdx.x * X + tx, o = blockIdx.y, base = o * red * inner + col;
+  const int run = (red + Y - 1) / Y, k0 = ty * run, k1 = k0 + run < red ? k0 + run : red;
+  acc_t acc = R::init();
+  if (col < inner && k0 < k1) {
+    acc = R::seed(acc, k0);
+    for (int k = k0; k < k1; k += 8) {
+      CT v[8];
+#pragma unroll
+      for (int u = 0; u < 8; u++) v[u] = load_one<CT>(in, IDT, base + (int64_t)(k + u < k1 ? k + u : k1 - 1) * inner);
+#pragma unroll
+      for (int u = 0; u < 8; u++)
+        if (k + u < k1) acc = R::accumulate(acc, v[u], k + u);
+    }
+  }
+  sm[threadIdx.x] = acc;
+  __syncthreads();
+#pragma unroll
+  for (int w = 1; w < Y; w *= 2) {  // neighbouring runs first: in order
+    if (ty % (2 * w) == 0) sm[threadIdx.x] = R::combine(sm[threadIdx.x], sm[threadIdx.x + w * X]);
+    __syncthreads();
+  }
+  if (ty == 0 && col < inner) finalize(out, odt, o * inner + col, sm[tx]);
+}
+
 // fold partial[outer, nseg, inner] -> out[outer, inner].  A work-group takes 32 adjacent outputs; its eight rows
 // of 32 lanes each fold a slice of the segments (four loads in flight per lane), and the first row folds the eight
 // slices in segment order.  (One lane per output walking all segments is a chain of up to 1024 dependent
@@ -426,6 +469,21 @@ static int run_reduce_t(hipnx_ctx *ctx, bool static_ws, int idt, int odt, int64_
     }
     partials_release(ctx, static_ws, ws, ws_cap);
   } else {
+    if constexpr (IDT >= 0 && IDT != HIPNX_F64 && std::is_floating_point<CT>::value) {
+      // (more work-groups than this and the kernel below, whose lanes have eight columns each, gives the chip its waves in longer
+      // runs of memory; with eight columns to a work-group that is sooner: f32 [4096, 1000] 11.5 us here, 9.3 there; [4096, 512] 6.1, 9.6)
+      const int X = cols_once_x(red, inner);
+      const int64_t groups = (inner + X - 1) / X;
+      if (red > 0 && red <= cols_once_run * (COLS_ONCE / X) && outer <= 65535 && outer * groups <= (X == 8 ? 64 : 128)) {
+        const dim3 g1((unsigned)groups, (unsigned)outer), b1(COLS_ONCE);
+        if (X == 8) hipLaunchKernelGGL((reduce_cols_once_kernel<R, CT, IDT, 8>), g1, b1, 0, ctx->stream, in, out, odt, (int)red, inner);
+        else if (X == 16) hipLaunchKernelGGL((reduce_cols_once_kernel<R, CT, IDT, 16>), g1, b1, 0, ctx->stream, in, out, odt, (int)red, inner);
+        else if (X == 32) hipLaunchKernelGGL((reduce_cols_once_kernel<R, CT, IDT, 32>), g1, b1, 0, ctx->stream, in, out, odt, (int)red, inner);
+        else hipLaunchKernelGGL((reduce_cols_once_kernel<R, CT, IDT, 64>), g1, b1, 0, ctx->stream, in, out, odt, (int)red, inner);
+        HIPNX_HIP(hipGetLastError());
+        return HIPNX_OK;
+      }
+    }
     const bool vec = inner % E == 0;
     const bool unal = !vec && inner >= 8 * E && IDT >= 0;  // long rows off the vector grid (compiled for the common element types)
     const int64_t lanes = outer * (unal ? (inner + E - 1) / E : inner / (vec ? E : 1));

@@ -390,3 +390,30 @@ def test_integer_ends_in_long_slabs_of_short_rows(red, inner, ty, op, hip, oracl
         x[red - 1, ::3] = info.max
     hx, ox = both(x, ty, hip, oracle)
     assert_bits_equal(getattr(Nx, op)(hx, axes=[0]), getattr(Nx, op)(ox, axes=[0]), f"{op} {ty} [{red}, {inner}]")
+
+
+# runs of the reduced axis of a lane: none, one row, whole and partial eights, the last run short; columns on either side of a
+# work-group's 8, 16, 32 and 64; the longest axis it takes and one more
+@pytest.mark.parametrize("ty", ["f32", "bf16", "f16"])
+@pytest.mark.parametrize("outer,red,inner", [(1, 2, 3), (3, 33, 5), (1, 48, 8), (2, 129, 9), (1, 1025, 33), (1, 1024, 32), (1, 4095, 8), (1, 4096, 8), (5, 31, 64),
+                                             (1, 512, 65), (1, 513, 64), (1, 2049, 16), (1, 300, 2048), (7, 1, 100), (1, 4096, 520)])
+def test_few_columns_in_one_launch(outer, red, inner, ty, hip, oracle):
+    """On whole numbers: every sum and position is the oracle's, of both zeros the one it meets first (the kernel for long narrow
+    slabs, from 4096 rows on, meets its rows in another order)."""
+    rng = np.random.default_rng(seed_of(outer, red, inner, ty))
+    v = rng.integers(-2, 3, size=(outer, red, inner)).astype(np.float32)
+    if red < 4096:
+        v[:, :, ::3] = np.where(rng.random(v[:, :, ::3].shape) < 0.5, 0.0, -0.0)
+    arr = (v.view(np.uint32) >> 16).astype(np.uint16) if ty == "bf16" else v.astype(np.float16 if ty == "f16" else np.float32)
+    h, o = from_numpy(arr, ty, hip), from_numpy(arr, ty, oracle)
+    for op in ("sum", "reduce_max", "reduce_min"):
+        assert_bits_equal(getattr(Nx, op)(h, axes=[1]), getattr(Nx, op)(o, axes=[1]), op)
+    for op in ("argmax", "argmin"):
+        for tie in ("low", "high"):
+            assert_bits_equal(getattr(Nx, op)(h, axis=1, tie_break=tie), getattr(Nx, op)(o, axis=1, tie_break=tie), op)
+    assert_bits_equal(Nx.all(h, axes=[1]), Nx.all(o, axes=[1]), "all")
+    v[0, red // 2, 0] = np.nan
+    arr = (v.view(np.uint32) >> 16).astype(np.uint16) if ty == "bf16" else v.astype(np.float16 if ty == "f16" else np.float32)
+    h, o = from_numpy(arr, ty, hip), from_numpy(arr, ty, oracle)
+    for op in ("sum", "reduce_max"):
+        assert_bits_equal(getattr(Nx, op)(h, axes=[1]), getattr(Nx, op)(o, axes=[1]), f"{op}, NaN")
