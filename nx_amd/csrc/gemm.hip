@@ -70,9 +70,8 @@ dot_generic_kernel(const void *__restrict__ l, const void *__restrict__ r, void 
   const int64_t m0 = (int64_t)blockIdx.x * T, n0 = (int64_t)(blockIdx.y / nseg) * T, m = m0 + ty, n = n0 + tx;
   const int64_t lbase = b * M * K, rbase = b * N * K;
   const int64_t k_begin = seg * seg_len, k_end = k_begin + seg_len < K ? k_begin + seg_len : K;
-  CT acc = 0;
-  for (int64_t k0 = k_begin; k0 < k_end; k0 += TK) {
-    CT a[PER], c[PER];
+  CT acc = 0, a[PER], c[PER];
+  auto request = [&](int64_t k0) {
 #pragma unroll
     for (int q = 0; q < PER; q++) {
       // consecutive lanes along the operand's contiguous axis
@@ -82,6 +81,9 @@ dot_generic_kernel(const void *__restrict__ l, const void *__restrict__ r, void 
       a[q] = (mm < M && ka < k_end) ? load_one<CT>(l, ldt, lbase + (lk ? mm * K + ka : ka * M + mm)) : (CT)0;
       c[q] = (nn < N && kb < k_end) ? load_one<CT>(r, rdt, rbase + (rk ? nn * K + kb : kb * N + nn)) : (CT)0;
     }
+  };
+  request(k_begin);
+  for (int64_t k0 = k_begin; k0 < k_end; k0 += TK) {
 #pragma unroll
     for (int q = 0; q < PER; q++) {
       const int e = tid + q * 256;
@@ -90,11 +92,14 @@ dot_generic_kernel(const void *__restrict__ l, const void *__restrict__ r, void 
       sB[bn][bk] = c[q];
     }
     __syncthreads();
+    if (k0 + TK < k_end) request(k0 + TK);  // under this slab's arithmetic
     const int steps = k_end - k0 < TK ? (int)(k_end - k0) : TK;
     for (int k16 = 0; k16 < steps; k16 += 16) {  // (behind K both are zero)
 #pragma unroll
       for (int kk = k16; kk < k16 + 16; kk++) {
-        if constexpr (std::is_same<CT, double>::value) acc = sA[ty][kk] * sB[tx][kk] + acc;
+        // (products of two f32 numbers or narrower ones are exact in f64: one rounding either way)
+        if constexpr (std::is_same<CT, double>::value && LDT >= 0 && LDT != HIPNX_F64 && RDT >= 0 && RDT != HIPNX_F64) acc = __builtin_fma(sA[ty][kk], sB[tx][kk], acc);
+        else if constexpr (std::is_same<CT, double>::value) acc = sA[ty][kk] * sB[tx][kk] + acc;
         else acc = (int64_t)((uint64_t)sA[ty][kk] * (uint64_t)sB[tx][kk] + (uint64_t)acc);
       }
     }
@@ -469,8 +474,8 @@ static int dot_impl(hipnx_ctx *ctx, int l_dt, int r_dt, int out_dt, int64_t batc
         return HIPNX_OK;
       }
       // Few outputs over a long K (the weight gradient of a layer with a handful of classes: [6377, 80]^T . [6377, 3] is five
-      // tiles): K is cut until every CU has two work-groups, where that saves more slabs than the second pass costs (eight
-      // and more: 1 us each against 5).  Not where a sum's order shows: an f64 operand or result adds over k in order.
+      // tiles): K is cut until every CU has two work-groups, where that saves more slabs than the second pass costs (four
+      // and more: 1 to 3 us each against 5).  Not where a sum's order shows: an f64 operand or result adds over k in order.
       const bool any_f64 = l_dt == HIPNX_F64 || r_dt == HIPNX_F64 || out_dt == HIPNX_F64;
       const int64_t tiles = (int64_t)grid.x * grid.y * batch, slabs = (K + 63) / 64;
       int64_t nseg = any_f64 ? 1 : std::min<int64_t>(2 * (int64_t)ctx->num_cus / tiles, slabs / 2);
@@ -479,7 +484,7 @@ static int dot_impl(hipnx_ctx *ctx, int l_dt, int r_dt, int out_dt, int64_t batc
         seg_len = (slabs + nseg - 1) / nseg * 64;
         nseg = (K + seg_len - 1) / seg_len;
       }
-      if (nseg < 2 || slabs - seg_len / 64 < 8 || grid.y * nseg > 65535) nseg = 1, seg_len = K;
+      if (nseg < 2 || slabs - seg_len / 64 < 4 || grid.y * nseg > 65535) nseg = 1, seg_len = K;
       void *ws = nullptr;
       size_t ws_cap = 0;
       if (nseg > 1 && pool_alloc(ctx, (size_t)(batch * M * N * nseg) * 8, &ws, &ws_cap) != HIPNX_OK) nseg = 1, seg_len = K;
