@@ -594,6 +594,8 @@ static int dot_impl(hipnx_ctx *ctx, int l_dt, int r_dt, int out_dt, int64_t batc
       else if (l_dt == HIPNX_S8 && big_ok && t256 * 2 >= ctx->num_cus)
         cfg = GEMM_CFG_256;  // int8 has no half-width tile: full tiles from half of the CUs on (3072^3: 46 us against 57 us)
       else cfg = GEMM_CFG_128;
+      // up to 32 rows against 2-byte weights stored K-outer: a stream of the weights through tiles of 32 rows
+      if (two_byte && l_kin && !r_kin && M <= 32 && N >= 128 && batch == 1) cfg = GEMM_CFG_32x128;
       // many rows against at most 32 columns (a layer with a few outputs): a 128-column tile would be three
       // quarters empty or more, and its MFMA work is what bounds f32
       if (N <= 32 && M > 64 && cfg == GEMM_CFG_128) cfg = GEMM_CFG_128x32;
@@ -649,6 +651,12 @@ static int dot_impl(hipnx_ctx *ctx, int l_dt, int r_dt, int out_dt, int64_t batc
             }
           }
         }
+      } else if (cfg == GEMM_CFG_32x128) {
+        // (us per call, 128-row tiles in one or two splits / these: bf16 8 x 11008 x 4096 23.8 / 19.5, 1 x 4096 x 4096 12.1 / 9.2, 8 x 1128 x 4992
+        // 12.4 / 8.9, 32 x 11008 x 4096 23.2 / 21.0)  A work-group takes about 0.35 us a slab; K is cut until every CU has two, four slabs or more each, where that saves
+        // more than the second pass takes
+        for (int cand = 16; cand >= 2; cand--)
+          if (t128 * cand <= 2 * (int64_t)ctx->num_cus && nslab / cand >= 4 && reaches(cand) && 0.35 * (double)(nslab - per_split(cand)) > 5.0) { splits = cand; break; }
       } else if (splittable && t128 * 2 <= ctx->num_cus && nslab >= (t128 * 4 <= ctx->num_cus ? 32 : 64))
         // (the second pass and the partial results cost about 10 us: worth it from K = 32 slabs on -- 64 where
         // the grid already covers more than a quarter of the CUs -- with at least 8 slabs left per split and no

@@ -14,6 +14,7 @@ enum {
   GEMM_CFG_128 = 1,  // 128 x 128: mid-size and batched problems; 4 waves (2 x 2, each 64 x 64), or two such groups sharing K
   GEMM_CFG_64x32 = 2, // 64 x 32, 2 waves: few rows against a long weight matrix (HBM streaming)
   GEMM_CFG_64x128 = 4, // 64 x 128, 4 waves (2 x 2, each 32 x 64): f32 and f64, wherever the cost model of gemm.hip has it cheapest
+  GEMM_CFG_32x128 = 6, // 32 x 128, 4 waves (1 x 4, each 32 x 32): few rows against 2-byte weights stored K-outer (HBM streaming)
   GEMM_CFG_128x32 = 5  // 128 x 32, 4 waves (4 x 1, each 32 x 32): many rows against up to 32 columns (a layer with a few outputs)
 };
 
@@ -131,6 +132,10 @@ static int launch_cfg(const hipnx_ctx *ctx, int cfg, const GemmArgs &a, int64_t 
     case GEMM_CFG_128x32:
       if constexpr (LK && RK) return launch_one<DT, 4, 1, 1, 1, LK, RK, 4>(ctx, a, batch);
       else return launch_one<DT, 4, 1, 1, 1, LK, RK>(ctx, a, batch);
+    case GEMM_CFG_32x128:
+      // four stages of 20 KiB: two work-groups and 96 KiB of weights in flight to a CU
+      if constexpr (LK && !RK && (DT == HIPNX_BF16 || DT == HIPNX_F16)) return launch_one<DT, 1, 4, 1, 1, LK, RK, 4>(ctx, a, batch);
+      return launch_one<DT, 2, 2, 2, 2, LK, RK>(ctx, a, batch);
     case GEMM_CFG_64x128:
       if constexpr (DT == HIPNX_F32) return launch_one<DT, 2, 2, 1, 2, LK, RK>(ctx, a, batch);
       return launch_one<DT, 2, 2, 2, 2, LK, RK>(ctx, a, batch);

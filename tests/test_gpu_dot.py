@@ -787,3 +787,18 @@ def test_few_outputs_over_a_long_k_are_cut_into_segments(lt, rt, M, N, K, layout
     a, b = values(oa) if layout[0] == "n" else values(oa).T, values(ob) if layout[1] == "n" else values(ob).T
     apart = np.abs(values(got) - values(want))
     assert (apart <= ULP[got.type] * np.abs(values(want)) + 2 * K * 2.0 ** -53 * (np.abs(a) @ np.abs(b))).all(), f"{lt} {layout}: {apart.max()}"
+
+
+@pytest.mark.parametrize("ty", ["bf16", "f16"])
+@pytest.mark.parametrize("M,N,K", [(1, 256, 64), (8, 1000, 4096), (32, 136, 520), (17, 2048, 1096), (5, 11008, 256), (32, 128, 8200), (31, 392, 72)])
+def test_few_rows_against_k_outer_weights_on_tiles_of_32(M, N, K, ty, hip):
+    """Whole and partial slabs of K, K cut and whole, the edges of 32 rows and 128 columns: whole numbers, exact in any order."""
+    rng = np.random.default_rng(seed_of(M, N, K, ty))
+    a, b = rng.integers(-2, 3, size=(M, K)).astype(np.float32), rng.integers(-2, 3, size=(K, N)).astype(np.float32)
+
+    def put(v):
+        return from_numpy((v.view(np.uint32) >> 16).astype(np.uint16) if ty == "bf16" else v.astype(np.float16), ty, hip)
+    exact = a.astype(np.float64) @ b
+    got = values(Nx.dot(put(a), [1], put(b), [0]))
+    want = (exact.astype(np.float32).view(np.uint32) & np.uint32(0xFFFF0000)).view(np.float32) if ty == "bf16" else exact.astype(np.float16)
+    np.testing.assert_array_equal(got, want.astype(np.float64))
