@@ -280,6 +280,12 @@ int hipnx_dot_scaled(hipnx_ctx *ctx, int l_dt, int r_dt, int64_t batch, int64_t 
                      int l_layout, int r_layout, const hipnx_buf *l, const hipnx_buf *r, int scale_mode,
                      const hipnx_buf *scale, hipnx_buf *out);
 
+/* The same for a K that need not be whole slabs: the partial slab is walked in place, rows that are not whole 16-byte pieces are
+ * copied first, as hipnx_dot does (from 16 M multiply-adds on; HIPNX_EUNSUPPORTED below). */
+int hipnx_dot_scaled_any_k(hipnx_ctx *ctx, int l_dt, int r_dt, int64_t batch, int64_t M, int64_t N, int64_t K,
+                           int l_layout, int r_layout, const hipnx_buf *l, const hipnx_buf *r, int scale_mode,
+                           const hipnx_buf *scale, hipnx_buf *out);
+
 /* ---- data movement -------------------------------------------------------------------------
  * replaces: transpose/3 (nx/lib/nx/backend.ex:73; oracle binary_backend.ex:280-319) */
 int hipnx_transpose(hipnx_ctx *ctx, int elem_bytes, int rank, const int64_t *in_dims,

@@ -100,6 +100,8 @@ PROTOTYPES = {
                           _i64p, _i64p, _buf_p, _buf_p, _buf_p],
     "hipnx_dot_scaled": [_ctx_p, C.c_int, C.c_int, C.c_int64, C.c_int64, C.c_int64, C.c_int64, C.c_int, C.c_int,
                          _buf_p, _buf_p, C.c_int, _buf_p, _buf_p],
+    "hipnx_dot_scaled_any_k": [_ctx_p, C.c_int, C.c_int, C.c_int64, C.c_int64, C.c_int64, C.c_int64, C.c_int, C.c_int,
+                         _buf_p, _buf_p, C.c_int, _buf_p, _buf_p],
     "hipnx_transpose": [_ctx_p, C.c_int, C.c_int, _i64p, _intp, _buf_p, _buf_p],
     "hipnx_broadcast": [_ctx_p, C.c_int, C.c_int, _i64p, _i64p, _buf_p, _buf_p],
     "hipnx_gather": [_ctx_p, C.c_int, C.c_int, _i64p, C.c_int, C.c_int64, C.c_int, C.c_int, _buf_p, _buf_p, _buf_p],

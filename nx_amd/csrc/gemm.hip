@@ -329,7 +329,7 @@ struct DotView {
 // and nothing has been launched)
 static int dot_impl(hipnx_ctx *ctx, int l_dt, int r_dt, int out_dt, int64_t batch, int64_t M, int64_t N,
                     int64_t K, int l_layout, int r_layout, const hipnx_buf *l, const hipnx_buf *r,
-                    hipnx_buf *out, int scale_mode, const hipnx_buf *scale, const DotView *view = nullptr) {
+                    hipnx_buf *out, int scale_mode, const hipnx_buf *scale, const DotView *view = nullptr, bool any_k = false) {
   if (view && batch > 65535) return set_error(HIPNX_EUNSUPPORTED, "dot_strided: more than 65535 batch items");
   // More batch items than a grid's second dimension holds (100000 small matrices): runs of 65535 items, each over
   // borrowed handles on its part of the three buffers.
@@ -348,7 +348,7 @@ static int dot_impl(hipnx_ctx *ctx, int l_dt, int r_dt, int out_dt, int64_t batc
       int st = hipnx_buf_wrap(ctx, (char *)l->ptr + b0 * lb, nb * lb > 0 ? nb * lb : 1, &lw);
       if (!st) st = hipnx_buf_wrap(ctx, (char *)r->ptr + b0 * rb, nb * rb > 0 ? nb * rb : 1, &rw);
       if (!st) st = hipnx_buf_wrap(ctx, (char *)out->ptr + b0 * ob, nb * ob, &ow);
-      if (!st) st = dot_impl(ctx, l_dt, r_dt, out_dt, nb, M, N, K, l_layout, r_layout, lw, rw, ow, scale_mode, scale);
+      if (!st) st = dot_impl(ctx, l_dt, r_dt, out_dt, nb, M, N, K, l_layout, r_layout, lw, rw, ow, scale_mode, scale, nullptr, any_k);
       if (lw) hipnx_buf_destroy(lw);
       if (rw) hipnx_buf_destroy(rw);
       if (ow) hipnx_buf_destroy(ow);
@@ -393,7 +393,7 @@ static int dot_impl(hipnx_ctx *ctx, int l_dt, int r_dt, int out_dt, int64_t batc
       if (l_pad || r_pad || l_dt != HIPNX_S8) mfma = (double)M * (double)N * (double)K * (double)batch >= 16777216.0;
     }
     if (scaled) {
-      if (!(int8_pair && mfma && row_bytes % SLAB == 0)) return set_error(HIPNX_EUNSUPPORTED, "dot_scaled: s8 x s8 with K a multiple of 128 and at most 65536, M * N >= 256");
+      if (!(int8_pair && mfma && (any_k || row_bytes % SLAB == 0))) return set_error(HIPNX_EUNSUPPORTED, "dot_scaled: s8 x s8 with K a multiple of 128 and at most 65536, M * N >= 256");
       if (scale_mode == HIPNX_SCALE_PER_ROW && batch != 1) return set_error(HIPNX_EUNSUPPORTED, "dot_scaled: a scale per row with more than one batch item");
       const int64_t need = scale_mode == HIPNX_SCALE_PER_COLUMN ? N : scale_mode == HIPNX_SCALE_PER_ROW ? M : 1;
       if (int st = check_buf(ctx, scale, (uint64_t)need * 4, "dot_scaled scale")) return st;
@@ -748,4 +748,12 @@ extern "C" int hipnx_dot_scaled(hipnx_ctx *ctx, int l_dt, int r_dt, int64_t batc
   if (scale_mode != HIPNX_SCALE_PER_COLUMN && scale_mode != HIPNX_SCALE_PER_ROW && scale_mode != HIPNX_SCALE_ONE)
     return set_error(HIPNX_EINVAL, "dot_scaled: scale mode %d", scale_mode);
   return dot_impl(ctx, l_dt, r_dt, HIPNX_F32, batch, M, N, K, l_layout, r_layout, l, r, out, scale_mode, scale);
+}
+
+extern "C" int hipnx_dot_scaled_any_k(hipnx_ctx *ctx, int l_dt, int r_dt, int64_t batch, int64_t M, int64_t N, int64_t K,
+                                      int l_layout, int r_layout, const hipnx_buf *l, const hipnx_buf *r, int scale_mode,
+                                      const hipnx_buf *scale, hipnx_buf *out) {
+  if (scale_mode != HIPNX_SCALE_PER_COLUMN && scale_mode != HIPNX_SCALE_PER_ROW && scale_mode != HIPNX_SCALE_ONE)
+    return set_error(HIPNX_EINVAL, "dot_scaled_any_k: scale mode %d", scale_mode);
+  return dot_impl(ctx, l_dt, r_dt, HIPNX_F32, batch, M, N, K, l_layout, r_layout, l, r, out, scale_mode, scale, nullptr, true);
 }

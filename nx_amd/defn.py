@@ -1589,7 +1589,7 @@ class _Run:
             one_call = getattr(mod, "dot_scaled", None)
             if one_call is not None:
                 try:
-                    return one_call(out, lv, c1, b1, rv, c2, b2, sv, mode)
+                    return one_call(out, lv, c1, b1, rv, c2, b2, sv, mode, any_k=True)
                 except Exception as err:  # a shape the kernel leaves to the separate callbacks
                     if getattr(err, "status", None) != _EUNSUPPORTED:
                         raise

@@ -20,7 +20,7 @@ from ._lib import native
 
 # entry points whose effect is their result buffer's content, a function of their arguments
 _RECORDED = frozenset("hipnx_" + n for n in (
-    "binary", "unary", "as_type", "reduce", "argreduce", "dot", "dot_strided", "dot_scaled", "transpose", "broadcast", "gather", "select", "clip",
+    "binary", "unary", "as_type", "reduce", "argreduce", "dot", "dot_strided", "dot_scaled", "dot_scaled_any_k", "transpose", "broadcast", "gather", "select", "clip",
     "concat", "strided_copy", "iota", "eye", "narrow_int", "threefry2x32", "threefry_key", "fused_elementwise", "fused_words", "fused_scores"))
 _lock = threading.Lock()
 

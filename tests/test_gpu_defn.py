@@ -689,6 +689,29 @@ def test_scaled_dot_with_batches_and_with_the_weights_k_outer(hip):
     assert_bits_equal(planned(x, w, sc), defn.compile(fun, x, w, sc)(x, w, sc), "batched")
 
 
+# partial slabs in place, rows copied to whole pieces, transposed first, both; fewer than 16 M multiply-adds: three calls
+@pytest.mark.parametrize("M,N,K,contract", [(64, 512, 607, 1), (8, 4098, 607, 0), (33, 2000, 272, 0), (512, 300, 1008, 1), (128, 1040, 129, 0), (64, 640, 494, 1), (16, 32, 100, 1)])
+@pytest.mark.parametrize("scales", ["column", "row", "one"])
+def test_scaled_dot_of_any_k(M, N, K, contract, scales, hip):
+    rng = np.random.default_rng(seed_of(M, N, K, contract, scales))
+    x, w = rand_s8(rng, (M, K), hip), rand_s8(rng, (N, K) if contract else (K, N), hip)
+    sc = from_numpy(rng.uniform(1e-3, 1e-2, size={"column": (N,), "row": (M, 1), "one": (1,)}[scales]).astype(np.float32), "f32", hip)
+
+    def fun(xq, wq, s):
+        return Nx.multiply(Nx.as_type(Nx.dot(xq, [1], wq, [contract], out_type="s32"), "f32"), s)
+    planned = defn.compile(fun, x, w, sc, fuse="compiled")
+    assert planned.roots[0].data.op == "dot_scaled"
+    calls = []
+    original = hip.as_type.__func__
+    hip.as_type = classmethod(lambda cls, *a: (calls.append(1), original(cls, *a))[1])
+    try:
+        got = planned(x, w, sc)
+    finally:
+        hip.as_type = classmethod(original)
+    assert bool(calls) == (M * N * K < 1 << 24 and (K % 16 != 0)), calls
+    assert_bits_equal(got, defn.compile(fun, x, w, sc)(x, w, sc), f"{M} x {N} x {K}")
+
+
 def test_scaled_dot_entry_point_refuses_what_it_does_not_take(hip):
     from nx_amd._lib import EUNSUPPORTED, SCALE_PER_COLUMN, HipNxError
     rng = np.random.default_rng(5)
