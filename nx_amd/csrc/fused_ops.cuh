@@ -273,7 +273,7 @@ __device__ __forceinline__ void fetch_static(KernArgs a, const Saved &S, const R
 template <typename P, int PC>
 constexpr bool divides_exponentials() {
   constexpr auto is_exp = [](int i) { return P::kind[i] == HIPNX_FUSED_UNARY && P::op[i] == HIPNX_EXP; };
-  if (PC < 1 || P::nv > 2 || (P::nv == 0 && P::form != ROW_LANE)) return false;
+  if (PC < 1 || P::nv > (P::scores >= 0 ? 4 : 2) || (P::nv == 0 && P::form != ROW_LANE)) return false;
   if (is_exp(PC - 1)) return true;
   if (P::kind[PC - 1] != HIPNX_FUSED_SET || P::src[PC - 1] != HIPNX_FUSED_SRC_CARRY) return false;
   for (int i = PC - 1; i > 0; i--)  // what the stage before left: the value its reduction was taken over

@@ -90,6 +90,10 @@ static void share_row(const FusedArgs &a, bool walk, Keeps &k) {
   k.tpr = class_lanes(a);
   // (a wave per row of 64 had an eighth of its lanes at work)
   if (a.cols <= 256) k.tpr = a.cols <= 16 ? 1 : a.cols <= 64 ? 8 : a.cols <= 128 ? 16 : 32;
+  // (a contraction's rows are in LDS: with up to four vectors a lane, two or four rows share a wave's reductions, which are a fifth of
+  // the instructions when a row of 512 takes it alone; the order of a sum is this kernel's own.
+  // bf16 4 x 8 x 512 x 512: 20.9 -> 19.3 us a pass.  One row alone -- a step of decoding -- is faster with a wave: 784 columns 7.7, 9.9 so)
+  if (a.scores >= 0 && a.cols > 256 && a.scores_rows >= 8) k.tpr = a.cols <= 512 ? 16 : a.cols <= 1024 ? 32 : WAVE;
   k.form = a.cols <= 16 ? ROW_LANE : a.cols % FE == 0 ? ROW_WHOLE : a.cols <= 256 ? ROW_GROUP : ROW_RAGGED;
   if (k.form == ROW_LANE) k.trips = (int)(a.cols / FE), k.tail = (int)(a.cols % FE);
 }
