@@ -5,7 +5,7 @@
  * conversions of the call, of the allocation in front of it and of the release behind its operands.  A traced function
  * paid 5-7 us more per node to its evaluator.  Here a callback's arguments are laid out once per signature (Call), a traced
  * function's calls are recorded once and issued again from C (Replay); the library is called through the same entry points
- * with the same arguments.  (add, multiply, exp, sum of 1024 x 1024: see DESIGN, 6.1, for what a pass took before and after.)
+ * with the same arguments.  add, multiply, exp, sum of 1024 x 1024, one callback at a time: 30.6 -> 18.6 us a pass.
  *
  * Every entry point of include/hipnx.h takes integers and pointers only, at most MAX_ARGS of them: they are called through
  * one function type of 64-bit arguments (an int argument is the low half of its register or stack slot). */

@@ -9,7 +9,8 @@
 //       contraction is large enough to pay for it (16 M multiply-adds).
 //   everything else (f64 whose K is not whole slabs, wide integers, mixed operand types, fewer than 256 outputs, and below
 //     16 M multiply-adds a float K that is not whole 16-byte pieces, in every layout): dot_generic_kernel,
-//     a plain tiled kernel accumulating in f64 or wrapping 64-bit integers.
+//     a plain tiled kernel accumulating in f64 or wrapping 64-bit integers, K cut into segments where few outputs would leave
+//     the chip idle; dot_blocked_kernel for many outputs, dot_reduce_kernel for a handful, dot_small_batched_kernel for many small matrices.
 //
 // Algorithmic work: 2*B*M*N*K flop; minimum traffic bytes(l) + bytes(r) + bytes(out).
 #include <type_traits>
@@ -626,16 +627,19 @@ static int dot_impl(hipnx_ctx *ctx, int l_dt, int r_dt, int out_dt, int64_t batc
         //   `resident` of them (as the LDS holds) share a CU and take `shared` us per slab and work-group together,
         //   near what the MFMAs take: a split that puts two or three work-groups on a CU pays for its second pass
         //   (784 x 512 x 4096, 52 tiles: 4 splits 58 us, 8 splits 50; 1000 x 700 x 1500, 96 tiles: 2 splits 45 us,
-        //   8 splits 35; 300 x 1000 x 900, 40 tiles: 64 x 32 tiles 29 us, 6 splits of 64 x 128 18.5; 2048^3: 128 x 128
+        //   8 splits 33; 300 x 1000 x 900, 40 tiles: 64 x 32 tiles 29 us, 6 splits of 64 x 128 16; 2048^3: 128 x 128
         //   174 us, 64 x 128, two to a CU, 152).  Fitted to f32 contractions of 100 to 8192 a side in three layouts,
         //   within a tenth.  (Both operands K-inner: 128 x 128 tiles on the two-group kernel, which holds its CU alone,
         //   and six stages of 64 x 32 tiles, two to a CU.)
-        struct Tile { int cfg, rows, cols, resident; double alone, shared; };
-        const bool kk = l_kin && r_kin, f64 = l_dt == HIPNX_F64;
+        //   An operand that is not K-inner: the figures of eight waves to a work-group (two_waves_a_simd, gemm_launch.cuh); two and
+        //   three work-groups of 64 x 32 that start together share a CU no better than `pair` (1024^3, 512 of them: 46 us; two splits
+        //   of 64 x 128 31; 6000 x 100 x 500 24.8 / 17.9; 4096 x 512 x 784 40.7 -> 35.3; 2048^3 152 -> 144, both K-outer 160 -> 150).
+        struct Tile { int cfg, rows, cols, resident; double alone, pair, shared; };
+        const bool kk = l_kin && r_kin, oo = !l_kin && !r_kin, f64 = l_dt == HIPNX_F64;
         const Tile tiles[3] = {
-            {GEMM_CFG_128, 128, 128, f64 || kk ? 1 : 2, f64 ? 2.6 : kk ? 2.05 : 2.5, f64 ? 2.6 : kk ? 2.05 : 2.15},
-            {GEMM_CFG_64x128, 64, 128, f64 ? 1 : 3, f64 ? 1.3 : 1.44, f64 ? 1.3 : 1.15},
-            {GEMM_CFG_64x32, 64, 32, f64 ? 1 : kk ? 2 : 6, f64 ? 0.55 : kk ? 0.75 : 0.79, f64 ? 0.55 : kk ? 0.65 : 0.36}};
+            {GEMM_CFG_128, 128, 128, f64 || kk ? 1 : 2, f64 ? 2.6 : kk ? 2.05 : 2.25, 0, f64 ? 2.6 : kk ? 2.05 : 2.15},
+            {GEMM_CFG_64x128, 64, 128, f64 ? 1 : 3, f64 ? 1.3 : kk ? 1.44 : 1.25, 0, f64 ? 1.3 : kk || oo ? 1.15 : 1.12},
+            {GEMM_CFG_64x32, 64, 32, f64 ? 1 : kk ? 2 : 6, f64 ? 0.55 : kk ? 0.75 : 0.9, f64 || kk ? 0 : 1.38, f64 ? 0.55 : kk ? 0.65 : 0.36}};
         if (cfg == GEMM_CFG_128) {
           const int64_t cus = ctx->num_cus;
           double best = 0;
@@ -644,7 +648,7 @@ static int dot_impl(hipnx_ctx *ctx, int l_dt, int r_dt, int out_dt, int64_t batc
             for (int cand : {1, 2, 3, 4, 6, 8, 12, 16, 24, 32, 48, 64}) {
               if (cand > 1 && (!splittable || t.cfg == GEMM_CFG_64x32 || count * cand > t.resident * cus || nslab / cand < 2 || !reaches(cand))) continue;
               const int64_t per_cu = (count * cand + cus - 1) / cus, last = per_cu % t.resident;
-              double us = (double)per_split(cand) * ((double)(per_cu - last) * t.shared + (last ? std::max(t.alone, (double)last * t.shared) : 0.0));
+              double us = (double)per_split(cand) * ((double)(per_cu - last) * t.shared + (last ? std::max(last > 1 && last == per_cu ? std::max(t.alone, t.pair) : t.alone, (double)last * t.shared) : 0.0));
               // a split's second launch, then the partial results written and read once (mostly from cache: ~8 MB per us)
               if (cand > 1) us += 5.0 + 2.0 * (double)cand * (double)(M * N) * 4.0 / 8.0e6;
               if (best == 0 || us < best) { best = us; cfg = t.cfg; splits = cand; }

@@ -1149,7 +1149,7 @@ def _cluster_rows(roots: List[Tensor]) -> int:
     last axis -- of a fused group's value or of a tensor as it is -- followed by a chain of
     element-wise nodes on the one value per row.  The node that is rewritten is an element-wise fused
     group over the full shape (a softmax, a layer normalisation), or itself such a per-row value
-    (a log-sum-exp).  A row is walked by a wave, or by a block when it has more than 4096 elements: as the
+    (a log-sum-exp).  A row is walked by a lane, part of a wave, a wave or -- above 4096 elements -- a block: as the
     separate reduction walks it, whose order the stages keep."""
     order, readers, seen = [], {}, set()
 

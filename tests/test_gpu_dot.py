@@ -802,3 +802,18 @@ def test_few_rows_against_k_outer_weights_on_tiles_of_32(M, N, K, ty, hip):
     got = values(Nx.dot(put(a), [1], put(b), [0]))
     want = (exact.astype(np.float32).view(np.uint32) & np.uint32(0xFFFF0000)).view(np.float32) if ty == "bf16" else exact.astype(np.float16)
     np.testing.assert_array_equal(got, want.astype(np.float64))
+
+
+# f32 with an operand that is not K-inner: tiles of 64 x 128 and 128 x 128 on eight waves up to one or two work-groups to a CU and
+# on four beyond, one slab, a partial slab, K cut
+@pytest.mark.parametrize("layout", ["nn", "tn", "tt"])
+@pytest.mark.parametrize("M,N,K", [(64, 256, 32), (68, 132, 36), (60, 384, 68), (1000, 132, 64), (2044, 1028, 40), (4100, 1024, 36), (4096, 2052, 100),
+                                   (2048, 2048, 96), (300, 1000, 900), (1024, 1024, 260), (132, 260, 4100)])
+def test_f32_tiles_on_four_and_eight_waves(M, N, K, layout, hip):
+    """Whole numbers whose sums are exact in f32 in any order, so every output is the same number on any kernel."""
+    rng = np.random.default_rng(seed_of(M, N, K, layout))
+    a, b = rng.integers(-3, 4, size=(M, K)).astype(np.float32), rng.integers(-3, 4, size=(K, N)).astype(np.float32)
+    l, lc = (a, [1]) if layout[0] == "n" else (np.ascontiguousarray(a.T), [0])
+    r, rc = (b, [0]) if layout[1] == "n" else (np.ascontiguousarray(b.T), [1])
+    got = values(Nx.dot(from_numpy(l, "f32", hip), lc, from_numpy(r, "f32", hip), rc))
+    np.testing.assert_array_equal(got, a.astype(np.float64) @ b.astype(np.float64))
