@@ -247,8 +247,9 @@ int hipnx_argreduce(hipnx_ctx *ctx, int op, int tie, int in_dt, int out_dt, int6
  * out_dt (f32 accumulation for f16/bf16/f32 operands, exact s32 for s8, f64 accumulation on the matrix cores for
  * f64 operands whose K is a multiple of 16 and whose result has 256 elements or more, then one encode; other f64
  * shapes, wider integers, mixed operand types, results of fewer than 256 elements and, below 16 M multiply-adds, float
- * operands whose K is not whole 16-byte pieces accumulate in f64 / wrapping 64-bit integers over k in order, as do
- * a handful of outputs over a long K -- the dot of two vectors -- whose segments of K are summed in f64).
+ * operands whose K is not whole 16-byte pieces accumulate in f64 / wrapping 64-bit integers: over k in order where an operand
+ * or the result is f64; otherwise K may be cut into segments, each over k in order, that are added in f64 in their order.
+ * A handful of outputs over a long K -- the dot of two vectors -- are such segments of interleaved sums for every type).
  * out_dt may be HIPNX_BF16_RNE (bf16 rounded to nearest even).  Any batch count is taken (beyond 65535 items in
  * several launches).  The call may take workspace from the context's pool and return it before it ends: a re-laid
  * operand whose K-outer rows are not whole 16-byte blocks, a K-inner operand copied to rows of whole 16-byte pieces
@@ -406,7 +407,7 @@ enum { HIPNX_FUSED_FLAG_SWAP = 1, HIPNX_FUSED_FLAG_INT = 2, HIPNX_FUSED_FLAG_RES
 enum { HIPNX_FUSED_SRC_CONST = 0, HIPNX_FUSED_SRC_INPUT, HIPNX_FUSED_SRC_SAVED, HIPNX_FUSED_SRC_ROWSTAT,
        HIPNX_FUSED_SRC_CARRY };
 /* Stages over the same rows.  HIPNX_FUSED_ROW_REDUCE reduces the accumulator along the row (op =
- * HIPNX_RED_SUM / MAX / MIN, exactly as the reduction of the separate entry point would, the result stored
+ * HIPNX_RED_SUM / MAX / MIN, exactly as the reduction of the separate entry point would (rows of any length), the result stored
  * in type dt) and leaves that one value per row in the accumulator; the instructions that follow work on
  * it (a sum divided by the row length, an rsqrt of a variance, ...; operands are constants or earlier row
  * statistics) until HIPNX_FUSED_ROW_STAT ends the stage: the accumulator becomes row statistic number `arg`
@@ -460,7 +461,8 @@ int hipnx_fused_scores(hipnx_ctx *ctx, int n_instr, const hipnx_fused_instr *pro
  * cache plays for a whole function, here for one element-wise group.  Results are bit-identical in
  * both modes.  A program first met while the context is capturing runs interpreted in that capture (one that exists only
  * compiled is refused there: HIPNX_EUNSUPPORTED).  A program of stages that keeps an input or values of its rows in registers
- * is compiled once per number of 512-element steps (2048 above 4096 elements, up to 32768) in a row; a capture that meets
+ * is compiled once per number of 512-element steps (2048 above 4096 elements, up to 32768) in a row, and per way that rows
+ * which are not whole vectors of eight, or shorter than 512 elements, are divided among lanes; a capture that meets
  * it at another row length takes a kernel that reads the rows again, unless it reads HIPNX_FUSED_SRC_CARRY, provided the
  * program was compiled at some length on the same side of 4096.
  * A program's constants are part of what it is compiled for: one whose constant changes from call to
