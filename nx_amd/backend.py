@@ -1214,6 +1214,9 @@ class HipNxBackend:
             return cls._take_along(out, args[0], args[1], struct.axis)
         if isinstance(struct, BlockThreefry):
             return cls.threefry2x32(out, args[0])
+        recorder = _recorder[0]
+        if recorder is not None:
+            recorder.unrecordable()  # (the function may read tensors of its own, one of them also a parameter)
         return fun(struct, *args)
 
 

@@ -72,6 +72,9 @@ class _Recorder:
             return status
         return call
 
+    def unrecordable(self):
+        self.failed |= threading.get_ident() == self._thread
+
     def allocated(self, ref):
         if threading.get_ident() == self._thread:
             self._drain()
@@ -135,17 +138,38 @@ def record(evaluate, params):
     if not data or B._capturing or any(d.__class__ is not B.HipNxBackend or d.released or d.device != data[0].device for d in data) or not _lock.acquire(blocking=False):
         return evaluate(params), None
     try:
-        recorder = _Recorder(data[0].device, params)
+        private = [_private(p) for p in params]
+        recorder = _Recorder(data[0].device, private)
         real, L.lib, B._recorder[0] = L.lib, recorder, recorder
         native.log_freed(recorder.freed)
         try:
-            results = evaluate(params)
+            results = evaluate(private)
         finally:
             native.log_freed(None)
             L.lib, B._recorder[0] = real, None
     finally:
         _lock.release()
-    return results, None if recorder.failed else _finish(recorder, results)
+    replay = None if recorder.failed else _finish(recorder, results)
+    return [_callers(t, private, params) for t in results], replay
+
+
+def _private(p):
+    """The parameter in a buffer that the function cannot know as its own: a call's operands are told apart by their handles, and
+    a number given as an argument and the same number written in the function are one shared constant (of one element)."""
+    return B.HipNxBackend.backend_copy(p, B.HipNxBackend, {"device": p.data.device}) if p.data.ref.nbytes <= 8 else p
+
+
+def _callers(t, private, params):
+    """A result that is a parameter, or shares its buffer, over the caller's own."""
+    for q, p in zip(private, params):
+        if q is p:
+            continue
+        if t.data is q.data:
+            return t.with_(data=p.data)
+        if getattr(t.data, "ref", None) is q.data.ref:
+            p.data.ref.sharers += 1
+            return t.with_(data=B.HipNxBackend(p.data.ref, p.data.device))
+    return t
 
 
 def _finish(rec, results):

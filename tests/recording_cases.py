@@ -1,0 +1,69 @@
+"""Traced functions and callbacks issued natively (nx_amd/replay.py, csrc/calls.c), over the stand-in for the library: one case per
+function, run by name in a process of its own (test_recording.py)."""
+import sys
+
+import library_standin as standin
+
+standin.install()
+
+import numpy as np  # noqa: E402
+
+from nx_amd import HostBinary, HipNxBackend as Hip  # noqa: E402
+from nx_amd import backend as B  # noqa: E402
+from nx_amd import defn  # noqa: E402
+from nx_amd import nx as Nx  # noqa: E402
+from support import from_numpy  # noqa: E402
+
+Nx.default_backend(Hip)
+FUSE = (False, True, "compiled")
+
+
+def f32(*values):
+    return from_numpy(np.asarray(values, np.float32), "f32", Hip)
+
+
+def read(t):
+    return Nx.to_numpy(t).tolist()
+
+
+def a_number_given_as_an_argument_is_not_the_functions_own():
+    """The number that is an argument when the recording is made is also written in the function."""
+    for fuse in FUSE:
+        x = f32(1, 2, 4)
+        f = defn.compile(lambda x, s: (Nx.multiply(x, s), Nx.add(x, 0.5)), x, 0.5, fuse=fuse)
+        for _ in range(4):
+            f(x, 0.5)
+        assert f.replay is not None
+        scaled, shifted = f(x, 2.0)
+        assert read(scaled) == [2, 4, 8] and read(shifted) == [1.5, 2.5, 4.5], (fuse, read(scaled), read(shifted))
+
+
+def a_tensor_of_a_blocks_own_given_as_the_functions_argument():
+    """A block's default function reads a tensor that the traced function is called with."""
+    w, x = f32(1, 2, 4), f32(10, 20, 40)
+    f = defn.compile(lambda v: Nx.block(object(), [v], v.with_(data=None), lambda struct, t: Nx.negate(w)), w)
+    for _ in range(5):
+        assert read(f(w)) == [-1, -2, -4]
+    assert read(f(x)) == [-1, -2, -4]
+
+
+def arguments_handed_through_stay_the_callers():
+    x = f32(1, 2, 4)
+    f = defn.compile(lambda v: (v, Nx.reshape(v, (3, 1)), Nx.multiply(v, 3.0)), x)
+    for i in range(6):
+        x = f32(i, 2, 4)
+        same, alias, tripled = f(x)
+        assert same.data is x.data and alias.data.ref is x.data.ref and read(tripled) == [3 * i, 6, 12]
+        before = x.data.ref.sharers
+        assert Nx.backend_deallocate(alias) == "ok" and x.data.ref.sharers == before - 1
+        assert read(same) == [i, 2, 4]
+    f = defn.compile(lambda s, v: (s, Nx.reshape(s, (1,)), Nx.multiply(v, s)), 2.0, x)
+    for i in range(6):
+        s = f32(3.0 + i) if i % 2 else Nx.to_tensor(2.0)
+        s = Nx.reshape(s, ())
+        same, alias, scaled = f(s, x)
+        assert same.data is s.data and alias.data.ref is s.data.ref and alias.shape == (1,) and read(scaled) == [read(s) * v for v in read(x)]
+
+
+if __name__ == "__main__":
+    globals()[sys.argv[1]]()
