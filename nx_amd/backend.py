@@ -1262,7 +1262,7 @@ def _install():
 
 
 _install()
-native.setup(C.cast(L.lib.hipnx_buf_alloc, C.c_void_p).value, C.cast(L.lib.hipnx_buf_destroy, C.c_void_p).value, Tensor, HipNxBackend)
+native.setup(C.cast(L.lib.hipnx_buf_alloc, C.c_void_p).value, C.cast(L.lib.hipnx_buf_destroy, C.c_void_p).value, Tensor, HipNxBackend, L.check)
 
 
 def sync(device: int = 0) -> None:

@@ -13,6 +13,7 @@
 #include <Python.h>
 #include <structmember.h>
 #include <stdint.h>
+#include "../../include/hipnx.h"
 
 #define MAX_ARGS 20
 typedef int (*entry_t)(int64_t, int64_t, int64_t, int64_t, int64_t, int64_t, int64_t, int64_t, int64_t, int64_t, int64_t, int64_t,
@@ -26,9 +27,21 @@ static int enter(int64_t fn, const int64_t *a) {
 static int (*buf_alloc)(void *, size_t, void **);
 static int (*buf_destroy)(void *);
 static PyTypeObject *tensor_type, *backend_type;
+static PyObject *raise_status;        /* raises what the library reports with a status */
 static PyObject *s_data, *s_type, *s_shape, *s_names, *s_ref, *s_device, *s_released;
 static PyObject *freed_log;           /* the list that takes the handles `freed_thread` releases, while a function is recorded */
 static unsigned long freed_thread;
+
+/* Whether a status is an error of the call to raise at once.  The others (an operand gone, no memory, nothing that the kernels
+ * take) are found again by the general path, which reports them; these may not be: what an earlier kernel recorded is
+ * reported once, to the call that waits, and so is an error of the device. */
+static int is_raised(int status) { return status == HIPNX_EHIP || status == HIPNX_EINDEX || status == HIPNX_ERAISED; }
+static PyObject *raised(int status) {
+  PyObject *r = PyObject_CallFunction(raise_status, "i", status);
+  Py_XDECREF(r);
+  if (r) PyErr_Format(PyExc_RuntimeError, "status %d", status);
+  return NULL;
+}
 
 /* ---- Ref: owns one buffer handle ------------------------------------------------------------- */
 typedef struct {
@@ -160,7 +173,7 @@ static PyTypeObject CallType = {PyVarObject_HEAD_INIT(NULL, 0).tp_name = "hipnx_
                                 .tp_flags = Py_TPFLAGS_DEFAULT, .tp_dealloc = (destructor)call_dealloc,
                                 .tp_call = (ternaryfunc)call_call,
                                 .tp_doc = "call(*tensors) -> the result, or None where the tensors are not what it was made for, or the "
-                                          "library refused (the general path then reports it)"};
+                                          "library refused (the general path then reports it); raises what the call itself reports"};
 
 /* prepare(fn, args, in_at, out_at, nbytes, ctx, ctx_value, device, type, shape, names, keep) */
 static PyObject *prepare(PyObject *mod, PyObject *a) {
@@ -192,7 +205,7 @@ static PyObject *call_call(Call *self, PyObject *args, PyObject *kw) {
   Ref *in[4] = {NULL, NULL, NULL, NULL};
   int64_t a[MAX_ARGS];
   void *out = NULL;
-  int ok = PyTuple_GET_SIZE(args) == self->n_in, status = 1;
+  int ok = PyTuple_GET_SIZE(args) == self->n_in, status = HIPNX_EINVAL;
   memcpy(a, self->args, sizeof(a));
   for (int i = 0; ok && i < self->n_in; i++) {
     in[i] = live_ref(PyTuple_GET_ITEM(args, i), self->device);
@@ -210,6 +223,7 @@ static PyObject *call_call(Call *self, PyObject *args, PyObject *kw) {
     Py_END_ALLOW_THREADS
   }
   for (int i = 0; i < self->n_in; i++) Py_XDECREF(in[i]);
+  if (is_raised(status)) return raised(status);
   if (status) Py_RETURN_NONE;
   Ref *ref = new_ref(self->ctx, out, self->nbytes);
   if (!ref) {
@@ -260,7 +274,8 @@ static PyTypeObject ReplayType = {PyVarObject_HEAD_INIT(NULL, 0).tp_name = "hipn
                                   .tp_flags = Py_TPFLAGS_DEFAULT, .tp_dealloc = (destructor)replay_dealloc,
                                   .tp_call = (ternaryfunc)replay_call,
                                   .tp_doc = "replay(*tensors) -> [results], or None where the tensors are not what it was recorded for, or a "
-                                            "call was refused (nothing is kept then: the function is evaluated the general way)"};
+                                            "call was refused (nothing is kept then: the function is evaluated the general way); raises what a call "
+                                            "itself reports"};
 
 /* record(ops, n_params, n_slots, outs, ctx, ctx_value, device, keep)
  * ops: ("alloc", slot, nbytes) | ("free", slot) | ("call", fn, [argument | ("slot", s) | ("list", [s, ...])])
@@ -410,7 +425,7 @@ static PyObject *replay_call(Replay *self, PyObject *args, PyObject *kw) {
       for (int l = 0; l < o->n_lists; l++) {
         const HandleList *h = &self->lists[o->first_list + l];
         if (used + h->count > MAX_ARGS * 2) {
-          status = 1;
+          status = HIPNX_EINVAL;
           break;
         }
         a[h->at] = (int64_t)(intptr_t)&handles[used];
@@ -423,6 +438,10 @@ static PyObject *replay_call(Replay *self, PyObject *args, PyObject *kw) {
     for (int s = self->n_params; s < self->n_slots; s++)
       if (slot[s]) buf_destroy(slot[s]);
   Py_END_ALLOW_THREADS
+  if (is_raised(status)) {
+    raised(status);
+    goto done;
+  }
   if (status) goto refused;
   result = PyList_New(self->n_outs);
   for (int i = 0; result && i < self->n_outs; i++) {
@@ -451,11 +470,14 @@ done:
 static PyObject *setup(PyObject *mod, PyObject *a) {
   unsigned long long alloc, destroy;
   PyTypeObject *tensor, *backend;
-  if (!PyArg_ParseTuple(a, "KKO!O!", &alloc, &destroy, &PyType_Type, &tensor, &PyType_Type, &backend)) return NULL;
+  PyObject *check;
+  if (!PyArg_ParseTuple(a, "KKO!O!O", &alloc, &destroy, &PyType_Type, &tensor, &PyType_Type, &backend, &check)) return NULL;
   buf_alloc = (int (*)(void *, size_t, void **))(uintptr_t)alloc;
   buf_destroy = (int (*)(void *))(uintptr_t)destroy;
   Py_INCREF(tensor);
   Py_INCREF(backend);
+  Py_INCREF(check);
+  raise_status = check;
   tensor_type = tensor, backend_type = backend;
   Py_RETURN_NONE;
 }

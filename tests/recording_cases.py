@@ -65,5 +65,31 @@ def arguments_handed_through_stay_the_callers():
         assert same.data is s.data and alias.data.ref is s.data.ref and alias.shape == (1,) and read(scaled) == [read(s) * v for v in read(x)]
 
 
+def raises(call, text):
+    try:
+        call()
+    except Exception as e:  # noqa: BLE001
+        assert text in str(e), e
+    else:
+        raise AssertionError(f"no error, where {text!r} was due")
+
+
+def what_an_earlier_kernel_recorded_is_raised_by_the_call_that_waits():
+    """The library reports it once, to whichever call waits first: a callback laid out or recorded raises it, as any other does."""
+    t, at = f32([1, 2], [3, 4], [5, 6]), from_numpy(np.array([2, 0], np.int32), "s32", Hip)
+    f = defn.compile(lambda t, i: Nx.add(Nx.take(t, i), 1.0), t, at)
+    for _ in range(5):
+        assert read(Nx.take(t, at)) == [[5, 6], [1, 2]] and read(f(t, at)) == [[6, 7], [2, 3]]
+    assert f.replay is not None
+    for call in (lambda: Nx.take(t, at), lambda: f(t, at)):
+        standin.deferred.append(b"ArithmeticError: divided by zero a while ago")
+        raises(call, "divided by zero a while ago")
+        assert not standin.deferred
+        call()
+    far = from_numpy(np.array([2, 3], np.int32), "s32", Hip)
+    for call in (lambda: Nx.take(t, far), lambda: f(t, far)):
+        raises(call, "index out of bounds")
+
+
 if __name__ == "__main__":
     globals()[sys.argv[1]]()
