@@ -429,7 +429,7 @@ class HipNxBackend:
             fn, laid = "hipnx_gather", [T.size_bytes(t.type), len(t.shape), C.addressof(arrays[0]), T.code(indices.type), indices.size, 1, _bounds["policy"]]
         laid = [ctx.value] + laid
         first, n = len(laid), len(tensors)
-        return native.prepare(C.cast(getattr(L.lib, fn), C.c_void_p).value, laid + [0] * (n + 1), list(range(first, first + n)), first + n,
+        return native.prepare(_entry_points[fn], laid + [0] * (n + 1), list(range(first, first + n)), first + n,
                               out.size * T.size_bytes(out.type), ctx, ctx.value, device, out.type, out.shape, out.names, arrays)
 
     @classmethod
@@ -1262,6 +1262,8 @@ def _install():
 
 
 _install()
+_entry_points = {name: C.cast(getattr(L.lib, name), C.c_void_p).value for name in
+                 ("hipnx_binary", "hipnx_unary", "hipnx_reduce", "hipnx_argreduce", "hipnx_dot", "hipnx_gather")}  # (L.lib is stood in for while a function is recorded)
 native.setup(C.cast(L.lib.hipnx_buf_alloc, C.c_void_p).value, C.cast(L.lib.hipnx_buf_destroy, C.c_void_p).value, Tensor, HipNxBackend, L.check)
 
 

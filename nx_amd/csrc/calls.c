@@ -32,6 +32,9 @@ static PyObject *s_data, *s_type, *s_shape, *s_names, *s_ref, *s_device, *s_rele
 static PyObject *freed_log;           /* the list that takes the handles `freed_thread` releases, while a function is recorded */
 static unsigned long freed_thread;
 
+/* While a thread's evaluation is recorded its calls go through the library's stand-in, which writes them down. */
+static int is_recording(void) { return freed_log && freed_thread == PyThread_get_thread_ident(); }
+
 /* Whether a status is an error of the call to raise at once.  The others (an operand gone, no memory, nothing that the kernels
  * take) are found again by the general path, which reports them; these may not be: what an earlier kernel recorded is
  * reported once, to the call that waits, and so is an error of the device. */
@@ -53,7 +56,7 @@ typedef struct {
 
 static void ref_dealloc(Ref *self) {
   if (self->handle && buf_destroy) {
-    if (freed_log && freed_thread == PyThread_get_thread_ident()) {
+    if (is_recording()) {
       PyObject *h = PyLong_FromVoidPtr(self->handle);
       if (!h || PyList_Append(freed_log, h) < 0) PyErr_Clear();
       Py_XDECREF(h);
@@ -205,7 +208,7 @@ static PyObject *call_call(Call *self, PyObject *args, PyObject *kw) {
   Ref *in[4] = {NULL, NULL, NULL, NULL};
   int64_t a[MAX_ARGS];
   void *out = NULL;
-  int ok = PyTuple_GET_SIZE(args) == self->n_in, status = HIPNX_EINVAL;
+  int ok = PyTuple_GET_SIZE(args) == self->n_in && !is_recording(), status = HIPNX_EINVAL;
   memcpy(a, self->args, sizeof(a));
   for (int i = 0; ok && i < self->n_in; i++) {
     in[i] = live_ref(PyTuple_GET_ITEM(args, i), self->device);
@@ -389,7 +392,7 @@ static PyObject *replay_call(Replay *self, PyObject *args, PyObject *kw) {
   void *stack_slots[ON_STACK], *handles[MAX_ARGS * 2], **slot = stack_slots;
   Ref *stack_refs[ON_STACK], **in = stack_refs;
   PyObject *result = NULL;
-  if (PyTuple_GET_SIZE(args) != self->n_params) Py_RETURN_NONE;
+  if (PyTuple_GET_SIZE(args) != self->n_params || is_recording()) Py_RETURN_NONE;
   if (self->n_slots > ON_STACK) {
     slot = PyMem_Calloc(self->n_slots, sizeof(void *));
     in = PyMem_Calloc(self->n_slots, sizeof(Ref *));

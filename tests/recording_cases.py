@@ -91,5 +91,18 @@ def what_an_earlier_kernel_recorded_is_raised_by_the_call_that_waits():
         raises(call, "index out of bounds")
 
 
+def a_block_evaluated_by_its_default_function_while_a_recording_is_made():
+    """Its callbacks come through the front end, which lays their calls out: after a setting changed, or after operands elsewhere."""
+    for first in ("settings", "host"):
+        x = f32(0, 2, 0)
+        f = defn.compile(lambda a: Nx.logical_not(a), x)
+        for i in range(6):
+            if i == 2:
+                previous = B.bounds_policy("clamp")
+            here = x if first == "settings" or i > 1 else Nx.backend_copy(x, HostBinary, {})
+            assert read(f(here)) == [1, 0, 1], (first, i)
+        B.bounds_policy(previous)
+
+
 if __name__ == "__main__":
     globals()[sys.argv[1]]()
