@@ -98,8 +98,9 @@ def _fresh_ref(ctx, nbytes: int, _fresh=native.fresh) -> _Ref:
     ref = _fresh(ctx, ctx.value, nbytes)
     if ref.__class__ is int:
         L.check(ref)
-    if _recorder[0] is not None:
-        _recorder[0].allocated(ref)
+    recorder = _recorder[0]  # (read once: the thread that records may end its recording here)
+    if recorder is not None:
+        recorder.allocated(ref)
     return ref
 
 

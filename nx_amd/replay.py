@@ -67,7 +67,7 @@ class _Recorder:
                     self.ops.append(("call", C.cast(real, C.c_void_p).value, [self._argument(a, t) for a, t in zip(args, real.argtypes)]))
                     if name in ("hipnx_fused_elementwise", "hipnx_fused_words", "hipnx_fused_scores"):
                         self.modes.add(B._fused_set.get(self.device, "interpreted"))
-                except _Unrecordable:
+                except Exception:  # the evaluation goes on, whatever becomes of its recording
                     self.failed = True
             return status
         return call
@@ -91,7 +91,7 @@ class _Recorder:
     def _buffer(self, handle):
         slot = self.slots.get(handle)
         if slot is None:  # a constant the backend keeps: an operand of every call from now on
-            ref = next((r for r in B.HipNxBackend._scalar_cache.values() if r.handle == handle), None)
+            ref = next((r for r in B.HipNxBackend._scalar_cache.copy().values() if r.handle == handle), None)  # (other threads add to it)
             if ref is None:
                 raise _Unrecordable
             slot = self._slot(handle)

@@ -104,5 +104,36 @@ def a_block_evaluated_by_its_default_function_while_a_recording_is_made():
         B.bounds_policy(previous)
 
 
+def other_threads_make_constants_while_a_function_is_recorded():
+    """The recorder looks its constants up in a table that grows meanwhile, and other threads' buffers are made while it begins and
+    ends."""
+    class Growing(dict):
+        def values(self):
+            for v in super().values():
+                yield v
+                self[len(self)] = v
+    x = f32(1, 2, 4)
+    f = defn.compile(lambda v: Nx.multiply(Nx.add(v, 0.25), 3.0), x)
+    cache, Hip._scalar_cache = Hip._scalar_cache, Growing(Hip._scalar_cache)
+    read(Nx.add(x, 7.0))
+    try:
+        for _ in range(5):
+            assert read(f(x)) == [3.75, 6.75, 12.75]
+    finally:
+        Hip._scalar_cache = cache
+
+    class Ending(list):  # (another thread ends its recording between two reads)
+        def __getitem__(self, i):
+            now, self[0] = list.__getitem__(self, i), None
+            return now
+
+    class Other:
+        def allocated(self, ref):
+            pass
+    B._recorder = Ending([Other()])
+    assert read(Nx.negate(x)) == [-1, -2, -4]
+    B._recorder = [None]
+
+
 if __name__ == "__main__":
     globals()[sys.argv[1]]()
