@@ -1376,18 +1376,25 @@ def bf16_rounding(mode: str) -> str:
     return previous
 
 
-_epoch = [0]
+_fused_modes = {}  # device -> the mode chosen with fused_mode/2: what a call that names none runs in
+_settings = [None]
 
 
-def settings_epoch() -> int:
-    """Grows with every change of a setting that calls are laid out under (bounds policy, bf16 rounding, fused mode)."""
-    return _epoch[0]
+def settings():
+    """The settings that calls are laid out under (bounds policy, bf16 rounding, fused modes), as one value: equal again once
+    they are set back."""
+    return _settings[0]
 
 
 def _settings_changed() -> None:
+    """After the change: what is laid out from here on goes to a new table, and what another thread is laying out under the
+    old settings to the old one."""
     from . import nx
-    _epoch[0] += 1
-    nx._ready.clear()
+    _settings[0] = (_bounds["policy"], _bf16["rounding"], tuple(sorted(kv for kv in _fused_modes.items() if kv[1] != "interpreted")))
+    nx._ready = {}
+
+
+_settings_changed()
 
 
 def fused_mode(mode: str, device: int = 0) -> None:
@@ -1429,7 +1436,6 @@ def _advise_huge_pages(address: int, n: int) -> None:
 _REDUCTIONS = {"sum": RED_SUM, "product": RED_PRODUCT, "reduce_max": RED_MAX, "reduce_min": RED_MIN, "all": RED_ALL, "any": RED_ANY}
 _reduce_plans = {}  # (types, shape and axes of a reduction callback) -> its type codes, [outer, red, inner] view, result bytes
 _binary_plans = {}  # (types and shapes of a binary callback) -> its type codes, shape and stride arrays, result bytes
-_fused_modes = {}  # device -> the mode chosen with fused_mode/2: what a call that names none runs in
 _fused_set = {}    # device -> the mode the library is in at this moment (a call that names one leaves it there)
 _fused_arrays = {}  # (id of a layout, input types) -> (the layout itself, so the id stays its own; C arrays of types and strides)
 

@@ -215,11 +215,12 @@ _ready = {}
 
 def _make_ready(key, mod, *args):
     if "prepared" in mod.__dict__:  # (not asked of the expression builder, to which any name is an operation)
-        if len(_ready) >= 4096:
-            _ready.clear()
+        table = _ready  # (replaced when a setting changes: a call laid out under the old one goes where nobody looks)
+        if len(table) >= 4096:
+            table.clear()
         call = mod.prepared(*args)
         if call is not None:
-            _ready[key] = call
+            table[key] = call
 
 
 def _number_or_type(x):

@@ -37,7 +37,7 @@ class _Recorder:
         self.ctx, self.device = B._Context.get(device), device
         self.slots, self.n_slots = {}, 0  # handle -> slot while the buffer lives
         self.ops, self.keep, self.freed, self.externals, self.modes = [], [], [], [], set()
-        self.failed = False
+        self.failed, self.settings = False, B.settings()
         for p in params:
             handle = p.data.ref.handle
             self.failed |= handle in self.slots  # (one buffer twice: which of the two a call reads cannot be told)
@@ -117,12 +117,12 @@ class _Recorder:
 class Replay:
     """A recorded evaluation: `run(params)` gives its results, or None where it does not apply."""
 
-    def __init__(self, calls, device, mode, constants):
+    def __init__(self, calls, device, mode, constants, settings):
         self.calls, self.device, self.mode, self.constants = calls, device, mode, constants
-        self.settings, self.backend = B.settings_epoch(), Nx.default_backend()
+        self.settings, self.backend = settings, Nx.default_backend()
 
     def run(self, params):
-        if B._capturing or self.settings != B.settings_epoch():
+        if B._capturing or self.settings != B.settings():
             return None
         mod, opts = Nx.default_backend()
         if mod is not self.backend[0] or opts != self.backend[1]:
@@ -181,8 +181,8 @@ def _finish(rec, results):
             return None
         outs.append((rec.slots.get(d.ref.handle, -1), d.ref.nbytes, t.type, t.shape, t.names))
     late = [slot for slot, _ in rec.late]
-    if len(rec.modes) > 1 or len({o[0] for o in outs}) < len(outs) or any(o[0] < rec.n_params or o[0] in late for o in outs):
-        return None  # (a parameter or a constant handed through, or one buffer under two results)
+    if rec.settings is not B.settings() or len(rec.modes) > 1 or len({o[0] for o in outs}) < len(outs) or any(o[0] < rec.n_params or o[0] in late for o in outs):
+        return None  # (a parameter or a constant handed through, or one buffer under two results; settings that another thread changed meanwhile)
     # slots in the order the native side wants them: parameters, constants, then what is allocated
     order = list(range(rec.n_params)) + late + [s for s in range(rec.n_params, rec.n_slots) if s not in late]
     to = {s: i for i, s in enumerate(order)}
@@ -194,4 +194,4 @@ def _finish(rec, results):
     ops = [(op[0], op[1], [moved(a) for a in op[2]]) if op[0] == "call" else (op[0], to[op[1]], op[2] if op[0] == "alloc" else 0) for op in rec.ops]
     calls = native.record(ops, rec.n_params + len(late), rec.n_slots, [(to[o[0]],) + o[1:] for o in outs], rec.ctx, rec.ctx.value, rec.device, rec.keep)
     constants = [Nx.Tensor(B.HipNxBackend(ref, rec.device), "u8", ()) for _, ref in rec.late]
-    return Replay(calls, rec.device, rec.modes.pop() if rec.modes else None, constants)
+    return Replay(calls, rec.device, rec.modes.pop() if rec.modes else None, constants, rec.settings)

@@ -135,5 +135,36 @@ def other_threads_make_constants_while_a_function_is_recorded():
     B._recorder = [None]
 
 
+def a_setting_changed_while_a_call_is_laid_out_or_recorded():
+    """Another thread changes the bounds policy between the call's layout and its place in the table, or within the evaluation that
+    is recorded: neither is kept under the new policy."""
+    t, near, far = f32([1, 2], [3, 4], [5, 6]), from_numpy(np.array([2, 0], np.int32), "s32", Hip), from_numpy(np.array([2, 9], np.int32), "s32", Hip)
+    prepared, armed = Hip.prepared.__func__, [1]
+
+    def slowly(cls, *args):
+        call = prepared(cls, *args)
+        if armed:
+            armed.clear()
+            B.bounds_policy("clamp")
+        return call
+    Hip.prepared = classmethod(slowly)
+    Nx.take(t, near)
+    Hip.prepared = classmethod(prepared)
+    assert read(Nx.take(t, far)) == [[5, 6], [5, 6]]
+    f, evaluations = defn.compile(lambda t, i: Nx.take(t, i), t, near), []
+    walk = f._walk
+
+    def changing(params):
+        evaluations.append(params)
+        results = walk(params)
+        if len(evaluations) == 3:
+            B.bounds_policy("raise")
+        return results
+    f._walk = changing
+    for _ in range(3):
+        f(t, near)
+    raises(lambda: f(t, far), "index out of bounds")
+
+
 if __name__ == "__main__":
     globals()[sys.argv[1]]()
