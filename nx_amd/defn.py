@@ -1638,9 +1638,6 @@ class _Run:
         return self.backend[0] if mod is HostBinary else mod
 
 
-_RECORD_AT = 3
-
-
 class Compiled:
     """A traced function: call it with arguments of the traced shapes and types."""
 
@@ -1649,7 +1646,8 @@ class Compiled:
         self.n_params = len(templates)
         self.plans: Dict[Any, _Plan] = {}
         self.plan = _Plan(roots, 0, self.plans)
-        self.calls, self.replay = 0, None
+        self.replay = None     # the recording in use (replay.py)
+        self.recordings = {}   # settings -> what is known of recordings under them
 
     def _params(self, args):
         leaves: list = []
@@ -1663,18 +1661,15 @@ class Compiled:
         return params
 
     def _evaluate(self, params):
-        """Through the recorded library calls where there is a recording that applies (replay.py): the third evaluation is
-        recorded, by which time every program is compiled and every fallback has been found."""
+        """Through the recorded library calls where there is a recording that applies (replay.py)."""
         if self.replay is not None:
             results = self.replay.run(params)
             if results is not None:
                 return results
-        self.calls += 1
-        if self.calls == _RECORD_AT and (backend := sys.modules.get(__package__ + ".backend")) is not None:
-            if all(p.data.__class__ is backend.HipNxBackend for p in params):
-                from .replay import record
-                results, self.replay = record(self._walk, params)
-                return results
+        backend = sys.modules.get(__package__ + ".backend")
+        if backend is not None and not backend._capturing and all(p.data.__class__ is backend.HipNxBackend for p in params):
+            from .replay import evaluate
+            return evaluate(self, params)
         return self._walk(params)
 
     def _walk(self, params):

@@ -5,8 +5,8 @@ calling -- which entry points, with which extents, on which buffers, allocated a
 the traced shapes and types alone unless a node looks at values (`while`, `cond`) or moves data between host and device.
 So one evaluation is recorded at the boundary of the library (every call through `_lib.lib`, every buffer made and
 released), and later calls issue the same list natively (`csrc/calls.c`) on that call's own operands and fresh buffers:
-no result and no address is kept.  A recording holds for the settings it was made under; whatever it does not cover --
-operands elsewhere, a device that is capturing, a call the library refuses -- is evaluated as before.
+no result and no address is kept.  A recording holds for the settings it was made under, kept for when they come back; whatever
+it does not cover -- operands elsewhere, a device that is capturing, a call the library refuses -- is evaluated as before.
 """
 from __future__ import annotations
 
@@ -36,12 +36,10 @@ class _Recorder:
         self._lib, self._thread = L.lib, threading.get_ident()
         self.ctx, self.device = B._Context.get(device), device
         self.slots, self.n_slots = {}, 0  # handle -> slot while the buffer lives
-        self.ops, self.keep, self.freed, self.externals, self.modes = [], [], [], [], set()
+        self.ops, self.keep, self.freed, self.modes = [], [], [], set()
         self.failed, self.settings = False, B.settings()
         for p in params:
-            handle = p.data.ref.handle
-            self.failed |= handle in self.slots  # (one buffer twice: which of the two a call reads cannot be told)
-            self._slot(handle)
+            self._slot(p.data.ref.handle)
         self.n_params = self.n_slots
         self.late = []  # handles of buffers made before the recording (constants): slots behind the parameters
 
@@ -132,26 +130,72 @@ class Replay:
         return self.calls(*params, *self.constants)
 
 
-def record(evaluate, params):
-    """(the results of `evaluate(params)`, a Replay of it or None)."""
-    data = [p.data for p in params]
-    if not data or B._capturing or any(d.__class__ is not B.HipNxBackend or d.released or d.device != data[0].device for d in data) or not _lock.acquire(blocking=False):
-        return evaluate(params), None
-    try:
-        private = [_private(p) for p in params]
-        recorder = _Recorder(data[0].device, private)
-        real, L.lib, B._recorder[0] = L.lib, recorder, recorder
-        native.log_freed(recorder.freed)
+RECORD_AT = 3   # by the third evaluation every program is compiled and every fallback has been found
+ATTEMPTS = 3     # a function whose calls cannot be written down is not tried for ever
+SETTINGS = 8     # settings whose recordings a function keeps
+
+
+class _History:
+    """A function's evaluations on the device under one value of the settings."""
+
+    __slots__ = ("calls", "attempts", "replay")
+
+    def __init__(self):
+        self.calls = self.attempts = 0
+        self.replay = None
+
+
+def evaluate(compiled, params):
+    """An evaluation of `compiled` on operands of the device backend that its present recording, if any, did not answer: by the
+    recording of the present settings, or the general way, writing it down if it is time to."""
+    mod, opts = Nx.default_backend()
+    key = (B.settings(), mod, repr(opts))
+    known = compiled.recordings.get(key)
+    if known is None:
+        if len(compiled.recordings) >= SETTINGS:
+            compiled.recordings.clear()
+        known = compiled.recordings.setdefault(key, _History())
+    if known.replay is not None:
+        if known.replay is not compiled.replay:  # these settings were in force before
+            compiled.replay = known.replay
+            results = known.replay.run(params)
+            if results is not None:
+                return results
+        return compiled._walk(params)
+    known.calls += 1
+    if known.calls >= RECORD_AT and known.attempts < ATTEMPTS and _recordable(params) and _lock.acquire(blocking=False):
         try:
-            results = evaluate(private)
+            results, replay = record(compiled._walk, params)
+            known.attempts += 1
         finally:
-            native.log_freed(None)
-            L.lib, B._recorder[0] = real, None
+            _lock.release()
+        if replay is not None:
+            compiled.replay = known.replay = replay
+        return results
+    return compiled._walk(params)
+
+
+def _recordable(params):
+    """Whether an evaluation on these operands can be told apart by its calls.  (One buffer twice: which of the two a call reads
+    cannot be.)"""
+    data = [p.data for p in params]
+    return bool(data) and not any(d.released or d.device != data[0].device for d in data) and len({id(d.ref) for d in data}) == len(data)
+
+
+def record(evaluate, params):
+    """(the results of `evaluate(params)`, a Replay of it or None).  One thread at a time."""
+    device = params[0].data.device
+    private = [_private(p) for p in params]
+    recorder = _Recorder(device, private)
+    real, L.lib, B._recorder[0] = L.lib, recorder, recorder
+    native.log_freed(recorder.freed)
+    try:
+        results = evaluate(private)
     finally:
-        _lock.release()
+        native.log_freed(None)
+        L.lib, B._recorder[0] = real, None
     replay = None if recorder.failed else _finish(recorder, results)
     return [_callers(t, private, params) for t in results], replay
-
 
 def _private(p):
     """The parameter in a buffer that the function cannot know as its own: a call's operands are told apart by their handles, and

@@ -166,5 +166,75 @@ def a_setting_changed_while_a_call_is_laid_out_or_recorded():
     raises(lambda: f(t, far), "index out of bounds")
 
 
+def recorded(f):
+    """Whether a call of `f` is answered by its recording: nothing is evaluated."""
+    walk, evaluated = f._walk, []
+    f._walk = lambda params: (evaluated.append(1), walk(params))[1]
+    try:
+        yield lambda *args: (evaluated.clear(), f(*args), not evaluated)[2]
+    finally:
+        f._walk = walk
+
+
+def recordings_are_made_again_and_come_back_with_their_settings():
+    x, y = f32(1, 2, 4), f32(3, 5, 7)
+    f = defn.compile(lambda a, b: Nx.subtract(Nx.multiply(a, 2.0), b), x, y)
+    for by_recording in recorded(f):
+        assert [by_recording(x, y) for _ in range(5)] == [False, False, False, True, True]
+        B.bounds_policy("clamp")
+        assert [by_recording(x, y) for _ in range(5)] == [False, False, False, True, True]
+        B.bounds_policy("raise")     # back: the recording of these settings applies at once
+        assert by_recording(x, y)
+        B.bounds_policy("clamp")
+        assert by_recording(x, y)
+        Nx.default_backend(HostBinary)
+        assert [by_recording(x, y) for _ in range(4)] == [False, False, False, True]
+        Nx.default_backend(Hip)
+        assert by_recording(x, y) and read(f(x, y)) == [-1, -1, 1]
+        B.bounds_policy("raise")
+        for i in range(20):          # any number of settings, a bounded number of recordings
+            B.fused_mode("compiled", device=i)
+            f(x, y)
+            assert len(f.recordings) <= 8
+        for i in range(20):
+            B.fused_mode("interpreted", device=i)
+
+
+def a_third_call_that_cannot_be_recorded_is_not_the_last_chance():
+    import threading
+    from nx_amd import replay
+    x, y = f32(1, 2, 4), f32(3, 5, 7)
+    host = Nx.backend_copy(x, HostBinary, {})
+    f = defn.compile(lambda a, b: Nx.subtract(Nx.multiply(a, 2.0), b), x, y)
+    for by_recording in recorded(f):
+        assert not any(by_recording(x, x) for _ in range(4)) and f.replay is None  # one buffer twice
+        assert not by_recording(x, y) and by_recording(x, y)
+    f = defn.compile(lambda a, b: Nx.subtract(Nx.multiply(a, 2.0), b), x, y)
+    for by_recording in recorded(f):
+        assert not any(by_recording(host, y) for _ in range(4))                    # operands elsewhere count for nothing
+        assert [by_recording(x, y) for _ in range(4)] == [False, False, False, True]
+    f = defn.compile(lambda a, b: Nx.subtract(Nx.multiply(a, 2.0), b), x, y)
+    for by_recording in recorded(f):
+        assert not by_recording(x, y) and not by_recording(x, y)
+        with replay._lock:                                                          # another thread records
+            assert not by_recording(x, y)
+        assert not by_recording(x, y) and by_recording(x, y)
+    f = defn.compile(lambda a: Nx.logical_not(a), x)                                # never: tried a few times
+    attempts, record = [], replay.record
+    replay.record = lambda *a: (attempts.append(1), record(*a))[1]
+    for _ in range(12):
+        assert read(f(x)) == [0, 0, 0]
+    replay.record = record
+    assert f.replay is None and len(attempts) == replay.ATTEMPTS
+    # two threads at once: whoever does not record leaves the other's recording alone
+    f = defn.compile(lambda a, b: Nx.subtract(Nx.multiply(a, 2.0), b), x, y)
+    threads = [threading.Thread(target=lambda: [f(x, y) for _ in range(50)]) for _ in range(4)]
+    [t.start() for t in threads], [t.join() for t in threads]
+    Nx.default_backend(Hip)
+    for _ in range(3):
+        assert read(f(x, y)) == [-1, -1, 1]
+    assert f.replay is not None
+
+
 if __name__ == "__main__":
     globals()[sys.argv[1]]()
