@@ -365,8 +365,8 @@ static int fused_impl(hipnx_ctx *ctx, int n_instr, const hipnx_fused_instr *prog
       const int64_t *st = side ? c.r_strides : c.l_strides;
       for (int i = 0; i < 3; i++)
         if (st[i] < 0 || st[i] > (1ll << 40)) return set_error(HIPNX_EINVAL, "fused_scores: a stride of %lld elements", (long long)st[i]);
-      const int64_t last = (c.batch_outer - 1) * st[0] + (c.batch_inner - 1) * st[1] + ((side ? cols : c.M) - 1) * st[2] + c.K;
-      if (int s = check_buf(ctx, side ? c.r : c.l, (uint64_t)last * 2, side ? "fused_scores rhs" : "fused_scores lhs")) return s;
+      const uint64_t bytes = strided_bytes(c.batch_outer, st[0], c.batch_inner, st[1], side ? cols : c.M, st[2], c.K, 2);
+      if (int s = check_buf(ctx, side ? c.r : c.l, bytes, side ? "fused_scores rhs" : "fused_scores lhs")) return s;
     }
     a.scores_inner = (int)c.batch_inner;
     a.scores_rows = c.M;

@@ -331,6 +331,11 @@ struct DotView {
 static int dot_impl(hipnx_ctx *ctx, int l_dt, int r_dt, int out_dt, int64_t batch, int64_t M, int64_t N,
                     int64_t K, int l_layout, int r_layout, const hipnx_buf *l, const hipnx_buf *r,
                     hipnx_buf *out, int scale_mode, const hipnx_buf *scale, const DotView *view = nullptr, bool any_k = false) {
+  if (batch > 0 && M > 0 && N > 0 && K > 0) {  // (the products below are 64 bits wide)
+    const __int128 most = INT64_MAX / 8;
+    if ((__int128)M * N > most / batch || (__int128)M * K > most / batch || (__int128)N * K > most / batch)
+      return set_error(HIPNX_EINVAL, "dot: extents beyond any buffer");
+  }
   if (view && batch > 65535) return set_error(HIPNX_EUNSUPPORTED, "dot_strided: more than 65535 batch items");
   // More batch items than a grid's second dimension holds (100000 small matrices): runs of 65535 items, each over
   // borrowed handles on its part of the three buffers.
@@ -728,7 +733,7 @@ extern "C" int hipnx_dot_strided(hipnx_ctx *ctx, int l_dt, int r_dt, int out_dt,
   if ((l_layout != HIPNX_K_INNER && l_layout != HIPNX_K_OUTER) || (r_layout != HIPNX_K_INNER && r_layout != HIPNX_K_OUTER))
     return set_error(HIPNX_EINVAL, "dot_strided: unknown operand layout");
   const int64_t batch = batch_outer * batch_inner;
-  if (batch * M * N > 0 && K > 0) {
+  if (batch > 0 && M > 0 && N > 0 && K > 0) {
     Enter in(ctx);
     if (in.status) return in.status;
     for (int side = 0; side < 2; side++) {
@@ -738,8 +743,8 @@ extern "C" int hipnx_dot_strided(hipnx_ctx *ctx, int l_dt, int r_dt, int out_dt,
         if (s[i] < 0 || s[i] > (1ll << 40)) return set_error(HIPNX_EINVAL, "dot_strided: a stride of %lld elements", (long long)s[i]);
       // runs that overlap within an item, or that are read as neighbours without being ones, are no operand
       if (s[2] < (kin ? K : rows)) return set_error(HIPNX_EINVAL, "dot_strided: rows of an operand overlap");
-      const int64_t last = (batch_outer - 1) * s[0] + (batch_inner - 1) * s[1] + ((kin ? rows : K) - 1) * s[2] + (kin ? K : rows);
-      if (int st = check_buf(ctx, side ? r : l, (uint64_t)last * (side ? rsz : lsz), side ? "dot_strided rhs" : "dot_strided lhs")) return st;
+      const uint64_t bytes = strided_bytes(batch_outer, s[0], batch_inner, s[1], kin ? rows : K, s[2], kin ? K : rows, side ? rsz : lsz);
+      if (int st = check_buf(ctx, side ? r : l, bytes, side ? "dot_strided rhs" : "dot_strided lhs")) return st;
     }
   }
   const DotView v{batch_inner, l_strides[2] * lsz, l_strides[0] * lsz, l_strides[1] * lsz, r_strides[2] * rsz, r_strides[0] * rsz, r_strides[1] * rsz};

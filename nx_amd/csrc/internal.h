@@ -134,6 +134,13 @@ inline int check_buf(const hipnx_ctx *ctx, hipnx_buf *b, uint64_t need_bytes, co
   return st;
 }
 
+// Bytes that an operand reaches over: n2 runs of `run` elements s2 elements apart, in n0 x n1 items s0 and s1 apart (no extent is
+// 0).  Extents and strides are the caller's, and their products need more than 64 bits; what does is more than any buffer holds.
+inline uint64_t strided_bytes(int64_t n0, int64_t s0, int64_t n1, int64_t s1, int64_t n2, int64_t s2, int64_t run, int size) {
+  const __int128 bytes = ((__int128)(n0 - 1) * s0 + (__int128)(n1 - 1) * s1 + (__int128)(n2 - 1) * s2 + run) * size;
+  return bytes > (__int128)INT64_MAX ? UINT64_MAX : (uint64_t)bytes;
+}
+
 // pooled device memory; both expect the context mutex to be held (i.e. inside an Enter scope)
 int pool_alloc(hipnx_ctx *ctx, size_t bytes, void **ptr_out, size_t *cap_out);
 int pool_free(hipnx_ctx *ctx, void *ptr, size_t cap);

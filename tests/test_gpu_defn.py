@@ -1229,6 +1229,9 @@ def test_other_orders_of_a_dots_operands(hip, oracle):
 
 def test_dot_strided_refuses_what_is_not_there(hip):
     """Strides that reach past an operand's end, overlapping rows, extents below zero: an error, and nothing is launched."""
+    import ctypes as C
+
+    from nx_amd import backend as B
     from nx_amd.backend import K_INNER
     x = rand_float(np.random.default_rng(1), "bf16", (4, 32, 64), hip)
     out = rand_float(np.random.default_rng(2), "bf16", (4, 32, 32), hip)
@@ -1243,6 +1246,32 @@ def test_dot_strided_refuses_what_is_not_there(hip):
     for bad in ((0, 32 * 64 + 8, 64), (0, 32 * 64, 72), (8, 32 * 64, 64), (0, 32 * 64, 56), (0, -64, 64), (0, 32 * 64, 1 << 41)):
         assert call(bad, good, outer=2 if bad[0] else 1, inner=4) != 0 and call(good, bad, outer=2 if bad[0] else 1) != 0, bad
     assert call(good, good, M=-1) != 0 and call(good, good, K=72) != 0
+    # products that are small numbers, or none, in 64 bits: rows 2^40 elements apart, batches of 2^62 items
+    for M, stride in (((1 << 23) + 1, 1 << 40), ((1 << 24) + 1, 1 << 40), ((1 << 25) + 1, 1 << 39), ((1 << 60) + 1, 64), ((1 << 59) + 1, 64)):
+        for inner in (1, 4):
+            assert call((0, 32 * 64, stride), good, M=M, inner=inner) == L.EINVAL and "dot_strided lhs" in L.last_error(), (M, stride)
+    assert call((1 << 40, 0, 64), good, outer=(1 << 24) + 1, inner=1) != 0 and call(good, (0, 1 << 40, 64), inner=(1 << 23) + 1) != 0
+    assert call(good, good, outer=1 << 32, inner=1 << 31) != 0
+    for shape in ((1 << 31, 1 << 33, 64), (1 << 62, 4, 8), (4, 1 << 62, 8), (32, 32, 1 << 61)):
+        assert L.lib.hipnx_dot(_Context.get(0), T_BF16, T_BF16, T_BF16, 1, *shape, K_INNER, K_INNER, x.data.ref.handle, x.data.ref.handle,
+                               out.data.ref.handle) == L.EINVAL, shape
+    row_reduce, row_stat = L.FUSED_BITCAST + 1, L.FUSED_BITCAST + 2
+    instr = (L.FusedInstr * 3)()
+    for q, (kind, op, src) in zip(instr, ((L.FUSED_SET, 0, L.FUSED_SRC_INPUT), (row_reduce, 0, 0), (row_stat, 0, 0))):
+        q.kind, q.op, q.src, q.dt, q.flags = kind, op, src, T.code(("f", 32)), kind == row_stat
+
+    def scores(M, l, r):
+        handles = (C.c_void_p * 1)(x.data.ref.handle)
+        return L.lib.hipnx_fused_scores(_Context.get(0), 3, C.cast(instr, C.c_void_p), 1, handles, (C.c_int * 1)(T_BF16), (C.c_int64 * 1)(32), (C.c_int * 1)(1),
+                                        32, 0, 1, 4, M, 64, (C.c_int64 * 6)(*l, *r), (C.c_void_p * 2)(x.data.ref.handle, x.data.ref.handle),
+                                        T.code(("f", 32)), out.data.ref.handle)
+    B._set_fused_mode("compiled", 0)
+    try:
+        assert scores(32, good, good) == 0
+        for M, stride in (((1 << 23) + 1, 1 << 40), ((1 << 24) + 1, 1 << 40), ((1 << 25) + 1, 1 << 39)):
+            assert scores(M, (0, 32 * 64, stride), good) == L.EINVAL and "fused_scores lhs" in L.last_error(), (M, stride)
+    finally:
+        B._set_fused_mode("interpreted", 0)
 
 
 # ---- traced functions and callbacks issued natively (nx_amd/replay.py, csrc/calls.c) ----------------------
