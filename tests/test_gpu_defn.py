@@ -1171,7 +1171,8 @@ def split_heads(t, heads):
 # kernel the tile choice can come to; K that is not whole 16-byte pieces is copied as before
 @pytest.mark.parametrize("ty", ["bf16", "f16", "f32", "s8"])
 @pytest.mark.parametrize("batch,heads,queries,keys,dim", [(2, 3, 40, 72, 64), (1, 4, 1, 333, 128), (3, 2, 130, 257, 72), (2, 8, 256, 512, 64),
-                                                          (1, 2, 512, 640, 1024), (2, 2, 17, 65, 33), (1, 1, 24, 48, 64)])
+                                                          (1, 2, 512, 640, 1024), (2, 2, 17, 65, 33), (1, 1, 24, 48, 64),
+                                                          (2, 3, 16, 24, 4096), (1, 2, 1, 300, 1024), (2, 2, 4, 64, 2048)])
 def test_a_dot_reads_transposed_operands_where_they_lie(batch, heads, queries, keys, dim, ty, hip):
     rng = np.random.default_rng(seed_of(batch, heads, queries, keys, dim, ty))
 
@@ -1206,6 +1207,8 @@ def test_a_dot_reads_transposed_operands_where_they_lie(batch, heads, queries, k
         assert_bits_equal(got, want, f"{fun.__name__} {ty}")
         esz, K = {"s8": 1, "f32": 4}.get(ty, 2), dim if fun is scores else keys
         direct = K * esz % 16 == 0 and (fun is scores or dim % row_block == 0) and queries * (keys if fun is scores else dim) >= 256
+        if (queries <= 32 and keys <= 32 and K >= 4096) or (fun is scores and esz == 4 and queries <= 4 and K >= 1024):
+            direct = False  # (few outputs over a long K are summed in f64 -- s8 exactly -- by the separate contraction)
         assert (not copies) == direct, (fun.__name__, ty, copies)
 
 
