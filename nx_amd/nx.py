@@ -410,7 +410,10 @@ def _argmin_or_max(t, op, axis=None, tie_break="low", keep_axis=False, type=("s"
         raise ValueError(f"unknown value for :tie_break, expected :high or :low, got: {tie_break!r}")
     t = to_tensor(t)
     key = (op, t.type, t.shape, axis, tie_break, keep_axis, type) if axis is None or axis.__class__ is int else None
-    ready = _ready.get(key)
+    try:
+        ready = _ready.get(key)
+    except TypeError:  # options that are no key: the general path takes or refuses them
+        key = ready = None
     if ready is not None:
         res = ready(t)
         if res is not None:

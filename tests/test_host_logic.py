@@ -7,6 +7,7 @@ from nx_amd import HostBinary, nx as Nx
 from nx_amd import shape as S
 from nx_amd import types as T
 from nx_amd.tensor import list_to_binary, number_to_binary
+from support import from_numpy
 
 
 def test_merge_follows_type_ex_doctests():  # nx/lib/nx/type.ex:405-461
@@ -150,3 +151,14 @@ def test_pad_merges_its_type_before_the_number_becomes_a_tensor(oracle):
     assert Nx.pad(bf, 0.0, [(1, 1, 0)]).type == ("bf", 16)
     assert Nx.pad(Nx.tensor([1, 2]), 0, [(1, 1, 0)]).type == ("s", 32)
     assert Nx.to_flat_list(Nx.pad(bf, 0.0, [(1, 2, 0)])) == [0.0, 1.0, 2.0, 0.0, 0.0]
+
+
+def test_argmax_takes_a_type_as_a_list(oracle):
+    """The type of the result as any pair; a pair that names no type is refused for what it is."""
+    t = from_numpy(np.array([[3, 1, 2], [4, 6, 5]], np.float32), "f32", oracle)
+    for axis, want in ((0, [1, 1, 1]), (1, [0, 1]), (None, 4)):
+        for type in (["s", 16], ("s", 16), "s16"):
+            got = Nx.argmax(t, axis=axis, type=type)
+            assert got.type == ("s", 16) and Nx.to_numpy(got).tolist() == want
+    with pytest.raises(ValueError, match="invalid numerical type"):
+        Nx.argmin(t, axis=0, type=["s", 33])
