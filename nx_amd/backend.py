@@ -420,9 +420,10 @@ class HipNxBackend:
                                            T.code(out.type), outer, red, inner]
         elif kind == "dot":
             l, c1, b1, r, c2, _ = args
-            _, _, _, K, batch, ((l_layout, M), (r_layout, N)) = cls._dot_plans[(l.shape, tuple(c1), len(b1), r.shape, tuple(c2))]
-            if l_layout is None or r_layout is None:
+            plan = cls._dot_plans.get((l.shape, tuple(c1), len(b1), r.shape, tuple(c2)))  # (another thread may have cleared the table)
+            if plan is None or None in (plan[5][0][0], plan[5][1][0]):
                 return None
+            _, _, _, K, batch, ((l_layout, M), (r_layout, N)) = plan
             fn, laid = "hipnx_dot", [T.code(l.type), T.code(r.type), _out_code(out.type), batch, M, N, K, l_layout, r_layout]
         else:  # "take": whole entries of the first axis
             t, indices = tensors

@@ -446,13 +446,16 @@ def dot(t1, *args, out_type=None):
     `out_type` is not part of the reference's front end: it sets the template type handed to the
     `dot` callback (both reference backends honour `out.type` whatever the operand types,
     binary_backend.ex:549-559) and is how a s8 x s8 -> s32 contraction is requested."""
+    t2 = args[len(args) // 2] if len(args) in (1, 3, 5) else None
+    if t1.__class__ is not Tensor or t2.__class__ is not Tensor:  # numbers, lists (values are no key), anything to refuse
+        return _dot(t1, args, out_type, None)
     try:
-        key = ("dot", out_type, t1.type, t1.shape) + tuple([(a.type, a.shape) if a.__class__ is Tensor else tuple(a) for a in args])
+        key = ("dot", out_type, t1.type, t1.shape) + tuple([(a.type, a.shape) if a is t2 else tuple(a) for a in args])
         ready = _ready.get(key)
-    except (TypeError, AttributeError):  # numbers, axes that are no lists of integers: the general path and its checks
+    except TypeError:  # axes that are no lists of integers: the general path and its checks
         return _dot(t1, args, out_type, None)
     if ready is not None:
-        res = ready(t1, args[0] if len(args) == 1 else args[len(args) // 2])
+        res = ready(t1, t2)
         if res is not None:
             return res
     return _dot(t1, args, out_type, key)

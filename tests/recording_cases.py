@@ -236,5 +236,22 @@ def a_third_call_that_cannot_be_recorded_is_not_the_last_chance():
     assert f.replay is not None
 
 
+def a_lists_values_are_no_key():
+    """A contraction with a list of numbers is laid out for no one: the table neither grows with its values nor holds them."""
+    t = f32([1, 2], [3, 4])
+    Hip.dot, plain = classmethod(lambda cls, out, *args: out.with_(data=t.data)), Hip.dot.__func__
+    for i in range(20):
+        Nx.dot(t, [float(i), 1.0])
+        Nx.dot(t, np.array([1.0, float(i)], np.float32))
+        Nx.dot(t, [1], [float(i), 2.0], [0])
+    assert len(Nx._ready) == 0, list(Nx._ready)
+    for axes in ([1], (1,)):
+        Nx.dot(t, axes, t, axes)
+    assert len(Nx._ready) <= 1
+    # the plans that a call is laid out from may be gone, cleared by another thread
+    Hip.dot, Hip._dot_plans = classmethod(plain), {}
+    assert Hip.prepared("dot", "dot", t.with_(data=None), t, [1], [], t, [1], []) is None
+
+
 if __name__ == "__main__":
     globals()[sys.argv[1]]()
