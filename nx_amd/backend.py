@@ -678,19 +678,21 @@ class HipNxBackend:
         that way: the caller then makes the separate calls."""
         dev = cls._device_of(l, r)
         l, r = cls._from_nx(l, dev), cls._from_nx(r, dev)
-        key = (l.shape, l_axes, tuple(c1), r.shape, r_axes, tuple(c2), len(b1), out.type)
+        key = (l.type, l.shape, l_axes, tuple(c1), r.type, r.shape, r_axes, tuple(c2), len(b1), out.type)
         plan = cls._view_plans.get(key)
         if plan is None:
             if len(cls._view_plans) >= 4096:
                 cls._view_plans.clear()
             plan = cls._view_plans[key] = cls._plan_views(l.shape, l_axes, c1, r.shape, r_axes, c2, len(b1)) or ()
         if not plan or out.type[1] < 8:
-            raise L.HipNxError(L.EUNSUPPORTED, "dot_views: operands that are not strided matrices")
+            raise L.HipNxError(L.EUNSUPPORTED, "dot_views: operands that the kernels do not take where they lie")
         outer, inner, K, l_layout, M, l_strides, r_layout, N, r_strides = plan
         res = cls._alloc(out, dev)
         status = L.lib.hipnx_dot_strided(res.data.ref.ctx, T.code(l.type), T.code(r.type), _out_code(out.type), outer, inner, M, N, K,
                                          l_layout, r_layout, l_strides, r_strides, cls._handle(l), cls._handle(r), res.data.ref.handle)
         if status:
+            if status == L.EUNSUPPORTED:  # it follows from what is in the key: known from here on, before a result is allocated
+                cls._view_plans[key] = ()
             L.check(status)
         return res
 
@@ -1149,16 +1151,19 @@ class HipNxBackend:
         key = ("scores", id(layout), id(program), out.type, out.shape, l.type, l.shape, l_axes, r.type, r.shape, r_axes, *[t.type for t in inputs])
         cached = _fused_arrays.get(key)
         if cached is None or cached[0] is not layout or cached[1] is not program:
-            views = cls._plan_views(l.shape, l_axes, c1, r.shape, r_axes, c2, len(b1))
-            if views is None or views[3] != K_INNER or views[6] != K_INNER or views[7] != cols or l.type != r.type:
-                raise L.HipNxError(L.EUNSUPPORTED, "fused_scores: operands that are not rows of contiguous elements")
-            outer, inner, K, _, M, l_strides, _, _, r_strides = views
-            n, types = len(inputs), [l.type if i == at else t.type for i, t in enumerate(inputs)]
             if len(_fused_arrays) > 4096:
                 _fused_arrays.clear()
-            cached = _fused_arrays[key] = (layout, program, (C.c_int * n)(*[T.code(t) for t in types]), (C.c_int64 * n)(*[s[0] for s in strides]),
-                                           (C.c_int * n)(*[s[1] for s in strides]), (C.c_int64 * 6)(*l_strides, *r_strides),
-                                           (outer, inner, M, K), T.code(out.type), out.size * T.size_bytes(out.type), _packed(program))
+            views = cls._plan_views(l.shape, l_axes, c1, r.shape, r_axes, c2, len(b1))
+            if views is None or views[3] != K_INNER or views[6] != K_INNER or views[7] != cols or l.type != r.type:
+                cached = _fused_arrays[key] = (layout, program)
+            else:
+                outer, inner, K, _, M, l_strides, _, _, r_strides = views
+                n, types = len(inputs), [l.type if i == at else t.type for i, t in enumerate(inputs)]
+                cached = _fused_arrays[key] = (layout, program, (C.c_int * n)(*[T.code(t) for t in types]), (C.c_int64 * n)(*[s[0] for s in strides]),
+                                               (C.c_int * n)(*[s[1] for s in strides]), (C.c_int64 * 6)(*l_strides, *r_strides),
+                                               (outer, inner, M, K), T.code(out.type), out.size * T.size_bytes(out.type), _packed(program))
+        if len(cached) == 2:
+            raise L.HipNxError(L.EUNSUPPORTED, "fused_scores: operands that are not rows of contiguous elements, or extents that two calls are for")
         _, _, dts, rs, cs, operand_strides, extents, out_code, nbytes, prog_ptr = cached
         handles = (C.c_void_p * len(inputs))(*[cls._handle(t) for t in inputs])
         operands = (C.c_void_p * 2)(cls._handle(l), cls._handle(r))
@@ -1167,6 +1172,10 @@ class HipNxBackend:
         status = L.lib.hipnx_fused_scores(ctx, len(program), prog_ptr, len(inputs), handles, dts, rs, cs, cols, at, *extents, operand_strides,
                                           operands, out_code, ref.handle)
         if status:
+            # a refusal follows from what is in the key -- but for a program first met while capturing -- and is known from here
+            # on, before a result is allocated
+            if status == L.EUNSUPPORTED and wanted == "compiled" and dev not in _capturing:
+                _fused_arrays[key] = (layout, program)
             L.check(status)
         return out.with_(data=HipNxBackend(ref, dev))
 

@@ -253,5 +253,28 @@ def a_lists_values_are_no_key():
     assert Hip.prepared("dot", "dot", t.with_(data=None), t, [1], [], t, [1], []) is None
 
 
+def a_refused_attempt_is_not_made_again():
+    """What the library does not take at these extents is known from the first refusal on: no buffer is made for it again, and none
+    is part of a recording."""
+    q = from_numpy(np.ones((2, 4, 6, 8), np.float32), "f32", Hip)
+    out = q.with_(data=None, shape=(2, 6, 4, 4))
+    for _ in range(3):
+        raises(lambda: Hip.dot_views(out, q, (0, 2, 1, 3), [3], [0, 1], q, (0, 2, 1, 3), [3], [0, 1]), "")
+    assert standin.counts.get("hipnx_dot_strided") == 1
+    b = from_numpy(np.ones((2, 4, 6, 64), np.uint16), "bf16", Hip)
+    out = b.with_(data=None, type="f32", shape=(2, 6, 4, 4))
+    program, layout = defn._Program([{"kind": B.L.FUSED_SET, "src": B.L.FUSED_SRC_INPUT, "dt": ("f", 32)}]), (48, 4, [(4, 1)])
+    before = dict(standin.counts)
+    for _ in range(3):
+        raises(lambda: Hip.fused_scores(out, program, [b], layout, 0, (b, (0, 2, 1, 3), [3], [0, 1], b, (0, 2, 1, 3), [3], [0, 1]), mode="compiled"), "")
+    assert standin.counts["hipnx_fused_scores"] == 1 and standin.counts["hipnx_buf_alloc"] == before["hipnx_buf_alloc"] + 1
+    B._capturing.add(0)      # (a program is not compiled while capturing, whatever its extents)
+    program = defn._Program(program)
+    raises(lambda: Hip.fused_scores(out, program, [b], layout, 0, (b, (0, 2, 1, 3), [3], [0, 1], b, (0, 2, 1, 3), [3], [0, 1]), mode="compiled"), "")
+    B._capturing.discard(0)
+    raises(lambda: Hip.fused_scores(out, program, [b], layout, 0, (b, (0, 2, 1, 3), [3], [0, 1], b, (0, 2, 1, 3), [3], [0, 1]), mode="compiled"), "")
+    assert standin.counts["hipnx_fused_scores"] == 3
+
+
 if __name__ == "__main__":
     globals()[sys.argv[1]]()
