@@ -55,6 +55,7 @@ typedef struct {
 } Ref;
 
 static void ref_dealloc(Ref *self) {
+  PyObject_GC_UnTrack(self);
   if (self->handle && buf_destroy) {
     if (is_recording()) {
       PyObject *h = PyLong_FromVoidPtr(self->handle);
@@ -92,21 +93,36 @@ static int ref_init(Ref *self, PyObject *args, PyObject *kw) {
   return 0;
 }
 
+/* The owner of borrowed memory may lead back here (an object that holds the tensor it lends its memory to). */
+static int ref_traverse(Ref *self, visitproc visit, void *arg) {
+  Py_VISIT(self->ctx);
+  Py_VISIT(self->keep);
+  return 0;
+}
+static int ref_clear(Ref *self) {
+  PyObject *keep = self->keep;
+  Py_INCREF(Py_None);
+  self->keep = Py_None;
+  Py_XDECREF(keep);
+  return 0;
+}
+
 static PyObject *ref_get_handle(Ref *self, void *unused) { return PyLong_FromVoidPtr(self->handle); }
 static PyMemberDef ref_members[] = {{"ctx", T_OBJECT, offsetof(Ref, ctx), READONLY, NULL},
-                                    {"keep", T_OBJECT, offsetof(Ref, keep), 0, NULL},
+                                    {"keep", T_OBJECT, offsetof(Ref, keep), READONLY, NULL},
                                     {"nbytes", T_PYSSIZET, offsetof(Ref, nbytes), READONLY, NULL},
                                     {"sharers", T_PYSSIZET, offsetof(Ref, sharers), 0, NULL},
                                     {NULL}};
 static PyGetSetDef ref_getset[] = {{"handle", (getter)ref_get_handle, NULL, "the hipnx_buf pointer", NULL}, {NULL}};
 static PyTypeObject RefType = {PyVarObject_HEAD_INIT(NULL, 0).tp_name = "hipnx_calls.Ref", .tp_basicsize = sizeof(Ref),
-                               .tp_flags = Py_TPFLAGS_DEFAULT, .tp_new = PyType_GenericNew, .tp_init = (initproc)ref_init,
-                               .tp_dealloc = (destructor)ref_dealloc, .tp_members = ref_members, .tp_getset = ref_getset,
+                               .tp_flags = Py_TPFLAGS_DEFAULT | Py_TPFLAGS_HAVE_GC, .tp_new = PyType_GenericNew, .tp_init = (initproc)ref_init,
+                               .tp_traverse = (traverseproc)ref_traverse, .tp_clear = (inquiry)ref_clear, .tp_dealloc = (destructor)ref_dealloc, .tp_members = ref_members, .tp_getset = ref_getset,
                                .tp_doc = "Owns one device buffer; shared by metadata-only callbacks."};
 
 static Ref *new_ref(PyObject *ctx, void *handle, Py_ssize_t nbytes) {
   Ref *r = (Ref *)RefType.tp_alloc(&RefType, 0);
   if (!r) return NULL;
+  PyObject_GC_UnTrack(r); /* it owns its memory: nothing for the collector to follow */
   Py_INCREF(ctx);
   r->ctx = ctx;
   Py_INCREF(Py_None);

@@ -276,5 +276,22 @@ def a_refused_attempt_is_not_made_again():
     assert standin.counts["hipnx_fused_scores"] == 3
 
 
+def a_lender_that_holds_what_it_lent_to_is_collected():
+    import gc
+    import weakref
+
+    class Lender:
+        pass
+    owner = f32(1, 2, 4)
+    lender = Lender()
+    lender.tensor = Nx.from_pointer(Hip, Nx.Pointer(kind="local", address=Nx.to_pointer(owner).address, data_size=12), "f32", (3,), keep=lender)
+    assert read(lender.tensor) == [1, 2, 4]
+    gone, handles = weakref.ref(lender), len(standin.memory)
+    del lender
+    gc.collect()
+    assert gone() is None and len(standin.memory) == handles - 1
+    assert read(owner) == [1, 2, 4]
+
+
 if __name__ == "__main__":
     globals()[sys.argv[1]]()
