@@ -1213,7 +1213,7 @@ def test_a_dot_reads_transposed_operands_where_they_lie(batch, heads, queries, k
 
 
 def test_other_orders_of_a_dots_operands(hip, oracle):
-    """Operands whose kept or contracted axes are not neighbours, three batch axes, a transposed operand with a second reader."""
+    """Operands whose kept or contracted axes are not neighbours, batch axes in two orders, a transposed operand with a second reader."""
     rng = np.random.default_rng(77)
     a, b = rand_float(rng, "bf16", (4, 32, 6, 64), hip), rand_float(rng, "bf16", (6, 4, 48, 64), hip)
 
@@ -1561,3 +1561,172 @@ def test_scores_that_are_left_to_the_contraction(ty, hip):
         assert_bits_equal(planned(q, k), defn.compile(fun, q, k)(q, k), "nearest even")
     finally:
         B.bf16_rounding(previous)
+
+
+def test_a_dot_over_three_batch_axes(hip):
+    """Batches that fold to two axes are read where they lie, others are copied: the same bits."""
+    rng = np.random.default_rng(78)
+    x, y = rand_float(rng, "bf16", (2, 3, 20, 4, 64), hip), rand_float(rng, "bf16", (2, 3, 24, 4, 64), hip)
+    z, w = rand_float(rng, "f32", (3, 20, 2, 4, 32), hip), rand_float(rng, "f32", (4, 3, 2, 24, 32), hip)
+
+    def heads_last(a, b):     # batch axes 0 and 1 are neighbours, the third lies behind the rows
+        return Nx.dot(Nx.transpose(a, axes=[0, 1, 3, 2, 4]), [4], [0, 1, 2], Nx.transpose(b, axes=[0, 1, 3, 2, 4]), [4], [0, 1, 2])
+
+    def all_apart(a, b):      # no two of them are neighbours in the same order on either side
+        return Nx.dot(Nx.transpose(a, axes=[2, 0, 3, 1, 4]), [4], [0, 1, 2], Nx.transpose(b, axes=[2, 1, 0, 3, 4]), [4], [0, 1, 2])
+    for fun, args in ((heads_last, (x, y)), (all_apart, (z, w))):
+        planned = defn.compile(fun, *args, fuse="compiled")
+        assert planned.roots[0].data.op == "dot_views"
+        for _ in range(4):  # (the last one from its recording)
+            assert_bits_equal(planned(*args), defn.compile(fun, *args)(*args), fun.__name__)
+        assert planned.replay is not None
+
+
+# both layouts on either side; rows, and items of the two batch axes, any number of elements apart
+@pytest.mark.parametrize("ty", ["bf16", "f16", "f32", "s8"])
+@pytest.mark.parametrize("layouts", ["nn", "nt", "tn", "tt"])
+@pytest.mark.parametrize("M,N,K,gap", [(32, 48, 64, 1), (144, 272, 128, 3), (272, 528, 208, 8), (64, 1040, 1072, 5)])
+def test_strided_operands_lie_anywhere(M, N, K, gap, layouts, ty, hip):
+    """Whole numbers, exact in any order.  What is between the rows is no operand: numbers that would show."""
+    from nx_amd import types as T
+    from nx_amd.backend import K_INNER, K_OUTER
+    rng = np.random.default_rng(seed_of(M, N, K, gap, layouts, ty))
+    outer, inner = 2, 3
+
+    def operand(rows, k_inner):
+        runs, run = (rows, K) if k_inner else (K, rows)
+        ld = run + gap
+        item = runs * ld + gap
+        strides = (inner * item + gap, item, ld)
+        v = np.full(outer * strides[0] + gap, 77.0, np.float32)
+        values = rng.integers(-2, 3, size=(outer, inner, runs, run)).astype(np.float32)
+        for o in range(outer):
+            for i in range(inner):
+                np.lib.stride_tricks.as_strided(v[o * strides[0] + i * item:], (runs, run), (4 * ld, 4))[:] = values[o, i]
+        held = (v.view(np.uint32) >> 16).astype(np.uint16) if ty == "bf16" else v.astype({"f16": np.float16, "f32": np.float32, "s8": np.int8}[ty])
+        return from_numpy(held, ty, hip), L.i64_array(strides), values if k_inner else values.transpose(0, 1, 3, 2), K_INNER if k_inner else K_OUTER
+    l, ls, a, l_layout = operand(M, layouts[0] == "n")
+    r, rs, b, r_layout = operand(N, layouts[1] == "t")
+    ot = T.normalize("s32" if ty == "s8" else "f32")
+    out = from_numpy(np.zeros((outer, inner, M, N), np.int32 if ty == "s8" else np.float32), ot, hip)
+    code = T.code(T.normalize(ty))
+    L.check(L.lib.hipnx_dot_strided(_Context.get(0), code, code, T.code(ot), outer, inner, M, N, K, l_layout, r_layout, ls, rs,
+                                    l.data.ref.handle, r.data.ref.handle, out.data.ref.handle))
+    np.testing.assert_array_equal(hip.to_numpy(out).astype(np.float64), a.astype(np.float64) @ b.astype(np.float64).transpose(0, 1, 3, 2))
+
+
+@pytest.mark.parametrize("fuse", [False, True, "compiled"])
+def test_a_recorded_function_tells_its_numbers_from_its_arguments(fuse, hip):
+    """A rate given as an argument, equal to a number of the function while it is recorded."""
+    x = rand_float(np.random.default_rng(4), "f32", (12, 16), hip)
+
+    def fun(t, rate):
+        return Nx.subtract(t, Nx.multiply(Nx.exp(t), rate)), Nx.add(t, 0.5), Nx.max(t, rate)
+    previous = Nx.default_backend(hip)  # (where numbers go)
+    try:
+        planned, plain = defn.compile(fun, x, 0.5, fuse=fuse), defn.compile(fun, x, 0.5)
+        for rate in (0.5, 0.5, 0.5, 0.5, 2.0, 0.25, 0.5):
+            for g, w in zip(planned(x, rate), plain._walk([x, Nx.to_tensor(rate)])):
+                assert_bits_equal(g, w, f"rate {rate}")
+        assert planned.replay is not None
+    finally:
+        Nx.default_backend(*previous)
+
+
+def groups_and_operands(hip):
+    rng = np.random.default_rng(17)
+    key = Random.key(3, backend=hip)
+    q, k = rand_float(rng, "bf16", (2, 40, 128), hip), rand_float(rng, "bf16", (2, 72, 128), hip)
+    ragged = rand_float(rng, "f32", (37, 185), hip), rand_float(rng, "f32", (185,), hip)
+    return {"words": (lambda kk: Random.normal(kk, shape=(1001,))[0], (key,)), "scores": (lambda a, b: attention_probabilities(a, b, 2), (q, k)),
+            "ragged rows": (centred_and_scaled, ragged), "ragged sums": (lambda a, b: Nx.sum(Nx.exp(Nx.add(a, b)), axes=[1]), ragged)}
+
+
+@pytest.mark.parametrize("met", ["inside the capture", "before the capture"])
+@pytest.mark.parametrize("name", ["words", "scores", "ragged rows", "ragged sums"])
+def test_groups_met_inside_a_capture(name, met, hip):
+    """A group that a capture meets first is evaluated without its kernel there, one met before with it: every replay gives the bits
+    of the evaluator, on new operands too, with work of its own between the replays.  (Scores on whole numbers: the kernel
+    that contracts them adds in another order.)"""
+    from nx_amd import backend as B
+    fun, args = groups_and_operands(hip)[name]
+
+    def fresh(i):
+        out = []
+        for t in args:
+            v = np.roll(hip.to_numpy(t), i + 1, axis=0)
+            if name == "scores":
+                v = np.random.default_rng(i).integers(-2, 3, size=t.shape).astype(np.float32)
+                v = (v.view(np.uint32) >> 16).astype(np.uint16)
+            out.append(from_numpy(v + np.uint32(i) if name == "words" else v, t.type, hip))
+        return out
+    held = fresh(0)
+    planned, plain = defn.compile(fun, *args, fuse="compiled"), defn.compile(fun, *args)
+    if met == "before the capture":
+        for _ in range(2):
+            planned._walk(held)
+    plain._walk(held)  # (the pool has the blocks that a capture takes)
+    B.sync()
+    B.capture_begin(0)
+    try:
+        results = planned._evaluate(held)
+    finally:
+        graph = B.capture_end(0)
+    try:
+        for i in (1, 2, 1, 3):
+            now = fresh(i)
+            for h, n in zip(held, now):
+                B.copy_into(h, n)
+            graph.launch()
+            for g, w in zip(results, plain._walk(now)):
+                assert_bits_equal(g, w, f"{name}, replay {i}")
+            B.sync()
+    finally:
+        graph.destroy()
+
+
+# K of one to eight steps of 32, whole and partial slabs of the contraction's own kernel; every form of the row, odd queries
+@pytest.mark.parametrize("ty", ["bf16", "f16"])
+@pytest.mark.parametrize("queries,keys,K", [(17, 64, 32), (16, 100, 96), (40, 300, 96), (33, 513, 64), (31, 1000, 160), (20, 1001, 256), (64, 776, 128), (1, 272, 64)])
+def test_contracted_scores_are_rounded_sums(queries, keys, K, ty, hip):
+    """The scores themselves, carried out of the kernel (halves, less nothing of their row's maximum).  Each is the operands' type's rounding (bf16 drops the
+    low bits, f16 rounds to nearest: both rise with their argument) of an f32 sum of K exact products, which is at most K * 2^-24
+    of the sum of their magnitudes away from the exact one: it lies between the roundings of the ends of that range."""
+    rng = np.random.default_rng(seed_of(queries, keys, K, ty, "rounded"))
+    heads = 2
+    batch = 2 if keys * K <= 65536 else 128 // ((queries + 15) // 16)  # (over a large right operand: blocks for every CU)
+    q, k = rand_float(rng, ty, (batch, queries, heads * K), hip), rand_float(rng, ty, (batch, keys, heads * K), hip)
+
+    def fun(a, b):
+        s = Nx.dot(split_heads(a, heads), [3], [0, 1], split_heads(b, heads), [3], [0, 1])
+        half = Nx.multiply(Nx.as_type(s, "f32"), 0.5)
+        return Nx.subtract(half, Nx.multiply(Nx.reduce_max(half, axes=[-1], keep_axes=True), 0.0))
+    planned = defn.compile(fun, q, k, fuse="compiled")
+    assert planned.roots[0].data.args[0].scores is not None
+    calls, original = [], hip.fused_scores.__func__
+
+    def counting(cls, *a, **kw):
+        out = original(cls, *a, **kw)
+        calls.append(1)
+        return out
+    hip.fused_scores = classmethod(counting)
+    try:
+        got = 2.0 * hip.to_numpy(planned(q, k)).astype(np.float64)
+    finally:
+        hip.fused_scores = classmethod(original)
+    assert calls == [1]
+
+    def heads_of(t):
+        v = Nx.to_float64(t).reshape(t.shape[0], t.shape[1], heads, K)
+        return v.transpose(0, 2, 1, 3)
+    a, b = heads_of(q), heads_of(k).transpose(0, 1, 3, 2)
+    exact, away = a @ b, K * 2.0 ** -24 * (np.abs(a) @ np.abs(b))
+
+    def rounded(v):
+        v = v.astype(np.float32)
+        return (v.view(np.uint32) & np.uint32(0xFFFF0000)).view(np.float32) if ty == "bf16" else v.astype(np.float16)
+    lo, hi = rounded(exact - away).astype(np.float64), rounded(exact + away).astype(np.float64)
+    assert (lo <= got).all() and (got <= hi).all(), (np.abs(got - exact).max(), int(((got < lo) | (got > hi)).sum()))
+    # the range is 2 K 2^-24 * 0.64 K wide on these operands, at most two thirds of a unit of the results around sqrt(K) (f16, K = 256): a
+    # quarter of them and more are decided to the bit, the others to a unit
+    assert (lo == hi).mean() > 0.25
