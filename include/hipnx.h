@@ -263,7 +263,8 @@ int hipnx_dot(hipnx_ctx *ctx, int l_dt, int r_dt, int out_dt, int64_t batch, int
  * first batch axis, along the second, and from row to row (HIPNX_K_INNER: the K elements of a row are contiguous) or from k to k
  * (HIPNX_K_OUTER: the rows are).  The heads of [batch, positions, heads, dim] are {positions * heads * dim, dim, heads * dim}.
  * The bits are those of the two calls.  Contractions on the matrix cores whose operands can be read as they lie (K of
- * whole 16-byte pieces, K-outer rows of whole blocks); anything else is HIPNX_EUNSUPPORTED: copy, then hipnx_dot. */
+ * whole 16-byte pieces, K-outer rows of whole blocks; any strides and addresses); anything else -- among it few outputs over a long K,
+ * which hipnx_dot sums in f64 -- is HIPNX_EUNSUPPORTED: copy, then hipnx_dot. */
 int hipnx_dot_strided(hipnx_ctx *ctx, int l_dt, int r_dt, int out_dt, int64_t batch_outer, int64_t batch_inner, int64_t M, int64_t N,
                       int64_t K, int l_layout, int r_layout, const int64_t *l_strides, const int64_t *r_strides, const hipnx_buf *l,
                       const hipnx_buf *r, hipnx_buf *out);
@@ -447,7 +448,9 @@ int hipnx_fused_words(hipnx_ctx *ctx, int n_instr, const hipnx_fused_instr *prog
  * columns (the scores of an attention under their softmax).  strides: {first batch axis, second, row} of the left operand, then of
  * the right one; operands: the two buffers; inputs[scores] is not looked at.  K of 32 to 256 in whole steps of 32, at most 4096
  * columns, HIPNX_FUSED_COMPILED; anything else, and shapes that are faster in two calls, are HIPNX_EUNSUPPORTED.  A sum over K is
- * added in order of k in f32, rounded to the operands' type once. */
+ * added in order of k in f32, rounded to the operands' type once; hipnx_dot may add the same products in another order and round some
+ * sums to the neighbouring number.  A stage's sum along the row is added in f64, in an order of this entry point's own, the same for every
+ * call of the same extents. */
 int hipnx_fused_scores(hipnx_ctx *ctx, int n_instr, const hipnx_fused_instr *prog, int n_inputs, const hipnx_buf *const *inputs,
                        const int *in_dts, const int64_t *in_row_strides, const int *in_col_strides, int64_t cols, int scores,
                        int64_t batch_outer, int64_t batch_inner, int64_t M, int64_t K, const int64_t *strides,
@@ -459,7 +462,7 @@ int hipnx_fused_scores(hipnx_ctx *ctx, int n_instr, const hipnx_fused_instr *pro
  * out over the same device functions, compiled for the device once by the run-time compiler (a few
  * hundred milliseconds) and kept with the context -- the role exla/lib/exla/defn.ex's compilation
  * cache plays for a whole function, here for one element-wise group.  Results are bit-identical in
- * both modes.  A program first met while the context is capturing runs interpreted in that capture (one that exists only
+ * both modes (hipnx_fused_words and hipnx_fused_scores exist compiled only).  A program first met while the context is capturing runs interpreted in that capture (one that exists only
  * compiled is refused there: HIPNX_EUNSUPPORTED).  A program of stages that keeps an input or values of its rows in registers
  * is compiled once per number of 512-element steps (2048 above 4096 elements, up to 32768) in a row, and per way that rows
  * which are not whole vectors of eight, or shorter than 512 elements, are divided among lanes; a capture that meets

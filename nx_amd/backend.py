@@ -1139,7 +1139,8 @@ class HipNxBackend:
     def fused_scores(cls, out: Tensor, program, inputs, layout, at: int, dot, mode=None) -> Tensor:
         """`fused_elementwise` for a program of stages whose input number `at` is the contraction `dot` = (left, its axes,
         contracted axes, batch axes, right, its axes, contracted axes, batch axes; see `dot_views`): its result is made
-        inside the kernel and never stored.  Raises HipNxError with status EUNSUPPORTED where the two calls have to be made."""
+        inside the kernel and never stored.  The sums over K and along the rows are added in orders of the kernel's own: a score may be the
+        neighbouring number of its type, and a sum along a row differ in its last bit.  Raises HipNxError with status EUNSUPPORTED where the two calls have to be made."""
         l, l_axes, c1, b1, r, r_axes, c2, b2 = dot
         dev = cls._device_of(l, r)
         if any(t.data.__class__ is not HipNxBackend for t in inputs) or r.data.__class__ is not HipNxBackend or _bf16["rounding"] != "truncate":
@@ -1410,7 +1411,8 @@ _settings_changed()
 def fused_mode(mode: str, device: int = 0) -> None:
     """How fused groups run on the device from now on: "interpreted" (one pair of kernels decodes any
     program; the default) or "compiled" (each distinct program is compiled for the device once, on
-    first use, and kept).  Results are bit-identical."""
+    first use, and kept).  Results are bit-identical.  (A function planned with fuse="compiled" gives the bits of its nodes run one by
+    one, but where a contraction's scores are made inside the stages that read them: `fused_scores`.)"""
     _set_fused_mode(mode, device)
     _fused_modes[device] = mode
     _settings_changed()

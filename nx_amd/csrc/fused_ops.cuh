@@ -193,7 +193,8 @@ struct RowVector {
 };
 
 // How the lanes of a row share it (P::form).  In every form a lane meets its elements in the order in which the separate
-// reduction of rows of that length folds them (reduce_rows_kernel and its short-row forms).
+// reduction of rows of that length folds them (reduce_rows_kernel and its short-row forms) -- but for the rows of contracted
+// scores, which may have fewer lanes (share_row, fused_rtc.hip): a sum along them is added in an order of its own.
 //   ROW_WHOLE: rows of whole vectors; lane l takes the vectors l, l + tpr, ...
 //   ROW_LANE: rows of at most 16 elements; a lane takes a row (tpr = 1): its vectors, then the P::tail elements behind them.
 //   ROW_GROUP: rows of 17 to 256 elements that are not whole vectors; 8, 16 or 32 lanes, so that each has one vector at most;
@@ -266,9 +267,11 @@ __device__ __forceinline__ void fetch_static(KernArgs a, const Saved &S, const R
 }
 
 // Exponentials over one value of their row (a softmax's last stage) in programs of a few vectors a lane, which vector instructions
-// bound: x / y by the correctly rounded reciprocal r of y, q = x r, q + r (x - q y) -- the last two fused -- is the correctly rounded
-// quotient while nothing leaves the normal numbers: every 24-bit x against 2000 24-bit y, and 3 10^8 random pairs over the ranges tested
-// below, give division's bits.  Three instructions an element and two for the test instead of seventeen slots.  (With more
+// bound: x / y by Markstein's corrected quotient: the correctly rounded reciprocal r of y, q = x r, q + r (x - q y), the last two fused.
+// The correction is at most 1.5 units of q and wrong by 2^-24 of itself, its residual by a unit of the product's last place: the result can
+// miss the correctly rounded quotient only where x / y lies within 5 / (2 y) units (y as a 24-bit integer) of a midpoint between
+// two numbers.  All 4.6 10^7 pairs of 24-bit significands within 8 / (2 y) were tried: each gives division's bits.  (While nothing
+// leaves the normal numbers: the ranges tested below.)  Three instructions an element and two for the test instead of seventeen slots.  (With more
 // vectors a lane the branch costs the overlap of their trips: f32 8192 x 32000, sixteen vectors, 385 -> 539 us.)
 template <typename P, int PC>
 constexpr bool divides_exponentials() {

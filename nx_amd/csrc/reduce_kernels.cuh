@@ -271,7 +271,7 @@ reduce_cols_kernel(const void *__restrict__ in, void *__restrict__ out, typename
 // work-group of 1024 lanes takes X adjacent columns, its 1024 / X rows of lanes a run of the reduced axis each, eight loads in
 // flight, and the runs are folded in order in LDS.  Bound by latency: four round trips of a lane and ten steps in LDS.  (One lane
 // per column walked all of it, or it was two launches; us per call, then / now: f32 [48, 3] 12.2 / 3.5, [144, 915] 16.7 / 3.7,
-// [2048, 8] 9.4 / 4.0, [4000, 100] 23.2 / 5.8, [2000, 2000] 9.4 / 6.3.)
+// [2048, 8] 9.4 / 4.0, [4000, 100] 23.2 / 5.8, [2000, 2000] 9.4 / 6.3, each on an input that was read just before.)
 constexpr int COLS_ONCE = 1024;
 constexpr int cols_once_run = 32;  // rows of a lane at most
 inline int cols_once_x(int64_t red, int64_t inner) {  // the widest group that covers the axis
@@ -471,7 +471,8 @@ static int run_reduce_t(hipnx_ctx *ctx, bool static_ws, int idt, int odt, int64_
   } else {
     if constexpr (IDT >= 0 && IDT != HIPNX_F64 && std::is_floating_point<CT>::value) {
       // (more work-groups than this and the kernel below, whose lanes have eight columns each, gives the chip its waves in longer
-      // runs of memory; with eight columns to a work-group that is sooner: f32 [4096, 1000] 11.5 us here, 9.3 there; [4096, 512] 6.1, 9.6)
+      // runs of memory; with eight columns to a work-group that is sooner: f32 [4096, 1000] 11.5 us here, 9.3 there; [4096, 512] 6.1, 9.6 on
+      // an input read just before.  Behind the pass that wrote it the latter takes 10.3 us here and 6.5 + 4.1 there: one launch less)
       const int X = cols_once_x(red, inner);
       const int64_t groups = (inner + X - 1) / X;
       if (red > 0 && red <= cols_once_run * (COLS_ONCE / X) && outer <= 65535 && outer * groups <= (X == 8 ? 64 : 128)) {
