@@ -1638,6 +1638,10 @@ class _Run:
         return self.backend[0] if mod is HostBinary else mod
 
 
+_BACKEND = __package__ + ".backend"
+_evaluate_on_device = None  # replay.evaluate, once there are operands for it
+
+
 class Compiled:
     """A traced function: call it with arguments of the traced shapes and types."""
 
@@ -1666,11 +1670,16 @@ class Compiled:
             results = self.replay.run(params)
             if results is not None:
                 return results
-        backend = sys.modules.get(__package__ + ".backend")
-        if backend is not None and not backend._capturing and all(p.data.__class__ is backend.HipNxBackend for p in params):
-            from .replay import evaluate
-            return evaluate(self, params)
-        return self._walk(params)
+        device = getattr(sys.modules.get(_BACKEND), "HipNxBackend", None)
+        for p in params:
+            if p.data.__class__ is not device:
+                return self._walk(params)
+        if not params:
+            return self._walk(params)
+        global _evaluate_on_device
+        if _evaluate_on_device is None:
+            from .replay import evaluate as _evaluate_on_device
+        return _evaluate_on_device(self, params)
 
     def _walk(self, params):
         run = _Run(self.plans, _runtime_backend(params))

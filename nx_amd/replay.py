@@ -148,6 +148,8 @@ class _History:
 def evaluate(compiled, params):
     """An evaluation of `compiled` on operands of the device backend that its present recording, if any, did not answer: by the
     recording of the present settings, or the general way, writing it down if it is time to."""
+    if B._capturing:
+        return compiled._walk(params)
     mod, opts = Nx.default_backend()
     key = (B.settings(), mod, repr(opts))
     known = compiled.recordings.get(key)
