@@ -3,10 +3,8 @@
 //
 //   bf16 / f16 / f32 operand pairs (f32 accumulation) and s8 pairs (exact s32 accumulation):
 //     the MFMA kernels (gemm_mfma.cuh, gemm_pingpong.cuh), which take both operand layouts and any K directly
-//       (a partial slab of K is walked with zeros behind its end).  What they cannot take is first copied: a K-outer
-//       operand whose row count is not a multiple of its transpose block (16 s8 / 8 bf16,f16 / 4 f32 rows) by the
-//       tiled transpose, a K-inner one whose rows are not whole 16-byte pieces to rows that are -- where the
-//       contraction is large enough to pay for it (16 M multiply-adds).
+//       (a partial slab of K is walked with zeros behind its end; rows and k-rows need not be whole 16-byte pieces).  What
+//       is shorter than a piece is first copied, and K-inner rows on no dword that many tiles re-read (rows_worth_copying).
 //   everything else (f64 whose K is not whole slabs, wide integers, mixed operand types, fewer than 256 outputs, and below
 //     16 M multiply-adds a float K that is not whole 16-byte pieces, in every layout): dot_generic_kernel,
 //     a plain tiled kernel accumulating in f64 or wrapping 64-bit integers, K cut into segments where few outputs would leave
@@ -302,6 +300,26 @@ splitk_combine_kernel(const AT *__restrict__ part, void *__restrict__ out, int o
   }
 }
 
+// Whether a K-inner operand is copied to rows of whole pieces though the kernels take its rows as they lie.  Sixteen bytes at an
+// address that is no multiple of four cost a CU three times its intake of aligned ones (measured from L2: 30 TB/s aligned, 18
+// with rows on any multiple of four -- never worth a copy --, 15 on any multiple of two, 11.7 on any byte), which a tile pays per
+// slab where its multiplications do not cover it; a copy costs a launch and reads and writes the operand once.  So the
+// operand that many tiles re-read is copied, the long one that few do is not.  us per call, both copied / neither / by this rule:
+// int8 512 x 11007 x 11005 142 / 157 / 119, 512 x 1001 x 11006 56 / 66 / 53, 128 x 11007 x 4094 43 / 32 / 29; bf16 168 x 4000 x 1597
+// 25.3 / 25.7 / 21.1.
+static bool rows_worth_copying(const hipnx_ctx *ctx, int dt, int64_t batch, int64_t M, int64_t N, int64_t row_bytes, bool right) {
+  if (row_bytes % 4 == 0) return false;
+  const bool big = M >= 192 && N >= 192 && ((M + 255) / 256) * ((N + 255) / 256) * batch * 4 >= (int64_t)ctx->num_cus * 3;
+  const int bm = M <= 64 ? 64 : big ? 256 : 128, bn = M <= 64 ? 64 : big ? 256 : 128;
+  const int64_t groups = ((M + bm - 1) / bm) * ((N + bn - 1) / bn) * batch, slabs = (row_bytes + SLAB - 1) / SLAB;
+  const double intake = 78e3, flops = 7.8e6;  // bytes and 2-byte multiply-adds x 2 a CU takes per us
+  const double aligned = (double)(bm + bn) * SLAB / intake, side = (double)(right ? bn : bm) * SLAB / intake * (row_bytes % 2 ? 1.4 : 0.85);
+  const double work = (double)bm * bn * SLAB / (dt == HIPNX_F32 ? 0.5 : 1.0) / flops;
+  const double extra = (double)((groups + ctx->num_cus - 1) / ctx->num_cus) * (double)slabs * std::max(0.0, aligned + side - std::max(aligned, work));
+  const double copy = 2.5 + (double)batch * (double)(right ? N : M) * (double)row_bytes * 2.0 / 4.5e6;
+  return extra > copy;
+}
+
 // A K-inner operand ([rows, K]) copied to rows of whole 16-byte pieces.
 static int pad_rows(hipnx_ctx *ctx, int esz, int64_t rows, int64_t K, const hipnx_buf *in, hipnx_buf **out) {
   const int64_t pieces = (K * esz + 15) / 16;
@@ -363,10 +381,12 @@ static int dot_impl(hipnx_ctx *ctx, int l_dt, int r_dt, int out_dt, int64_t batc
     return HIPNX_OK;
   }
   bool mfma = false, l_pad = false, r_pad = false;
-  // the MFMA kernels transpose K-outer operands themselves when the rows come in whole blocks
+  // the MFMA kernels transpose K-outer operands themselves, k-rows that are not whole pieces too (not f64: its last slab would
+  // have to be walked first, and it adds over k in order), but for k-rows shorter than one
   const int row_block = dtype_size(l_dt) == 1 ? 16 : dtype_size(l_dt) == 2 ? 8 : dtype_size(l_dt) == 4 ? 4 : 2;
-  const bool l_relay = l_layout == HIPNX_K_OUTER && M % row_block != 0;
-  const bool r_relay = r_layout == HIPNX_K_OUTER && N % row_block != 0;
+  const bool l_ragged = l_layout == HIPNX_K_OUTER && M % row_block != 0, r_ragged = r_layout == HIPNX_K_OUTER && N % row_block != 0;
+  const bool l_relay = l_ragged && (M < row_block || l_dt == HIPNX_F64);
+  const bool r_relay = r_ragged && (N < row_block || l_dt == HIPNX_F64);
   {
     Enter in(ctx);
     if (in.status) return in.status;
@@ -379,7 +399,7 @@ static int dot_impl(hipnx_ctx *ctx, int l_dt, int r_dt, int out_dt, int64_t batc
     if (int st = check_buf(ctx, r, (uint64_t)batch * N * K * dtype_size(r_dt), "dot rhs")) return st;
     if (int st = check_buf(ctx, out, (uint64_t)batch * M * N * out_dtype_size(out_dt), "dot out")) return st;
     if (batch * M * N == 0) return HIPNX_OK;
-    if (view && (l_relay || r_relay || K * dtype_size(l_dt) % 16 != 0))
+    if (view && (l_ragged || r_ragged || K * dtype_size(l_dt) % 16 != 0))
       return set_error(HIPNX_EUNSUPPORTED, "dot_strided: operands that the kernels cannot take as they lie");
     if (batch > 65535) return set_error(HIPNX_EUNSUPPORTED, "dot: more than 65535 batch items");
 
@@ -390,13 +410,15 @@ static int dot_impl(hipnx_ctx *ctx, int l_dt, int r_dt, int out_dt, int64_t batc
     mfma = (float_pair || int8_pair) && K > 0 && M * N >= 256;
     if (mfma && l_dt == HIPNX_F64) mfma = row_bytes % SLAB == 0;  // (f64 otherwise adds over k in order, on the plain kernels)
     else if (mfma && row_bytes % 16 != 0) {
-      // rows that are not whole pieces: only a K-inner operand minds, and a copy of it is worth a launch from 16 M
-      // multiply-adds on.  Below that floats are summed in f64 on the plain kernels whatever the layout (two K-outer
-      // operands need no copy, but their sums would be f32 where the same product stored otherwise has f64); int8 is
-      // exact on either.
-      l_pad = l_layout == HIPNX_K_INNER || l_relay;
-      r_pad = r_layout == HIPNX_K_INNER || r_relay;
+      // rows that are not whole pieces: below 16 M multiply-adds floats are summed in f64 on the plain kernels, whatever the
+      // layout; int8 is exact on either.  Rows shorter than a piece are copied to one.
+      l_pad = row_bytes < 16 && (l_layout == HIPNX_K_INNER || l_relay);
+      r_pad = row_bytes < 16 && (r_layout == HIPNX_K_INNER || r_relay);
       if (l_pad || r_pad || l_dt != HIPNX_S8) mfma = (double)M * (double)N * (double)K * (double)batch >= 16777216.0;
+      if (mfma && row_bytes >= 16) {
+        l_pad = l_layout == HIPNX_K_INNER && !l_relay && rows_worth_copying(ctx, l_dt, batch, M, N, row_bytes, false);
+        r_pad = r_layout == HIPNX_K_INNER && !r_relay && rows_worth_copying(ctx, l_dt, batch, M, N, row_bytes, true);
+      }
     }
     if (scaled) {
       if (!(int8_pair && mfma && (any_k || row_bytes % SLAB == 0))) return set_error(HIPNX_EUNSUPPORTED, "dot_scaled: s8 x s8 with K a multiple of 128 and at most 65536, M * N >= 256");
@@ -575,8 +597,10 @@ static int dot_impl(hipnx_ctx *ctx, int l_dt, int r_dt, int out_dt, int64_t batc
         a.ld_r = view->ld_r, a.bs_r = view->bs_r, a.ts_r = view->ts_r;
         a.batch_inner = (int)view->inner;
       }
-      a.tail_l = (int)(l_kin ? (over + 15) / 16 * 16 : over / esz);
-      a.tail_r = (int)(r_kin ? (over + 15) / 16 * 16 : over / esz);
+      // (the last k-row of a ragged K-outer operand is read with care, which the walk does for a partial slab only)
+      const int64_t last = over == 0 && ((l_ragged && !l_relay) || (r_ragged && !r_relay)) ? SLAB : over;
+      a.tail_l = (int)(!l_kin ? last / esz : l_pad ? (last + 15) / 16 * 16 : last);
+      a.tail_r = (int)(!r_kin ? last / esz : r_pad ? (last + 15) / 16 * 16 : last);
       a.scale = scale_mode != HIPNX_SCALE_NONE ? (const float *)scale->ptr : nullptr;
       a.scale_mode = scale_mode;
       // tile choice: the largest tile that still gives every CU work; few rows against a long

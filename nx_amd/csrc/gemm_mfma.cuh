@@ -118,6 +118,24 @@ __device__ __forceinline__ void lds_dma16(const unsigned char *g, unsigned char 
 // behind the operands holds.
 static __device__ __attribute__((aligned(16))) const unsigned g_zero16[4] = {0, 0, 0, 0};
 
+// The last `rem` (1 .. 15) of the 16 bytes that end at `end`, moved to the front, zeros behind them: the end of a row that is not
+// whole pieces.  One load that lies inside the row, whatever is behind it (the row has sixteen bytes, the host sees to it).
+__device__ __forceinline__ v4i row_end_piece(const unsigned char *end, int rem) {
+  typedef unsigned long long v2ul __attribute__((ext_vector_type(2)));
+  typedef v4i __attribute__((aligned(1))) v4i_any;
+  const v2ul w = __builtin_bit_cast(v2ul, *reinterpret_cast<const v4i_any *>(end - 16));
+  const int shift = (16 - rem) * 8;
+  v2ul out;
+  if (shift >= 64) {
+    out[0] = w[1] >> (shift - 64);
+    out[1] = 0;
+  } else {
+    out[0] = (w[0] >> shift) | (w[1] << (64 - shift));
+    out[1] = w[1] >> shift;
+  }
+  return __builtin_bit_cast(v4i, out);
+}
+
 // K-inner slab loader: ROWS x 128 B, direct to LDS.  The per-lane source pointers (row clamp,
 // row * stride, swizzled chunk) are computed once; per slab only the K offset moves.
 // Rows past `rows_valid` are clamped (loaded from the last valid row; their results are never
@@ -148,13 +166,24 @@ struct KInnerLoader {
     for (int i = 0; i < PER; i++)
       lds_dma16(src[i] + kbyte0, lds + lds_off[i]);
   }
-  // a slab of which only the first `valid` bytes of each row exist (whole 16-byte pieces)
+  // a slab of which only the first `valid` bytes of each row exist; a row's last piece, where it is not whole, is zero until
+  // finish_partial writes it, behind the wave's wait for these requests
   __device__ __forceinline__ void issue_partial(int64_t kbyte0, int valid, unsigned char *lds, int wave, int lane) const {
 #pragma unroll
     for (int i = 0; i < PER; i++) {
       const int r = (wave + NWAVES * i) * 8 + (lane >> 3);
-      lds_dma16(lds_slot(r, lane & 7) * 16 < valid ? src[i] + kbyte0 : (const unsigned char *)g_zero16, lds + lds_off[i]);
+      lds_dma16(lds_slot(r, lane & 7) * 16 + 16 <= valid ? src[i] + kbyte0 : (const unsigned char *)g_zero16, lds + lds_off[i]);
     }
+  }
+  __device__ __forceinline__ void finish_partial(int64_t kbyte0, int valid, unsigned char *lds, int wave, int lane) const {
+    if ((valid & 15) == 0) return;
+    v4i v[PER];
+#pragma unroll
+    for (int i = 0; i < PER; i++)
+      if (lds_slot((wave + NWAVES * i) * 8 + (lane >> 3), lane & 7) == valid >> 4) v[i] = row_end_piece(src[i] + kbyte0 + (valid & 15), valid & 15);
+#pragma unroll
+    for (int i = 0; i < PER; i++)
+      if (lds_slot((wave + NWAVES * i) * 8 + (lane >> 3), lane & 7) == valid >> 4) *reinterpret_cast<v4i *>(lds + lds_off[i] + lane * 16) = v[i];
   }
   // instruction i of the slab goes out at step i * spread / PER + phase (+ skew, which may be a
   // run-time value); with t, spread and phase known after unrolling the tests fold away
@@ -171,8 +200,9 @@ struct KInnerLoader {
 //   ES = 2:  8 k x  8 rows -> eight 16-byte K-runs (v_perm_b32 pairs halves)
 //   ES = 4:  4 k x  4 rows -> four 16-byte K-runs (pure register renaming)
 //   ES = 1:  4 k x 16 rows -> sixteen 4-byte K-runs (4 x 4 byte transposes with v_perm_b32)
-// `rows_valid` must be a multiple of the block's row count (the host falls back to a transpose
-// pass otherwise); of a partial slab the k past the end of K are zero (fetch_partial).
+// A k-row that is not whole pieces (rows_valid no multiple of RB): its last piece runs into the next k-row, which only rows of
+// the tile past the edge see; the very last k-row has nothing behind it, so its piece is read so as to end with the row
+// (fetch_partial: the host makes the last slab a partial one).  Of a partial slab the k past the end of K are zero.
 template <int ES> struct KOuterShape;
 template <> struct KOuterShape<2> { static constexpr int KB = 8, RB = 8; };
 template <> struct KOuterShape<4> { static constexpr int KB = 4, RB = 4; };
@@ -186,6 +216,7 @@ struct KOuterStage {
   static constexpr int BLOCKS = (ROWS / RB) * (KSLAB / KB);
   static constexpr int PER = (BLOCKS + NTHREADS - 1) / NTHREADS;
   static constexpr int LOADS = PER * KB;                        // vector-memory ops per slab per lane
+  typedef v4i __attribute__((aligned(1))) v4i_any;  // (one load at whatever address)
   v4i v[PER][KB];
 
   __device__ __forceinline__ void fetch(const unsigned char *__restrict__ g, int64_t ld, int64_t row0, int64_t rows_valid,
@@ -196,10 +227,10 @@ struct KOuterStage {
       if (blk >= BLOCKS) break;
       const int rb = blk % (ROWS / RB), kb = blk / (ROWS / RB);
       int64_t col = row0 + rb * RB;
-      col = col + RB <= rows_valid ? col : rows_valid - RB;  // tile rows past the edge: any valid run
+      col = col < rows_valid ? col : (rows_valid - 1) / RB * RB;  // tile rows past the edge: any piece
 #pragma unroll
       for (int j = 0; j < KB; j++)
-        v[p][j] = *reinterpret_cast<const v4i *>(g + (k0 + kb * KB + j) * ld + col * ES);
+        v[p][j] = *reinterpret_cast<const v4i_any *>(g + (k0 + kb * KB + j) * ld + col * ES);
     }
   }
 
@@ -212,11 +243,15 @@ struct KOuterStage {
       if (blk >= BLOCKS) break;
       const int rb = blk % (ROWS / RB), kb = blk / (ROWS / RB);
       int64_t col = row0 + rb * RB;
-      col = col + RB <= rows_valid ? col : rows_valid - RB;
+      col = col < rows_valid ? col : (rows_valid - 1) / RB * RB;
+      const bool runs_over = col + RB > rows_valid;
 #pragma unroll
       for (int j = 0; j < KB; j++) {
         const int k = kb * KB + j;
-        v[p][j] = k < valid ? *reinterpret_cast<const v4i *>(g + (k0 + k) * ld + col * ES) : v4i{0, 0, 0, 0};
+        const unsigned char *q = g + (k0 + k) * ld;
+        if (k >= valid) v[p][j] = v4i{0, 0, 0, 0};
+        else if (runs_over && k == valid - 1) v[p][j] = row_end_piece(q + rows_valid * ES, (int)(rows_valid - col) * ES);
+        else v[p][j] = *reinterpret_cast<const v4i_any *>(q + col * ES);
       }
     }
   }
@@ -314,9 +349,10 @@ struct KOuterDmaLoader {
   static_assert(RBYTES >= 256 && INSTR % NWAVES == 0, "needs at least 16 chunks per k-row");
   const unsigned char *src[PER];
   int lds_off[PER];
+  int rem[PER];  // bytes of this lane's piece that lie inside its k-row, 0: all of them
 
-  // g: [K, cols] with `ld` bytes per k; the tile covers columns col0 .. col0+ROWS-1, of which
-  // cols_valid (a multiple of 16 bytes' worth) exist: chunks past the edge re-read the last valid one
+  // g: [K, cols] with `ld` bytes per k; the tile covers columns col0 .. col0+ROWS-1, of which cols_valid exist: chunks past the
+  // edge re-read the last one, which runs into the next k-row where k-rows are not whole pieces (see KOuterStage)
   __device__ __forceinline__ void init(const unsigned char *__restrict__ g, int64_t ld, int64_t col0, int64_t cols_valid,
                                        int wave, int lane) {
 #pragma unroll
@@ -325,8 +361,9 @@ struct KOuterDmaLoader {
       const int o = t * 1024 + lane * 16;
       const int k = o / RBYTES, slot = (o % RBYTES) / 16;
       int64_t byte = col0 * ES + tr_slot<ES>(k, slot) * 16;
-      const int64_t last = cols_valid * ES - 16;
+      const int64_t last = (cols_valid * ES - 1) & ~(int64_t)15;
       byte = byte <= last ? byte : last;
+      rem[i] = byte == last ? (int)(cols_valid * ES) & 15 : 0;
       src[i] = g + (int64_t)k * ld + byte;
       lds_off[i] = t * 1024;
     }
@@ -336,13 +373,19 @@ struct KOuterDmaLoader {
     for (int i = 0; i < PER; i++)
       lds_dma16(src[i] + k0 * ld, lds + lds_off[i]);
   }
-  // a slab of which only the first `valid` k-rows exist
+  // a slab of which only the first `valid` k-rows exist; the last one's piece that is not whole is zero until finish_partial
   __device__ __forceinline__ void issue_partial(int64_t k0, int64_t ld, int valid, unsigned char *lds, int wave, int lane) const {
 #pragma unroll
     for (int i = 0; i < PER; i++) {
       const int k = ((wave + NWAVES * i) * 1024 + lane * 16) / RBYTES;
-      lds_dma16(k < valid ? src[i] + k0 * ld : (const unsigned char *)g_zero16, lds + lds_off[i]);
+      lds_dma16(k < valid - (rem[i] != 0) ? src[i] + k0 * ld : (const unsigned char *)g_zero16, lds + lds_off[i]);
     }
+  }
+  __device__ __forceinline__ void finish_partial(int64_t k0, int64_t ld, int valid, unsigned char *lds, int wave, int lane) const {
+#pragma unroll
+    for (int i = 0; i < PER; i++)
+      if (rem[i] != 0 && ((wave + NWAVES * i) * 1024 + lane * 16) / RBYTES == valid - 1)
+        *reinterpret_cast<v4i *>(lds + lds_off[i] + lane * 16) = row_end_piece(src[i] + k0 * ld + rem[i], rem[i]);
   }
   __device__ __forceinline__ void issue_at(int t, int spread, int phase, int skew, int64_t k0, int64_t ld, unsigned char *lds) const {
 #pragma unroll
@@ -396,8 +439,8 @@ struct GemmArgs {
   int batch_inner;
   int64_t ts_l, ts_r;
   int all_slabs;         // > 0: grid index y is not a batch item but a range of Kb of the all_slabs slabs of K (the last may be shorter)
-  // What exists of a partial last slab, 0 = every slab is whole: bytes of each row of a K-inner operand (a multiple of
-  // 16), k of a K-outer one.  The kernels walk the partial slab FIRST, in the prologue, where its requests are code of
+  // What exists of a partial last slab, 0 = every slab is whole: bytes of each row of a K-inner operand, k of a K-outer one
+  // (all of them where the slab is whole and only the end of the last k-row needs care).  The kernels walk the partial slab FIRST, in the prologue, where its requests are code of
   // their own (lanes past the end read g_zero16): the loop over the whole slabs pays nothing for it.  (bf16
   // 2000 x 3000 x 1000: 21.0 us per call.  Contracting the whole slabs in place, the rest from two zero-extended
   // copies, and adding the two results was seven launches and 48.8 us.)
@@ -420,6 +463,34 @@ __device__ __forceinline__ void gemm_batch_item(const GemmArgs &a, int b, const 
     l = a.l + b * a.bs_l;
     r = a.r + b * a.bs_r;
   }
+}
+
+// Stores of results at any address: rows of N outputs begin wherever N puts them, and global memory takes a vector at any address
+// (bf16 2048 x 2047 x 2048 with a store per output / with these: 26.1 / 21.1 us).
+typedef v4i __attribute__((aligned(1))) v4i_store;
+typedef int __attribute__((ext_vector_type(2), aligned(1))) v2i_store;
+typedef int __attribute__((aligned(1))) int_store;
+// the first `n` of the 16 / ES outputs of a piece, n > 0
+template <int ES>
+__device__ __forceinline__ void put_piece(unsigned char *q, v4i v, int64_t n) {
+  if (n >= 16 / ES) {
+    *reinterpret_cast<v4i_store *>(q) = v;
+    return;
+  }
+  const int bytes = (int)n * ES;
+  if (bytes & 8) {
+    *reinterpret_cast<v2i_store *>(q) = v2i_store{v[0], v[1]};
+    q += 8;
+    v[0] = v[2];
+    v[1] = v[3];
+  }
+  if (bytes & 4) {
+    *reinterpret_cast<int_store *>(q) = v[0];
+    q += 4;
+    v[0] = v[1];
+  }
+  if constexpr (ES == 2)
+    if (bytes & 2) *reinterpret_cast<short *>(q) = (short)v[0];
 }
 
 // Epilogue of one wave: for 16x16 tile (i, j) a lane holds m = 16*i + lane%16 and
@@ -452,7 +523,6 @@ __device__ __forceinline__ void gemm_epilogue(typename Mma16<DT>::acc_t (&acc)[T
   } else if constexpr (int_acc && ODT == HIPNX_F32) {
     // as_type(s32 -> f32) then multiply, each rounding once, as the two separate kernels would
     if (scale_mode == HIPNX_SCALE_NONE) return;  // the host pairs them only with a scale
-    const bool vec_ok = (N % 4) == 0;
     const float one = scale_mode == HIPNX_SCALE_ONE ? scale[0] : 0.0f;
 #pragma unroll
     for (int i = 0; i < TM; i++) {
@@ -461,21 +531,13 @@ __device__ __forceinline__ void gemm_epilogue(typename Mma16<DT>::acc_t (&acc)[T
 #pragma unroll
       for (int j = 0; j < TN; j++) {
         const int64_t gn = col0 + 16 * j + 4 * (lane >> 4);
-        float v[4];
+        v4i v;
 #pragma unroll
         for (int e = 0; e < 4; e++) {
           const float sc = scale_mode == HIPNX_SCALE_PER_COLUMN ? (gn + e < N ? scale[gn + e] : 0.0f) : per_row;
-          v[e] = (float)(int32_t)acc[i][j][e] * sc;
+          v[e] = (int)f32_canon_bits((float)(int32_t)acc[i][j][e] * sc);
         }
-        const int64_t idx = obase + gm * N + gn;
-        if (gm < M) {
-          if (vec_ok && gn + 4 <= N) store_vec<float, 4>(out, HIPNX_F32, idx, v);
-          else {
-#pragma unroll
-            for (int e = 0; e < 4; e++)
-              if (gn + e < N) store_one<float>(out, HIPNX_F32, idx + e, v[e]);
-          }
-        }
+        if (gm < M && gn < N) put_piece<4>((unsigned char *)out + (obase + gm * N + gn) * 4, v, N - gn);
       }
     }
   } else if constexpr (int_acc != int_out) return;  // the host never pairs them
@@ -493,8 +555,6 @@ __device__ __forceinline__ void gemm_epilogue(typename Mma16<DT>::acc_t (&acc)[T
       else if constexpr (ODT == HIPNX_BF16_RNE) return (uint32_t)f32_to_bf16_bits_rne(lo) | ((uint32_t)f32_to_bf16_bits_rne(hi) << 16);
       else return (uint32_t)f32_to_f16_bits(lo) | ((uint32_t)f32_to_f16_bits(hi) << 16);
     };
-    // N % 8 == 0: a group of 8 columns lies wholly inside or outside, and row starts keep the 16-byte alignment
-    const bool paired = (N % 8) == 0 && ((uintptr_t)out & 15) == 0;
     // A second exchange makes the runs whole cache lines: of two neighbouring PAIRS of tiles the lanes of
     // rows 8..15 hand their first pair's 16 bytes to the lane 8 rows up and take that lane's second pair, so
     // that one store instruction covers rows 0..7 with 128 contiguous bytes each (four tiles wide) and the
@@ -510,10 +570,10 @@ __device__ __forceinline__ void gemm_epilogue(typename Mma16<DT>::acc_t (&acc)[T
       return v;
     };
     auto put16 = [&](int64_t gm, int64_t gn, const v4i &v) {
-      if (gm < M && gn < N) *reinterpret_cast<v4i *>((unsigned char *)out + (obase + gm * N + gn) * 2) = v;
+      if (gm < M && gn < N) put_piece<2>((unsigned char *)out + (obase + gm * N + gn) * 2, v, N - gn);
     };
     if constexpr (TN % 4 == 0) {
-      if (wave_lds != nullptr && paired) {
+      if (wave_lds != nullptr) {
         // with LDS of its own the wave turns four tiles (16 rows x 128 bytes) around instead, as the 4-byte
         // branch below describes: every cache line leaves as one run of eight neighbouring lanes
         const int wr = lane & 15, wc = lane >> 4, rr = lane >> 3, rp = lane & 7;
@@ -549,44 +609,21 @@ __device__ __forceinline__ void gemm_epilogue(typename Mma16<DT>::acc_t (&acc)[T
     for (int i = 0; i < TM; i++) {
       const int64_t gm = row0 + 16 * i + (lane & 15);
       if constexpr (TN % 4 == 0) {
-        if (paired) {
 #pragma unroll
-          for (int j = 0; j < TN; j += 4) {
-            const v4i v = pair16(i, j), w = pair16(i, j + 2);
-            v4i got;  // the partner's other pair: rows 0..7 receive the second pair of rows 8..15 and vice versa
+        for (int j = 0; j < TN; j += 4) {
+          const v4i v = pair16(i, j), w = pair16(i, j + 2);
+          v4i got;  // the partner's other pair: rows 0..7 receive the second pair of rows 8..15 and vice versa
 #pragma unroll
-            for (int e = 0; e < 4; e++) got[e] = __shfl_xor(hi ? v[e] : w[e], 8, 64);
-            const int64_t gn0 = gc + 16 * (j + (odd ? 1 : 0)), gn1 = gn0 + 32;
-            // rows 0..7 of the 16: own first pair (rows < 8) | the partner's second pair, stored for row - 8
-            put16(hi ? gm - 8 : gm, hi ? gn1 : gn0, hi ? got : v);
-            // rows 8..15: own second pair stays with rows >= 8 | rows < 8 store the partner's first pair for row + 8
-            put16(hi ? gm : gm + 8, hi ? gn1 : gn0, hi ? w : got);
-          }
-          continue;
+          for (int e = 0; e < 4; e++) got[e] = __shfl_xor(hi ? v[e] : w[e], 8, 64);
+          const int64_t gn0 = gc + 16 * (j + (odd ? 1 : 0)), gn1 = gn0 + 32;
+          // rows 0..7 of the 16: own first pair (rows < 8) | the partner's second pair, stored for row - 8
+          put16(hi ? gm - 8 : gm, hi ? gn1 : gn0, hi ? got : v);
+          // rows 8..15: own second pair stays with rows >= 8 | rows < 8 store the partner's first pair for row + 8
+          put16(hi ? gm : gm + 8, hi ? gn1 : gn0, hi ? w : got);
         }
-      }
+      } else {
 #pragma unroll
-      for (int j = 0; j < TN; j += 2) {
-        if (paired) {
-          put16(gm, gc + 16 * (j + (odd ? 1 : 0)), pair16(i, j));
-        } else {
-#pragma unroll
-          for (int jj = j; jj < j + 2; jj++) {
-            const int64_t gn = col0 + 16 * jj + 4 * (lane >> 4);
-            float v[4];
-#pragma unroll
-            for (int e = 0; e < 4; e++) v[e] = acc[i][jj][e];
-            const int64_t idx = obase + gm * N + gn;
-            if (gm < M) {
-              if ((N % 4) == 0 && gn + 4 <= N) store_vec<float, 4>(out, ODT, idx, v);
-              else {
-#pragma unroll
-                for (int e = 0; e < 4; e++)
-                  if (gn + e < N) store_one<float>(out, ODT, idx + e, v[e]);
-              }
-            }
-          }
-        }
+        for (int j = 0; j < TN; j += 2) put16(gm, gc + 16 * (j + (odd ? 1 : 0)), pair16(i, j));
       }
     }
   } else if constexpr ((ODT == HIPNX_S32 || ODT == HIPNX_U32 || ODT == HIPNX_F32) && TN % 2 == 0) {
@@ -600,11 +637,10 @@ __device__ __forceinline__ void gemm_epilogue(typename Mma16<DT>::acc_t (&acc)[T
       else return (int)f32_canon_bits(c[e]);
     };
     const bool hi = (lane >> 3) & 1;
-    const bool lines = (N % 4) == 0 && ((uintptr_t)out & 15) == 0;
     auto put16 = [&](int64_t gm, int64_t gn, const v4i &v) {
-      if (gm < M && gn < N) *reinterpret_cast<v4i *>((unsigned char *)out + (obase + gm * N + gn) * 4) = v;
+      if (gm < M && gn < N) put_piece<4>((unsigned char *)out + (obase + gm * N + gn) * 4, v, N - gn);
     };
-    if (wave_lds != nullptr && lines) {
+    if (wave_lds != nullptr) {
       // With 4 KiB of LDS of its own a wave turns each pair of tiles (16 rows x 128 bytes) around first:
       // written as the accumulators hold it (lane = row, 16-byte piece c of either tile), read back with
       // eight consecutive lanes along one row, so that every cache line of the result leaves as ONE
@@ -647,19 +683,11 @@ __device__ __forceinline__ void gemm_epilogue(typename Mma16<DT>::acc_t (&acc)[T
         v4i v, w;
 #pragma unroll
         for (int e = 0; e < 4; e++) { v[e] = word(acc[i][j], e); w[e] = word(acc[i][j + 1], e); }
-        if (lines) {
-          v4i got;
+        v4i got;
 #pragma unroll
-          for (int e = 0; e < 4; e++) got[e] = __shfl_xor(hi ? v[e] : w[e], 8, 64);
-          put16(hi ? gm - 8 : gm, hi ? gn1 : gn0, hi ? got : v);  // rows 0..7 of the 16, both tiles
-          put16(hi ? gm : gm + 8, hi ? gn1 : gn0, hi ? w : got);  // rows 8..15
-        } else {
-#pragma unroll
-          for (int e = 0; e < 4; e++) {
-            if (gm < M && gn0 + e < N) *reinterpret_cast<int *>((unsigned char *)out + (obase + gm * N + gn0 + e) * 4) = v[e];
-            if (gm < M && gn1 + e < N) *reinterpret_cast<int *>((unsigned char *)out + (obase + gm * N + gn1 + e) * 4) = w[e];
-          }
-        }
+        for (int e = 0; e < 4; e++) got[e] = __shfl_xor(hi ? v[e] : w[e], 8, 64);
+        put16(hi ? gm - 8 : gm, hi ? gn1 : gn0, hi ? got : v);  // rows 0..7 of the 16, both tiles
+        put16(hi ? gm : gm + 8, hi ? gn1 : gn0, hi ? w : got);  // rows 8..15
       }
     }
   } else {
@@ -805,6 +833,14 @@ gemm_pipelined_kernel(GemmArgs a) {
     else if constexpr (R_TR) rtr.issue_partial(k_first / ES, a.ld_r, a.tail_r, sB, wave, lane);
     else rregs.fetch_partial(rb, a.ld_r, n0, a.N, k_first / ES, a.tail_r, tid);
   };
+  // the pieces that end a row, behind the wave's own wait for the rest of the slab (register-staged operands have them already)
+  auto finish_partial = [&]() {
+    unsigned char *sA = smem, *sB = sA + BM * SLAB;
+    if constexpr (L_KIN) lload.finish_partial(k_first, a.tail_l, sA, wave, lane);
+    else if constexpr (L_TR) ltr.finish_partial(k_first / ES, a.ld_l, a.tail_l, sA, wave, lane);
+    if constexpr (R_KIN) rload.finish_partial(k_first, a.tail_r, sB, wave, lane);
+    else if constexpr (R_TR) rtr.finish_partial(k_first / ES, a.ld_r, a.tail_r, sB, wave, lane);
+  };
   auto commit = [&](int stage) {  // register-staged K-outer operands: transposed LDS writes
     unsigned char *sA = smem + stage * STAGE, *sB = sA + BM * SLAB;
     if constexpr (!L_KIN && !L_TR) lregs.store(sA, tid);
@@ -876,6 +912,7 @@ gemm_pipelined_kernel(GemmArgs a) {
   commit(0);
   if (nslab >= NSTAGE - 1) wait_vmcnt<INFLIGHT>();
   else wait_vmcnt<0>();
+  if (partial) finish_partial();
   __syncthreads();
   if constexpr (AHEAD)
     if (1 < nslab) issue(1, SLAB + k_shift);

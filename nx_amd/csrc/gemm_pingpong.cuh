@@ -93,14 +93,27 @@ struct PPKInnerLoader {
 #pragma unroll
     for (int i = 0; i < PER; i++) lds_dma16_at(b, off[i], lds + (wave + NWAVES * i) * 1024);
   }
-  // a slab of which only the first `valid` bytes of each row exist (whole 16-byte pieces)
+  // a slab of which only the first `valid` bytes of each row exist; a row's last piece, where it is not whole, is zero until
+  // finish_partial writes it, behind the wave's wait for these requests
   __device__ __forceinline__ void issue_partial(int64_t kbyte0, int valid, unsigned char *lds, int wave, int lane) const {
     const unsigned char *b = base + kbyte0;
 #pragma unroll
     for (int i = 0; i < PER; i++) {
       const int r = (wave + NWAVES * i) * 8 + (lane >> 3);
-      lds_dma16(lds_slot16(r, lane & 7) * 16 < valid ? b + off[i] : (const unsigned char *)g_zero16, lds + (wave + NWAVES * i) * 1024);
+      lds_dma16(lds_slot16(r, lane & 7) * 16 + 16 <= valid ? b + off[i] : (const unsigned char *)g_zero16, lds + (wave + NWAVES * i) * 1024);
     }
+  }
+  __device__ __forceinline__ void finish_partial(int64_t kbyte0, int valid, unsigned char *lds, int wave, int lane) const {
+    if ((valid & 15) == 0) return;
+    const unsigned char *b = base + kbyte0 + (valid & 15);
+    v4i v[PER];
+#pragma unroll
+    for (int i = 0; i < PER; i++)
+      if (lds_slot16((wave + NWAVES * i) * 8 + (lane >> 3), lane & 7) == valid >> 4) v[i] = row_end_piece(b + off[i], valid & 15);
+#pragma unroll
+    for (int i = 0; i < PER; i++)
+      if (lds_slot16((wave + NWAVES * i) * 8 + (lane >> 3), lane & 7) == valid >> 4)
+        *reinterpret_cast<v4i *>(lds + (wave + NWAVES * i) * 1024 + lane * 16) = v[i];
   }
 };
 
@@ -114,8 +127,9 @@ struct PPKOuterLoader {
   static_assert(RBYTES >= 256 || ES == 1, "a 2-byte k-row must span all LDS banks");
   const unsigned char *base;
   unsigned off[PER];
+  int rem[PER];  // bytes of this lane's piece that lie inside its k-row, 0: all of them (KOuterDmaLoader)
   __device__ __forceinline__ void init(const unsigned char *g, int64_t ld, int64_t col0, int64_t cols_valid, int wave, int lane) {
-    const int64_t last = cols_valid * ES - 16;
+    const int64_t last = (cols_valid * ES - 1) & ~(int64_t)15;
     const int64_t first = col0 * ES <= last ? col0 * ES : last;
     base = wave_uniform(g + first);
 #pragma unroll
@@ -124,6 +138,7 @@ struct PPKOuterLoader {
       const int k = o / RBYTES, slot = (o % RBYTES) / 16;
       int64_t byte = col0 * ES + tr_slot_w<ES, RBYTES>(k, slot) * 16;
       byte = byte <= last ? byte : last;
+      rem[i] = byte == last ? (int)(cols_valid * ES) & 15 : 0;
       off[i] = (unsigned)((int64_t)k * ld + (byte - first));
     }
   }
@@ -132,14 +147,21 @@ struct PPKOuterLoader {
 #pragma unroll
     for (int i = 0; i < PER; i++) lds_dma16_at(b, off[i], lds + (wave + NWAVES * i) * 1024);
   }
-  // a slab of which only the first `valid` k-rows exist
+  // a slab of which only the first `valid` k-rows exist; the last one's piece that is not whole is zero until finish_partial
   __device__ __forceinline__ void issue_partial(int64_t k0, int64_t ld, int valid, unsigned char *lds, int wave, int lane) const {
     const unsigned char *b = base + k0 * ld;
 #pragma unroll
     for (int i = 0; i < PER; i++) {
       const int k = ((wave + NWAVES * i) * 1024 + lane * 16) / RBYTES;
-      lds_dma16(k < valid ? b + off[i] : (const unsigned char *)g_zero16, lds + (wave + NWAVES * i) * 1024);
+      lds_dma16(k < valid - (rem[i] != 0) ? b + off[i] : (const unsigned char *)g_zero16, lds + (wave + NWAVES * i) * 1024);
     }
+  }
+  __device__ __forceinline__ void finish_partial(int64_t k0, int64_t ld, int valid, unsigned char *lds, int wave, int lane) const {
+    const unsigned char *b = base + k0 * ld;
+#pragma unroll
+    for (int i = 0; i < PER; i++)
+      if (rem[i] != 0 && ((wave + NWAVES * i) * 1024 + lane * 16) / RBYTES == valid - 1)
+        *reinterpret_cast<v4i *>(lds + (wave + NWAVES * i) * 1024 + lane * 16) = row_end_piece(b + off[i] + rem[i], rem[i]);
   }
 };
 
@@ -251,6 +273,16 @@ gemm_pingpong_kernel(GemmArgs a) {
     wait_vmcnt<RPER + 4>();
   } else {
     wait_vmcnt<0>();
+  }
+  if (partial) {  // the pieces that end a row
+    const int64_t k0 = (int64_t)(nslab - 1) * SLAB;
+    unsigned char *sA = smem + lhalf * (HALF * SLAB), *sB = smem + BM * SLAB;
+    if constexpr (R_KIN) rload.finish_partial(k0, a.tail_r, sB, wave, lane);
+    else rtr.finish_partial(k0 / ES, a.ld_r, a.tail_r, sB, wave, lane);
+    if constexpr (L_KIN) lload.finish_partial(k0, a.tail_l, sA, wave & 3, lane);
+    else ltr.finish_partial(k0 / ES, a.ld_l, a.tail_l, sA, wave & 3, lane);
+    __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): they are in LDS before the barrier
+    __builtin_amdgcn_sched_barrier(0);
   }
   __builtin_amdgcn_s_barrier();
   if (grp) __builtin_amdgcn_s_barrier();  // group 1 runs one phase behind
@@ -495,6 +527,15 @@ gemm_pingpong128_kernel(GemmArgs a) {
   if (grp == 1) {
     if (nslab >= AHEAD) wait_vmcnt<(AHEAD - 1) / 2 * REQ>();
     else wait_vmcnt<0>();
+    if (partial) {  // the pieces that end a row
+      const int64_t k0 = (int64_t)(nslab1 - 1) * SLAB;
+      if constexpr (L_KIN) lkin.finish_partial(k0, a.tail_l, smem, w4, lane);
+      else lkout.finish_partial(k0 / ES, a.ld_l, a.tail_l, smem, w4, lane);
+      if constexpr (R_KIN) rkin.finish_partial(k0, a.tail_r, smem + BM * SLAB, w4, lane);
+      else rkout.finish_partial(k0 / ES, a.ld_r, a.tail_r, smem + BM * SLAB, w4, lane);
+      __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): they are in LDS before the barrier
+      __builtin_amdgcn_sched_barrier(0);
+    }
   }
   __builtin_amdgcn_s_barrier();
   HIPNX_TL_STAMP(tl_walk);

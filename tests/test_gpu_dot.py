@@ -382,6 +382,39 @@ def test_what_lies_behind_the_end_of_k_is_not_read(ty, M, N, K, layout, hip):
     assert np.isnan(got[0, 1::2]).all() and not np.isfinite(got[0, ::2][:, ~finite]).any() and np.isnan(got[1:]).all()
 
 
+# Rows and k-rows one element longer or shorter than whole 16-byte pieces, in every kernel: the smallest operands the matrix
+# kernels take, few rows, 32- to 256-row tiles, K split, whole slabs of K under a k-row that is not whole pieces.
+@pytest.mark.parametrize("ty,M,N,K", [("s8", 17, 17, 17), ("s8", 33, 31, 15), ("s8", 7, 1057, 296), ("s8", 43, 379, 2049), ("s8", 65, 4097, 1024),
+                                      ("s8", 271, 130, 129), ("s8", 1025, 2063, 640), ("bf16", 9, 20, 64), ("bf16", 1, 1031, 2047), ("bf16", 31, 1027, 512),
+                                      ("f16", 257, 393, 321), ("bf16", 1281, 515, 1093), ("bf16", 2061, 3075, 576), ("f16", 131, 1037, 4097),
+                                      ("f32", 21, 13, 32), ("f32", 785, 131, 1025), ("f32", 1021, 10, 1669), ("f32", 66, 515, 992)])
+@pytest.mark.parametrize("layout", ["nn", "nt", "tn", "tt"])
+def test_rows_that_are_not_whole_pieces(ty, M, N, K, layout, hip):
+    """Integer-valued operands: the product is exact in any order.  What is not a number behind the operands, which the loads of
+    a last piece must not reach, would show in the last row and column."""
+    rng = np.random.default_rng(seed_of(ty, M, N, K, layout, "not whole pieces"))
+    a, b = rng.integers(-4, 5, size=(M, K)), rng.integers(-4, 5, size=(K, N))
+    la = a if layout[0] == "n" else np.ascontiguousarray(a.T)
+    lb = b if layout[1] == "n" else np.ascontiguousarray(b.T)
+
+    def followed_by_garbage(x):
+        held = HELD[ty](x)
+        behind = np.full(256, 77, np.int8) if ty == "s8" else HELD[ty](np.full(256, np.nan))
+        owner = from_numpy(np.concatenate([held.ravel(), behind]), ty, hip)
+        pointer = Nx.Pointer(kind="local", address=Nx.to_pointer(owner).address, data_size=held.size * held.itemsize)
+        return Nx.from_pointer(hip, pointer, ty, held.shape, keep=owner)
+    c1, c2 = [1 if layout[0] == "n" else 0], [0 if layout[1] == "n" else 1]
+    want = a.astype(np.float64) @ b.astype(np.float64)
+    for out in ["s32", "s8"] if ty == "s8" else ["f32", ty]:
+        got = Nx.dot(followed_by_garbage(la), c1, followed_by_garbage(lb), c2, out_type=out)
+        if out == "s8":
+            assert np.array_equal(hip.to_numpy(got), want.astype(np.int64).astype(np.int8))
+        elif out == "s32" or ty == "f32":
+            assert np.array_equal(hip.to_numpy(got).astype(np.float64), want)
+        else:  # rounded once: toward zero in bf16, to nearest in f16
+            assert (np.abs(values(got).reshape(M, N) - want) <= ULP[got.type] * np.abs(want)).all()
+
+
 def at_odd_address(arr, ty, hip, elements):
     """`arr` on the device, `elements` behind the start of an allocation, as a tensor over borrowed memory."""
     flat = np.concatenate([np.zeros(elements, arr.dtype), arr.ravel(), np.zeros(3, arr.dtype)])
