@@ -421,6 +421,9 @@ static int dot_impl(hipnx_ctx *ctx, int l_dt, int r_dt, int out_dt, int64_t batc
       }
     }
     if (scaled) {
+      // (below 16 M multiply-adds callers of a K off whole pieces make the conversion and the product calls of their own)
+      if (any_k && row_bytes % 16 != 0 && (l_layout == HIPNX_K_INNER || r_layout == HIPNX_K_INNER || l_ragged || r_ragged) && (double)M * (double)N * (double)K * (double)batch < 16777216.0)
+        return set_error(HIPNX_EUNSUPPORTED, "dot_scaled: a K off whole 16-byte pieces from 16 M multiply-adds on");
       if (!(int8_pair && mfma && (any_k || row_bytes % SLAB == 0))) return set_error(HIPNX_EUNSUPPORTED, "dot_scaled: s8 x s8 with K a multiple of 128 and at most 65536, M * N >= 256");
       if (scale_mode == HIPNX_SCALE_PER_ROW && batch != 1) return set_error(HIPNX_EUNSUPPORTED, "dot_scaled: a scale per row with more than one batch item");
       const int64_t need = scale_mode == HIPNX_SCALE_PER_COLUMN ? N : scale_mode == HIPNX_SCALE_PER_ROW ? M : 1;
