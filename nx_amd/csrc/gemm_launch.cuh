@@ -12,9 +12,9 @@ enum {
   GEMM_CFG_256x128 = 3,  // 256 x 128, the two-group kernel with half-width wave tiles: 2-byte types whose 256 x 256 grid is too small
   GEMM_CFG_256 = 0,  // 256 x 256, 8 waves (4 x 2, each 64 x 128): large square-ish problems
   GEMM_CFG_128 = 1,  // 128 x 128: mid-size and batched problems; 4 waves (2 x 2, each 64 x 64), or two such groups sharing K
-  GEMM_CFG_64x32 = 2, // 64 x 32, 2 waves: few rows against a long weight matrix (HBM streaming)
-  GEMM_CFG_64x128 = 4, // 64 x 128, 4 waves (2 x 2, each 32 x 64): f32 and f64, wherever the cost model of gemm.hip has it cheapest
-  GEMM_CFG_32x128 = 6, // 32 x 128, 4 waves (1 x 4, each 32 x 32): few rows against 2-byte weights stored K-outer (HBM streaming)
+  GEMM_CFG_64 = 2,  // 64 x 64 on the two-group kernel (2-byte K-inner pairs, int8): small and mid-size problems, few rows; otherwise 64 x 32, 2 waves
+  GEMM_CFG_64x128 = 4, // 64 x 128, wherever the cost models of gemm.hip have it cheapest: the two-group kernel (2-byte, int8) or 4 waves (2 x 2, each 32 x 64)
+  GEMM_CFG_32x128 = 6, // 32 x 128, 4 waves (1 x 4, each 32 x 32): 2-byte weights stored K-outer, few rows or small problems
   GEMM_CFG_128x32 = 5  // 128 x 32, 4 waves (4 x 1, each 32 x 32): many rows against up to 32 columns (a layer with a few outputs)
 };
 
@@ -95,7 +95,7 @@ static int launch_cfg(const hipnx_ctx *ctx, int cfg, const GemmArgs &a, int64_t 
         if constexpr (LK && RK) return launch_one<DT, 4, 1, 1, 1, LK, RK, 4>(ctx, a, batch);
         else return launch_one<DT, 4, 1, 1, 1, LK, RK>(ctx, a, batch);
       case GEMM_CFG_64x128: return launch_one<DT, 2, 2, 1, 2, LK, RK>(ctx, a, batch);
-      case GEMM_CFG_64x32:
+      case GEMM_CFG_64:
         if constexpr (LK && RK) return launch_one<DT, 2, 1, 1, 1, LK, RK, 6>(ctx, a, batch);
         else return launch_one<DT, 2, 1, 1, 1, LK, RK>(ctx, a, batch);
       default: {
@@ -127,13 +127,13 @@ static int launch_cfg(const hipnx_ctx *ctx, int cfg, const GemmArgs &a, int64_t 
       // operand is copied straight into LDS (the condition of the kernel's L_TR / R_TR)
       constexpr int ES = DT == HIPNX_S8 ? 1 : DT == HIPNX_F32 ? 4 : 2;
       constexpr bool tr = ES <= 2 && 128 * ES >= 256;
-      // From 8 slabs of K on, the two-group kernel (2-byte types and int8; f32 with both operands K-inner): 730 clocks per
-      // slab against the 1600-2100 below.  It holds a CU's LDS alone, so for the 2-byte types only where no
+      // From two slabs of K on (f32: eight), the two-group kernel (2-byte types and int8; f32 with both operands K-inner): 730
+      // clocks per slab against the 1600-2100 below (int8 512 x 512 x 512, four slabs: 14.8 us, 9.9 so).  It holds a CU's LDS alone, so for the 2-byte types only where no
       // second work-group would share the CU; int8 has no wider two-group tile to fall back on and takes it
       // for every grid (2048 x 4096 x 4096, 512 tiles: 52 -> 42 us).
       if constexpr (DT == HIPNX_BF16 || DT == HIPNX_F16 || DT == HIPNX_S8 || (DT == HIPNX_F32 && LK && RK)) {
         const int64_t groups = ((a.M + 127) / 128) * ((a.N + 127) / 128) * batch;
-        if (a.Kb >= 8 * SLAB && a.ld_l < (1ll << 23) && a.ld_r < (1ll << 23) && (DT == HIPNX_S8 || DT == HIPNX_F32 || groups <= ctx->num_cus))
+        if (a.Kb >= (DT == HIPNX_F32 ? 8 : 2) * SLAB && a.ld_l < (1ll << 23) && a.ld_r < (1ll << 23) && (DT == HIPNX_S8 || DT == HIPNX_F32 || groups <= ctx->num_cus))
           return launch_pingpong128<DT, LK, RK>(ctx, a, batch);
       }
       if constexpr ((LK || tr) && (RK || tr)) {
@@ -156,20 +156,16 @@ static int launch_cfg(const hipnx_ctx *ctx, int cfg, const GemmArgs &a, int64_t 
           return launch_one<DT, 2, 4, 1, 1, LK, RK>(ctx, a, batch);
         return launch_one<DT, 2, 2, 1, 2, LK, RK>(ctx, a, batch);
       }
+      if constexpr (LK && (DT == HIPNX_BF16 || DT == HIPNX_F16 || DT == HIPNX_S8))
+        if (a.ld_l < (1ll << 24) && a.ld_r < (1ll << 24)) return launch_pingpong128<DT, LK, RK, 64, 128, 6, 1>(ctx, a, batch);
       return launch_one<DT, 2, 2, 2, 2, LK, RK>(ctx, a, batch);
     default:
-      // K-inner 2-byte operands and int8 in either layout: the two-group kernel on 64 x 64 tiles -- 64 rows of the weights per
-      // work-group, their slabs requested three phases (six slabs) ahead, two slabs per phase where K allows
-      // (int8 64 x 11008 x 4096: kernel 13.0 us; the 64 x 32 tiles below 18.7 us)
+      // K-inner 2-byte operands and int8 in either layout: the two-group kernel on 64 x 64 tiles, slabs requested three phases
+      // (six slabs) ahead, two slabs per phase where K allows (int8 64 x 11008 x 4096: kernel 13.0 us; the 64 x 32 tiles
+      // below 18.7 us; of one slab too: 600 x 1500 x 200 bf16 5.1 us against 6.6)
       if constexpr ((LK && RK && (DT == HIPNX_BF16 || DT == HIPNX_F16)) || DT == HIPNX_S8) {
-        if (a.Kb >= 8 * SLAB && a.ld_l < (1ll << 24) && a.ld_r < (1ll << 24)) {
-          if constexpr (DT == HIPNX_S8 && !RK) {
-            // int8 weights stored [K, N]: a k-row of a 64-column tile is half a cache line; where 128-column tiles
-            // still give 3/8 of the CUs work they stream the weights as fast as the K-inner layout
-            // (64 x 32000 x 4096: 50 -> 28 us; with 32 such tiles, 64 x 4096 x 4096, they are slower: 12 -> 18 us)
-            if (((a.N + 127) / 128) * batch * 8 >= (int64_t)ctx->num_cus * 3) return launch_pingpong128<DT, LK, RK, 64, 128, 6, 1>(ctx, a, batch);
-          }
-          if (a.Kb % (2 * SLAB) == 0) return launch_pingpong128<DT, LK, RK, 64, 64, 4, 2>(ctx, a, batch);
+        if (a.ld_l < (1ll << 24) && a.ld_r < (1ll << 24)) {
+          if (a.Kb % (2 * SLAB) == 0 && a.all_slabs % 2 == 0) return launch_pingpong128<DT, LK, RK, 64, 64, 4, 2>(ctx, a, batch);
           return launch_pingpong128<DT, LK, RK, 64, 64, 8, 1>(ctx, a, batch);
         }
       }

@@ -850,3 +850,35 @@ def test_f32_tiles_on_four_and_eight_waves(M, N, K, layout, hip):
     r, rc = (b, [0]) if layout[1] == "n" else (np.ascontiguousarray(b.T), [1])
     got = values(Nx.dot(from_numpy(l, "f32", hip), lc, from_numpy(r, "f32", hip), rc))
     np.testing.assert_array_equal(got, a.astype(np.float64) @ b.astype(np.float64))
+
+
+# Tiles and ranges by the cost model: 64 x 64 and 64 x 128 on the two-group kernel, 32 x 128 against K-outer weights, one slab and odd
+# numbers of them, K cut with ranges of unequal length, the batch beside them
+@pytest.mark.parametrize("ty", ["bf16", "f16", "s8"])
+@pytest.mark.parametrize("right", ["n", "t"])
+@pytest.mark.parametrize("batch,M,N,K", [(1, 500, 500, 500), (1, 65, 129, 64), (1, 1000, 2000, 504), (1, 100, 300, 8000), (1, 256, 1025, 4160), (3, 200, 328, 1336),
+                                         (1, 129, 1000, 128), (1, 66, 4096, 11016), (1, 260, 520, 2240)])
+def test_tiles_of_small_and_middling_contractions(ty, right, batch, M, N, K, hip):
+    """Whole numbers whose sums are exact in f32 in any order, so every output is the same number on any kernel."""
+    rng = np.random.default_rng(seed_of(ty, right, batch, M, N, K))
+    a, b = rng.integers(-3, 4, size=(batch, M, K)), rng.integers(-3, 4, size=(batch, K, N))
+    lb = b if right == "n" else np.ascontiguousarray(b.transpose(0, 2, 1))
+    got = Nx.dot(from_numpy(HELD[ty](a), ty, hip), [2], [0], from_numpy(HELD[ty](lb), ty, hip), [1 if right == "n" else 2], [0], out_type="s32" if ty == "s8" else "f32")
+    assert np.array_equal(hip.to_numpy(got).astype(np.float64), a.astype(np.float64) @ b.astype(np.float64))
+
+
+@pytest.mark.parametrize("M,N,K,contract", [(48, 384, 9568, 1), (256, 1025, 8192, 0), (130, 257, 9999, 1), (64, 4098, 11008, 1)])
+@pytest.mark.parametrize("mode", ["column", "row", "one"])
+def test_scaled_int8_sums_of_cut_contractions(M, N, K, contract, mode, hip):
+    """K cut into ranges: their whole sums, converted and scaled once each, as numpy gives them in f32."""
+    from nx_amd._lib import SCALE_ONE, SCALE_PER_COLUMN, SCALE_PER_ROW
+    rng = np.random.default_rng(seed_of(M, N, K, contract, mode, "cut and scaled"))
+    x, w = rng.integers(-127, 128, size=(M, K)).astype(np.int8), rng.integers(-127, 128, size=(N, K)).astype(np.int8)
+    s = rng.uniform(1e-3, 1e-2, size={"column": N, "row": M, "one": 1}[mode]).astype(np.float32)
+    sums = (x.astype(np.float64) @ w.T.astype(np.float64)).astype(np.float32)  # exact below 2^53, rounded once
+    want = sums * (s[None, :] if mode == "column" else s[:, None] if mode == "row" else s)
+    held = w if contract else np.ascontiguousarray(w.T)
+    sc = from_numpy(s, "f32", hip)
+    out = hip.dot_scaled(sc.with_(data=None, shape=(M, N)), from_numpy(x, "s8", hip), [1], [], from_numpy(held, "s8", hip), [contract], [], sc,
+                         {"column": SCALE_PER_COLUMN, "row": SCALE_PER_ROW, "one": SCALE_ONE}[mode], any_k=True)
+    np.testing.assert_array_equal(hip.to_numpy(out), want)
