@@ -442,6 +442,11 @@ int hipnx_fused_elementwise(hipnx_ctx *ctx, int n_instr, const hipnx_fused_instr
 int hipnx_fused_words(hipnx_ctx *ctx, int n_instr, const hipnx_fused_instr *prog, int n_inputs, const hipnx_buf *const *inputs,
                       const int *in_dts, const int *in_col_strides, int words, int key_parts, int key_index, int64_t n,
                       int out_dt, hipnx_buf *out);
+/* The same (key_parts > 0, n > 0), and key number other_index of the key_parts in `other` (two u32 words): what a sample and the key
+ * for the next one take of a split. */
+int hipnx_fused_words_key(hipnx_ctx *ctx, int n_instr, const hipnx_fused_instr *prog, int n_inputs, const hipnx_buf *const *inputs,
+                          const int *in_dts, const int *in_col_strides, int words, int key_parts, int key_index, int64_t n,
+                          int out_dt, hipnx_buf *out, int other_index, hipnx_buf *other);
 
 /* A program of stages of which input `scores` is the result of a contraction that is not stored: out[b, m, n] of hipnx_dot_strided
  * for bf16 or f16 operands whose rows are K-inner and a result of their type, with rows = batch_outer * batch_inner * M and n along the

@@ -124,6 +124,8 @@ PROTOTYPES = {
     "hipnx_threefry_key": [_ctx_p, _buf_p, C.c_int, C.c_int, _buf_p],
     "hipnx_fused_words": [_ctx_p, C.c_int, C.c_void_p, C.c_int, C.POINTER(C.c_void_p), _intp, _intp, C.c_int, C.c_int, C.c_int, C.c_int64,
                           C.c_int, _buf_p],
+    "hipnx_fused_words_key": [_ctx_p, C.c_int, C.c_void_p, C.c_int, C.POINTER(C.c_void_p), _intp, _intp, C.c_int, C.c_int, C.c_int, C.c_int64,
+                              C.c_int, _buf_p, C.c_int, _buf_p],
     "hipnx_fused_scores": [_ctx_p, C.c_int, C.c_void_p, C.c_int, C.POINTER(C.c_void_p), _intp, _i64p, _intp, C.c_int64, C.c_int, C.c_int64,
                            C.c_int64, C.c_int64, C.c_int64, _i64p, C.POINTER(C.c_void_p), C.c_int, _buf_p],
     "hipnx_capture_begin": [_ctx_p],

@@ -1084,7 +1084,7 @@ class HipNxBackend:
         return Tensor(cls(ref, backend_opts["device"]), ty, tuple(shape), tuple(opts.get("names") or ()))
 
     @classmethod
-    def fused_elementwise(cls, out: Tensor, program, inputs, layout, reduce_op: int = -1, mode=None, words=None) -> Tensor:
+    def fused_elementwise(cls, out: Tensor, program, inputs, layout, reduce_op: int = -1, mode=None, words=None, beside=None):
         """A group of element-wise nodes in one kernel (the evaluator offers it groups it has found
         in a traced function).  `program` is a list of dicts with the fields of `hipnx_fused_instr`
         (`dt` as a type tuple); `layout` is (rows, cols, [(row_stride, col_stride) per input]).
@@ -1093,7 +1093,8 @@ class HipNxBackend:
         EUNSUPPORTED when the shapes do not fit the kernel: the caller then runs the nodes one by one.
         `mode` ("interpreted" / "compiled") runs this call in that mode whatever the device is set to.
         `words` (input number, parts, index): that input is a key (key `index` of the `parts` it splits into, if any), and what
-        the program reads are the random words of `threefry2x32` under it, made where they are used."""
+        the program reads are the random words of `threefry2x32` under it, made where they are used.  `beside` (template, index):
+        also that one of the `parts`, returned behind the result."""
         dev = cls._device_of(*inputs) if inputs else 0
         # the library is switched when a call wants another mode than the last call had, not around every call:
         # the groups of a traced function all want the same one
@@ -1126,14 +1127,20 @@ class HipNxBackend:
         handles = handle_array(*[t.data.ref.handle for t in inputs])
         ctx = _Context.get(dev)
         ref = _fresh_ref(ctx, nbytes)
-        if words is not None:
+        other = None
+        if beside is not None:
+            other = _fresh_ref(ctx, 8)
+            status = L.lib.hipnx_fused_words_key(ctx, len(program), prog_ptr, len(inputs), handles, dts, cs, *words, cols, out_code, ref.handle,
+                                                 beside[1], other.handle)
+        elif words is not None:
             status = L.lib.hipnx_fused_words(ctx, len(program), prog_ptr, len(inputs), handles, dts, cs, *words, cols, out_code, ref.handle)
         else:
             status = L.lib.hipnx_fused_elementwise(ctx, len(program), prog_ptr, len(inputs), handles, dts, rs, cs, rows, cols,
                                                    reduce_op, out_code, ref.handle)
         if status:
             L.check(status)
-        return out.with_(data=HipNxBackend(ref, dev))
+        res = out.with_(data=HipNxBackend(ref, dev))
+        return res if other is None else (res, beside[0].with_(data=HipNxBackend(other, dev)))
 
     @classmethod
     def fused_scores(cls, out: Tensor, program, inputs, layout, at: int, dot, mode=None) -> Tensor:

@@ -195,7 +195,7 @@ struct Scores {
 static int fused_impl(hipnx_ctx *ctx, int n_instr, const hipnx_fused_instr *prog, int n_inputs,
                       const hipnx_buf *const *inputs, const int *in_dts, const int64_t *in_row_strides,
                       const int *in_col_strides, int64_t rows, int64_t cols, int reduce_op, int out_dt,
-                      hipnx_buf *out, int words, int key_parts, int key_index, const Scores &scores = Scores()) {
+                      hipnx_buf *out, int words, int key_parts, int key_index, const Scores &scores = Scores(), int beside_index = 0, hipnx_buf *beside = nullptr) {
   Enter in(ctx);
   if (in.status) return in.status;
   if (n_instr < 1 || n_instr > HIPNX_FUSED_MAX_INSTR || !prog)
@@ -213,6 +213,11 @@ static int fused_impl(hipnx_ctx *ctx, int n_instr, const hipnx_fused_instr *prog
   a.words = words;
   a.key_parts = key_parts;
   a.key_index = key_index;
+  a.beside_index = beside_index;
+  if (beside) {
+    if (int st = check_buf(ctx, beside, 8, "fused_words key")) return st;
+    a.beside = (uint32_t *)beside->ptr;
+  }
   a.scores = scores.input;
   if (words >= 0 && ctx->fused_mode != HIPNX_FUSED_COMPILED) return set_error(HIPNX_EUNSUPPORTED, "fused: random words need the compiled mode");
   unsigned saved = 0;  // slots that hold a value so far
@@ -509,6 +514,19 @@ extern "C" int hipnx_fused_words(hipnx_ctx *ctx, int n_instr, const hipnx_fused_
     return set_error(HIPNX_EINVAL, "fused_words: key %d of %d", key_index, key_parts);
   const int64_t row_strides[HIPNX_FUSED_MAX_INPUTS] = {};
   return fused_impl(ctx, n_instr, prog, n_inputs, inputs, in_dts, row_strides, in_col_strides, 1, n, -1, out_dt, out, words, key_parts, key_index);
+}
+
+extern "C" int hipnx_fused_words_key(hipnx_ctx *ctx, int n_instr, const hipnx_fused_instr *prog, int n_inputs, const hipnx_buf *const *inputs,
+                                     const int *in_dts, const int *in_col_strides, int words, int key_parts, int key_index, int64_t n,
+                                     int out_dt, hipnx_buf *out, int other_index, hipnx_buf *other) {
+  if (words < 0 || words >= n_inputs || n_inputs > HIPNX_FUSED_MAX_INPUTS) return set_error(HIPNX_EINVAL, "fused_words_key: input %d of %d", words, n_inputs);
+  if (key_parts < 1 || key_parts > 1 << 30 || key_index < 0 || key_index >= key_parts || other_index < 0 || other_index >= key_parts)
+    return set_error(HIPNX_EINVAL, "fused_words_key: keys %d and %d of %d", key_index, other_index, key_parts);
+  if (!other) return set_error(HIPNX_EINVAL, "fused_words_key: null key");
+  if (n < 1) return set_error(HIPNX_EUNSUPPORTED, "fused_words_key: no words");
+  const int64_t row_strides[HIPNX_FUSED_MAX_INPUTS] = {};
+  return fused_impl(ctx, n_instr, prog, n_inputs, inputs, in_dts, row_strides, in_col_strides, 1, n, -1, out_dt, out, words, key_parts, key_index, Scores(),
+                    other_index, other);
 }
 
 extern "C" int hipnx_fused_scores(hipnx_ctx *ctx, int n_instr, const hipnx_fused_instr *prog, int n_inputs, const hipnx_buf *const *inputs,

@@ -44,7 +44,8 @@ struct FusedArgs {
   const void *l, *r;
   int64_t l_outer, l_inner, l_ld, r_outer, r_inner, r_ld;
   int key_parts, key_index;  // the key is number key_index of the key_parts that in[words] splits into (0 parts: in[words] itself)
-  int unused;
+  int beside_index;          // which of the key's parts goes to `beside`, where that is not null
+  uint32_t *beside;
 };
 
 // The argument block is read where the launch put it (the kernel-argument segment, constant address
@@ -506,6 +507,11 @@ __device__ __forceinline__ void fused_words_body() {
   KernArgs a = (KernArgs)__builtin_amdgcn_kernarg_segment_ptr();
   const uint32_t *key = (const uint32_t *)a->in[P::words];
   uint32_t key1 = __builtin_amdgcn_readfirstlane(key[0]), key2 = __builtin_amdgcn_readfirstlane(key[1]);
+  if (a->beside && blockIdx.x == 0) {  // (uniform: a launch of its own cost 1.6 us on the device and 2.4 on the host)
+    uint32_t b1 = key1, b2 = key2;
+    threefry_sub_key(b1, b2, a->key_parts, a->beside_index);
+    if (threadIdx.x == 0) ((uint32_t *)a->beside)[0] = b1, ((uint32_t *)a->beside)[1] = b2;
+  }
   if (a->key_parts > 0) threefry_sub_key(key1, key2, a->key_parts, a->key_index);
   const int64_t n = a->cols, half = (n + 1) / 2, groups = (half + FE - 1) / FE;
   for (int64_t g = (int64_t)blockIdx.x * FBLOCK + threadIdx.x; g < groups; g += (int64_t)gridDim.x * FBLOCK) {

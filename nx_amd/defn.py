@@ -560,6 +560,7 @@ class _Group:
     for the backend's accumulator machine (None when the group does not fit it)."""
 
     words = None  # (input number, parts, index): that operand is a key, and the input its random words (_absorb_random)
+    beside = None  # another of the keys that operand splits into, which the launch leaves too
 
     def __init__(self, root: Tensor, members: List[Tensor], inputs: List[Tensor]):
         self.root, self.members, self.inputs = root, members, inputs
@@ -691,7 +692,8 @@ class _Group:
                 return None
         return program
 
-    def run(self, run: "_Run", out: Tensor, values: List[Tensor]):
+    def run(self, run: "_Run", out: Tensor, values: List[Tensor], results=None):
+        """`results`: where `beside` goes, if this launch is to make it."""
         mod = run.pick(values)
         fused = getattr(mod, "fused_elementwise", None) if self.program and self.layout else None
         if self.reduce is not None:
@@ -709,6 +711,10 @@ class _Group:
             return getattr(run.pick([value]), name)(out, value, opts)
         if fused is not None:
             try:
+                if results is not None:
+                    key = self.beside
+                    value, results[key.data.id] = fused(out, self.program, values, self.layout, **self.how, words=self.words, beside=(key.with_(data=None), key.data.args[2]))
+                    return value
                 return fused(out, self.program, values, self.layout, **self.how, **({"words": self.words} if self.words else {}))
             except Exception as e:  # e.g. integer instructions met while the device is capturing
                 if getattr(e, "status", None) != _EUNSUPPORTED:
@@ -1078,10 +1084,17 @@ def _absorb_random(order: List[Tensor], uses) -> None:
                 group.words = (k, parts, index)
                 e.args = [group, inputs[:k] + [key] + inputs[k + 1:]]
                 break
+    keys = []
     for node in order:
         split = _split_of(node)
         if split is not None:
             node.data.op, node.data.args = "random_key", list(split)
+            keys.append(node)
+    for node in order:  # (a sample and the key for the next one: one launch)
+        group = node.data.args[0] if node.data.op == "fused" else None
+        if isinstance(group, _Group) and group.words and group.words[1]:
+            key = node.data.args[1][group.words[0]]
+            group.beside = next((k for k in keys if k.data.args[0].data.id == key.data.id and k.data.args[1:2] == [group.words[1]] and k.data.args[2] != group.words[2]), None)
 
 
 def _over_last_axis(opts, rank: int) -> bool:
@@ -1581,7 +1594,11 @@ class _Run:
             return result
         if op == "fused":
             group, inputs = e.args
-            return group.run(self, x.with_(data=None), [self.eval(t, scope) for t in inputs])
+            values = [self.eval(t, scope) for t in inputs]
+            key = group.beside.data.id if group.__class__ is _Group and group.beside is not None else None
+            if key is not None and scope is not None and scope.counts.get(key, 0) > 0 and key not in scope.results:
+                return group.run(self, x.with_(data=None), values, scope.results)
+            return group.run(self, x.with_(data=None), values)
         if op == "dot_scaled":
             l, c1, b1, r, c2, b2, scale, mode = e.args
             lv, rv, sv = self.eval(l, scope), self.eval(r, scope), self.eval(scale, scope)

@@ -21,7 +21,7 @@ from ._lib import native
 # entry points whose effect is their result buffer's content, a function of their arguments
 _RECORDED = frozenset("hipnx_" + n for n in (
     "binary", "unary", "as_type", "reduce", "argreduce", "dot", "dot_strided", "dot_scaled", "dot_scaled_any_k", "transpose", "broadcast", "gather", "select", "clip",
-    "concat", "strided_copy", "iota", "eye", "narrow_int", "threefry2x32", "threefry_key", "fused_elementwise", "fused_words", "fused_scores"))
+    "concat", "strided_copy", "iota", "eye", "narrow_int", "threefry2x32", "threefry_key", "fused_elementwise", "fused_words", "fused_words_key", "fused_scores"))
 _lock = threading.Lock()
 
 
@@ -63,7 +63,7 @@ class _Recorder:
                 try:
                     self._drain()
                     self.ops.append(("call", C.cast(real, C.c_void_p).value, [self._argument(a, t) for a, t in zip(args, real.argtypes)]))
-                    if name in ("hipnx_fused_elementwise", "hipnx_fused_words", "hipnx_fused_scores"):
+                    if name in ("hipnx_fused_elementwise", "hipnx_fused_words", "hipnx_fused_words_key", "hipnx_fused_scores"):
                         self.modes.add(B._fused_set.get(self.device, "interpreted"))
                 except Exception:  # the evaluation goes on, whatever becomes of its recording
                     self.failed = True

@@ -135,3 +135,23 @@ def test_words_made_inside_a_compiled_group(shape, hip):
         assert not calls or shape == (1,), name
         for g, w in zip(got, defn.compile(fun, key, other)._walk([key, other])):
             assert_bits_equal(g, w, f"{name} {shape}")
+
+
+# The sample and the key for the next one, in one launch where the split's other part is what is asked for
+@pytest.mark.parametrize("count", [2, 7, 8, 513, 70001])
+@pytest.mark.parametrize("order", ["sample first", "key first", "both keys", "three parts"])
+def test_a_sample_and_the_next_key_of_one_split(count, order, hip):
+    from nx_amd import defn
+    from nx_amd import random as Random
+
+    def program(key):
+        keys = Random.split(key, 3 if order == "three parts" else 2)
+        sample, after = Random.normal_split(Nx.squeeze(Nx.slice(keys, [1, 0], [1, 2]), axes=[0]), shape=(count,)), Nx.squeeze(Nx.slice(keys, [0, 0], [1, 2]), axes=[0])
+        if order == "key first":
+            return after, sample
+        return (sample, after, Nx.squeeze(Nx.slice(keys, [1, 0], [1, 2]), axes=[0])) if order == "both keys" else (sample, after)
+    key = Random.key(2024 + count, backend=hip)
+    planned = defn.compile(program, key, fuse="compiled")
+    want = [Nx.to_binary(t) for t in program(key)]
+    for _ in range(5):  # (evaluated, recorded, issued from the recording)
+        assert [Nx.to_binary(t) for t in planned(key)] == want
