@@ -1409,7 +1409,7 @@ def _settings_changed() -> None:
     old settings to the old one."""
     from . import nx
     _settings[0] = (_bounds["policy"], _bf16["rounding"], tuple(sorted(kv for kv in _fused_modes.items() if kv[1] != "interpreted")))
-    nx._ready = {}
+    nx._ready, nx._bound, nx._capturing = {}, {}, _capturing
 
 
 _settings_changed()

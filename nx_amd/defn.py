@@ -1668,6 +1668,9 @@ class Compiled:
         self.plans: Dict[Any, _Plan] = {}
         self.plan = _Plan(roots, 0, self.plans)
         self.replay = None     # the recording in use (replay.py)
+        # how results are handed out: one, a tuple of them in order, or what _unflatten makes of them
+        self.one = isinstance(structure, _Leaf)
+        self.row = structure.__class__ is tuple and [getattr(s, "index", -1) for s in structure] == list(range(len(roots)))
         self.recordings = {}   # settings -> what is known of recordings under them
 
     def _params(self, args):
@@ -1709,6 +1712,10 @@ class Compiled:
         return results
 
     def __call__(self, *args):
+        if self.replay is not None:  # tensors as they were traced, one by one: the recording looks at them itself
+            results = self.replay.run(args)
+            if results is not None:
+                return results[0] if self.one else tuple(results) if self.row else _unflatten(self.structure, results)
         return _unflatten(self.structure, self._evaluate(self._params(args)))
 
     def capture(self, *args) -> "Captured":

@@ -223,6 +223,21 @@ def _make_ready(key, mod, *args):
             table[key] = call
 
 
+# Of those, the ones with a number: the call with the number's constant in it, and the default backend the constant is on.  Not
+# while a device is capturing, whose constants are the graph's own.
+_bound = {}
+_capturing = ()  # (the device backend's devices that are)
+
+
+def _bind(key, call, number):
+    table = _bound  # (replaced together with _ready)
+    if len(table) >= 1024:
+        table.clear()
+    bound = call.bind(1, number)
+    if bound is not None:
+        table[key] = (bound, getattr(_state, "backend", None) or _global_default[0])
+
+
 def _number_or_type(x):
     return x if isinstance(x, (int, float)) and not isinstance(x, bool) else to_tensor(x).type
 
@@ -236,10 +251,19 @@ def _binary(name, left, right, out_type_fun):
         elif right.__class__ is float or (right.__class__ is int and left.type[0] != "u" and left.type[0] != "s"):
             key, r = (name, left.type, left.shape, right.__class__), None
         if key is not None:
+            if r is None and right:  # (zeros: two of them are equal)
+                bound = _bound.get((key, right))
+                if bound is not None and bound[1] is (getattr(_state, "backend", None) or _global_default[0]) and not _capturing:
+                    out = bound[0](left)
+                    if out is not None:
+                        return out
             ready = _ready.get(key)
             if ready is not None:
-                out = ready(left, to_tensor(right) if r is None else r)
+                number = to_tensor(right) if r is None else r
+                out = ready(left, number)
                 if out is not None:
+                    if r is None and right and not _capturing:
+                        _bind((key, right), ready, number)
                     return out
     if left.__class__ is Tensor and right.__class__ is Tensor:  # the common case: no number to look at
         ty = left.type if left.type == right.type else T.merge(left.type, right.type)

@@ -38,6 +38,7 @@ class _Recorder:
         self.slots, self.n_slots = {}, 0  # handle -> slot while the buffer lives
         self.ops, self.keep, self.freed, self.modes = [], [], [], set()
         self.failed, self.settings = False, B.settings()
+        self.shapes = tuple((p.type, p.shape) for p in params)
         for p in params:
             self._slot(p.data.ref.handle)
         self.n_params = self.n_slots
@@ -113,7 +114,8 @@ class _Recorder:
 
 
 class Replay:
-    """A recorded evaluation: `run(params)` gives its results, or None where it does not apply."""
+    """A recorded evaluation: `run(params)` gives its results, or None where it does not apply (to tensors of other types and
+    shapes, or to what is no tensor, too)."""
 
     def __init__(self, calls, device, mode, constants, settings):
         self.calls, self.device, self.mode, self.constants = calls, device, mode, constants
@@ -122,8 +124,8 @@ class Replay:
     def run(self, params):
         if B._capturing or self.settings != B.settings():
             return None
-        mod, opts = Nx.default_backend()
-        if mod is not self.backend[0] or opts != self.backend[1]:
+        backend = Nx.default_backend()
+        if backend is not self.backend and (backend[0] is not self.backend[0] or backend[1] != self.backend[1]):
             return None
         if self.mode is not None and B._fused_set.get(self.device, "interpreted") != self.mode:
             B._set_fused_mode(self.mode, self.device)
@@ -238,6 +240,6 @@ def _finish(rec, results):
             return a
         return (a[0], [to[s] for s in a[1]] if a[0] == "list" else to[a[1]])
     ops = [(op[0], op[1], [moved(a) for a in op[2]]) if op[0] == "call" else (op[0], to[op[1]], op[2] if op[0] == "alloc" else 0) for op in rec.ops]
-    calls = native.record(ops, rec.n_params + len(late), rec.n_slots, [(to[o[0]],) + o[1:] for o in outs], rec.ctx, rec.ctx.value, rec.device, rec.keep)
+    calls = native.record(ops, rec.n_params + len(late), rec.n_slots, [(to[o[0]],) + o[1:] for o in outs], rec.ctx, rec.ctx.value, rec.device, rec.keep, rec.shapes)
     constants = [Nx.Tensor(B.HipNxBackend(ref, rec.device), "u8", ()) for _, ref in rec.late]
     return Replay(calls, rec.device, rec.modes.pop() if rec.modes else None, constants, rec.settings)

@@ -276,6 +276,50 @@ def a_refused_attempt_is_not_made_again():
     assert standin.counts["hipnx_fused_scores"] == 3
 
 
+def a_number_laid_out_with_its_call_is_that_number():
+    """Numbers of both kinds, zeros of both signs, other tensors, other default backends, more numbers than are kept."""
+    x, y = f32(1, 2, 4), f32(3, 5, 7)
+    for _ in range(4):
+        assert read(Nx.multiply(x, 0.5)) == [0.5, 1, 2] and read(Nx.multiply(y, 0.5)) == [1.5, 2.5, 3.5] and read(Nx.multiply(x, 3)) == [3, 6, 12]
+        assert read(Nx.multiply(x, 3.0)) == [3, 6, 12] and str(read(Nx.multiply(x, 0.0))) == "[0.0, 0.0, 0.0]"
+        assert str(read(Nx.multiply(x, -0.0))) == "[-0.0, -0.0, -0.0]" and read(Nx.multiply(x, True)) == [1, 2, 4]
+        assert all(v != v for v in read(Nx.add(x, float("nan"))))
+    assert any(k[1] == 0.5 for k in Nx._bound) and not any(k[1] == 0 for k in Nx._bound)
+    gone = f32(1, 2, 4)
+    assert Nx.backend_deallocate(gone) == "ok"
+    raises(lambda: Nx.multiply(gone, 0.5), "deallocated")
+    for i in range(3000):
+        assert read(Nx.add(x, i + 0.5)) == [1 + i + 0.5, 2 + i + 0.5, 4 + i + 0.5]
+    assert len(Nx._bound) <= 1024 and read(Nx.multiply(x, 0.5)) == [0.5, 1, 2]
+    previous = B.bf16_rounding("nearest_even")
+    assert not Nx._bound and read(Nx.multiply(x, 0.5)) == [0.5, 1, 2]
+    B.bf16_rounding(previous)
+    for _ in range(3):
+        Nx.multiply(x, 0.5)
+    Nx.default_backend(HostBinary)  # (its constants follow the tensor: no number of the device's is taken for one of its own)
+    assert read(Nx.multiply(x, 0.5)) == [0.5, 1, 2]
+    Nx.default_backend(Hip)
+
+
+def what_a_recording_was_not_made_for_is_evaluated_or_refused():
+    """Arguments of other types, shapes and kinds go the general way, with what it says of them."""
+    x, y = f32(1, 2, 4), f32(3, 5, 7)
+    f = defn.compile(lambda a, b: (Nx.add(a, b), Nx.multiply(a, 2.0)), x, y)
+    for _ in range(5):
+        total, twice = f(x, y)
+    assert f.replay is not None and read(total) == [4, 7, 11] and read(twice) == [2, 4, 8]
+    raises(lambda: f(x, f32(1, 2)), "traced for")
+    raises(lambda: f(x, from_numpy(np.asarray([1, 2, 4], np.int32), "s32", Hip)), "traced for")
+    raises(lambda: f(x), "expected 2")
+    raises(lambda: f(x, y, y), "expected 2")
+    one = defn.compile(lambda a, s: Nx.multiply(a, s), x, 2.0)
+    for k in range(6):
+        assert read(one(x, float(k))) == [k, 2 * k, 4 * k]
+    pair = defn.compile(lambda ab: {"d": Nx.subtract(ab[0], ab[1])}, (x, y))
+    for _ in range(6):
+        assert read(pair((x, y))["d"]) == [-2, -3, -3]
+
+
 def a_lender_that_holds_what_it_lent_to_is_collected():
     import gc
     import weakref
