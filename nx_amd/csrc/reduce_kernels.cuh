@@ -18,6 +18,7 @@
 // (tie HIGH) index.
 // Algorithmic traffic: bytes(in) + bytes(out).
 #pragma once
+#include <algorithm>
 #include <type_traits>
 #include <utility>
 
@@ -310,6 +311,68 @@ reduce_cols_once_kernel(const void *__restrict__ in, void *__restrict__ out, int
   if (ty == 0 && col < inner) finalize(out, odt, o * inner + col, sm[tx]);
 }
 
+// Columns under a long axis, in segments: a work-group takes 16 X bytes of adjacent columns, 16 bytes a lane at whatever address
+// they have, its rows of X lanes a run of the reduced axis each, eight loads in flight; the runs are folded in order in LDS, so that a
+// segment leaves one partial result a column however many waves shared it.  Bound by memory from some 64 MB on and by
+// two launches below.  (A lane per eight columns and segment, as below, needs a segment per wave: hundreds of partial results a
+// column, or a chip that is idle; and the last lane of a ragged row reads its columns one by one while the others wait.
+// us per call, so / here: f32 [20000, 300] 34.1 / 9.6, [200000, 300] 216 / 49, [25000, 2047] 100 / 41, [6000, 10007] 116 / 46,
+// [16384, 4096] 50.8 / 43.6, [5000, 1600] 12.4 / 8.9; bf16 [20000, 300] 31.5 / 9.2, [60000, 1024] 37.6 / 27.7, [16384, 4096] 33.5 / 26.2.)
+constexpr int cols_tile_lanes(int dt) { return reduce_type_bytes(dt) == 4 ? 1024 : 512; }  // (32 KiB of f64 sums in LDS)
+template <int IDT, int X_>
+struct ColsTile {
+  static constexpr int V = 16 / reduce_type_bytes(IDT), X = X_, Y = cols_tile_lanes(IDT) / X, C = X * V, LANES = cols_tile_lanes(IDT), BATCH = 8;
+};
+template <typename R, typename CT, int IDT, int X_>
+__global__ void __launch_bounds__(cols_tile_lanes(IDT))
+reduce_cols_tile_kernel(const void *__restrict__ in, void *__restrict__ out, typename R::acc_t *__restrict__ partial, int odt,
+                        int64_t red, int64_t inner, int64_t run, int nseg) {
+  typedef ColsTile<IDT, X_> T;
+  typedef typename R::acc_t acc_t;
+  constexpr int V = T::V, X = T::X, Y = T::Y, C = T::C, BATCH = T::BATCH;
+  __shared__ acc_t sm[Y][C];
+  const int tx = threadIdx.x % X, ty = threadIdx.x / X, seg = blockIdx.y;
+  const int64_t o = blockIdx.z, col = (int64_t)blockIdx.x * C + tx * V;
+  const int64_t first = col + V <= inner ? col : inner - V;  // a row's last vector ends with it (a row has one, the host sees to it)
+  const int64_t k0 = ((int64_t)seg * Y + ty) * run, k1 = k0 + run < red ? k0 + run : red;
+  acc_t acc[V];
+#pragma unroll
+  for (int i = 0; i < V; i++) acc[i] = R::init();
+  if (col < inner && k0 < k1) {
+#pragma unroll
+    for (int i = 0; i < V; i++) acc[i] = R::seed(acc[i], k0);
+    const int64_t base = o * red * inner + first;
+    for (int64_t k = k0; k < k1; k += BATCH) {
+      CT v[BATCH][V];
+#pragma unroll
+      for (int u = 0; u < BATCH; u++) load_vec<CT, V, false>(in, IDT, base + (k + u < k1 ? k + u : k1 - 1) * inner, v[u]);
+#pragma unroll
+      for (int u = 0; u < BATCH; u++)
+        if (k + u < k1)
+#pragma unroll
+          for (int i = 0; i < V; i++) acc[i] = R::accumulate(acc[i], v[u][i], k + u);
+    }
+  }
+  const int over = (int)(col - first);  // columns of the vector that are the lane before's
+#pragma unroll
+  for (int i = 0; i < V; i++)
+    if (col < inner && i >= over) sm[ty][tx * V + i - over] = acc[i];
+  __syncthreads();
+#pragma unroll
+  for (int w = 1; w < Y; w *= 2) {  // neighbouring runs first: in order
+    for (int j = threadIdx.x; j < Y / (2 * w) * C; j += T::LANES) {
+      const int r = j / C * 2 * w, c = j % C;
+      sm[r][c] = R::combine(sm[r][c], sm[r + w][c]);
+    }
+    __syncthreads();
+  }
+  const int64_t c = (int64_t)blockIdx.x * C + threadIdx.x;
+  if ((int)threadIdx.x < C && c < inner) {
+    if (nseg == 1) finalize(out, odt, o * inner + c, sm[0][threadIdx.x]);
+    else partial[(o * nseg + seg) * inner + c] = sm[0][threadIdx.x];
+  }
+}
+
 // fold partial[outer, nseg, inner] -> out[outer, inner].  A work-group takes 32 adjacent outputs; its eight rows
 // of 32 lanes each fold a slice of the segments (four loads in flight per lane), and the first row folds the eight
 // slices in segment order.  (One lane per output walking all segments is a chain of up to 1024 dependent
@@ -484,6 +547,41 @@ static int run_reduce_t(hipnx_ctx *ctx, bool static_ws, int idt, int odt, int64_
         HIPNX_HIP(hipGetLastError());
         return HIPNX_OK;
       }
+    }
+    if constexpr (std::is_floating_point<acc_t>::value && (IDT == HIPNX_F32 || IDT == HIPNX_BF16 || IDT == HIPNX_F16)) {
+      auto tile = [&](auto x) -> int {
+        typedef ColsTile<IDT, decltype(x)::value> T;
+        const int64_t groups = (inner + T::C - 1) / T::C, want = (int64_t)ctx->num_cus * 2 * (1024 / T::LANES);
+        if (red < T::Y * T::BATCH || outer > 65535 || outer * groups >= want) return -1;
+        int64_t nseg = std::min<int64_t>(want / (outer * groups), red / (T::Y * T::BATCH));
+        if (nseg < 1) nseg = 1;
+        const int64_t run = (red + nseg * T::Y - 1) / (nseg * T::Y);
+        nseg = (red + run * T::Y - 1) / (run * T::Y);
+        if (static_ws && sizeof(acc_t) * (size_t)(outer * nseg * inner) > HIPNX_REDUCE_STATIC_SCRATCH_BYTES) return -1;
+        acc_t *partial = nullptr;
+        void *ws = nullptr;
+        size_t ws_cap = 0;
+        if (nseg > 1) {
+          if (int st = partials_acquire(ctx, static_ws, sizeof(acc_t) * (size_t)(outer * nseg * inner), &ws, &ws_cap)) return st;
+          partial = (acc_t *)ws;
+        }
+        hipLaunchKernelGGL((reduce_cols_tile_kernel<R, CT, IDT, T::X>), dim3((unsigned)groups, (unsigned)nseg, (unsigned)outer), dim3(T::LANES), 0, ctx->stream,
+                           in, out, partial, odt, red, inner, run, (int)nseg);
+        if (nseg > 1) {
+          const int64_t b2 = (outer * inner + COMBINE_COLS_X - 1) / COMBINE_COLS_X;
+          hipLaunchKernelGGL((combine_cols_kernel<R>), dim3((unsigned)(b2 < MAX_BLOCKS ? b2 : MAX_BLOCKS)), dim3(BLOCK), 0, ctx->stream, partial, out, odt, outer, inner, (int)nseg);
+        }
+        partials_release(ctx, static_ws, ws, ws_cap);
+        HIPNX_HIP(hipGetLastError());
+        return HIPNX_OK;
+      };
+      // Rows of 32 KiB and more of whole vectors stay with the kernel below (f32 [16384, 8192] 90 us there, 100 here); so do rows
+      // that leave most of a work-group's columns empty.  Wider work-groups read a large input in longer runs (f32 [200000, 300] 55 us
+      // by 16 lanes to a row, 49 by 32, 55 by 64), narrower ones leave more of them to a small one (bf16 [20000, 300] 9.2 / 11.4 / 12.4).
+      const int64_t bytes = outer * red * inner * dtype_size(idt), row = inner * dtype_size(idt);
+      const int st = row < 128 || (inner % E == 0 && row >= 32768) ? -1 : bytes >= (32ll << 20) && row >= 512 ? tile(std::integral_constant<int, 32>{})
+                                                                                                 : tile(std::integral_constant<int, 16>{});
+      if (st >= 0) return st;
     }
     const bool vec = inner % E == 0;
     const bool unal = !vec && inner >= 8 * E && IDT >= 0;  // long rows off the vector grid (compiled for the common element types)

@@ -417,3 +417,39 @@ def test_few_columns_in_one_launch(outer, red, inner, ty, hip, oracle):
     h, o = from_numpy(arr, ty, hip), from_numpy(arr, ty, oracle)
     for op in ("sum", "reduce_max"):
         assert_bits_equal(getattr(Nx, op)(h, axes=[1]), getattr(Nx, op)(o, axes=[1]), f"{op}, NaN")
+
+
+# columns under a long axis in segments: one segment and several, the last run of a segment short or empty, columns on either side of a
+# work-group's 64, 128 and 256, a row's last vector off its end, outer items beside them, inputs on either side of 32 MiB
+@pytest.mark.parametrize("ty", ["f32", "bf16", "f16"])
+@pytest.mark.parametrize("outer,red,inner", [(1, 4096, 257), (1, 4097, 300), (1, 5000, 777), (3, 513, 65), (2, 1025, 128), (70, 512, 64), (5, 700, 33), (1, 9001, 1001),
+                                             (1, 520, 20003), (1, 17000, 1030), (2, 40007, 259), (1, 4096, 4096)])
+def test_columns_in_segments(outer, red, inner, ty, hip):
+    """On whole numbers, whose sums are exact and of which the extremes are the same in any order."""
+    rng = np.random.default_rng(seed_of(outer, red, inner, ty, "segments"))
+    v = rng.integers(-2, 3, size=(outer, red, inner)).astype(np.float32)
+    v[0, red - 1, inner - 1], v[-1, 0, 0] = 7, -7  # the ends of the slab
+    arr = (v.view(np.uint32) >> 16).astype(np.uint16) if ty == "bf16" else v.astype(np.float16 if ty == "f16" else np.float32)
+    h = from_numpy(arr, ty, hip)
+    sums = v.sum(axis=1, dtype=np.float64)
+    want = (sums.astype(np.float32).view(np.uint32) & np.uint32(0xFFFF0000)).view(np.float32) if ty == "bf16" else sums.astype(np.float16 if ty == "f16" else np.float32)
+    np.testing.assert_array_equal(values(Nx.sum(h, axes=[1])), want.astype(np.float64))
+    np.testing.assert_array_equal(values(Nx.reduce_max(h, axes=[1])), v.max(axis=1))
+    np.testing.assert_array_equal(values(Nx.reduce_min(h, axes=[1])), v.min(axis=1))
+
+
+@pytest.mark.parametrize("ty", ["f32", "bf16", "f16"])
+@pytest.mark.parametrize("op", ["sum", "product", "reduce_max", "reduce_min", "all", "any"])
+def test_special_values_in_columns_in_segments(ty, op, hip, oracle):
+    """Infinities, NaN, zeros of either sign: the oracle's results, of two zeros the first."""
+    red, inner = 4099, 300
+    rng = np.random.default_rng(seed_of(ty, op, "special"))
+    v = np.where(rng.random((red, inner)) < 0.5, 0.0, -0.0).astype(np.float32)
+    if op in ("product", "all"):
+        v = np.where(rng.random((red, inner)) < 0.5, 1.0, -1.0).astype(np.float32)
+        v[red // 2, 40:80] = -0.0
+    v[red - 1, 0:20], v[0, 10:30], v[red // 3, 15:25] = np.inf, -np.inf, 1.0
+    v[red // 2, 100:110] = np.nan
+    v[7, 250:] = np.inf
+    arr = (v.view(np.uint32) >> 16).astype(np.uint16) if ty == "bf16" else v.astype(np.float16 if ty == "f16" else np.float32)
+    assert_bits_equal(getattr(Nx, op)(from_numpy(arr, ty, hip), axes=[0]), getattr(Nx, op)(from_numpy(arr, ty, oracle), axes=[0]), f"{op} {ty}")
