@@ -348,6 +348,7 @@ as_type_kernel(const void *__restrict__ in, void *__restrict__ out, int idt_, in
 // ---- host side ------------------------------------------------------------------------------
 
 // elementwise_flat.hip: whether it took the call
+bool binary_mixed(const hipnx_ctx *ctx, int op, int l_dt, int r_dt, int out_dt, const void *l, const void *r, void *out, int64_t n, int64_t ls, int64_t rs);
 bool binary_flat(const hipnx_ctx *ctx, int op, int dt, const void *l, const void *r, void *out, int64_t total, int64_t cols,
                  int64_t l0, int64_t l1, int64_t r0, int64_t r1);
 
@@ -555,6 +556,11 @@ extern "C" int hipnx_binary(hipnx_ctx *ctx, int op, int l_dt, int r_dt, int out_
     }
   }
   if (m == 0) { dims[0] = 1; ls[0] = 0; rs[0] = 0; m = 1; }
+
+  if (m == 1 && binary_mixed(ctx, op, l_dt, r_dt, out_dt, l->ptr, r->ptr, out->ptr, n, ls[0], rs[0])) {
+    HIPNX_HIP(hipGetLastError());
+    return HIPNX_OK;
+  }
 
   bool vec_ok = false;
   BinArgs a{};

@@ -1,5 +1,6 @@
 // Binary operations of a dense [rows, cols] tensor with a row [cols] or one value per row where a row is not whole vectors of
-// eight elements (a table of 100 features and their means, a bias of 10 classes): float types, one type throughout.
+// eight elements (a table of 100 features and their means, a bias of 10 classes): float types, one type throughout.  And
+// two forms of mixed types: a mean's quotient of sums and a whole number, and values times a mask.
 #include <type_traits>
 
 #include "elementwise_ops.cuh"
@@ -92,6 +93,54 @@ static bool flat_any(std::integer_sequence<int, OPS...>, const hipnx_ctx *ctx, i
   bool took = false;
   (void)((op == OPS ? (took = flat_op<OPS>(ctx, dt, l_dense, per_row, dense, other, out, total, cols, step), true) : false) || ...);
   return took;
+}
+
+// W consecutive elements a lane.  NUMBER: the right operand is one element.
+// (The kernel that reads its operands' types as it runs is some thousand instructions, which a launch of a few waves spends its time
+// fetching, the more so behind a pass that went through the caches.  us, there / here: 100 f32 sums over an s32 count behind
+// 268 MB 8.0 / 4.8, 300 behind 24 MB 6.4 / 1.9; f32 [4096, 512] times a u8 mask 6.9 / 3.4.)
+template <int OP, typename CT, int LDT, int RDT, int W, bool NUMBER>
+__global__ void __launch_bounds__(BLOCK)
+binary_mixed_kernel(const void *__restrict__ l, const void *__restrict__ r, void *__restrict__ out, uint32_t n) {
+  const uint32_t f0 = (blockIdx.x * (uint32_t)BLOCK + threadIdx.x) * W;
+  if (f0 >= n) return;
+  CT a[W], b[W], c[W];
+  if (n - f0 >= (uint32_t)W) {
+    load_vec<CT, W>(l, LDT, f0, a);
+    if constexpr (NUMBER) {
+      b[0] = load_one<CT>(r, RDT, 0);
+#pragma unroll
+      for (int i = 1; i < W; i++) b[i] = b[0];
+    } else load_vec<CT, W>(r, RDT, f0, b);
+#pragma unroll
+    for (int i = 0; i < W; i++) c[i] = binary_apply<OP, CT, false>(a[i], b[i]);
+    store_vec<CT, W>(out, LDT, f0, c);
+  } else {
+    for (uint32_t f = f0; f < n; f++)
+      store_one<CT>(out, LDT, f, binary_apply<OP, CT, false>(load_one<CT>(l, LDT, f), load_one<CT>(r, RDT, NUMBER ? 0 : f)));
+  }
+}
+
+// Flat operands of n elements, ls / rs 1 or (one element for all) 0, the result of the float operand's type:
+//   float / one s32 number, computed in f64 as any operation with a 32-bit integer is, of up to 2^16 elements (a lane each; more are
+//   bound by memory, not by the launch);
+//   f32 * u8, either way round (a product commutes), below 2^31 elements.
+bool binary_mixed(const hipnx_ctx *ctx, int op, int l_dt, int r_dt, int out_dt, const void *l, const void *r, void *out, int64_t n, int64_t ls, int64_t rs) {
+  if (op == HIPNX_DIVIDE && r_dt == HIPNX_S32 && l_dt == out_dt && (ls == 1 || n == 1) && (rs == 0 || n == 1) && n <= (1 << 16)) {
+    const dim3 grid((unsigned)((n + BLOCK - 1) / BLOCK)), block(BLOCK);
+    if (l_dt == HIPNX_F32) hipLaunchKernelGGL((binary_mixed_kernel<HIPNX_DIVIDE, double, HIPNX_F32, HIPNX_S32, 1, true>), grid, block, 0, ctx->stream, l, r, out, (uint32_t)n);
+    else if (l_dt == HIPNX_BF16) hipLaunchKernelGGL((binary_mixed_kernel<HIPNX_DIVIDE, double, HIPNX_BF16, HIPNX_S32, 1, true>), grid, block, 0, ctx->stream, l, r, out, (uint32_t)n);
+    else if (l_dt == HIPNX_F16) hipLaunchKernelGGL((binary_mixed_kernel<HIPNX_DIVIDE, double, HIPNX_F16, HIPNX_S32, 1, true>), grid, block, 0, ctx->stream, l, r, out, (uint32_t)n);
+    else return false;
+    return true;
+  }
+  const bool masked = l_dt == HIPNX_F32 && r_dt == HIPNX_U8, mask_first = l_dt == HIPNX_U8 && r_dt == HIPNX_F32;
+  if (op == HIPNX_MULTIPLY && out_dt == HIPNX_F32 && (masked || mask_first) && ls == 1 && rs == 1 && n < (1ll << 31)) {
+    const dim3 grid((unsigned)((n + 4 * BLOCK - 1) / (4 * BLOCK))), block(BLOCK);
+    hipLaunchKernelGGL((binary_mixed_kernel<HIPNX_MULTIPLY, float, HIPNX_F32, HIPNX_U8, 4, false>), grid, block, 0, ctx->stream, masked ? l : r, masked ? r : l, out, (uint32_t)n);
+    return true;
+  }
+  return false;
 }
 
 // Strides per row (l0, r0) and column (l1, r1; 0 or 1) of both operands; total < 2^31.  Taken where one operand is as dense as

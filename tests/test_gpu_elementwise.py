@@ -498,3 +498,29 @@ def test_short_rows_on_special_values(rows, cols, ty, op, hip, oracle):
             assert np.array_equal(g.view(_uint(g.dtype))[fixed], w.view(_uint(w.dtype))[fixed]), f"{op} {ty} {rows}x{cols} {shape}"
             tol = {"f16": 2e-3, "bf16": 1.6e-2, "f32": 2e-6}[ty] if op == "atan2" else 0.0  # (a library function on either side)
             assert (np.abs(gf[~fixed] - wf[~fixed]) <= tol * np.abs(wf[~fixed])).all(), f"{op} {ty} {rows}x{cols} {shape}"
+
+
+SPECIAL = [0.0, -0.0, 1.0, -1.5, np.inf, -np.inf, np.nan, 1e-40, -1e36, 6e-8, 60000.0]
+
+
+# a whole number that counts, behind sums: one element, a wave, blocks and one element more, the longest the small kernel takes and one more
+@pytest.mark.parametrize("ty", ["f32", "bf16", "f16"])
+@pytest.mark.parametrize("n", [1, 7, 256, 257, 65536, 65537])
+@pytest.mark.parametrize("count", [1, 3, -7, 0, 20000, 16777217, -2147483648])
+def test_quotients_by_a_whole_number(ty, n, count, hip, oracle):
+    rng = np.random.default_rng(seed_of(ty, n, count, "count"))
+    x = np.resize(np.concatenate([SPECIAL if ty != "f16" else [v for v in SPECIAL if abs(v) < 1e30 or not np.isfinite(v)], rng.uniform(-1e4, 1e4, size=256)]), n).astype(np.float32)
+    arr = (x.view(np.uint32) >> 16).astype(np.uint16) if ty == "bf16" else x.astype(np.float16 if ty == "f16" else np.float32)
+    h, o = both(arr, ty, hip, oracle)
+    hc, oc = both(np.array(count, np.int32), "s32", hip, oracle)
+    assert_bits_equal(Nx.divide(h, hc), Nx.divide(o, oc), f"{ty} [{n}] / {count}")
+
+
+@pytest.mark.parametrize("shape", [(1,), (3,), (1024,), (1025,), (333, 250), (4, 5, 7)])
+def test_values_times_a_mask(shape, hip, oracle):
+    rng = np.random.default_rng(seed_of(shape, "mask"))
+    x = np.resize(np.concatenate([SPECIAL, rng.uniform(-1e4, 1e4, size=500)]), shape).astype(np.float32)
+    m = rng.choice(np.array([0, 1, 1, 255], np.uint8), size=shape)
+    (hx, ox), (hm, om) = both(x, "f32", hip, oracle), both(m, "u8", hip, oracle)
+    assert_bits_equal(Nx.multiply(hx, hm), Nx.multiply(ox, om), "x * mask")
+    assert_bits_equal(Nx.multiply(hm, hx), Nx.multiply(om, ox), "mask * x")
