@@ -195,40 +195,43 @@ __device__ __forceinline__ double fma_const(double p, double w, double c) {
   return d;
 }
 
+// the first step of one, w * c1 + c0: one constant in scalar registers (an instruction reads one such pair), the other in vector registers,
+// which the compiler fills once for all elements of a lane
+__device__ __forceinline__ double fma_consts(double w, double c1, double c0) {
+  double d;
+  asm("v_fma_f64 %0, %1, %2, %3" : "=v"(d) : "v"(w), "s"(c1), "v"(c0));
+  return d;
+}
+
 // The same for an f32 operand (the f32 class of the kernels).  Bound by f64 instructions, each of which costs a SIMD as
 // much as an f32 one; the form above takes about 190, most of them in the library's log, which serves every double, and
-// in separate products and sums.  Here the logarithm is written for what can occur, y = (1 - x)(1 + x) in [2^-23, 1]:
-// y = 2^k m with m in [1/sqrt(2), sqrt(2)), found by adding to the high word (as the logarithms of the FreeBSD and musl math
-// libraries do), log m = 2 atanh(s), s = (m - 1) / (m + 1), the series of atanh in z = s^2
+// in separate products and sums.  Here the logarithm is written for what can occur, y = 1 - x^2 in [2^-23, 1]:
+// y = 2^e m with m in [1/2, 1), c = 1/sqrt(2), log(m / c) = 2 atanh(s), s = (m - c) / (m + c), the series of atanh in z = s^2
 // beyond its first term as a polynomial of degree 6 (interpolated at the Chebyshev points of z in [0, 0.02945]; its
-// error is below 2^-57 of log m), the quotient from v_rcp_f64 and two Newton steps; the polynomials are fused
-// multiply-adds.  The polynomials' argument w - 2.5 has one rounding of its own size as above, p one less per step: against
-// the same polynomials in 80 bits either form is within 3.6e-16 (2^26 arguments, half of them next to +-1, the forms written
-// out for the CPU; none of them rounded to another f32 by either).  So a result is the reference's but where the f64 value
-// lies that close to halfway between two floats: the last bit, about once in 2^25.  No branch but the rare one: w >= 5 is |x| > 0.99662, and everything that is
-// not inside (-1, 1) goes the same way.  2^26 normal samples, the chain behind the cipher: 320 us by the form above,
-// 195 with this log and the compiler's v_fmac, 151 as it is.
+// error is below 2^-57 of the logarithm), the quotient from v_rcp_f64 and one correction by its remainder; the polynomials are fused
+// multiply-adds.  Only w - 2.5 is wanted, in absolute terms, so that log c may stand in its constant although e ln 2 cancels it near y = 1.
+// The polynomials' argument has one rounding of its own size as above, p one less per step: against
+// the same polynomials in 80 bits either form is within 3.7e-16 (every multiple of 2^-23 in (-1, 1) and 7.7 M arguments spread over the
+// exponents and towards +-1, the forms written out for the CPU with a reciprocal of 2^-25; none of them rounded to another f32 by either).  So a result is
+// the reference's but where the f64 value lies that close to halfway between two floats: the last bit, about once in 2^25.  No branch but the
+// rare one: w >= 5 is |x| > 0.99662, and everything that is not inside (-1, 1) goes the same way.  2^26 normal samples, the chain behind the
+// cipher: 320 us by the form above, 195 with the logarithm about m = 1 and the compiler's v_fmac, 151 with constants in scalar registers;
+// cipher and chain in one kernel then 186.6, and 174.4 as it is.
 __device__ __forceinline__ float erf_inv_f32(float xf) {
-  const double x = (double)xf, y = (1.0 - x) * (1.0 + x);
-  const uint64_t bits = __builtin_bit_cast(uint64_t, y);
-  const uint32_t hi = (uint32_t)(bits >> 32) + (0x3FF00000u - 0x3FE6A09Eu);  // (0x3FE6A09E: the high word of 1/sqrt(2))
-  const double k = (double)((int)(hi >> 20) - 0x3FF);
-  const double m = __builtin_bit_cast(double, ((uint64_t)((hi & 0xFFFFFu) + 0x3FE6A09Eu) << 32) | (uint32_t)bits);
-  const double f = m - 1.0, d = m + 1.0;
-  double r = __builtin_amdgcn_rcp(d);
-  r = __builtin_fma(__builtin_fma(-d, r, 1.0), r, r);
-  r = __builtin_fma(__builtin_fma(-d, r, 1.0), r, r);
-  const double s = f * r, z = s * s;
-  double q = __builtin_fma(z, 0x1.2b5b5fb2eac92p-3, 0x1.39fe208c33457p-3);
+  const double x = (double)xf, y = __builtin_fma(-x, x, 1.0);
+  const double e = (double)__builtin_amdgcn_frexp_exp(y), m = __builtin_amdgcn_frexp_mant(y);
+  const double f = m - 0x1.6a09e667f3bcdp-1, d = m + 0x1.6a09e667f3bcdp-1, r = __builtin_amdgcn_rcp(d), s0 = f * r;
+  const double s = __builtin_fma(__builtin_fma(-d, s0, f), r, s0), z = s * s;
+  double q = fma_consts(z, 0x1.2b5b5fb2eac92p-3, 0x1.39fe208c33457p-3);
   q = fma_const(q, z, 0x1.7462b69705382p-3);
   q = fma_const(q, z, 0x1.c71c62debf86bp-3);
   q = fma_const(q, z, 0x1.2492492df6947p-2);
   q = fma_const(q, z, 0x1.99999999952b2p-2);
   q = fma_const(q, z, 0x1.5555555555558p-1);
   q = fma_const(q, z, 2.0);
-  // w - 2.5, w = -(k ln 2 + log m)
-  double w = __builtin_fma(-s, q, __builtin_fma(k, -0x1.62e42fefa39efp-1, -2.5));
-  double p = __builtin_fma(w, 2.81022636e-08, 3.43273939e-07);
+  // w - 2.5, w = -(e ln 2 + log c + 2 atanh(s))
+  double w = __builtin_fma(-s, q, fma_consts(e, -0x1.62e42fefa39efp-1, 0x1.62e42fefa39efp-2 - 2.5));
+  double p = fma_consts(w, 2.81022636e-08, 3.43273939e-07);
   p = fma_const(p, w, -3.5233877e-06);
   p = fma_const(p, w, -4.39150654e-06);
   p = fma_const(p, w, 0.00021858087);
