@@ -42,14 +42,14 @@ static int launch_one(const hipnx_ctx *ctx, GemmArgs a, int64_t batch) {
 }
 
 // Whether an f32 tile goes to eight waves in place of four: a wave alone on its SIMD leaves the matrix pipe idle from the barrier of
-// a slab to its next fragments, two take turns.  Only with an operand staged through registers (both K-inner: 40.1 / 40.7 us),
-// and only while the CUs hold every work-group at once -- `per_cu` of them by the registers of eight waves.  us per call, four waves
-// / eight: 64 x 128 tiles 4096 x 512 x 784, W stored [K, N] 41.9 / 37.5, both operands K-outer 43.6 / 38.7; two to a CU 2048^3 151 /
+// a slab to its next fragments, two take turns.  Only while the CUs hold every work-group at once -- `per_cu` of them by the registers of eight waves.  us per call, four waves
+// / eight: 64 x 128 tiles 4096 x 512 x 784, W stored [K, N] 41.9 / 37.5, both operands K-outer 43.6 / 38.7, both K-inner 40.9 / 35.3 (2000 x 1000 x 500
+// 27.5 / 23.5; beyond one to a CU 2048^3 136 on 128 x 128 tiles, 151 so; deeper stages, three or four, 34.6 to 36.9 and 149 to 159); two to a CU 2048^3 151 /
 // 144 (both K-outer, where one fills the registers: 162 / 180); 128 x 128 tiles 2048^3 169 / 146, 784 x 512 x 4096 in 4 splits 92 / 80.
 // (A K of one slab has LDS for one stage, which is less than the epilogue of eight waves takes.)
 template <int DT, bool LK, bool RK>
 static bool two_waves_a_simd(const hipnx_ctx *ctx, const GemmArgs &a, int64_t groups, int per_cu) {
-  return DT == HIPNX_F32 && !(LK && RK) && a.Kb > SLAB && groups <= per_cu * (int64_t)ctx->num_cus;
+  return DT == HIPNX_F32 && a.Kb > SLAB && groups <= per_cu * (int64_t)ctx->num_cus;
 }
 
 // the two-group 256 x 256 kernel (gemm_pingpong.cuh): bf16 / f16 in every layout, s8 with a K-inner
@@ -119,7 +119,7 @@ static int launch_cfg(const hipnx_ctx *ctx, int cfg, const GemmArgs &a, int64_t 
       }
       return launch_one<DT, 2, 2, 2, 2, LK, RK>(ctx, a, batch);
     case GEMM_CFG_128: {
-      if constexpr (DT == HIPNX_F32)
+      if constexpr (DT == HIPNX_F32 && !(LK && RK))
         if (two_waves_a_simd<DT, LK, RK>(ctx, a, ((a.M + 127) / 128) * ((a.N + 127) / 128) * batch, 1))
           return launch_one<DT, 4, 2, 1, 2, LK, RK>(ctx, a, batch);
       // one wave per SIMD and 0.25 us of MFMA work per slab: two stages cannot cover the latency of the next
@@ -152,7 +152,7 @@ static int launch_cfg(const hipnx_ctx *ctx, int cfg, const GemmArgs &a, int64_t 
       return launch_one<DT, 2, 2, 2, 2, LK, RK>(ctx, a, batch);
     case GEMM_CFG_64x128:
       if constexpr (DT == HIPNX_F32) {
-        if (two_waves_a_simd<DT, LK, RK>(ctx, a, ((a.M + 63) / 64) * ((a.N + 127) / 128) * batch, LK || RK ? 2 : 1))
+        if (two_waves_a_simd<DT, LK, RK>(ctx, a, ((a.M + 63) / 64) * ((a.N + 127) / 128) * batch, LK != RK ? 2 : 1))
           return launch_one<DT, 2, 4, 1, 1, LK, RK>(ctx, a, batch);
         return launch_one<DT, 2, 2, 1, 2, LK, RK>(ctx, a, batch);
       }
