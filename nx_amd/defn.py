@@ -491,7 +491,7 @@ def _fusable(t: Tensor) -> bool:
                 return True
             c = _const(a)
             return binary_op in _EXACT_WITH_INT_CONSTANT and T.is_integer(a.type) and abs(c) <= 1 << 24
-        return a.type in _NARROW
+        return a.type in _NARROW or (binary_op == "multiply" and a.type == _TRUTH)  # (values times a mask)
 
     if op in UNARY_OPS and op not in _INT_ONLY_UNARY:
         out_ok = t.type == _TRUTH if op in ("is_nan", "is_infinity") else t.type in _NARROW

@@ -236,7 +236,26 @@ def reuse_and_square(x, y):
     return Nx.multiply(Nx.multiply(s, s), Nx.subtract(s, x))   # op(s, s) and three reads of one value
 
 
+def masked_products(x, y):
+    kept = Nx.greater(x, 0.0)
+    return Nx.subtract(Nx.multiply(kept, Nx.add(x, y)), Nx.multiply(Nx.multiply(y, Nx.is_nan(Nx.divide(x, x))), kept))
+
+
+def product_with_a_given_mask(x, y, mask):
+    return Nx.multiply(Nx.add(x, y), mask)
+
+
+def not_finite(rng, ty, shape, b):
+    v = rng.standard_normal(shape).astype(np.float32)
+    v.reshape(-1)[::3] = np.resize(np.array([0.0, -0.0, np.inf, -np.inf, np.nan, 1e-40], np.float32), v.reshape(-1)[::3].shape)
+    return from_numpy((v.view(np.uint32) >> 16).astype(np.uint16) if ty == "bf16" else v.astype(np.float16 if ty == "f16" else np.float32), ty, b)
+
+
 FUSED_CASES = {
+    "masked_products": (masked_products, lambda rng, b: (not_finite(rng, "f32", (64, 40), b), not_finite(rng, "f32", (64, 40), b))),
+    "masked_products_ragged": (masked_products, lambda rng, b: (not_finite(rng, "f16", (13, 7), b), not_finite(rng, "f16", (13, 7), b))),
+    "product_with_a_given_mask": (product_with_a_given_mask, lambda rng, b: (not_finite(rng, "bf16", (24, 64), b), not_finite(rng, "bf16", (24, 64), b),
+                                                                             from_numpy(rng.integers(0, 256, size=(24, 64), dtype=np.uint8), "u8", b))),
     "reuse_and_square": (reuse_and_square, lambda rng, b: (rand_float(rng, "f32", (40, 64), b), rand_float(rng, "f32", (40, 64), b))),
     "long_rows_tail": (gelu_like, lambda rng, b: (rand_float(rng, "f32", (3, 4104), b), rand_float(rng, "f32", (4104,), b))),
     "gelu_like": (gelu_like, lambda rng, b: (rand_float(rng, "f32", (64, 256), b), rand_float(rng, "f32", (256,), b))),
