@@ -272,27 +272,23 @@ splitk_combine_kernel(const AT *__restrict__ part, void *__restrict__ out, int o
   for (int64_t v = (int64_t)blockIdx.x * 256 + threadIdx.x; v < nvec; v += (int64_t)gridDim.x * 256) {
     typedef __attribute__((ext_vector_type(4), aligned(4))) AT vec_t;
     vec_t acc = *reinterpret_cast<const vec_t *>(part + v * 4);
+    // sixteen loads in flight (eight or four where there are no more), added in order of the ranges: what the pass waits for is round trips
+    // (us per call with four in flight / so: f16 30 x 1000 x 8000 9.5 / 8.8, int8 8 x 500 x 4000 7.9 / 7.0, the pass alone, f32 512 x 10 in 64 ranges, 7.2 / 5.3)
+    auto add = [&](auto many, int s) {
+      constexpr int B = decltype(many)::value;
+      vec_t p[B];
+#pragma unroll
+      for (int u = 0; u < B; u++) p[u] = *reinterpret_cast<const vec_t *>(part + (int64_t)(s + u < splits ? s + u : splits - 1) * mn + v * 4);
+#pragma unroll
+      for (int u = 0; u < B; u++)
+        if (s + u < splits)
+#pragma unroll
+          for (int e = 0; e < 4; e++) acc[e] += p[u][e];
+    };
     int s = 1;
-    for (; s + 3 < splits; s += 4) {  // four loads in flight; added in split order
-      vec_t p[4];
-#pragma unroll
-      for (int u = 0; u < 4; u++) p[u] = *reinterpret_cast<const vec_t *>(part + (s + u) * mn + v * 4);
-#pragma unroll
-      for (int u = 0; u < 4; u++)
-#pragma unroll
-        for (int e = 0; e < 4; e++) acc[e] += p[u][e];
-    }
-    if (s + 1 < splits) {
-      const vec_t p = *reinterpret_cast<const vec_t *>(part + s * mn + v * 4), q = *reinterpret_cast<const vec_t *>(part + (s + 1) * mn + v * 4);
-#pragma unroll
-      for (int e = 0; e < 4; e++) acc[e] = acc[e] + p[e] + q[e];
-      s += 2;
-    }
-    if (s < splits) {
-      const vec_t p = *reinterpret_cast<const vec_t *>(part + s * mn + v * 4);
-#pragma unroll
-      for (int e = 0; e < 4; e++) acc[e] += p[e];
-    }
+    for (; s + 8 < splits; s += 16) add(std::integral_constant<int, 16>{}, s);
+    if (s + 4 < splits) add(std::integral_constant<int, 8>{}, s);
+    else if (s < splits) add(std::integral_constant<int, 4>{}, s);
     if constexpr (SCALED) {
       float x[4];
 #pragma unroll
@@ -377,14 +373,14 @@ static GemmChoice gemm_choice(const hipnx_ctx *ctx, int l_dt, int out_dt, int64_
     //   174 us, 64 x 128, two to a CU, 152).  Fitted to f32 contractions of 100 to 8192 a side in three layouts,
     //   within a tenth.  (Both operands K-inner: 128 x 128 tiles on the two-group kernel, which holds its CU alone,
     //   and six stages of 64 x 32 tiles, two to a CU.)
-    //   An operand that is not K-inner: the figures of eight waves to a work-group (two_waves_a_simd, gemm_launch.cuh); two and
+    //   64 x 128 tiles, and an operand that is not K-inner: the figures of eight waves to a work-group (two_waves_a_simd, gemm_launch.cuh); two and
     //   three work-groups of 64 x 32 that start together share a CU no better than `pair` (1024^3, 512 of them: 46 us; two splits
     //   of 64 x 128 31; 6000 x 100 x 500 24.8 / 17.9; 4096 x 512 x 784 40.7 -> 35.3; 2048^3 152 -> 144, both K-outer 160 -> 150).
     struct Tile { int cfg, rows, cols, resident; double alone, pair, shared; };
     const bool kk = l_kin && r_kin, oo = !l_kin && !r_kin, f64 = l_dt == HIPNX_F64;
     const Tile tiles[3] = {
         {GEMM_CFG_128, 128, 128, f64 || kk ? 1 : 2, f64 ? 2.6 : kk ? 2.05 : 2.25, 0, f64 ? 2.6 : kk ? 2.05 : 2.15},
-        {GEMM_CFG_64x128, 64, 128, f64 ? 1 : 3, f64 ? 1.3 : kk ? 1.44 : 1.25, 0, f64 ? 1.3 : kk || oo ? 1.15 : 1.12},
+        {GEMM_CFG_64x128, 64, 128, f64 ? 1 : 3, f64 ? 1.3 : 1.25, 0, f64 ? 1.3 : kk || oo ? 1.15 : 1.12},
         {GEMM_CFG_64, 64, 32, f64 ? 1 : kk ? 2 : 6, f64 ? 0.55 : kk ? 0.75 : 0.9, f64 || kk ? 0 : 1.38, f64 ? 0.55 : kk ? 0.65 : 0.36}};
     if (cfg == GEMM_CFG_128) {
       const int64_t cus = ctx->num_cus;
