@@ -272,23 +272,27 @@ splitk_combine_kernel(const AT *__restrict__ part, void *__restrict__ out, int o
   for (int64_t v = (int64_t)blockIdx.x * 256 + threadIdx.x; v < nvec; v += (int64_t)gridDim.x * 256) {
     typedef __attribute__((ext_vector_type(4), aligned(4))) AT vec_t;
     vec_t acc = *reinterpret_cast<const vec_t *>(part + v * 4);
-    // sixteen loads in flight (eight or four where there are no more), added in order of the ranges: what the pass waits for is round trips
-    // (us per call with four in flight / so: f16 30 x 1000 x 8000 9.5 / 8.8, int8 8 x 500 x 4000 7.9 / 7.0, the pass alone, f32 512 x 10 in 64 ranges, 7.2 / 5.3)
-    auto add = [&](auto many, int s) {
-      constexpr int B = decltype(many)::value;
+    // up to sixteen loads in flight, as many as there are ranges left, added in order of the ranges: what the pass waits for is round trips
+    // (us per call with four in flight / so: f16 30 x 1000 x 8000 9.5 / 9.0, int8 8 x 500 x 4000 7.9 / 7.3, bf16 1 x 4096 x 11008 20.5 / 19.9, the pass alone, f32 512 x 10 in 64 ranges, 7.2 / 5.3)
+    int s = 1;
+    auto add = [&](auto count) {
+      constexpr int B = decltype(count)::value;
       vec_t p[B];
 #pragma unroll
-      for (int u = 0; u < B; u++) p[u] = *reinterpret_cast<const vec_t *>(part + (int64_t)(s + u < splits ? s + u : splits - 1) * mn + v * 4);
+      for (int u = 0; u < B; u++) p[u] = *reinterpret_cast<const vec_t *>(part + (int64_t)(s + u) * mn + v * 4);
 #pragma unroll
       for (int u = 0; u < B; u++)
-        if (s + u < splits)
 #pragma unroll
-          for (int e = 0; e < 4; e++) acc[e] += p[u][e];
+        for (int e = 0; e < 4; e++) acc[e] += p[u][e];
+      s += B;
     };
-    int s = 1;
-    for (; s + 8 < splits; s += 16) add(std::integral_constant<int, 16>{}, s);
-    if (s + 4 < splits) add(std::integral_constant<int, 8>{}, s);
-    else if (s < splits) add(std::integral_constant<int, 4>{}, s);
+    while (s + 16 <= splits) add(std::integral_constant<int, 16>{});
+    if (s + 8 <= splits) add(std::integral_constant<int, 8>{});
+    switch (splits - s) {
+#define HIPNX_LEFT(N) case N: add(std::integral_constant<int, N>{}); break;
+      HIPNX_LEFT(1) HIPNX_LEFT(2) HIPNX_LEFT(3) HIPNX_LEFT(4) HIPNX_LEFT(5) HIPNX_LEFT(6) HIPNX_LEFT(7)
+#undef HIPNX_LEFT
+    }
     if constexpr (SCALED) {
       float x[4];
 #pragma unroll
