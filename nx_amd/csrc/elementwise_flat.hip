@@ -98,7 +98,7 @@ static bool flat_any(std::integer_sequence<int, OPS...>, const hipnx_ctx *ctx, i
 // W consecutive elements a lane.  NUMBER: the right operand is one element.
 // (The kernel that reads its operands' types as it runs is some thousand instructions, which a launch of a few waves spends its time
 // fetching, the more so behind a pass that went through the caches.  us, there / here: 100 f32 sums over an s32 count behind
-// 268 MB 8.0 / 4.8, 300 behind 24 MB 6.4 / 1.9; f32 [4096, 512] times a u8 mask 6.9 / 3.4.)
+// 268 MB 8.0 / 4.8, 300 behind 24 MB 6.4 / 1.5; f32 [4096, 512] times a u8 mask 5.4 / 4.0 a call.)
 template <int OP, typename CT, int LDT, int RDT, int W, bool NUMBER>
 __global__ void __launch_bounds__(BLOCK)
 binary_mixed_kernel(const void *__restrict__ l, const void *__restrict__ r, void *__restrict__ out, uint32_t n) {

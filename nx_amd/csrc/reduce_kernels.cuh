@@ -575,11 +575,12 @@ static int run_reduce_t(hipnx_ctx *ctx, bool static_ws, int idt, int odt, int64_
         HIPNX_HIP(hipGetLastError());
         return HIPNX_OK;
       };
-      // Rows of 32 KiB and more of whole vectors stay with the kernel below (f32 [16384, 8192] 90 us there, 100 here); so do rows
+      // Rows of 20 KiB and more of whole vectors stay with the kernel below (f32 [16384, 8192] 90 us there, 100 here, bf16 [16384, 12000] 67 / 72;
+      // f32 [16384, 4096] 51 / 44, bf16 [16384, 8192] 57 / 45); so do rows
       // that leave most of a work-group's columns empty.  Wider work-groups read a large input in longer runs (f32 [200000, 300] 55 us
       // by 16 lanes to a row, 49 by 32, 55 by 64), narrower ones leave more of them to a small one (bf16 [20000, 300] 9.2 / 11.4 / 12.4).
       const int64_t bytes = outer * red * inner * dtype_size(idt), row = inner * dtype_size(idt);
-      const int st = row < 128 || (inner % E == 0 && row >= 32768) ? -1 : bytes >= (32ll << 20) && row >= 512 ? tile(std::integral_constant<int, 32>{})
+      const int st = row < 128 || (inner % E == 0 && row >= 20480) ? -1 : bytes >= (32ll << 20) && row >= 512 ? tile(std::integral_constant<int, 32>{})
                                                                                                  : tile(std::integral_constant<int, 16>{});
       if (st >= 0) return st;
     }
