@@ -206,21 +206,24 @@ __device__ __forceinline__ double fma_consts(double w, double c1, double c0) {
 // The same for an f32 operand (the f32 class of the kernels).  Bound by f64 instructions, each of which costs a SIMD as
 // much as an f32 one; the form above takes about 190, most of them in the library's log, which serves every double, and
 // in separate products and sums.  Here the logarithm is written for what can occur, y = 1 - x^2 in [2^-23, 1]:
-// y = 2^e m with m in [1/2, 1), c = 1/sqrt(2), log(m / c) = 2 atanh(s), s = (m - c) / (m + c), the series of atanh in z = s^2
+// y = 2^e m with m in [1/2, 1), log(m / c) = 2 atanh(s), s = (m - c) / (m + c), c next to 1/sqrt(2), the series of atanh in z = s^2
 // beyond its first term as a polynomial of degree 6 (interpolated at the Chebyshev points of z in [0, 0.02945]; its
 // error is below 2^-57 of the logarithm), the quotient from v_rcp_f64 and one correction by its remainder; the polynomials are fused
-// multiply-adds.  Only w - 2.5 is wanted, in absolute terms, so that log c may stand in its constant although e ln 2 cancels it near y = 1.
-// The polynomials' argument has one rounding of its own size as above, p one less per step: against
-// the same polynomials in 80 bits either form is within 3.7e-16 (every multiple of 2^-23 in (-1, 1) and 7.7 M arguments spread over the
-// exponents and towards +-1, the forms written out for the CPU with a reciprocal of 2^-25; none of them rounded to another f32 by either).  So a result is
-// the reference's but where the f64 value lies that close to halfway between two floats: the last bit, about once in 2^25.  No branch but the
+// multiply-adds.  Only w - 2.5 is wanted, in absolute terms, so that log c may stand in its constant although e ln 2 cancels it near y = 1:
+// of the doubles about 1/sqrt(2), c is one whose -2.5 - log c is a double to 2^-57 (1/sqrt(2) itself misses by 2^-53, which
+// took the error of the f64 value from 2.98e-16 to 3.09e-16).  The correction squares the reciprocal's error, 2^-24.5 at most over [1.2, 1.71)
+// (measured, 2^32 divisors); a Newton step in front of it changes the largest error by a hundredth.
+// The f64 value against the same polynomials in 80 bits, measured on the device over every float in [2^-10, 1) and a quarter of the exponents from 2^-30: at most
+// 2.89e-16 up to 0.9966 (with the logarithm about m = 1, exact at y = 1: 2.98e-16), 3.55e-16 beyond (3.55e-16), 2.73e-16 below 2^-10 (2.73e-16); none of the
+// 1.3e8 rounded to another f32.  So a result is the reference's but where the f64 value lies that close to halfway between two floats: the last
+// bit, about once in 2^25.  No branch but the
 // rare one: w >= 5 is |x| > 0.99662, and everything that is not inside (-1, 1) goes the same way.  2^26 normal samples, the chain behind the
 // cipher: 320 us by the form above, 195 with the logarithm about m = 1 and the compiler's v_fmac, 151 with constants in scalar registers;
 // cipher and chain in one kernel then 186.6, and 174.4 as it is.
 __device__ __forceinline__ float erf_inv_f32(float xf) {
   const double x = (double)xf, y = __builtin_fma(-x, x, 1.0);
   const double e = (double)__builtin_amdgcn_frexp_exp(y), m = __builtin_amdgcn_frexp_mant(y);
-  const double f = m - 0x1.6a09e667f3bcdp-1, d = m + 0x1.6a09e667f3bcdp-1, r = __builtin_amdgcn_rcp(d), s0 = f * r;
+  const double c = 0x1.6a09e667f3dep-1, f = m - c, d = m + c, r = __builtin_amdgcn_rcp(d), s0 = f * r;
   const double s = __builtin_fma(__builtin_fma(-d, s0, f), r, s0), z = s * s;
   double q = fma_consts(z, 0x1.2b5b5fb2eac92p-3, 0x1.39fe208c33457p-3);
   q = fma_const(q, z, 0x1.7462b69705382p-3);
@@ -229,8 +232,8 @@ __device__ __forceinline__ float erf_inv_f32(float xf) {
   q = fma_const(q, z, 0x1.99999999952b2p-2);
   q = fma_const(q, z, 0x1.5555555555558p-1);
   q = fma_const(q, z, 2.0);
-  // w - 2.5, w = -(e ln 2 + log c + 2 atanh(s))
-  double w = __builtin_fma(-s, q, fma_consts(e, -0x1.62e42fefa39efp-1, 0x1.62e42fefa39efp-2 - 2.5));
+  // w - 2.5, w = -(e ln 2 + log c + 2 atanh(s)); the constant is -2.5 - log c
+  double w = __builtin_fma(-s, q, fma_consts(e, -0x1.62e42fefa39efp-1, -0x1.13a37a020b97ep+1));
   double p = fma_consts(w, 2.81022636e-08, 3.43273939e-07);
   p = fma_const(p, w, -3.5233877e-06);
   p = fma_const(p, w, -4.39150654e-06);

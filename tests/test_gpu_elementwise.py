@@ -187,6 +187,22 @@ def test_f32_erf_inv_is_the_reference_but_for_last_bits_next_to_a_tie(where, hip
     assert apart.max() <= 1 and (apart != 0).sum() <= 2
 
 
+def test_f32_erf_inv_rounds_its_nearest_misses_of_a_tie_as_the_exact_formula_does(hip):
+    """Of the floats in [2^-10, 1) those whose value lies nearest to halfway between two floats, 3.9e-16 to 3.7e-15 of it away: the
+    kernel's f64 value is within 2.9e-16 up to 0.9966, so each rounds as the formula in 80 bits does."""
+    x = np.array([0x3C73BC07, 0x3BC4B808, 0x3F78AE99, 0x3C2A3771, 0x3B3C23F9], dtype=np.uint32).view(np.float32)
+    x = np.concatenate([x, -x])
+    wide = x.astype(np.longdouble)
+    if np.finfo(np.longdouble).nmant < 63:
+        pytest.skip("no 80-bit floats here")
+    w = -np.log((1 - wide) * (1 + wide)) - np.longdouble(2.5)
+    p = np.zeros_like(w)
+    for c in (2.81022636e-08, 3.43273939e-07, -3.5233877e-06, -4.39150654e-06, 0.00021858087, -0.00125372503, -0.00417768164, 0.246640727, 1.50140941):
+        p = p * w + np.longdouble(np.float64(c))
+    got = values(Nx.erf_inv(from_numpy(x, "f32", hip))).astype(np.float32)
+    assert np.array_equal(got.view(np.uint32), (p * wide).astype(np.float32).view(np.uint32))
+
+
 @pytest.mark.parametrize("op", ["abs", "negate", "sign", "ceil", "floor", "round", "is_nan", "is_infinity"])
 @pytest.mark.parametrize("ty", FLOAT_TYPES + ["s8", "s32", "s64", "u8", "u32"])
 def test_unary_exact(op, ty, hip, oracle):

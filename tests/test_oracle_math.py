@@ -12,6 +12,8 @@ function under test returns).
 A swapped pair (sin / cos, sinh / asinh, log / log1p), a dropped term (`exp(x) - 1`, `log(x + 1)`), a
 wrong sign or a transposed `atan2` operand fails at least one of these."""
 import math
+import re
+from pathlib import Path
 
 import mpmath as mp
 import numpy as np
@@ -92,6 +94,17 @@ def test_erf_inv_inverts_erf_and_follows_giles_polynomial_accuracy(oracle):
     got = values(run("erf_inv", p, "f64", oracle))
     assert np.abs(got - true).max() < 2e-6 and np.array_equal(np.sign(got), np.sign(p))
     assert values(run("erf_inv", [0.0], "f64", oracle)).item() == 0.0
+
+
+def test_the_logarithm_of_the_f32_erf_inv_kernel_has_a_constant_to_2_57():
+    """Its -2.5 - log c stands in one double that cancels e ln 2 next to zero: c is chosen for it (1/sqrt(2) misses by 2^-53)."""
+    source = (Path(__file__).resolve().parent.parent / "nx_amd" / "csrc" / "elementwise_ops.cuh").read_text()
+    body = source[source.index("float erf_inv_f32("):]
+    c = float.fromhex(re.search(r"const double c = (\S+?),", body).group(1))
+    constant = float.fromhex(re.search(r"fma_consts\(e, -0x1.62e42fefa39efp-1, (\S+?)\)", body).group(1))
+    assert abs(c - 2 ** -0.5) < 1e-12
+    with mp.workdps(50):
+        assert abs(mp.mpf(constant) + mp.mpf(2.5) + mp.log(mp.mpf(c))) < mp.mpf(2) ** -57
 
 
 INVERSE_PAIRS = [("acos", "cos", grid(0.01, 3.1, 31)), ("asin", "sin", grid(-1.5, 1.5, 31)), ("atan", "tan", grid(-1.5, 1.5, 31)),
