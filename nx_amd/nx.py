@@ -223,18 +223,27 @@ def _make_ready(key, mod, *args):
             table[key] = call
 
 
-# Of those, the ones with a number: the call with the number's constant in it, and the default backend the constant is on.  Not
-# while a device is capturing, whose constants are the graph's own.
+# Of those, by call and number, the ones with a number: the call with the number's constant in it, and the default backend the constant is on.  Not
+# while a device is capturing, whose constants are the graph's own.  A number is laid out when it is met again (a rate that changes from
+# step to step never is: laid out at once it cost such a call some 2 us, and the table its other numbers), and NaN, which no look-up finds, not at all.
 _bound = {}
+_met = {}  # the numbers met once
 _capturing = ()  # (the device backend's devices that are)
 
 
-def _bind(key, call, number):
-    table = _bound  # (replaced together with _ready)
-    if len(table) >= 1024:
-        table.clear()
-    bound = call.bind(1, number)
+def _bind(table, key, number):
+    """`table`: what `_bound` was before the call (it is replaced together with `_ready`)."""
+    if _met.pop(key, False) is False:
+        if key[1] == key[1]:
+            if len(_met) >= 1024:
+                _met.clear()
+            _met[key] = None
+        return
+    bound = key[0].bind(1, number)
     if bound is not None:
+        if len(table) >= 1024:
+            for old in list(table)[:64]:
+                table.pop(old, None)
         table[key] = (bound, getattr(_state, "backend", None) or _global_default[0])
 
 
@@ -251,20 +260,25 @@ def _binary(name, left, right, out_type_fun):
         elif right.__class__ is float or (right.__class__ is int and left.type[0] != "u" and left.type[0] != "s"):
             key, r = (name, left.type, left.shape, right.__class__), None
         if key is not None:
-            if r is None and right:  # (zeros: two of them are equal)
-                bound = _bound.get((key, right))
-                if bound is not None and bound[1] is (getattr(_state, "backend", None) or _global_default[0]) and not _capturing:
-                    out = bound[0](left)
-                    if out is not None:
-                        return out
             ready = _ready.get(key)
             if ready is not None:
-                number = to_tensor(right) if r is None else r
-                out = ready(left, number)
-                if out is not None:
-                    if r is None and right and not _capturing:
-                        _bind((key, right), ready, number)
-                    return out
+                if r is None:
+                    known = (ready, right)
+                    table, bound = _bound, _bound.get(known) if right else None  # (zeros: two of them are equal)
+                    if bound is not None and bound[1] is (getattr(_state, "backend", None) or _global_default[0]) and not _capturing:
+                        out = bound[0](left)
+                        if out is not None:
+                            return out
+                    number = to_tensor(right)
+                    out = ready(left, number)
+                    if out is not None:
+                        if right and not _capturing:
+                            _bind(table, known, number)
+                        return out
+                else:
+                    out = ready(left, r)
+                    if out is not None:
+                        return out
     if left.__class__ is Tensor and right.__class__ is Tensor:  # the common case: no number to look at
         ty = left.type if left.type == right.type else T.merge(left.type, right.type)
         l, r = left, right

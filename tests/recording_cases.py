@@ -301,6 +301,43 @@ def a_number_laid_out_with_its_call_is_that_number():
     Nx.default_backend(Hip)
 
 
+def a_number_is_laid_out_when_it_is_met_again():
+    """Numbers that are met once are not laid out, whatever their number, and leave those that are alone; NaN never is; a call that a
+    change of setting overtakes goes where nobody looks."""
+    x = f32(1, 2, 4)
+    for _ in range(4):
+        assert read(Nx.multiply(x, 0.5)) == [0.5, 1, 2]
+    assert [k[1] for k in Nx._bound] == [0.5]
+    kept = Nx._bound[next(iter(Nx._bound))]
+    for i in range(3000):
+        assert read(Nx.multiply(x, i + 0.25)) == [i + 0.25, 2 * i + 0.5, 4 * i + 1]
+        assert all(v != v for v in read(Nx.multiply(x, float("nan"))))
+    nan = float("nan")
+    for _ in range(4):
+        assert all(v != v for v in read(Nx.multiply(x, nan)))
+    assert list(Nx._bound.values()) == [kept] and len(Nx._met) <= 1024
+    for i in range(1200):  # (each met again: the oldest go, not all of them)
+        for _ in range(2):
+            Nx.multiply(x, i + 0.125)
+    assert 900 < len(Nx._bound) <= 1024 and any(k[1] == 1199.125 for k in Nx._bound)
+    for name, value in list(Nx._ready.items()):
+        if name[0] == "multiply":
+            class Overtaken:
+                def __call__(self, *args):
+                    B._settings_changed()
+                    return value(*args)
+
+                def bind(self, *args):
+                    return value.bind(*args)
+            Nx.multiply(x, 9000.5)  # (met once)
+            Nx._ready[name] = Overtaken()
+            assert read(Nx.multiply(x, 9000.5)) == [9000.5, 18001, 36002]
+            assert not Nx._bound and not Nx._ready
+            break
+    else:
+        raise AssertionError("no product is laid out")
+
+
 def what_a_recording_was_not_made_for_is_evaluated_or_refused():
     """Arguments of other types, shapes and kinds go the general way, with what it says of them."""
     x, y = f32(1, 2, 4), f32(3, 5, 7)
