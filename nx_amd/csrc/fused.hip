@@ -177,7 +177,7 @@ static void launch_fused_combine(const hipnx_ctx *ctx, const FusedArgs &a, int r
 static bool narrow(int dt) { return dt == HIPNX_BF16 || dt == HIPNX_F16 || dt == HIPNX_F32; }
 
 // fused_rtc.hip
-int fused_launch_compiled(hipnx_ctx *ctx, const FusedArgs &a, int reduce_op, bool block_per_row, bool walk, int scores_k, unsigned grid, bool *done);
+int fused_launch_compiled(hipnx_ctx *ctx, const FusedWordsArgs &a, int reduce_op, bool block_per_row, bool walk, int scores_k, unsigned grid, bool *done);
 
 }  // namespace hipnx
 
@@ -207,16 +207,17 @@ static int fused_impl(hipnx_ctx *ctx, int n_instr, const hipnx_fused_instr *prog
   if (!narrow(out_dt) && out_dt != HIPNX_U8 && !int_out) return set_error(HIPNX_EUNSUPPORTED, "fused: result type %d", out_dt);
   if (reduce_op != -1 && reduce_op != HIPNX_RED_SUM && reduce_op != HIPNX_RED_MAX && reduce_op != HIPNX_RED_MIN)
     return set_error(HIPNX_EUNSUPPORTED, "fused: reduction %d (sum, max and min along the rows are built)", reduce_op);
-  FusedArgs a{};
+  FusedWordsArgs block{};
+  FusedArgs &a = block;
   a.n_instr = n_instr;
   a.n_inputs = n_inputs;
   a.words = words;
   a.key_parts = key_parts;
   a.key_index = key_index;
-  a.beside_index = beside_index;
+  block.beside_index = beside_index;
   if (beside) {
     if (int st = check_buf(ctx, beside, 8, "fused_words key")) return st;
-    a.beside = (uint32_t *)beside->ptr;
+    block.beside = (uint32_t *)beside->ptr;
   }
   a.scores = scores.input;
   if (words >= 0 && ctx->fused_mode != HIPNX_FUSED_COMPILED) return set_error(HIPNX_EUNSUPPORTED, "fused: random words need the compiled mode");
@@ -471,7 +472,7 @@ static int fused_impl(hipnx_ctx *ctx, int n_instr, const hipnx_fused_instr *prog
     }
     if (scores.input >= 0) grid = scores.batch_outer * scores.batch_inner * ((scores.M + SCORE_ROWS - 1) / SCORE_ROWS);
     bool done = false;
-    if (int st = fused_launch_compiled(ctx, a, reduce_op, block_per_row, walk, scores.K, (unsigned)grid, &done)) return st;
+    if (int st = fused_launch_compiled(ctx, block, reduce_op, block_per_row, walk, scores.K, (unsigned)grid, &done)) return st;
     if (done) {
       if (a.nseg > 1) {
         launch_fused_combine(ctx, a, reduce_op);

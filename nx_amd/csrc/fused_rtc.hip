@@ -222,8 +222,8 @@ static std::string make_source(const FusedArgs &a, const Keeps &keeps, int reduc
            ";\n  static constexpr bool unal = " + (k.form == ROW_WHOLE && a.words < 0 ? "false" : "true") + ";\n  static constexpr int nv = " + std::to_string(k.trips) + ", written_out = " + std::to_string(k.written_out) + ", held = " + std::to_string(k.held) +
            ", held_stage = " + std::to_string(k.held_stage) + ";\n};\n";
   };
-  auto kernel = [](const std::string &called) {
-    return "extern \"C\" __global__ void __launch_bounds__(FBLOCK) " + called + "(FusedArgs by_value) {\n  (void)by_value;\n";
+  auto kernel = [&](const std::string &called) {
+    return "extern \"C\" __global__ void __launch_bounds__(FBLOCK) " + called + (a.words >= 0 ? "(FusedWordsArgs" : "(FusedArgs") + " by_value) {\n  (void)by_value;\n";
   };
   s += "};\n" + keeping("P", keeps);
   Keeps any;
@@ -304,8 +304,9 @@ static int trim_cache(hipnx_ctx *ctx) {
 // Launches the compiled kernel for `a`, compiling it first if this context has not seen the program.
 // *done = false (and HIPNX_OK) when the caller should run the interpreting kernel instead: the
 // program is new and the stream is capturing (compiling and loading a module is no work to record).
+// `a` holds what kernels over random words take too, the others are handed the block in front of it.
 // `walk`: a group of lanes takes a row, the grid follows from how many; `grid` is the grid otherwise.
-int fused_launch_compiled(hipnx_ctx *ctx, const FusedArgs &a, int reduce_op, bool block_per_row, bool walk, int scores_k, unsigned grid, bool *done) {
+int fused_launch_compiled(hipnx_ctx *ctx, const FusedWordsArgs &a, int reduce_op, bool block_per_row, bool walk, int scores_k, unsigned grid, bool *done) {
   *done = false;
   const Keeps keeps = what_is_kept(a, walk);
   int lanes = keeps.tpr;
@@ -341,7 +342,7 @@ int fused_launch_compiled(hipnx_ctx *ctx, const FusedArgs &a, int reduce_op, boo
   it->second.last_use = ++ctx->fused_clock;
   if (ctx->capture) it->second.in_graph = true;  // a recorded launch refers to the loaded module for as long as the graph lives
   // the argument block is the kernel's one by-value parameter: hand it over as the packed buffer it is
-  size_t size = sizeof(FusedArgs);
+  size_t size = a.words >= 0 ? sizeof(FusedWordsArgs) : sizeof(FusedArgs);
   if (walk && a.scores < 0) grid = (unsigned)((a.rows + FBLOCK / lanes - 1) / (FBLOCK / lanes));
   void *config[] = {HIP_LAUNCH_PARAM_BUFFER_POINTER, (void *)&a, HIP_LAUNCH_PARAM_BUFFER_SIZE, &size, HIP_LAUNCH_PARAM_END};
   HIPNX_HIP(hipModuleLaunchKernel(function, grid, 1, 1, FBLOCK, 1, 1, 0, ctx->stream, nullptr, config));
