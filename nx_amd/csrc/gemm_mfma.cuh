@@ -350,11 +350,13 @@ struct KOuterDmaLoader {
   const unsigned char *src[PER];
   int lds_off[PER];
   int rem[PER];  // bytes of this lane's piece that lie inside its k-row, 0: all of them
+  bool whole_pieces;  // (of a k-row, the same for all lanes: what nobody needs is jumped over, not looked at by each)
 
   // g: [K, cols] with `ld` bytes per k; the tile covers columns col0 .. col0+ROWS-1, of which cols_valid exist: chunks past the
   // edge re-read the last one, which runs into the next k-row where k-rows are not whole pieces (see KOuterStage)
   __device__ __forceinline__ void init(const unsigned char *__restrict__ g, int64_t ld, int64_t col0, int64_t cols_valid,
                                        int wave, int lane) {
+    whole_pieces = (int)(cols_valid * ES) % 16 == 0;
 #pragma unroll
     for (int i = 0; i < PER; i++) {
       const int t = wave + NWAVES * i;
@@ -382,6 +384,7 @@ struct KOuterDmaLoader {
     }
   }
   __device__ __forceinline__ void finish_partial(int64_t k0, int64_t ld, int valid, unsigned char *lds, int wave, int lane) const {
+    if (whole_pieces) return;
 #pragma unroll
     for (int i = 0; i < PER; i++)
       if (rem[i] != 0 && ((wave + NWAVES * i) * 1024 + lane * 16) / RBYTES == valid - 1)

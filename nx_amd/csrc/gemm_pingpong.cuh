@@ -128,7 +128,9 @@ struct PPKOuterLoader {
   const unsigned char *base;
   unsigned off[PER];
   int rem[PER];  // bytes of this lane's piece that lie inside its k-row, 0: all of them (KOuterDmaLoader)
+  bool whole_pieces;
   __device__ __forceinline__ void init(const unsigned char *g, int64_t ld, int64_t col0, int64_t cols_valid, int wave, int lane) {
+    whole_pieces = (int)(cols_valid * ES) % 16 == 0;
     const int64_t last = (cols_valid * ES - 1) & ~(int64_t)15;
     const int64_t first = col0 * ES <= last ? col0 * ES : last;
     base = wave_uniform(g + first);
@@ -157,6 +159,7 @@ struct PPKOuterLoader {
     }
   }
   __device__ __forceinline__ void finish_partial(int64_t k0, int64_t ld, int valid, unsigned char *lds, int wave, int lane) const {
+    if (whole_pieces) return;
     const unsigned char *b = base + k0 * ld;
 #pragma unroll
     for (int i = 0; i < PER; i++)
