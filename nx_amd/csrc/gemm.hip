@@ -314,148 +314,6 @@ splitk_combine_kernel(const AT *__restrict__ part, void *__restrict__ out, int o
   }
 }
 
-struct GemmChoice {
-  int cfg, splits, rows, cols;
-};
-// The tile of a contraction on the matrix cores and the number of ranges K is cut into.
-static GemmChoice gemm_choice(const hipnx_ctx *ctx, int l_dt, int out_dt, int64_t batch, int64_t M, int64_t N, int64_t K, bool l_kin, bool r_kin, bool scaled) {
-  const int esz = dtype_size(l_dt);
-  const int64_t nslab = (K * esz + SLAB - 1) / SLAB;
-  // tile choice: the largest tile that still gives every CU work; few rows against a long
-  // weight matrix stream the weights with many small tiles
-  const int64_t t256 = ((M + 255) / 256) * ((N + 255) / 256) * batch;
-  const int64_t t128 = ((M + 127) / 128) * ((N + 127) / 128);
-  const int64_t tw = ((M + 255) / 256) * ((N + 127) / 128) * batch;
-  const bool two_byte = l_dt == HIPNX_BF16 || l_dt == HIPNX_F16;
-  const bool big_ok = M >= 192 && N >= 192;
-  int cfg;
-  // few rows: 64-row tiles (f32: whatever its cost model below picks), except for a 2-byte K-outer operand
-  // (x . W with W stored [K, N]), which only the 128-row kernels read by transposing loads
-  // (64 x 4096 x 4096 bf16: 72 us on 64 x 32 tiles, 16.5 us there)
-  const bool wide = l_dt == HIPNX_F32 || l_dt == HIPNX_F64;  // (an f64 slab costs the matrix pipes what an f32 one does)
-  if (M <= 64 && !wide && !(two_byte && !(l_kin && r_kin) && N >= 128)) cfg = GEMM_CFG_64;
-  else if (t256 * 4 >= (int64_t)ctx->num_cus * 3 && big_ok) cfg = GEMM_CFG_256;
-  else if (two_byte && M >= 192 && N >= 128 && t128 * batch > ctx->num_cus)
-    // More 128 x 128 tiles than CUs: half-width tiles of the two-group kernel while they fit the CUs in one
-    // round, even where they leave some idle (1280 x 4096 x 4096, 160 tiles: 66 us; as 320 tiles of
-    // 128 x 128 in two rounds: 76 us); where they would need a second round, full tiles on what is then more
-    // than half of the CUs (3072^3: 144 tiles of 256 x 256 72 us, 288 half-width tiles 100 us)
-    cfg = tw <= ctx->num_cus || !big_ok ? GEMM_CFG_256x128 : GEMM_CFG_256;
-  else if (l_dt == HIPNX_S8 && big_ok && t256 * 2 >= ctx->num_cus)
-    cfg = GEMM_CFG_256;  // int8 has no half-width tile: full tiles from half of the CUs on (3072^3: 46 us against 57 us)
-  else cfg = GEMM_CFG_128;
-  // many rows against at most 32 columns (a layer with a few outputs): a 128-column tile would be three
-  // quarters empty or more, and its MFMA work is what bounds f32
-  if (N <= 32 && M > 64 && cfg == GEMM_CFG_128) cfg = GEMM_CFG_128x32;
-  // A grid of 128 x 128 tiles that leaves three quarters of the CUs idle (a few hundred rows against a long
-  // weight matrix: 128 x 4096 x 4096 is 32 tiles walking 64 slabs each) splits K over S work-groups per tile:
-  // f32 (s32) partial results in pool workspace, then one pass that adds them in split order.
-  int splits = 1;
-  auto per_split = [&](int cand) { return (nslab + cand - 1) / cand; };
-  auto reaches = [&](int cand) { return per_split(cand) * (cand - 1) < nslab; };  // (every split has a slab)
-  const bool splittable = (cfg == GEMM_CFG_128 || cfg == GEMM_CFG_128x32) && batch == 1 && (l_dt == HIPNX_S8 ? scaled || !is_float(out_dt) : true) && l_dt != HIPNX_F64;  // (partial results are f32 / s32)
-  if (wide && cfg == GEMM_CFG_128x32) {
-    // (0.6 us per slab of a 128 x 32 tile; the split as below)
-    const int64_t cus = ctx->num_cus, tiles = t128 * batch;
-    double best = 10.0 + (double)((tiles + cus - 1) / cus) * (double)nslab * 0.6;
-    if (splittable)
-      for (int cand = 2; cand <= 64; cand *= 2) {
-        if (tiles * cand > cus || nslab / cand < 2 || !reaches(cand)) continue;
-        const double t = 10.0 + (double)per_split(cand) * 0.6 + 5.0 + 2.0 * (double)cand * (double)(M * N) * 4.0 / 8.0e6;
-        if (t < best) { best = t; splits = cand; }
-      }
-  } else if (wide) {
-    // An f32 slab is eight times the MFMA work of a 2-byte one, so a grid that leaves CUs idle is cut much earlier: the
-    // cheapest, by the figures below, of 128 x 128, 64 x 128 (up to 64 rows a 128-row tile would be half empty; and
-    // a last round that leaves most CUs idle ends sooner in halves) and 64 x 32 tiles, the first two also with K
-    // split up to 64 ways, 2 slabs or more each.  512^3: 41 -> 18 us; 256 x 256 x 16384: 84 -> 40 us.
-    //   A work-group takes `alone` us per slab while it has its CU to itself, waiting for memory much of it; up to
-    //   `resident` of them (as the LDS holds) share a CU and take `shared` us per slab and work-group together,
-    //   near what the MFMAs take: a split that puts two or three work-groups on a CU pays for its second pass
-    //   (784 x 512 x 4096, 52 tiles: 4 splits 58 us, 8 splits 50; 1000 x 700 x 1500, 96 tiles: 2 splits 45 us,
-    //   8 splits 33; 300 x 1000 x 900, 40 tiles: 64 x 32 tiles 29 us, 6 splits of 64 x 128 16; 2048^3: 128 x 128
-    //   174 us, 64 x 128, two to a CU, 152).  Fitted to f32 contractions of 100 to 8192 a side in three layouts,
-    //   within a tenth.  (Both operands K-inner: 128 x 128 tiles on the two-group kernel, which holds its CU alone,
-    //   and six stages of 64 x 32 tiles, two to a CU.)
-    //   64 x 128 tiles, and an operand that is not K-inner: the figures of eight waves to a work-group (two_waves_a_simd, gemm_launch.cuh); two and
-    //   three work-groups of 64 x 32 that start together share a CU no better than `pair` (1024^3, 512 of them: 46 us; two splits
-    //   of 64 x 128 31; 6000 x 100 x 500 24.8 / 17.9; 4096 x 512 x 784 40.7 -> 35.3; 2048^3 152 -> 144, both K-outer 160 -> 150).
-    struct Tile { int cfg, rows, cols, resident; double alone, pair, shared; };
-    const bool kk = l_kin && r_kin, oo = !l_kin && !r_kin, f64 = l_dt == HIPNX_F64;
-    const Tile tiles[3] = {
-        {GEMM_CFG_128, 128, 128, f64 || kk ? 1 : 2, f64 ? 2.6 : kk ? 2.05 : 2.25, 0, f64 ? 2.6 : kk ? 2.05 : 2.15},
-        {GEMM_CFG_64x128, 64, 128, f64 ? 1 : 3, f64 ? 1.3 : 1.25, 0, f64 ? 1.3 : kk || oo ? 1.15 : 1.12},
-        {GEMM_CFG_64, 64, 32, f64 ? 1 : kk ? 2 : 6, f64 ? 0.55 : kk ? 0.75 : 0.9, f64 || kk ? 0 : 1.38, f64 ? 0.55 : kk ? 0.65 : 0.36}};
-    if (cfg == GEMM_CFG_128) {
-      const int64_t cus = ctx->num_cus;
-      double best = 0;
-      for (const Tile &t : tiles) {
-        const int64_t count = ((M + t.rows - 1) / t.rows) * ((N + t.cols - 1) / t.cols) * batch;
-        for (int cand : {1, 2, 3, 4, 6, 8, 12, 16, 24, 32, 48, 64}) {
-          if (cand > 1 && (!splittable || t.cfg == GEMM_CFG_64 || count * cand > t.resident * cus || nslab / cand < 2 || !reaches(cand))) continue;
-          const int64_t per_cu = (count * cand + cus - 1) / cus, last = per_cu % t.resident;
-          double us = (double)per_split(cand) * ((double)(per_cu - last) * t.shared + (last ? std::max(last > 1 && last == per_cu ? std::max(t.alone, t.pair) : t.alone, (double)last * t.shared) : 0.0));
-          // a split's second launch, then the partial results written and read once (mostly from cache: ~8 MB per us)
-          if (cand > 1) us += 5.0 + 2.0 * (double)cand * (double)(M * N) * 4.0 / 8.0e6;
-          if (best == 0 || us < best) { best = us; cfg = t.cfg; splits = cand; }
-        }
-      }
-    }
-  } else if (l_kin && (two_byte || l_dt == HIPNX_S8) && (cfg == GEMM_CFG_128 || cfg == GEMM_CFG_64)) {
-    // The cheapest tile and number of ranges of K.  A work-group (`resident` of them share a CU) takes `slab` us a slab, `off`
-    // more where rows do not begin on cache lines; `base` is a launch with an empty walk, `round` what a further round of
-    // work-groups costs beside its slabs; a second launch adds the ranges' partial results, written and read once.  Fitted to
-    // 70 contractions of 8 to 4000 rows (profiles/dot_tile_choice.md), within a tenth in the middle.  us per call, 128 x 128 tiles
-    // (64 rows and fewer: 64 x 64) / the choice: bf16 500^3 10.3 / 5.9, 1000^3 10.9 / 6.8 (K-outer weights 12.8 / 10.6), 168 x 4000 x 1600 13.7 / 8.8,
-    // 100 x 300 x 8000 13.9 / 10.2, 600 x 1500 x 200 8.9 / 5.1; int8 180 x 1088 x 824 20.3 / 6.7, 256 x 1024 x 8192 31.2 / 11.6.
-    struct Tile { int cfg, rows, cols, resident; double base, round, slab, off, second, megabyte; };
-    static const Tile table[4][3] = {
-        {{GEMM_CFG_128, 128, 128, 1, 5.65, 0.0, 0.331, 0.086, 3.0, 0.216}, {GEMM_CFG_64, 64, 64, 1, 4.29, 2.23, 0.173, 0.064, 3.38, 0.134}, {GEMM_CFG_64x128, 64, 128, 1, 5.0, 1.74, 0.298, 0.031, 2.74, 0.219}},
-        {{GEMM_CFG_128, 128, 128, 1, 5.5, 0.0, 0.438, 0.033, 3.0, 0.207}, {GEMM_CFG_32x128, 32, 128, 2, 4.18, 0.155, 0.424, 0.052, 2.93, 0.205}, {GEMM_CFG_64x128, 64, 128, 1, 4.59, 1.54, 0.4, 0.0, 2.86, 0.217}},
-        {{GEMM_CFG_128, 128, 128, 1, 7.3, 3.04, 0.376, 0.281, 1.67, 0.16}, {GEMM_CFG_64, 64, 64, 1, 5.87, 2.87, 0.164, 0.106, 3.41, 0.024}, {GEMM_CFG_64x128, 64, 128, 1, 6.2, 3.98, 0.314, 0.173, 3.0, 0.057}},
-        {{GEMM_CFG_128, 128, 128, 1, 7.25, 3.43, 0.48, 0.235, 1.3, 0.168}, {GEMM_CFG_64, 64, 64, 1, 5.72, 2.1, 0.272, 0.086, 3.3, 0.0}, {GEMM_CFG_64x128, 64, 128, 1, 5.94, 4.14, 0.435, 0.093, 2.9, 0.052}}};
-    double best = 0;
-    for (const Tile &t : table[(two_byte ? 0 : 2) + (r_kin ? 0 : 1)]) {
-      const int64_t count = ((M + t.rows - 1) / t.rows) * ((N + t.cols - 1) / t.cols) * batch, at_once = t.resident * (int64_t)ctx->num_cus;
-      for (int cand = 1; cand <= 16; cand++) {
-        if (cand > 1 && (batch != 1 || (is_float(out_dt) && l_dt == HIPNX_S8 && !scaled) || nslab / cand < 2 || !reaches(cand))) continue;
-        const double rounds = (double)((count * cand + at_once - 1) / at_once);
-        double us = t.base + t.round * (rounds - 1) + rounds * (double)per_split(cand) * (t.slab + (K * esz % 128 ? t.off : 0.0));
-        if (cand > 1) us += t.second + t.megabyte * (double)cand * (double)(M * N) * 8.0 / 1e6;
-        if (best == 0 || us < best) { best = us; cfg = t.cfg; splits = cand; }
-      }
-    }
-  } else if (splittable && t128 * 2 <= ctx->num_cus && nslab >= (t128 * 4 <= ctx->num_cus ? 32 : 64))
-    // (the second pass and the partial results cost about 10 us: worth it from K = 32 slabs on -- 64 where
-    // the grid already covers more than a quarter of the CUs -- with at least 8 slabs left per split and no
-    // more work-groups than CUs; 1024 x 2048 x 2048, 128 tiles of 32 slabs, is faster whole: 21 us against
-    // 22 us in two halves and 27 us in four quarters)
-    for (int cand = 16; cand >= 2; cand /= 2)
-      if (t128 * cand <= (int64_t)ctx->num_cus && nslab / cand >= 8 && reaches(cand)) { splits = cand; break; }
-  const int rows = cfg == GEMM_CFG_256 || cfg == GEMM_CFG_256x128 ? 256 : cfg == GEMM_CFG_32x128 ? 32 : cfg == GEMM_CFG_64 || cfg == GEMM_CFG_64x128 ? 64 : 128;
-  const int cols = cfg == GEMM_CFG_256 ? 256 : cfg == GEMM_CFG_64 ? 64 : cfg == GEMM_CFG_128x32 ? 32 : 128;
-  return {cfg, splits, rows, cols};
-}
-
-// Whether a K-inner operand is copied to rows of whole pieces though the kernels take its rows as they lie.  Sixteen bytes at an
-// address that is no multiple of four cost a CU three times its intake of aligned ones (measured from L2: 30 TB/s aligned, 18
-// with rows on any multiple of four -- never worth a copy --, 15 on any multiple of two, 11.7 on any byte), which a tile pays per
-// slab where its multiplications do not cover it; a copy costs a launch and reads and writes the operand once.  So the
-// operand that many tiles re-read is copied, the long one that few do is not.  us per call, both copied / neither / by this rule:
-// int8 512 x 11007 x 11005 142 / 157 / 119, 512 x 1001 x 11006 56 / 66 / 53, 128 x 11007 x 4094 43 / 32 / 29; bf16 168 x 4000 x 1597
-// 25.3 / 25.7 / 21.1.
-static bool rows_worth_copying(const hipnx_ctx *ctx, const GemmChoice &c, int dt, int64_t batch, int64_t M, int64_t N, int64_t row_bytes, bool right) {
-  if (row_bytes % 4 == 0) return false;
-  const int64_t groups = ((M + c.rows - 1) / c.rows) * ((N + c.cols - 1) / c.cols) * batch * c.splits;
-  const int64_t slabs = ((row_bytes + SLAB - 1) / SLAB + c.splits - 1) / c.splits;
-  const double intake = 78e3, flops = 7.8e6;  // bytes and 2-byte multiply-adds x 2 a CU takes per us
-  const double aligned = (double)(c.rows + c.cols) * SLAB / intake, side = (double)(right ? c.cols : c.rows) * SLAB / intake * (row_bytes % 2 ? 1.4 : 0.85);
-  const double work = (double)c.rows * c.cols * SLAB / (dt == HIPNX_F32 ? 0.5 : 1.0) / flops;
-  const double extra = (double)((groups + ctx->num_cus - 1) / ctx->num_cus) * (double)slabs * std::max(0.0, aligned + side - std::max(aligned, work));
-  const double copy = 2.5 + (double)batch * (double)(right ? N : M) * (double)row_bytes * 2.0 / 4.5e6;
-  return extra > copy;
-}
-
 // A K-inner operand ([rows, K]) copied to rows of whole 16-byte pieces.
 static int pad_rows(hipnx_ctx *ctx, int esz, int64_t rows, int64_t K, const hipnx_buf *in, hipnx_buf **out) {
   const int64_t pieces = (K * esz + 15) / 16;
@@ -517,6 +375,7 @@ static int dot_impl(hipnx_ctx *ctx, int l_dt, int r_dt, int out_dt, int64_t batc
     return HIPNX_OK;
   }
   bool mfma = false, l_pad = false, r_pad = false;
+  const bool partials = l_dt == HIPNX_S8 ? scale_mode != HIPNX_SCALE_NONE || !is_float(out_dt) : l_dt != HIPNX_F64;  // (a split's sums are f32 / s32)
   // the MFMA kernels transpose K-outer operands themselves, k-rows that are not whole pieces too (not f64: its last slab would
   // have to be walked first, and it adds over k in order), but for k-rows shorter than one
   const int row_block = dtype_size(l_dt) == 1 ? 16 : dtype_size(l_dt) == 2 ? 8 : dtype_size(l_dt) == 4 ? 4 : 2;
@@ -552,9 +411,9 @@ static int dot_impl(hipnx_ctx *ctx, int l_dt, int r_dt, int out_dt, int64_t batc
       r_pad = row_bytes < 16 && (r_layout == HIPNX_K_INNER || r_relay);
       if (l_pad || r_pad || l_dt != HIPNX_S8) mfma = (double)M * (double)N * (double)K * (double)batch >= 16777216.0;
       if (mfma && row_bytes >= 16) {
-        const GemmChoice choice = gemm_choice(ctx, l_dt, out_dt, batch, M, N, K, l_layout == HIPNX_K_INNER || l_relay, r_layout == HIPNX_K_INNER || r_relay, scaled);
-        l_pad = l_layout == HIPNX_K_INNER && !l_relay && rows_worth_copying(ctx, choice, l_dt, batch, M, N, row_bytes, false);
-        r_pad = r_layout == HIPNX_K_INNER && !r_relay && rows_worth_copying(ctx, choice, l_dt, batch, M, N, row_bytes, true);
+        const GemmChoice choice = gemm_choice(ctx->num_cus, l_dt, batch, M, N, K, l_layout == HIPNX_K_INNER || l_relay, r_layout == HIPNX_K_INNER || r_relay, partials);
+        l_pad = l_layout == HIPNX_K_INNER && !l_relay && rows_worth_copying(ctx->num_cus, choice, batch, M, N, row_bytes, false);
+        r_pad = r_layout == HIPNX_K_INNER && !r_relay && rows_worth_copying(ctx->num_cus, choice, batch, M, N, row_bytes, true);
       }
     }
     if (scaled) {
@@ -720,7 +579,7 @@ static int dot_impl(hipnx_ctx *ctx, int l_dt, int r_dt, int out_dt, int64_t batc
     if (!st) {
       const void *lp = lt ? lt->ptr : l->ptr, *rp = rt ? rt->ptr : r->ptr;
       const bool l_kin = l_layout == HIPNX_K_INNER || l_relay, r_kin = r_layout == HIPNX_K_INNER || r_relay;
-      const GemmChoice choice = gemm_choice(ctx, l_dt, out_dt, batch, M, N, K, l_kin, r_kin, scale_mode != HIPNX_SCALE_NONE);
+      const GemmChoice choice = gemm_choice(ctx->num_cus, l_dt, batch, M, N, K, l_kin, r_kin, partials);
       GemmArgs a{};
       a.l = (const unsigned char *)lp;
       a.r = (const unsigned char *)rp;

@@ -7,17 +7,6 @@
 
 namespace hipnx {
 
-// tile configurations of gemm_pipelined_kernel<DT, WM, WN, TM, TN, ...>
-enum {
-  GEMM_CFG_256x128 = 3,  // 256 x 128, the two-group kernel with half-width wave tiles: 2-byte types whose 256 x 256 grid is too small
-  GEMM_CFG_256 = 0,  // 256 x 256, 8 waves (4 x 2, each 64 x 128): large square-ish problems
-  GEMM_CFG_128 = 1,  // 128 x 128: mid-size and batched problems; 4 waves (2 x 2, each 64 x 64), or two such groups sharing K
-  GEMM_CFG_64 = 2,  // 64 x 64 on the two-group kernel (2-byte K-inner pairs, int8): small and mid-size problems, few rows; otherwise 64 x 32, 2 waves
-  GEMM_CFG_64x128 = 4, // 64 x 128, wherever the cost models of gemm.hip have it cheapest: the two-group kernel (2-byte, int8) or 4 waves (2 x 2, each 32 x 64)
-  GEMM_CFG_32x128 = 6, // 32 x 128, 4 waves (1 x 4, each 32 x 32): 2-byte weights stored K-outer, few rows or small problems
-  GEMM_CFG_128x32 = 5  // 128 x 32, 4 waves (4 x 1, each 32 x 32): many rows against up to 32 columns (a layer with a few outputs)
-};
-
 int launch_gemm_bf16(const hipnx_ctx *ctx, int cfg, bool l_kin, bool r_kin, GemmArgs a, int64_t batch);
 int launch_gemm_f16(const hipnx_ctx *ctx, int cfg, bool l_kin, bool r_kin, GemmArgs a, int64_t batch);
 int launch_gemm_f32(const hipnx_ctx *ctx, int cfg, bool l_kin, bool r_kin, GemmArgs a, int64_t batch);

@@ -28,6 +28,7 @@
 #include <type_traits>
 
 #include "dtypes.cuh"
+#include "gemm_choice.h"
 
 namespace hipnx {
 
@@ -35,7 +36,6 @@ typedef int v4i __attribute__((ext_vector_type(4)));
 typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 
-constexpr int SLAB = 128;          // bytes of K per row per slab
 constexpr int CHUNKS = SLAB / 16;  // 16-byte chunks per row
 
 typedef float v4f __attribute__((ext_vector_type(4)));
