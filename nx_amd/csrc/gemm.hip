@@ -20,8 +20,8 @@
 
 namespace hipnx {
 
-// Rows of K elements copied to a pitch of whole 16-byte pieces, zeros behind K: what a K-inner operand
-// needs whose rows are not whole pieces, as the direct-to-LDS loads take whole pieces.  A lane writes one
+// Rows of K elements copied to a pitch of whole 16-byte pieces, zeros behind K: K-inner rows shorter than a piece, which the
+// contraction kernels cannot take, and longer ones on no dword that many tiles re-read (rows_worth_copying).  A lane writes one
 // piece; a piece inside its row is one load at whatever address it has, the row's last one is put together by elements.
 // Bound by memory: reads and writes the operand once ([2000, 999] bf16, 8 MB moved: 3 us).
 template <typename T>
@@ -562,9 +562,15 @@ static int dot_impl(hipnx_ctx *ctx, int l_dt, int r_dt, int out_dt, int64_t batc
     }
   }
   for (int side = 0; side < 2 && !st; side++) {
-    if (!(side ? r_pad : l_pad)) continue;
+    bool &pad = side ? r_pad : l_pad;
+    if (!pad) continue;
     hipnx_buf *&turned = side ? rt : lt, *padded = nullptr;
     st = pad_rows(ctx, esz, batch * (side ? N : M), K, turned ? turned : side ? r : l, &padded);
+    if (st == HIPNX_ENOMEM && K * esz >= 16) {  // (such rows are copied for speed alone: without room for it they are read as they lie)
+      pad = false;
+      st = HIPNX_OK;
+      continue;
+    }
     if (turned) hipnx_buf_destroy(turned);  // (back to the pool: later work is ordered on the same stream)
     turned = padded;
   }

@@ -176,3 +176,33 @@ def test_out_of_memory_is_an_error_and_the_pool_gives_way(hip):
     assert int(hip.to_numpy(Nx.slice(c, [n - 1], [1]))[0]) == (n - 1) % 256
     del c
     gc.collect()
+
+
+def test_a_contraction_that_would_copy_its_rows_reads_them_in_place_when_there_is_no_room(hip):
+    """int8 rows of 8191 bytes are copied to whole 16-byte pieces where many tiles re-read them, for speed alone: on a full
+    device the contraction is done without the copy, with the same (exact) result."""
+    import gc
+    from nx_amd._lib import ENOMEM, HipNxError
+    M, N, K = 2048, 4097, 8191
+    rng = np.random.default_rng(3)
+    a, b = rng.integers(-128, 128, size=(M, K), dtype=np.int8), rng.integers(-128, 128, size=(N, K), dtype=np.int8)
+    x, w = from_numpy(a, "s8", hip), from_numpy(b, "s8", hip)
+    first = Nx.dot(x, [1], w, [1], out_type="s32")  # (with room; and every kernel is on the device from here on)
+    rows = [0, 1, 255, M - 1]
+    want = hip.to_numpy(first)
+    assert np.array_equal(want[rows], a[rows].astype(np.float64) @ b.astype(np.float64).T)
+    held, size = [], 64 * 2 ** 30
+    while size >= 2 ** 24:
+        try:
+            held.append(Nx.iota((size,), type="u8", backend=hip))
+        except HipNxError as e:
+            assert e.status == ENOMEM
+            size //= 2
+    with pytest.raises(HipNxError) as err:
+        Nx.iota((N * (K + 1),), type="u8", backend=hip)  # (the copy of w)
+    assert err.value.status == ENOMEM
+    del first  # (its block is the next result's)
+    got = hip.to_numpy(Nx.dot(x, [1], w, [1], out_type="s32"))
+    del held
+    gc.collect()
+    assert np.array_equal(got, want)
