@@ -591,7 +591,7 @@ static int dot_impl(hipnx_ctx *ctx, int l_dt, int r_dt, int out_dt, int64_t batc
       a.r = (const unsigned char *)rp;
       a.out = out->ptr;
       a.odt = out_dt;
-      const int64_t row_bytes = K * esz, nslab = (row_bytes + SLAB - 1) / SLAB, over = row_bytes % SLAB;
+      const int64_t row_bytes = K * esz, nslab = (row_bytes + SLAB - 1) / SLAB;
       const int64_t pitch = (row_bytes + 15) / 16 * 16;
       a.M = M; a.N = N; a.Kb = nslab * SLAB;
       a.ld_l = !l_kin ? M * esz : l_pad ? pitch : row_bytes;
@@ -603,10 +603,9 @@ static int dot_impl(hipnx_ctx *ctx, int l_dt, int r_dt, int out_dt, int64_t batc
         a.ld_r = view->ld_r, a.bs_r = view->bs_r, a.ts_r = view->ts_r;
         a.batch_inner = (int)view->inner;
       }
-      // (the last k-row of a ragged K-outer operand is read with care, which the walk does for a partial slab only)
-      const int64_t last = over == 0 && ((l_ragged && !l_relay) || (r_ragged && !r_relay)) ? SLAB : over;
-      a.tail_l = (int)(!l_kin ? last / esz : l_pad ? (last + 15) / 16 * 16 : last);
-      a.tail_r = (int)(!r_kin ? last / esz : r_pad ? (last + 15) / 16 * 16 : last);
+      const bool ragged = (l_ragged && !l_relay) || (r_ragged && !r_relay);
+      a.tail_l = gemm_tail(row_bytes, esz, ragged, l_kin, l_pad);
+      a.tail_r = gemm_tail(row_bytes, esz, ragged, r_kin, r_pad);
       a.scale = scale_mode != HIPNX_SCALE_NONE ? (const float *)scale->ptr : nullptr;
       a.scale_mode = scale_mode;
       const int cfg = choice.cfg;

@@ -189,4 +189,12 @@ static inline bool rows_worth_copying(int64_t num_cus, const GemmChoice &c, int6
   return extra > copy;
 }
 
+// What exists of the last slab of K: bytes of each row of a K-inner operand, k of a K-outer one; 0, the slab is whole and walked as every other.
+// ragged: an operand is K-outer with k-rows that are not whole pieces.  The end of its last k-row, behind which there may be nothing, is
+// read with care, which the kernels do for a partial slab only: a whole last slab is walked as one.  copied: to rows of whole pieces.
+static inline int gemm_tail(int64_t row_bytes, int esz, bool ragged, bool k_inner, bool copied) {
+  const int64_t over = row_bytes % SLAB, last = over == 0 && ragged ? SLAB : over;
+  return (int)(!k_inner ? last / esz : copied ? (last + 15) / 16 * 16 : last);
+}
+
 }  // namespace hipnx

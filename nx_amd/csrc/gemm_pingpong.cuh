@@ -43,131 +43,6 @@ __device__ unsigned long long g_timeline[4096 * 8];
 #define HIPNX_PP_EXP 0
 #endif
 
-// Swizzle of the [row][k] LDS layout of this kernel: the 16-byte chunk index XOR the part of
-// lds_slot() that depends on the low four row bits only (the part that makes a fragment read of 16
-// consecutive rows conflict-free).  A fragment's address is then one per-lane base per K step plus
-// a compile-time multiple of 16 rows, which the LDS instruction carries as its immediate offset:
-// two address registers per operand instead of one per fragment.
-__device__ __forceinline__ int lds_slot16(int row, int chunk) {
-  return chunk ^ (((row ^ (row >> 2)) & 1) | ((((row >> 1) ^ (row >> 2)) & 1) << 1) | ((((row >> 2) ^ (row >> 3)) & 1) << 2));
-}
-
-// a pointer every lane of the wave holds the same value of, moved to scalar registers
-__device__ __forceinline__ const unsigned char *wave_uniform(const unsigned char *p) {
-  const uint64_t u = (uint64_t)p;
-  const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)u), hi = __builtin_amdgcn_readfirstlane((uint32_t)(u >> 32));
-  return (const unsigned char *)(((uint64_t)hi << 32) | lo);
-}
-
-// direct-to-LDS load with a wave-uniform 64-bit base and a 32-bit byte offset per lane
-__device__ __forceinline__ void lds_dma16_at(const unsigned char *base, unsigned off, unsigned char *lds) {
-  const unsigned dst = __builtin_amdgcn_readfirstlane((unsigned)(size_t)(lptr_t)lds);
-#pragma clang diagnostic push
-#pragma clang diagnostic ignored "-Winline-asm"
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(dst) : "memory", "m0");
-#pragma clang diagnostic pop
-}
-
-// K-inner rows [row0, row0 + ROWS) of an operand, ROWS x 128 B per slab, shared by NWAVES waves:
-// PER instructions per wave, each filling 1 KiB of LDS (8 rows x 8 chunks).  Offsets are relative
-// to the operand's first tile row (clamped into the matrix), so they fit 32 bits whenever
-// 2 * ROWS * ld does (the host checks).
-template <int ROWS, int NWAVES>
-struct PPKInnerLoader {
-  static constexpr int PER = ROWS / 8 / NWAVES;
-  const unsigned char *base;
-  unsigned off[PER];
-  __device__ __forceinline__ void init(const unsigned char *g, int64_t ld, int64_t row0, int64_t rows_valid, int wave, int lane) {
-    const int64_t first = row0 < rows_valid ? row0 : rows_valid - 1;
-    base = wave_uniform(g + first * ld);
-#pragma unroll
-    for (int i = 0; i < PER; i++) {
-      const int r = (wave + NWAVES * i) * 8 + (lane >> 3);
-      int64_t gr = row0 + r;
-      gr = gr < rows_valid ? gr : rows_valid - 1;
-      off[i] = (unsigned)((gr - first) * ld) + lds_slot16(r, lane & 7) * 16;
-    }
-  }
-  __device__ __forceinline__ void issue(int64_t kbyte0, unsigned char *lds, int wave) const {
-    const unsigned char *b = base + kbyte0;
-#pragma unroll
-    for (int i = 0; i < PER; i++) lds_dma16_at(b, off[i], lds + (wave + NWAVES * i) * 1024);
-  }
-  // a slab of which only the first `valid` bytes of each row exist; a row's last piece, where it is not whole, is zero until
-  // finish_partial writes it, behind the wave's wait for these requests
-  __device__ __forceinline__ void issue_partial(int64_t kbyte0, int valid, unsigned char *lds, int wave, int lane) const {
-    const unsigned char *b = base + kbyte0;
-#pragma unroll
-    for (int i = 0; i < PER; i++) {
-      const int r = (wave + NWAVES * i) * 8 + (lane >> 3);
-      lds_dma16(lds_slot16(r, lane & 7) * 16 + 16 <= valid ? b + off[i] : (const unsigned char *)g_zero16, lds + (wave + NWAVES * i) * 1024);
-    }
-  }
-  __device__ __forceinline__ void finish_partial(int64_t kbyte0, int valid, unsigned char *lds, int wave, int lane) const {
-    if ((valid & 15) == 0) return;
-    const unsigned char *b = base + kbyte0 + (valid & 15);
-    v4i v[PER];
-#pragma unroll
-    for (int i = 0; i < PER; i++)
-      if (lds_slot16((wave + NWAVES * i) * 8 + (lane >> 3), lane & 7) == valid >> 4) v[i] = row_end_piece(b + off[i], valid & 15);
-#pragma unroll
-    for (int i = 0; i < PER; i++)
-      if (lds_slot16((wave + NWAVES * i) * 8 + (lane >> 3), lane & 7) == valid >> 4)
-        *reinterpret_cast<v4i *>(lds + (wave + NWAVES * i) * 1024 + lane * 16) = v[i];
-  }
-};
-
-// K-outer columns [col0, col0 + ROWS) of an operand copied k-major ([k][ROWS * ES bytes]) for the
-// transposing fragment reads (tr_slot layout of gemm_mfma.cuh), with 32-bit offsets from the tile's
-// first column (clamped).
-template <int ES, int ROWS, int NWAVES>
-struct PPKOuterLoader {
-  static constexpr int RBYTES = ROWS * ES;
-  static constexpr int PER = ROWS / 8 / NWAVES;
-  static_assert(RBYTES >= 256 || ES == 1, "a 2-byte k-row must span all LDS banks");
-  const unsigned char *base;
-  unsigned off[PER];
-  int rem[PER];  // bytes of this lane's piece that lie inside its k-row, 0: all of them (KOuterDmaLoader)
-  bool whole_pieces;
-  __device__ __forceinline__ void init(const unsigned char *g, int64_t ld, int64_t col0, int64_t cols_valid, int wave, int lane) {
-    whole_pieces = (int)(cols_valid * ES) % 16 == 0;
-    const int64_t last = (cols_valid * ES - 1) & ~(int64_t)15;
-    const int64_t first = col0 * ES <= last ? col0 * ES : last;
-    base = wave_uniform(g + first);
-#pragma unroll
-    for (int i = 0; i < PER; i++) {
-      const int o = (wave + NWAVES * i) * 1024 + lane * 16;
-      const int k = o / RBYTES, slot = (o % RBYTES) / 16;
-      int64_t byte = col0 * ES + tr_slot_w<ES, RBYTES>(k, slot) * 16;
-      byte = byte <= last ? byte : last;
-      rem[i] = byte == last ? (int)(cols_valid * ES) & 15 : 0;
-      off[i] = (unsigned)((int64_t)k * ld + (byte - first));
-    }
-  }
-  __device__ __forceinline__ void issue(int64_t k0, int64_t ld, unsigned char *lds, int wave) const {
-    const unsigned char *b = base + k0 * ld;
-#pragma unroll
-    for (int i = 0; i < PER; i++) lds_dma16_at(b, off[i], lds + (wave + NWAVES * i) * 1024);
-  }
-  // a slab of which only the first `valid` k-rows exist; the last one's piece that is not whole is zero until finish_partial
-  __device__ __forceinline__ void issue_partial(int64_t k0, int64_t ld, int valid, unsigned char *lds, int wave, int lane) const {
-    const unsigned char *b = base + k0 * ld;
-#pragma unroll
-    for (int i = 0; i < PER; i++) {
-      const int k = ((wave + NWAVES * i) * 1024 + lane * 16) / RBYTES;
-      lds_dma16(k < valid - (rem[i] != 0) ? b + off[i] : (const unsigned char *)g_zero16, lds + (wave + NWAVES * i) * 1024);
-    }
-  }
-  __device__ __forceinline__ void finish_partial(int64_t k0, int64_t ld, int valid, unsigned char *lds, int wave, int lane) const {
-    if (whole_pieces) return;
-    const unsigned char *b = base + k0 * ld;
-#pragma unroll
-    for (int i = 0; i < PER; i++)
-      if (rem[i] != 0 && ((wave + NWAVES * i) * 1024 + lane * 16) / RBYTES == valid - 1)
-        *reinterpret_cast<v4i *>(lds + (wave + NWAVES * i) * 1024 + lane * 16) = row_end_piece(b + off[i] + rem[i], rem[i]);
-  }
-};
-
 // TALL = false: wave tile 64 x 128 (waves 4 x 2); TALL = true: 128 x 64 (waves 2 x 4).  Either way
 // waves 0-3 own the upper 128 rows.  A transposing fragment read moves 8 bytes per lane, a plain one
 // 16, so the operand that needs the transposing reads should be the one with fewer fragments per

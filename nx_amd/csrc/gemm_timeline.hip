@@ -9,10 +9,7 @@
 // Environment: HIPNX_TL_ZERO=1 fills the operands with zeros (the same instructions and traffic with the least
 // switching in the data paths: what the clock does to the figure); HIPNX_TL_HALF_WIDTH=1 runs 256 x 128 tiles
 // (two per compute unit at n = 4096); HIPNX_TL_TILE_128=1 runs the two-group kernel on 128 x 128 tiles (the mid-size
-// problems' kernel: one tile per compute unit at n = 2048); HIPNX_TL_GROUP_M sets the tile order's group height.  The Makefile also
-// builds hipnx_gemm_timeline_exp1 / _exp32 / _exp64 from this file with -DHIPNX_PP_EXP=1 / 32 / 64: the walk
-// without its requests, without its fragment reads, without the wait for its requests (timing only, results
-// wrong -- "sampled_outputs_wrong" says so) -- what each of the three costs the walk.
+// problems' kernel: one tile per compute unit at n = 2048); HIPNX_TL_GROUP_M sets the tile order's group height.
 //
 // bf16: left operand K-inner, right operand K-outer (the plain Nx.dot(a, b) of the headline), bf16 output;
 // s8: the same layouts, s32 output.  Operands are drawn like the benchmark's (normal / 64 cut to bf16; uniform
@@ -208,7 +205,7 @@ static int run(int n, double settle_ms, int launches) {
          "\"walk_us\": {\"min\": %.2f, \"avg\": %.2f, \"max\": %.2f}, \"epilogue_us_avg\": %.2f, \"after_last_store_us\": %.2f, "
          "\"walk_shader_clocks\": %.0f, \"walk_shader_clock_MHz\": %.0f, \"mfma_clocks_needed\": %.0f, \"mfma_share_of_walk_clocks\": %.4f, "
          "\"walk_us_avg_per_xcc\": [",
-         BM == 256 ? "gemm_pingpong_kernel" : "gemm_pingpong128_kernel", DT == HIPNX_S8 ? "s8" : "bf16", BM, BN, HIPNX_PP_EXP == 0 ? "the library's kernel" : HIPNX_PP_EXP == 1 ? "timing only: no requests after the prologue" : HIPNX_PP_EXP == 32 ? "timing only: no fragment reads after the first slab" : HIPNX_PP_EXP == 64 ? "timing only: no wait for the requests" : "timing only", getenv("HIPNX_TL_ZERO") ? "all zero" : "as the benchmark draws them", n, nb, launches, launch_us, ops / launch_us / 1e6, bad, start, start_max, walk0, walk0_max, walk1, walk1_max,
+         BM == 256 ? "gemm_pingpong_kernel" : "gemm_pingpong128_kernel", DT == HIPNX_S8 ? "s8" : "bf16", BM, BN, "the library's kernel", getenv("HIPNX_TL_ZERO") ? "all zero" : "as the benchmark draws them", n, nb, launches, launch_us, ops / launch_us / 1e6, bad, start, start_max, walk0, walk0_max, walk1, walk1_max,
          stored, stored_max, (tend - t0) * tick, dur_min, dur, dur_max, stored - walk1, launch_us - stored_max, clocks, clocks / dur,
          mfma_clocks, mfma_clocks / clocks);
   for (int x = 0; x < 8; x++) printf("%s%.2f", x ? ", " : "", xcc_n[x] ? xcc_dur[x] / xcc_n[x] : 0.0);

@@ -390,8 +390,9 @@ def test_what_lies_behind_the_end_of_k_is_not_read(ty, M, N, K, layout, hip):
                                       ("f32", 21, 13, 32), ("f32", 785, 131, 1025), ("f32", 1021, 10, 1669), ("f32", 66, 515, 992)])
 @pytest.mark.parametrize("layout", ["nn", "nt", "tn", "tt"])
 def test_rows_that_are_not_whole_pieces(ty, M, N, K, layout, hip):
-    """Integer-valued operands: the product is exact in any order.  What is not a number behind the operands, which the loads of
-    a last piece must not reach, would show in the last row and column."""
+    """Integer-valued operands: the product is exact in any order.  What is not a number behind a K-inner operand would show in its
+    last row or column if the end of a row were not cut off there; behind a K-outer one it would meet only rows and columns that are not
+    stored, whatever is read (that no load leaves either is test_dot_loads.py's)."""
     rng = np.random.default_rng(seed_of(ty, M, N, K, layout, "not whole pieces"))
     a, b = rng.integers(-4, 5, size=(M, K)), rng.integers(-4, 5, size=(K, N))
     la = a if layout[0] == "n" else np.ascontiguousarray(a.T)
