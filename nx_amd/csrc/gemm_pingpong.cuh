@@ -27,10 +27,8 @@ namespace hipnx {
 
 // Only the stand-alone timeline program (gemm_timeline.hip) defines HIPNX_GEMM_TIMELINE: the 256-row kernel then
 // leaves, per work-group, the constant-rate clock at its start, at the first phase of the walk, at the end of the
-// walk and after its last store was issued, the shader clocks the walk took, and the XCD it ran on.  The same
-// program sets HIPNX_PP_EXP for timing-only builds of the walk (their results are wrong): 1 = no requests after
-// the prologue, 32 = no fragment reads after the first slab, 64 = no wait for the requests.  The library is built
-// without either.
+// walk and after its last store was issued, the shader clocks the walk took, and the XCD it ran on.  The library is
+// built without it.
 #ifdef HIPNX_GEMM_TIMELINE
 __device__ unsigned long long g_timeline[4096 * 8];
 #define HIPNX_TL_STAMP(var) const unsigned long long var = wall_clock64()
@@ -38,9 +36,6 @@ __device__ unsigned long long g_timeline[4096 * 8];
 #else
 #define HIPNX_TL_STAMP(var)
 #define HIPNX_TL_CLOCK(var)
-#endif
-#ifndef HIPNX_PP_EXP
-#define HIPNX_PP_EXP 0
 #endif
 
 // TALL = false: wave tile 64 x 128 (waves 4 x 2); TALL = true: 128 x 64 (waves 2 x 4).  Either way
@@ -173,18 +168,11 @@ gemm_pingpong_kernel(GemmArgs a) {
 #pragma unroll
     for (int ks = 0; ks < 2; ks++) {
       // ---- memory phase: fragments of K step ks, then this phase's requests
-#if HIPNX_PP_EXP & 32
-      if (s == 0) {
-#endif
 #pragma unroll
       for (int i = 0; i < TM16; i++) fa[i] = read_l(cur, ks, i);
 #pragma unroll
       for (int j = 0; j < TN16; j++) fb[j] = read_r(cur, ks, j);
-#if HIPNX_PP_EXP & 32
-      }
-#endif
       bool issued = false, issued_r = false;
-#if !(HIPNX_PP_EXP & 1)
       if (ks == 0) {
         if (s >= 1 && s + 1 < nslab) {
           issue_r((s + 1) & 1, (int64_t)(s + 1) * SLAB + k_shift);
@@ -199,14 +187,11 @@ gemm_pingpong_kernel(GemmArgs a) {
         issue_l(s & 1, (int64_t)(s + 2) * SLAB + k_shift);
         issued = true;
       }
-#endif
       // what I requested a memory phase ago (or in the prologue) has to be in LDS before the barrier
       // that publishes it; in the very first phase nothing is due yet (slab 1 is first read in phase 4)
-#if !(HIPNX_PP_EXP & 64)
       if (issued) wait_vmcnt<4>();
       else if (issued_r) wait_vmcnt<RPER>();
       else if (!(s == 0 && ks == 0)) wait_vmcnt<0>();
-#endif
       __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): my fragments are in registers
       __builtin_amdgcn_s_barrier();
       __builtin_amdgcn_sched_barrier(0);
