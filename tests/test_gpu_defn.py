@@ -1086,6 +1086,35 @@ def spread_rows(x):               # the result reads two other statistics
     return Nx.divide(Nx.sum(Nx.subtract(x, lo), axes=[-1], keep_axes=True), hi)
 
 
+def sum_of_a_masked_product(x, y):
+    return Nx.sum(Nx.multiply(Nx.add(x, y), Nx.greater(x, 0.0)), axes=[1])
+
+
+def largest_masked_product(x, y):
+    return Nx.reduce_max(Nx.multiply(Nx.less_equal(y, 0.5), Nx.exp(x)), axes=[1], keep_axes=True)
+
+
+def masked_softmax_rows(x, y):      # one mask is made by the stages, of the row they read, the other is an operand of theirs
+    z = Nx.multiply(x, 0.125)
+    e = Nx.multiply(Nx.exp(Nx.subtract(z, Nx.reduce_max(z, axes=[-1], keep_axes=True))), Nx.greater(x, 0.0))
+    return Nx.multiply(Nx.greater(y, -1.0), Nx.divide(e, Nx.sum(e, axes=[-1], keep_axes=True)))
+
+
+# rows of whole vectors and ragged ones, one to a wave and one to a block; numbers that are not finite under the mask
+@pytest.mark.parametrize("ty", ["f32", "bf16", "f16"])
+@pytest.mark.parametrize("shape", [(64, 256), (9, 185), (1, 7), (5, 8200), (2049, 40)])
+@pytest.mark.parametrize("name", ["sum_of_a_masked_product", "largest_masked_product", "masked_softmax_rows"])
+def test_values_times_a_mask_feed_reductions_and_row_stages(name, shape, ty, hip):
+    fun = globals()[name]
+    rng = np.random.default_rng(seed_of(name, shape, ty, "mask"))
+    for make in (rand_float, not_finite):
+        args = (make(rng, ty, shape, hip), make(rng, ty, shape, hip))
+        planned = defn.compile(fun, *args, fuse="compiled")
+        group = planned.roots[0].data.args[0]
+        assert any(i["dt"] == ("u", 8) for i in group.program) and (type(group).__name__ == "_RowCluster" or group.reduce is not None)
+        assert_bits_equal(planned(*args), defn.compile(fun, *args)(*args), f"{name} {shape} {ty}")
+
+
 @pytest.mark.parametrize("ty", ["f32", "bf16"])
 @pytest.mark.parametrize("shape", [(32, 512, 512), (100, 64), (7, 4096), (3, 5, 8), (1, 1024), (2049, 40)])
 @pytest.mark.parametrize("name", ["log_sum_exp_rows", "mean_rows", "root_mean_square_rows", "spread_rows"])

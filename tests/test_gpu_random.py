@@ -152,6 +152,18 @@ def test_a_sample_and_the_next_key_of_one_split(count, order, hip):
         return (sample, after, Nx.squeeze(Nx.slice(keys, [1, 0], [1, 2]), axes=[0])) if order == "both keys" else (sample, after)
     key = Random.key(2024 + count, backend=hip)
     planned = defn.compile(program, key, fuse="compiled")
+    group = next(r.data.args[0] for r in planned.roots if r.data.op == "fused")
+    assert group.words is not None and group.beside is not None
     want = [Nx.to_binary(t) for t in program(key)]
+    beside, keys = [], []
+    fused, random_key = hip.fused_elementwise.__func__, hip.random_key.__func__
+    hip.fused_elementwise = classmethod(lambda cls, *a, **k: (beside.append(k.get("beside") is not None), fused(cls, *a, **k))[1])
+    hip.random_key = classmethod(lambda cls, *a: (keys.append(a[3]), random_key(cls, *a))[1])
+    try:
+        assert [Nx.to_binary(t) for t in planned._walk([key])] == want
+    finally:
+        hip.fused_elementwise, hip.random_key = classmethod(fused), classmethod(random_key)
+    # a key that is there before the sample is not made again; one that is the sample's own is never beside it
+    assert beside == [order != "key first"] and keys == {"key first": [0], "both keys": [1]}.get(order, [])
     for _ in range(5):  # (evaluated, recorded, issued from the recording)
         assert [Nx.to_binary(t) for t in planned(key)] == want
