@@ -252,8 +252,9 @@ int hipnx_argreduce(hipnx_ctx *ctx, int op, int tie, int in_dt, int out_dt, int6
  * A handful of outputs over a long K -- the dot of two vectors -- are such segments of interleaved sums for every type).
  * out_dt may be HIPNX_BF16_RNE (bf16 rounded to nearest even).  Any batch count is taken (beyond 65535 items in
  * several launches).  The call may take workspace from the context's pool and return it before it ends: a re-laid
- * operand whose K-outer rows are not whole 16-byte blocks, a K-inner operand copied to rows of whole 16-byte pieces
- * where its own are not, the partial results of a contraction whose K is split over several work-groups per tile or output. */
+ * K-outer operand whose k-rows are shorter than 16 bytes (f64: no whole number of them), a K-inner operand copied to rows of whole 16-byte
+ * pieces where its own are shorter than one or, for speed, on no dword and re-read by many tiles, the partial results of a contraction whose
+ * K is split over several work-groups per tile or output.  What is for speed alone is left out where there is no room for it. */
 int hipnx_dot(hipnx_ctx *ctx, int l_dt, int r_dt, int out_dt, int64_t batch, int64_t M, int64_t N,
               int64_t K, int l_layout, int r_layout, const hipnx_buf *l, const hipnx_buf *r,
               hipnx_buf *out);
@@ -282,8 +283,8 @@ int hipnx_dot_scaled(hipnx_ctx *ctx, int l_dt, int r_dt, int64_t batch, int64_t 
                      int l_layout, int r_layout, const hipnx_buf *l, const hipnx_buf *r, int scale_mode,
                      const hipnx_buf *scale, hipnx_buf *out);
 
-/* The same for a K that need not be whole slabs: the partial slab is walked in place, rows that are not whole 16-byte pieces are
- * copied first, as hipnx_dot does (from 16 M multiply-adds on; HIPNX_EUNSUPPORTED below). */
+/* The same for a K that need not be whole slabs: the partial slab is walked in place.  Rows that are not whole 16-byte pieces are
+ * taken as hipnx_dot takes them, from 16 M multiply-adds on (HIPNX_EUNSUPPORTED below). */
 int hipnx_dot_scaled_any_k(hipnx_ctx *ctx, int l_dt, int r_dt, int64_t batch, int64_t M, int64_t N, int64_t K,
                            int l_layout, int r_layout, const hipnx_buf *l, const hipnx_buf *r, int scale_mode,
                            const hipnx_buf *scale, hipnx_buf *out);
