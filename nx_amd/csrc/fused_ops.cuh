@@ -44,14 +44,15 @@ struct FusedArgs {
   const void *l, *r;
   int64_t l_outer, l_inner, l_ld, r_outer, r_inner, r_ld;
   int key_parts, key_index;  // the key is number key_index of the key_parts that in[words] splits into (0 parts: in[words] itself)
-  int unused;
+  int beside_index;          // which of the key's parts goes to `beside` (FusedWordsArgs), where that is not null
 };
-// What only the kernels over random words take, behind the block that every kernel does (with these two in it
-// the attention probabilities of 4 x 8 x 512 x 512 took 19.6 us a pass, 19.4 without).
+// What only the kernels over random words take, behind the block that every kernel does (with it in that block
+// the attention probabilities of 4 x 8 x 512 x 512 took 19.6 us a pass, 19.4 without).  It lies in the last of the block's 64-byte lines:
+// in one more, 63711 normal samples took 6.56 us, 6.39 so.
 struct FusedWordsArgs : FusedArgs {
-  int beside_index;  // which of the key's parts goes to `beside`, where that is not null
   uint32_t *beside;
 };
+static_assert(sizeof(FusedArgs) / 64 == (sizeof(FusedWordsArgs) - 1) / 64, "no line of its own");
 
 // The argument block is read where the launch put it (the kernel-argument segment, constant address
 // space) with wave-uniform indices: indexing the by-value copy would move it to per-lane scratch.
